@@ -396,6 +396,15 @@ QWIX_API int qwix_hip_gemv_wq_zp(const void* x, int64_t ldx, const void* q, int6
                         int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
                         const int8_t* zp, void* out, int out_dtype, int64_t ldo, void* stream);
 
+/* Weight-only product with the rows in groups, one weight per group (ragged_dot.py:229-241 without the dequantized copy,
+ * for a few rows per group): rows of x form G consecutive groups of group_sizes[g] rows (device memory, never read on the
+ * host; sizes are clamped to the M rows), group g meets the weight at q + g * q_group_bytes with the scales at
+ * s + g * s_group_stride elements.  Rows behind the last group come out as zeros.  Otherwise as qwix_hip_gemv_wq. */
+QWIX_API int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes,
+                        int b_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
+                        int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out, int out_dtype,
+                        int64_t ldo, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * Walsh-Hadamard rotation along the last axis (qwix/contrib/hadamard_rot.py:35-117):
  *     y[r, :] = ((x[r, :] * pre_sign) H_n) * post_sign * out_scale

@@ -280,21 +280,19 @@ __device__ __forceinline__ void consume_panel(const LaneOff<NT>& a, Block<QWIX_I
 }
 
 // NWAVE wavefronts per workgroup, each owning a slice of K; NT tiles of 16 output columns, RT tiles of 16 rows
-// (the weights are read, and widened, once per workgroup whatever RT is).
-template <int BQT, int NWAVE, int NT, bool SBF, int RT = 1, bool ZP = false>
-__global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
-  extern __shared__ float red_raw[];
+// (the weights are read, and widened, once per workgroup whatever RT is).  Rows row0 .. row_end - 1 of x and out
+// (at most 16 RT of them), columns from n_base on.
+template <int BQT, int NWAVE, int NT, bool SBF, int RT, bool ZP>
+__device__ __forceinline__ void gemv_wq_tile(const GemvArgs& p, int n_base, int row0, int row_end, float* red_raw) {
   float (*red)[RT * NT][4][64] = reinterpret_cast<float (*)[RT * NT][4][64]>(red_raw);  // [NWAVE]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, kq = lane >> 4;
-  const int n_base = blockIdx.x * (16 * NT);
   const int nblk = p.K / 128;
   // K is dealt out in pairs of blocks, so that a wavefront's slice starts on an even block
   const int per_wave = 2 * ((nblk + 2 * NWAVE - 1) / (2 * NWAVE));
   const int kb0 = min(nblk, wave * per_wave), kb1 = min(nblk, kb0 + per_wave);
 
-  const int row0 = blockIdx.y * (16 * RT);
   LaneOff<NT> a;
   a.bw = p.q + static_cast<int64_t>(n_base) * p.ldb;
   a.panel = reinterpret_cast<uint8_t*>(red_raw) + wave * (NT * 2048);
@@ -315,7 +313,7 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
 
   bool xrow[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) xrow[rt] = row0 + rt * 16 + col < p.M;
+  for (int rt = 0; rt < RT; ++rt) xrow[rt] = row0 + rt * 16 + col < row_end;
   a.x = static_cast<unsigned>(col) * static_cast<unsigned>(p.ldx) * 2u + kq * 64u;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -370,12 +368,12 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
   }
 
   if constexpr (BQT == QWIX_INT4) __syncthreads();  // the partial sums take the place of the weight panels
-  // result lane layout: column n = lane % 16, row m = 4 * (lane / 16) + r; rows past M are neither written nor summed
+  // result lane layout: column n = lane % 16, row m = 4 * (lane / 16) + r; rows past the last are neither written nor summed
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (row0 + rt * 16 + 4 * kq + r < p.M) {
+      if (row0 + rt * 16 + 4 * kq + r < row_end) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) red[wave][rt * NT + t][r][lane] = outacc[rt][t][r];
       }
@@ -384,7 +382,7 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
     const int t2 = idx >> 8, r = (idx >> 6) & 3, l = idx & 63;
     const int rt = t2 / NT, t = t2 % NT;
     const int mo = row0 + rt * 16 + 4 * (l >> 4) + r, n = n_base + t * 16 + (l & 15);
-    if (mo < p.M && n < p.N) {
+    if (mo < row_end && n < p.N) {
       float v = 0.f;
 #pragma unroll
       for (int w = 0; w < NWAVE; ++w) v += red[w][t2][r][l];
@@ -396,14 +394,59 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
   }
 }
 
+template <int BQT, int NWAVE, int NT, bool SBF, int RT = 1, bool ZP = false>
+__global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
+  extern __shared__ float red_raw[];
+  gemv_wq_tile<BQT, NWAVE, NT, SBF, RT, ZP>(p, blockIdx.x * (16 * NT), blockIdx.y * (16 * RT), p.M, red_raw);
+}
+
+// Rows in groups (mixture of experts): blockIdx.y is the group, whose rows every wavefront finds for itself from the group
+// sizes in device memory; the workgroup streams that group's weight columns once per 16 RT rows.  blockIdx.y == G clears
+// the rows that belong to no group.
+struct GemvGroups {
+  const int32_t* sizes;
+  int G;
+  int64_t q_stride, s_stride;  // bytes of weights, elements of scales between consecutive groups
+};
+
+template <int BQT, int NWAVE, int NT, bool SBF, int RT>
+__global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, GemvGroups gr) {
+  extern __shared__ float red_raw[];
+  const int g = blockIdx.y, lane = threadIdx.x & 63;
+  const int n_base = blockIdx.x * (16 * NT);
+  long long before = 0;
+  for (int i = lane; i < g; i += 64) before += max(gr.sizes[i], 0);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
+  // sizes are clamped so that no group reaches past row M
+  const int start = __builtin_amdgcn_readfirstlane(static_cast<int>(min(before, static_cast<long long>(p.M))));
+  if (g == gr.G) {
+    const int cols = min(16 * NT, p.N - n_base);
+    for (int idx = threadIdx.x; idx < (p.M - start) * cols; idx += NWAVE * 64) {
+      const int64_t at = static_cast<int64_t>(start + idx / cols) * p.ldo + n_base + idx % cols;
+      if (p.out_dtype == QWIX_BF16) reinterpret_cast<uint16_t*>(p.out)[at] = 0;
+      else reinterpret_cast<uint32_t*>(p.out)[at] = 0;
+    }
+    return;
+  }
+  const int size = min(max(gr.sizes[g], 0), p.M - start);
+  p.q += g * gr.q_stride;
+  p.s = static_cast<const char*>(p.s) + g * gr.s_stride * (SBF ? 2 : 4);
+  for (int row = 0; row < size; row += 16 * RT) {  // the trip count is the same for the whole workgroup
+    if (row > 0) __syncthreads();  // the partial sums in LDS are read to the end before the next pass writes there
+    gemv_wq_tile<BQT, NWAVE, NT, SBF, RT, false>(p, n_base, start + row, start + size, red_raw);
+  }
+}
+
 }  // namespace
 }  // namespace qwix
 
 using namespace qwix;
 
-static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int b_qtype, int64_t M, int64_t N,
+// Checks the operands and fills the kernel's arguments.
+static int gemv_wq_args(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int b_qtype, int64_t M, int64_t N,
                         int64_t K, int64_t group, const void* s, int s_dtype, const int8_t* zp, void* out, int out_dtype,
-                        int64_t ldo, void* stream) {
+                        int64_t ldo, GemvArgs* args) {
   if (!x || !q || !s || !out) return fail(QWIX_ERR_INVALID_ARGUMENT, "null argument");
   if (M <= 0 || N <= 0 || K <= 0 || N > INT32_MAX || K > INT32_MAX || M > 65535 * 16)
     return fail(QWIX_ERR_INVALID_ARGUMENT, "bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
@@ -422,7 +465,7 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
   const int64_t es = s_dtype == QWIX_BF16 ? 2 : 4;
   if (32 * ldx * 2 + K * 2 > INT32_MAX || 64 * ldb_bytes + brow > INT32_MAX || (K / group) * N * es > INT32_MAX)
     return fail(QWIX_ERR_UNSUPPORTED, "row strides too large for 32-bit lane offsets");
-  GemvArgs p;
+  GemvArgs& p = *args;
   p.x = static_cast<const uint16_t*>(x); p.ldx = ldx;
   p.q = static_cast<const uint8_t*>(q); p.ldb = ldb_bytes;
   p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
@@ -431,6 +474,15 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
   p.s = s; p.s_dtype = s_dtype;
   p.zp = zp;
   p.out = out; p.out_dtype = out_dtype; p.ldo = ldo;
+  return QWIX_OK;
+}
+
+static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int b_qtype, int64_t M, int64_t N,
+                        int64_t K, int64_t group, const void* s, int s_dtype, const int8_t* zp, void* out, int out_dtype,
+                        int64_t ldo, void* stream) {
+  GemvArgs p;
+  if (const int rc = gemv_wq_args(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, zp, out, out_dtype, ldo, &p))
+    return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Byte weights of 32 MB and more stream faster through the smallest workgroups (4 wavefronts, two row tiles, several
   // workgroups per CU) whatever the rows, even when the second row tile is empty: K 4096, N 14336, int8, 1 / 16 / 32
@@ -499,4 +551,57 @@ extern "C" int qwix_hip_gemv_wq_zp(const void* x, int64_t ldx, const void* q, in
                                    void* out, int out_dtype, int64_t ldo, void* stream) {
   if (!zp) return fail(QWIX_ERR_INVALID_ARGUMENT, "null zero points");
   return gemv_wq_impl(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, zp, out, out_dtype, ldo, stream);
+}
+
+extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes,
+                                       int b_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
+                                       int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out,
+                                       int out_dtype, int64_t ldo, void* stream) {
+  GemvArgs p;
+  if (const int rc = gemv_wq_args(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, nullptr, out, out_dtype, ldo, &p))
+    return rc;
+  if (!group_sizes || G <= 0 || G >= 65535)
+    return fail(QWIX_ERR_INVALID_ARGUMENT, "1..65534 group sizes are needed (G=%lld)", (long long)G);
+  if (q_group_bytes % 16 || q_group_bytes < 0 || s_group_stride < 0)
+    return fail(QWIX_ERR_INVALID_ARGUMENT, "bad group strides (weights: %lld bytes, scales: %lld elements)",
+                (long long)q_group_bytes, (long long)s_group_stride);
+  const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define QWIX_GEMVG_KERNEL(BQT, SBFF, NW, NTT, RTT)                                                         \
+  do {                                                                                                     \
+    constexpr size_t smem = NW * NTT * (RTT * 1024 > 2048 ? RTT * 1024 : 2048);                            \
+    gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT><<<dim3(static_cast<unsigned>((N + 16 * NTT - 1) / (16 * NTT)),  \
+                                                      static_cast<unsigned>(G + 1)), NW * 64, smem, st>>>(p, gr);   \
+  } while (0)
+#define QWIX_GEMVG_LAUNCH(NW, NTT, RTT)                                                                    \
+  do {                                                                                                     \
+    const bool sbf = s_dtype == QWIX_BF16;                                                                 \
+    if (b_qtype == QWIX_INT4 && sbf) QWIX_GEMVG_KERNEL(QWIX_INT4, true, NW, NTT, RTT);                     \
+    else if (b_qtype == QWIX_INT4) QWIX_GEMVG_KERNEL(QWIX_INT4, false, NW, NTT, RTT);                      \
+    else if (b_qtype == QWIX_E4M3 && sbf) QWIX_GEMVG_KERNEL(QWIX_E4M3, true, NW, NTT, RTT);                \
+    else if (b_qtype == QWIX_E4M3) QWIX_GEMVG_KERNEL(QWIX_E4M3, false, NW, NTT, RTT);                      \
+    else if (sbf) QWIX_GEMVG_KERNEL(QWIX_INT8, true, NW, NTT, RTT);                                        \
+    else QWIX_GEMVG_KERNEL(QWIX_INT8, false, NW, NTT, RTT);                                                \
+  } while (0)
+  // Many workgroups (several rounds of them) cover each other's latency, and few wavefronts in each leave the fewest partial
+  // sums to add; few workgroups need their wavefronts to keep the loads in flight.  Weights from HBM, int4 / int8 in us:
+  //   64 groups x 4 rows, K 2048, N 4096 (4096 workgroups of 64 columns): 2 wavefronts x 64 columns 53.7 / 97.7 (5.2 and
+  //     5.6 TB/s), 4 x 64 63.7 / 96.5, 8 x 32 80.3 / 119.7, 4 x 16 90.6 / 128.4
+  //   8 groups x 2 rows, K 2048, N 3072 (384): 4 x 64 8.3, 8 x 32 9.2, 2 x 64 11.6
+  //   8 groups x 2 rows, K 4096, N 1024 (128): 8 x 32 6.6 / 9.9, 4 x 64 10.4 / 15.8, 2 x 64 15.8 / 20.4
+  // Two row tiles pay for themselves where groups of more than 16 rows are common (64 groups of 8 / 12 / 16 / 30 rows on
+  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4); bytes take them always (64 x 4
+  // rows 96.5 against 97.5, 64 x 16 rows 157 against 119).
+  const int64_t wgs = G * ((N + 63) / 64);
+  const bool two = M > 10 * G;
+  if (wgs < 320) {
+    if (two) QWIX_GEMVG_LAUNCH(8, 2, 2); else QWIX_GEMVG_LAUNCH(8, 2, 1);
+  } else if (b_qtype == QWIX_INT4 && wgs >= 1024) {
+    if (two) QWIX_GEMVG_LAUNCH(2, 4, 2); else QWIX_GEMVG_LAUNCH(2, 4, 1);
+  } else {
+    if (two || b_qtype != QWIX_INT4) QWIX_GEMVG_LAUNCH(4, 4, 2); else QWIX_GEMVG_LAUNCH(4, 4, 1);
+  }
+#undef QWIX_GEMVG_LAUNCH
+#undef QWIX_GEMVG_KERNEL
+  return check_launch("gemv_wq (groups)");
 }

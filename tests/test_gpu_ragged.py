@@ -185,6 +185,36 @@ def test_ragged_dot_weight_only_experts(sizes, wq_type, tiled):
   assert np.all(got[min(sum(sizes), M):] == 0)
 
 
+@pytest.mark.parametrize('G,K,N,M,sizes', [
+    (4, 128, 200, 40, (0, 17, 16, 1)),           # few workgroups (8 wavefronts), one K block, rows left over
+    (4, 384, 72, 100, (33, 0, 70, 50)),          # two row tiles, an odd number of K blocks, sizes past the last row
+    (8, 256, 2568, 60, (1, 15, 0, 16, 3, 17, 2, 0)),   # 4 wavefronts x 64 columns, a column tile that ends early
+    (64, 256, 1000, 128, tuple(i % 4 for i in range(64))),        # several rounds: 2 wavefronts x 64 columns
+    (64, 384, 1000, 1100, tuple((7 * i) % 35 for i in range(64))),  # the same with two row tiles, several passes
+])
+@pytest.mark.parametrize('wq_type,tiled,dtype', [('int4', {1: 128}, O.BF16), ('int8', {1: 128}, O.BF16), ('int8', None, O.F32),
+                                                 ('float8_e4m3fn', {1: 128}, O.BF16), ('int4', None, O.F32)])
+def test_ragged_dot_weight_only_one_launch(G, K, N, M, sizes, wq_type, tiled, dtype):
+  """A few rows per group against weight-only experts in one launch, at the edges of its row tiles, column tiles and K
+  blocks.  The kernel keeps weight x scale in f32, so a bf16 result is off by its own rounding (half a step, 2^-8 of the
+  magnitude between powers of two) plus the f32 sums (below 1e-5 of the largest)."""
+  import qwix_amd
+  x_np, x_t = util.make((M, K), O.BF16, seed=81)
+  wq, owq = _quantized((G, K, N), dtype, 82, _how(wq_type, (0, 2), tiled), scale=0.05)
+  assert qwix_amd.core.ragged_dot._weight_only_groups(x_t, wq, _sizes(sizes), torch.float32) is not None
+  out = qwix_amd.ragged_dot(x_t, wq, _sizes(sizes), preferred_element_type=torch.float32)
+  q = O.qvalue_as_f32(owq).astype(np.float64) * np.repeat(owq.scale.v.astype(np.float64), K // owq.scale.v.shape[1], axis=1)
+  want, start = np.zeros((M, N)), 0
+  for g, size in enumerate(sizes):
+    stop = min(start + size, M)
+    want[start:stop] = x_np[start:stop].astype(np.float64) @ q[g]
+    start = stop
+  np.testing.assert_allclose(util.f32np(out), want, rtol=0, atol=1e-5 * np.abs(want).max())
+  low = qwix_amd.ragged_dot(x_t, wq, _sizes(sizes), preferred_element_type=torch.bfloat16)
+  np.testing.assert_allclose(util.f32np(low), want, rtol=2.0 ** -8, atol=2e-5 * np.abs(want).max())
+  assert np.all(util.f32np(out)[min(sum(sizes), M):] == 0)
+
+
 def test_ragged_dot_dequantize_first_path():
   """A raw float lhs or a zero point sends the call to the dequantize-first path (ragged_dot.py:278-292)."""
   import qwix_amd
