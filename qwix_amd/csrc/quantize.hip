@@ -329,16 +329,20 @@ struct ColGeom {
   int chunks_per_tile, col_blocks;
 };
 
+// The grid has at most 2^31 - 1 blocks, so the indices come apart with 32-bit divisions (the 64-bit ones of the first
+// version stood in front of a block's first load with some 200 scalar instructions).
 template <typename D>
-__device__ __forceinline__ void col_decode(const ColGeom& gm, int64_t b, int64_t* o, int64_t* t,
+__device__ __forceinline__ void col_decode(const ColGeom& gm, unsigned b, int64_t* o, int64_t* t,
                                            int* chunk, int64_t* c0) {
-  const int64_t cb = b % gm.col_blocks;
-  b /= gm.col_blocks;
-  *chunk = static_cast<int>(b % gm.chunks_per_tile);
-  b /= gm.chunks_per_tile;
-  *t = b % gm.ntiles;
-  *o = b / gm.ntiles;
-  *c0 = (cb * 16 + (threadIdx.x & 15)) * D::kVec;
+  const unsigned cbs = static_cast<unsigned>(gm.col_blocks), cpt = static_cast<unsigned>(gm.chunks_per_tile);
+  const unsigned nt = static_cast<unsigned>(gm.ntiles);
+  const unsigned cb = b % cbs;
+  b /= cbs;
+  *chunk = static_cast<int>(b % cpt);
+  b /= cpt;
+  *t = b % nt;
+  *o = b / nt;
+  *c0 = (static_cast<int64_t>(cb) * 16 + (threadIdx.x & 15)) * D::kVec;
 }
 
 template <typename D, int CAL>
@@ -402,7 +406,7 @@ __global__ void __launch_bounds__(256)
       atomicMax(ws + wbase + e, __float_as_uint(a));  // a >= 0: bit patterns order like values
       if constexpr (ASYM) {
         float b = fminf(fminf(red[1][0][tc][e], red[1][1][tc][e]), fminf(red[1][2][tc][e], red[1][3][tc][e]));
-        atomicMax(ws + plane + wbase + e, __float_as_uint(-b));
+        atomicMax(ws + plane + wbase + e, __float_as_uint(0.f - b));  // +0, not -0, for a block without negative values
       }
     }
   }
@@ -410,7 +414,8 @@ __global__ void __launch_bounds__(256)
 
 // The same reduction for tall scale groups (tile >= 256 rows): a workgroup covers 256 rows x 64 vectors of
 // columns, each wavefront reading whole 1 KiB row pieces, and issues one atomic per column for 256 rows
-// instead of one for 128.
+// instead of one for 128.  Bound by reading (8192 x 28672 bf16: 83 us, 5.7 TB/s; with eight loads in flight per thread,
+// each behind its own predicate, 114 us).
 constexpr int kWideRows = 256;
 template <typename D, int CAL>
 __global__ void __launch_bounds__(256)
@@ -420,12 +425,12 @@ __global__ void __launch_bounds__(256)
   constexpr bool ASYM = (CAL == QWIX_MINMAX);
   constexpr bool PACKED = !ASYM && D::kTag == QWIX_BF16;  // |x| of a bf16 pair orders like its low 15 bits
   __shared__ float red[ASYM ? 2 : 1][4][EV][64];
-  int64_t b = blockIdx.x;
-  const int64_t cb = b % wide_col_blocks;
-  b /= wide_col_blocks;
-  const int chunk = static_cast<int>(b % wide_chunks);
-  b /= wide_chunks;
-  const int64_t t = b % gm.ntiles, o = b / gm.ntiles;
+  unsigned b = blockIdx.x;
+  const int64_t cb = b % static_cast<unsigned>(wide_col_blocks);
+  b /= static_cast<unsigned>(wide_col_blocks);
+  const int chunk = static_cast<int>(b % static_cast<unsigned>(wide_chunks));
+  b /= static_cast<unsigned>(wide_chunks);
+  const int64_t t = b % static_cast<unsigned>(gm.ntiles), o = b / static_cast<unsigned>(gm.ntiles);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t c0 = (cb * 64 + lane) * EV;
   const bool col_ok = c0 < gm.inner;
@@ -437,15 +442,23 @@ __global__ void __launch_bounds__(256)
   for (int e = 0; e < EV; ++e) mx[e] = mn[e] = 0.f;
   const uint8_t* xp = x + ((o * gm.reduce + row0) * gm.inner + c0) * sizeof(typename D::storage);
   const int64_t step = 4 * gm.inner * sizeof(typename D::storage);
-  for (int it = 0; it < kWideRows / 32; ++it) {
-    uint4 raw[8];
+  // sixteen loads in flight per thread; blocks that lie inside the array (all but the last ones) load without predicates
+  constexpr int NB = 16;
+  const bool full = t * gm.tile + (static_cast<int64_t>(chunk) + 1) * kWideRows <= row_end && (cb + 1) * 64 * EV <= gm.inner;
+  for (int it = 0; it < kWideRows / (4 * NB); ++it) {
+    uint4 raw[NB];
+    if (full) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      raw[j] = make_uint4(0, 0, 0, 0);
-      if (col_ok && row0 + 4 * (it * 8 + j) < row_end) raw[j] = *reinterpret_cast<const uint4*>(xp + (it * 8 + j) * step);
+      for (int j = 0; j < NB; ++j) raw[j] = *reinterpret_cast<const uint4*>(xp + (it * NB + j) * step);
+    } else {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        raw[j] = make_uint4(0, 0, 0, 0);
+        if (col_ok && row0 + 4 * (it * NB + j) < row_end) raw[j] = *reinterpret_cast<const uint4*>(xp + (it * NB + j) * step);
+      }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < NB; ++j) {
       if constexpr (PACKED) {
         const uint32_t wd[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
@@ -489,7 +502,7 @@ __global__ void __launch_bounds__(256)
     atomicMax(ws + wbase + c, __float_as_uint(a));  // a >= 0: bit patterns order like values
     if constexpr (ASYM) {
       const float m = fminf(fminf(red[1][0][e][l], red[1][1][e][l]), fminf(red[1][2][e][l], red[1][3][e][l]));
-      atomicMax(ws + plane + wbase + c, __float_as_uint(-m));
+      atomicMax(ws + plane + wbase + c, __float_as_uint(0.f - m));  // +0, not -0, for a block without negative values
     }
   }
 }
@@ -559,162 +572,268 @@ __global__ void cols_finish_cal_kernel(const uint32_t* __restrict__ ws, int64_t 
   }
 }
 
+// One column's eight rows as packed codes (two words, int4: one).  SAFE: the scale was given, not derived from these rows.
+// A quotient carries the sign of its dividend, zero quotients included (the product with the positive reciprocal does).
+// clip (e4m3 from bf16): quotients by a scale that absmax gave stay inside e4m3's range once rounded to bf16 -- |x| / s is at
+// most 448 (1 + 2^-8), which rounds to 448 -- but a calibration factor below one lets them leave it.
+template <typename D, int QT, bool SAFE, bool ASYM>
+__device__ __forceinline__ void quantize_column(const float (&x)[8], float s, float zf, bool clip, uint32_t (&w)[2]) {
+  const Divider<D, SAFE, false> div(s);
+  if constexpr (QT == QWIX_E4M3 && D::kTag == QWIX_BF16 && !SAFE) {
+    // two bf16 quotients to two e4m3 codes in one instruction
+    typedef short s16x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    uint32_t p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = pack_bf16x2(div.raw(x[2 * j]), div.raw(x[2 * j + 1]));
+    if (clip) {  // wave-uniform; 0x43E0 is bf16 448
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        p[j] = (p[j] & 0x80008000u) | __builtin_bit_cast(uint32_t, __builtin_elementwise_min(
+                                          __builtin_bit_cast(u16x2, p[j] & 0x7FFF7FFFu), u16x2{0x43E0, 0x43E0}));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s16x2 r = {0, 0};
+      r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2_t, p[2 * h]), 1.f, false);
+      r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2_t, p[2 * h + 1]), 1.f, true);
+      w[h] = __builtin_bit_cast(uint32_t, r);
+    }
+    return;
+  }
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    v[j] = x[j];
+    v[j + 1] = x[j + 1];
+    div.pair_unsigned(v[j], v[j + 1]);
+    if constexpr (ASYM) {
+      v[j] += zf;
+      v[j + 1] += zf;
+      if constexpr (D::kTag == QWIX_BF16) round_bf16_pair(v[j], v[j + 1]);
+    }
+  }
+  if constexpr (QT == QWIX_INT8) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[h] = pack4_low_bytes(rne_bits_clamped(v[4 * h], -128.f, 127.f), rne_bits_clamped(v[4 * h + 1], -128.f, 127.f),
+                             rne_bits_clamped(v[4 * h + 2], -128.f, 127.f), rne_bits_clamped(v[4 * h + 3], -128.f, 127.f));
+  } else if constexpr (QT == QWIX_E4M3) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (SAFE)  // a given scale: NaN inputs stay NaN
+        w[h] = to_e4m3x2(v[4 * h], v[4 * h + 1]) | (to_e4m3x2(v[4 * h + 2], v[4 * h + 3]) << 16);
+      else
+        w[h] = to_e4m3x2_bounded(v[4 * h], v[4 * h + 1]) | (to_e4m3x2_bounded(v[4 * h + 2], v[4 * h + 3]) << 16);
+    }
+  } else {
+    w[0] = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[0] |= (rne_bits_clamped(v[j], -8.f, 7.f) & 0xFu) << (4 * j);
+  }
+}
+
 // Pass 2.  SRC 0: scale from ws (written out by chunk 0); SRC 1: scale given; SRC 2: the whole
 // scale group (at most 128 rows) lies inside this block, which then calibrates on its own registers:
 // one read of the input, no workspace, no atomics.
+//   What bounds it: memory, with the vector ALU close behind (91 us of 174 at 8192 x 28672 to e4m3 when a thread worked out
+// the scales of its eight columns itself and every element went through f32).  Each column's scale is worked out once
+// per block and shared through LDS, the input stays packed until a column is quantized (half the registers, twice the
+// wavefronts per CU), and bf16 quotients become e4m3 codes in pairs.
 template <typename D, int QT, int CAL, int LAYOUT, int SRC>
 __global__ void __launch_bounds__(256)
     cols_quantize_kernel(const uint8_t* __restrict__ x, ColGeom gm, const uint32_t* __restrict__ ws,
                          float factor, uint8_t* __restrict__ q, void* __restrict__ scale,
                          int8_t* __restrict__ zp) {
-  constexpr int EV = D::kVec;
+  constexpr int EV = D::kVec, NC = 16 * EV;  // columns per thread, per block
   constexpr bool ASYM = (CAL == QWIX_MINMAX);
-  __shared__ float red[SRC == 2 ? 2 : 1][SRC == 2 ? 4 : 1][SRC == 2 ? 16 : 1][EV];
+  __shared__ float red[SRC == 2 ? (ASYM ? 2 : 1) : 1][SRC == 2 ? 4 : 1][SRC == 2 ? NC : 1];
+  __shared__ __attribute__((aligned(16))) float sh_s[NC];
+  __shared__ __attribute__((aligned(16))) float sh_z[ASYM ? NC : 4];
   int64_t o, t, c0;
   int chunk;
   // After a calibration pass over the same array the blocks run in the opposite order: what that pass read
   // last is what the last-level cache still holds, so it is re-read first.
   col_decode<D>(gm, SRC == 0 ? gridDim.x - 1 - blockIdx.x : blockIdx.x, &o, &t, &chunk, &c0);
+  const int tid = threadIdx.x, tc = tid & 15, rb = tid >> 4;
   const bool col_ok = c0 < gm.inner;  // idle threads stay for the barriers
-  const int rb = threadIdx.x >> 4;
-  const int64_t sidx = (o * gm.ntiles + t) * gm.inner + c0;
+  const int64_t cb0 = c0 - tc * EV;   // first column of the block
   const int64_t row_end = (t + 1) * gm.tile;
-  const int64_t r0 = t * gm.tile + chunk * 128 + rb * 8;
-  float v[8][EV];
-  uint4 raw[8];
-  // The loads are issued before the scales are fetched, so that the two round trips overlap.
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    raw[j] = make_uint4(0, 0, 0, 0);
-    if (col_ok && r0 + j < row_end)
-      raw[j] = *reinterpret_cast<const uint4*>(x + ((o * gm.reduce + r0 + j) * gm.inner + c0) * sizeof(typename D::storage));
+  const int64_t row0 = t * gm.tile + chunk * 128, r0 = row0 + rb * 8;
+  const int64_t sidx = (o * gm.ntiles + t) * gm.inner + cb0 + tid;  // thread tid looks after column tid of the block
+  const bool owner = tid < NC && cb0 + tid < gm.inner;
+  uint32_t pre0 = 0, pre1 = 0;
+  if constexpr (SRC == 0) {  // in flight before the rows, so that the scales are ready when those arrive
+    if (owner) {
+      pre0 = ws[sidx];
+      if constexpr (ASYM) pre1 = ws[gm.outer * gm.ntiles * gm.inner + sidx];
+    }
   }
-  auto load_rows = [&]() {
+  uint4 raw[8];
+  {
+    const uint8_t* xp = x + ((o * gm.reduce + r0) * gm.inner + c0) * sizeof(typename D::storage);
+    const int64_t pitch = gm.inner * static_cast<int64_t>(sizeof(typename D::storage));
+    if (row0 + 128 <= row_end && cb0 + NC <= gm.inner) {  // all but the last blocks
 #pragma unroll
-    for (int j = 0; j < 8; ++j) unpack16<D>(raw[j], v[j]);
-  };
-  float s[EV];
-  int z[EV];
-  if constexpr (SRC == 2) {
-    load_rows();
-    float mx[EV], mn[EV];
-#pragma unroll
-    for (int e = 0; e < EV; ++e) {
-      mx[e] = mn[e] = 0.f;
+      for (int j = 0; j < 8; ++j) raw[j] = *reinterpret_cast<const uint4*>(xp + j * pitch);
+    } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if constexpr (ASYM) {
-          mx[e] = fmaxf(mx[e], v[j][e]);
-          mn[e] = fminf(mn[e], v[j][e]);
-        } else {
-          mx[e] = absmax_acc(mx[e], v[j][e]);
-        }
-      }
-      // lanes l, l^16, l^32 hold the same columns
-      mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], 16, 64));
-      mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], 32, 64));
-      if constexpr (ASYM) {
-        mn[e] = fminf(mn[e], __shfl_xor(mn[e], 16, 64));
-        mn[e] = fminf(mn[e], __shfl_xor(mn[e], 32, 64));
+        raw[j] = make_uint4(0, 0, 0, 0);
+        if (col_ok && r0 + j < row_end) raw[j] = *reinterpret_cast<const uint4*>(xp + j * pitch);
       }
     }
-    const int tc = threadIdx.x & 15;
-    if ((threadIdx.x & 63) < 16) {
+  }
+  auto value = [&](int j, int e) -> float {  // row j, column e of this thread
+    const uint32_t wd[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+    if constexpr (D::kTag == QWIX_BF16)
+      return __uint_as_float((e & 1) ? (wd[e >> 1] & 0xFFFF0000u) : (wd[e >> 1] << 16));
+    else
+      return __uint_as_float(wd[e]);
+  };
+  if constexpr (SRC == 2) {
+    float mx[EV], mn[EV];
+    if constexpr (!ASYM && D::kTag == QWIX_BF16) {  // |x| of a bf16 pair orders like its low 15 bits
+      u16x2 m[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t wd[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, wd[k] & 0x7FFF7FFFu));
+      }
+      // lanes l, l^16, l^32 hold the same columns
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 16, 64)));
+        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 32, 64)));
+        mx[2 * k] = bf16_bits_to_f32(m[k][0]);
+        mx[2 * k + 1] = bf16_bits_to_f32(m[k][1]);
+      }
+    } else {
 #pragma unroll
       for (int e = 0; e < EV; ++e) {
-        red[0][threadIdx.x >> 6][tc][e] = mx[e];
-        if constexpr (ASYM) red[1][threadIdx.x >> 6][tc][e] = mn[e];
+        mx[e] = mn[e] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float v = value(j, e);
+          if constexpr (ASYM) {
+            mx[e] = fmaxf(mx[e], v);
+            mn[e] = fminf(mn[e], v);
+          } else {
+            mx[e] = absmax_acc(mx[e], v);
+          }
+        }
+        mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], 16, 64));
+        mx[e] = fmaxf(mx[e], __shfl_xor(mx[e], 32, 64));
+        if constexpr (ASYM) {
+          mn[e] = fminf(mn[e], __shfl_xor(mn[e], 16, 64));
+          mn[e] = fminf(mn[e], __shfl_xor(mn[e], 32, 64));
+        }
+      }
+    }
+    if ((tid & 63) < 16) {
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        red[0][tid >> 6][tc * EV + e] = mx[e];
+        if constexpr (ASYM) red[1][tid >> 6][tc * EV + e] = mn[e];
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int e = 0; e < EV; ++e) {
-      z[e] = 0;
-      const float a = apply_factor<D>(
-          fmaxf(fmaxf(red[0][0][tc][e], red[0][1][tc][e]), fmaxf(red[0][2][tc][e], red[0][3][tc][e])), factor);
-      if constexpr (ASYM) {
-        const float b = apply_factor<D>(
-            fminf(fminf(red[1][0][tc][e], red[1][1][tc][e]), fminf(red[1][2][tc][e], red[1][3][tc][e])), factor);
-        s[e] = asym_scale_zp<D, QT>(b, a, &z[e]);
-      } else {
-        s[e] = sym_scale<D, QT>(a);
-      }
-      if (rb == 0 && col_ok) {
-        store1<D>(scale, sidx + e, s[e]);
-        if constexpr (ASYM) zp[sidx + e] = static_cast<int8_t>(z[e]);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < EV; ++e) {
-      z[e] = 0;
-      s[e] = 1.f;
-      if (!col_ok) continue;
-      if constexpr (SRC == 0) {
-        const float mx = apply_factor<D>(__uint_as_float(ws[sidx + e]), factor);
-        if constexpr (ASYM) {
-          const int64_t plane = gm.outer * gm.ntiles * gm.inner;
-          const float mn = apply_factor<D>(-__uint_as_float(ws[plane + sidx + e]), factor);
-          s[e] = asym_scale_zp<D, QT>(mn, mx, &z[e]);
-        } else {
-          s[e] = sym_scale<D, QT>(mx);
-        }
-        if (chunk == 0 && rb == 0) {
-          store1<D>(scale, sidx + e, s[e]);
-          if constexpr (ASYM) zp[sidx + e] = static_cast<int8_t>(z[e]);
-        }
-      } else {
-        s[e] = load1<D>(scale, sidx + e);
-        if constexpr (ASYM) z[e] = zp[sidx + e];
-      }
-    }
-    load_rows();
   }
+  if (tid < NC) {
+    float s = 1.f;
+    int z = 0;
+    if constexpr (SRC == 1) {
+      if (owner) {
+        s = load1<D>(scale, sidx);
+        if constexpr (ASYM) z = zp[sidx];
+      }
+    } else {
+      float a, b = 0.f;
+      if constexpr (SRC == 2) {
+        a = fmaxf(fmaxf(red[0][0][tid], red[0][1][tid]), fmaxf(red[0][2][tid], red[0][3][tid]));
+        if constexpr (ASYM) b = fminf(fminf(red[1][0][tid], red[1][1][tid]), fminf(red[1][2][tid], red[1][3][tid]));
+      } else {
+        a = __uint_as_float(pre0);
+        b = -__uint_as_float(pre1);
+      }
+      a = apply_factor<D>(a, factor);
+      if constexpr (ASYM)
+        s = asym_scale_zp<D, QT>(apply_factor<D>(b, factor), a, &z);
+      else
+        s = sym_scale<D, QT>(a);
+      if (owner && (SRC == 2 || chunk == 0)) {
+        store1<D>(scale, sidx, s);
+        if constexpr (ASYM) zp[sidx] = static_cast<int8_t>(z);
+      }
+    }
+    sh_s[tid] = s;
+    if constexpr (ASYM) sh_z[tid] = static_cast<float>(z);
+  }
+  // LDS only: the rows' loads stay in flight across the barrier
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  uint32_t codes[EV][2];
 #pragma unroll
   for (int e = 0; e < EV; ++e) {
-    const Divider<D, SRC == 1, QT == QWIX_E4M3> div(s[e]);
-    const float zf = static_cast<float>(z[e]);
+    float col[8];
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      div.pair(v[j][e], v[j + 1][e]);
-      if constexpr (ASYM) {
-        v[j][e] += zf;
-        v[j + 1][e] += zf;
-        if constexpr (D::kTag == QWIX_BF16) round_bf16_pair(v[j][e], v[j + 1][e]);
+    for (int j = 0; j < 8; ++j) col[j] = value(j, e);
+    quantize_column<D, QT, SRC == 1, ASYM>(col, sh_s[tc * EV + e], ASYM ? sh_z[tc * EV + e] : 0.f, factor > 0.f, codes[e]);
+  }
+  constexpr int EPB = (QT == QWIX_INT4) ? 2 : 1;  // elements per byte
+  if constexpr (LAYOUT == QWIX_LAYOUT_NATURAL) {
+    // back to rows: the codes of the EV columns of row j
+    if (col_ok) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (r0 + j >= row_end) continue;
+        uint8_t* dst = q + ((o * gm.reduce + r0 + j) * gm.inner + c0) / EPB;
+        if constexpr (QT == QWIX_INT4) {
+          uint32_t w = 0;
+#pragma unroll
+          for (int e = 0; e < EV; ++e) w |= ((codes[e][0] >> (4 * j)) & 0xFu) << (4 * e);
+          if constexpr (EV == 8) *reinterpret_cast<uint32_t*>(dst) = w;
+          else *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(w);
+        } else {
+          uint32_t w[EV / 4];
+#pragma unroll
+          for (int h = 0; h < EV / 4; ++h) {
+            const uint32_t sh = 8 * (j & 3);
+            w[h] = pack4_low_bytes(codes[4 * h][j >> 2] >> sh, codes[4 * h + 1][j >> 2] >> sh, codes[4 * h + 2][j >> 2] >> sh,
+                                   codes[4 * h + 3][j >> 2] >> sh);
+          }
+          if constexpr (EV == 8) nt_store8(reinterpret_cast<uint2*>(dst), make_uint2(w[0], w[1]));
+          else *reinterpret_cast<uint32_t*>(dst) = w[0];
+        }
       }
     }
-  }
-  constexpr bool kBounded = !(SRC == 1 && QT == QWIX_E4M3);  // a given scale: NaN inputs stay NaN in e4m3
-  if constexpr (LAYOUT == QWIX_LAYOUT_NATURAL) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (col_ok && r0 + j < row_end) store_q<QT, EV, kBounded>(v[j], q, (o * gm.reduce + r0 + j) * gm.inner + c0);
   } else {
-    // (outer, inner, reduce): the block's 128 rows x 128 columns leave as 128 column pieces of 128 rows.
+    // (outer, inner, reduce): the block's 128 rows x NC columns leave as NC column pieces of 128 rows.
     // A thread's 8 rows of one column are 8 consecutive output bytes, but a direct store would scatter
-    // 32-byte pieces over 128 output rows; staged through LDS the block writes whole 128-byte pieces.
-    constexpr int ROW_EL = 128 + 16;                       // staged row pitch in elements (keeps 8-byte alignment)
-    constexpr int EPB = (QT == QWIX_INT4) ? 2 : 1;         // elements per byte
-    __shared__ __attribute__((aligned(16))) uint8_t stage[16 * EV * ROW_EL / EPB];
-    const int tc = threadIdx.x & 15;
+    // 32-byte pieces over NC output rows; staged through LDS the block writes whole 128-byte pieces.
+    // 16-byte chunk p of a column sits at p ^ key of the thread column, which spreads the 8-byte writes of a wavefront
+    // over all 64 banks (at a plain pitch of 144 bytes they met eight to a bank).
+    constexpr int PITCH = 128 / EPB + 16, PIECES = 8 / EPB;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[NC * PITCH];
+    auto key = [](int thread_col) { return EPB == 2 ? (thread_col >> 1) & 3 : thread_col & 7; };
 #pragma unroll
     for (int e = 0; e < EV; ++e) {
-      float col[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) col[j] = v[j][e];
-      store_q<QT, 8, kBounded>(col, stage, (tc * EV + e) * ROW_EL + rb * 8);
+      uint8_t* row = stage + (tc * EV + e) * PITCH;
+      if constexpr (EPB == 2)
+        *reinterpret_cast<uint32_t*>(row + (((rb >> 2) ^ key(tc)) << 4) + (rb & 3) * 4) = codes[e][0];
+      else
+        *reinterpret_cast<uint2*>(row + (((rb >> 1) ^ key(tc)) << 4) + (rb & 1) * 8) = make_uint2(codes[e][0], codes[e][1]);
     }
     __syncthreads();
     // 16-byte pieces: piece p of column c covers rows 16*EPB*p .. of this block
-    constexpr int PIECES = 128 / (16 * EPB);
-    const int64_t row0 = t * gm.tile + chunk * 128;
-    const int64_t cb0 = c0 - tc * EV;                      // first column of the block
     const bool vec = (gm.reduce % (16 * EPB) == 0) && (row0 % (16 * EPB) == 0);
-    for (int i = threadIdx.x; i < 16 * EV * PIECES; i += 256) {
+    for (int i = tid; i < NC * PIECES; i += 256) {
       const int c = i / PIECES, pc = i % PIECES;
       const int64_t col = cb0 + c, r = row0 + pc * 16 * EPB;
       if (col >= gm.inner || r >= row_end) continue;
-      const uint8_t* src = stage + (c * ROW_EL + pc * 16 * EPB) / EPB;
+      const uint8_t* src = stage + c * PITCH + ((pc ^ key(c / EV)) << 4);
       uint8_t* dst = q + ((o * gm.inner + col) * gm.reduce + r) / EPB;
       if (vec && r + 16 * EPB <= row_end) {
         nt_store16(reinterpret_cast<uint4*>(dst), *reinterpret_cast<const uint4*>(src));
@@ -1199,58 +1318,102 @@ __global__ void __launch_bounds__(256)
   else store1<D>(out, idx, v[0]);
 }
 
-// Reduce-minor layout (values stored (outer, inner, reduce), output (outer, reduce, inner)): a 64 x 64 tile is
-// read along the reduced axis, turned in LDS, and written along the inner axis with its scales, 16 per thread.
+// Reduce-minor layout (values stored (outer, inner, reduce), output (outer, reduce, inner)): tiles of 128 columns (i) x one
+// 128-byte line of packed values per column.  Bound by memory: whole lines come in, 256-byte row pieces leave (bf16), and
+// nothing is turned byte by byte: the lines go to LDS as they are, a thread reads the same dword of eight columns and
+// converts its bytes (nibbles) in place, which yields eight consecutive outputs per row.  Chunk c of column i sits at
+// c ^ ((i >> 4) & 7) at a pitch of 144 bytes, so that those dword reads fall into 64 different banks.  Consecutive blocks
+// take consecutive columns: along the rows instead, blocks that run together write rows a power of two apart for such
+// widths (8192 x 8192, int4 / int8: 32 / 36 us against 45 / 46; 8192 x 28672 e4m3: 154 against 146).  8192 x 28672 e4m3 to
+// bf16 236 -> 154 us (4.6 TB/s), 4096 x 14336 59 -> 31, against tiles of 64 x 64 turned byte by byte.
 template <typename D, int QT>
 __global__ void __launch_bounds__(256)
     dequant_rm_kernel(const uint8_t* __restrict__ q, int64_t reduce, int64_t inner, int64_t tile,
                       const void* __restrict__ scale, const int8_t* __restrict__ zp, void* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) uint8_t turned[64][80];  // [r][i], rows padded to 80 bytes
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64, i0 = static_cast<int64_t>(blockIdx.y) * 64;
+  constexpr int EPB = QT == QWIX_INT4 ? 2 : 1, KT = 128 * EPB;  // values per byte, rows of the output per tile
+  constexpr int PITCH = 144;
+  __shared__ __attribute__((aligned(16))) uint8_t lines[128 * PITCH];
+  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * KT, i0 = static_cast<int64_t>(blockIdx.x) * 128;
   const int64_t o = blockIdx.z;
-  const int t = threadIdx.x;
-  {  // 64 rows (i) x 64 values (r): 16 values per thread
-    const int il = t >> 2, rc = (t & 3) * 16;
-    const int64_t i = i0 + il, r = r0 + rc;
-    uint32_t w[4] = {0, 0, 0, 0};
-    if (i < inner && r < reduce) {
-      const int64_t e = (o * inner + i) * reduce + r;
-      if constexpr (QT == QWIX_INT4) {
-        const uint2 p = *reinterpret_cast<const uint2*>(q + e / 2);
-        w[0] = p.x;
-        w[1] = p.y;
-      } else {
-        const uint4 p = *reinterpret_cast<const uint4*>(q + e);
-        w[0] = p.x; w[1] = p.y; w[2] = p.z; w[3] = p.w;
-      }
-    }
+  const int tid = threadIdx.x;
+  const int64_t row_bytes = reduce / EPB, b0 = r0 / EPB;  // reduce % 8 == 0
+  auto at = [](int col, int byte) { return col * PITCH + (((byte >> 4) ^ ((col >> 4) & 7)) << 4) + (byte & 15); };
+  if (i0 + 128 <= inner && b0 + 128 <= row_bytes && row_bytes % 16 == 0) {
+    uint4 v[4];
+    const uint8_t* src = q + (o * inner + i0 + (tid >> 3)) * row_bytes + b0 + (tid & 7) * 16;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      uint32_t b;
-      if constexpr (QT == QWIX_INT4) b = (w[k >> 3] >> (4 * (k & 7))) & 0xF;
-      else b = (w[k >> 2] >> (8 * (k & 3))) & 0xFF;
-      turned[rc + k][il] = static_cast<uint8_t>(b);
+    for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const uint4*>(src + j * 32 * row_bytes);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(lines + at((tid >> 3) + j * 32, (tid & 7) * 16)) = v[j];
+  } else {
+    for (int e = tid; e < 128 * 32; e += 256) {  // a dword each
+      const int col = e >> 5, byte = (e & 31) * 4;
+      uint32_t w = 0;
+      if (i0 + col < inner && b0 + byte < row_bytes)
+        w = *reinterpret_cast<const uint32_t*>(q + (o * inner + i0 + col) * row_bytes + b0 + byte);
+      *reinterpret_cast<uint32_t*>(lines + at(col, byte)) = w;
     }
   }
   __syncthreads();
-  const int rl = t >> 2, ic = (t & 3) * 16;
-  const int64_t r = r0 + rl, i = i0 + ic;
-  if (r >= reduce || i >= inner) return;
-  const uint4 pk = *reinterpret_cast<const uint4*>(&turned[rl][ic]);
-  const uint32_t w[4] = {pk.x, pk.y, pk.z, pk.w};
-  const int64_t si = (o * (reduce / tile) + r / tile) * inner + i;
-  const int64_t oi = (o * reduce + r) * inner + i;
+  const int cg = tid & 15;                // columns i0 + 8 cg ..
+  const int64_t i = i0 + cg * 8;
+  if (i >= inner) return;
+  const int left = static_cast<int>(min(static_cast<int64_t>(8), inner - i));
+  const bool vec = left == 8 && inner % D::kVec == 0;
+  int64_t have = -1;
+  float s[8], off[8];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    float v[8];
+  for (int it = 0; it < 2; ++it) {
+    const int d = (tid >> 4) + it * 16;   // dword of the line: 4 or 8 rows, all in one scale group (tile % 8 == 0)
+    const int64_t r = r0 + d * 4 * EPB;
+    if (r >= reduce) break;
+    const int64_t si = (o * (reduce / tile) + r / tile) * inner + i;
+    if (si != have) {
+      have = si;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        s[e] = e < left ? load1<D>(scale, si + e) : 0.f;
+        // what the offset-binary byte / nibble carries too much, zero point included; integers, exact in every type here
+        off[e] = QT == QWIX_INT8 ? 128.f : QT == QWIX_INT4 ? 8.f : 0.f;
+        if (zp != nullptr && e < left) off[e] += static_cast<float>(zp[si + e]);
+      }
+    }
+    uint32_t w[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int k = 8 * h + e;
-      float x = rnd<D>(q_to_f32<QT>((w[k >> 2] >> (8 * (k & 3))) & 0xFF));
-      if (zp != nullptr) x = rnd<D>(x - rnd<D>(static_cast<float>(zp[si + k])));
-      v[e] = rnd<D>(x * load1<D>(scale, si + k));
+      w[e] = *reinterpret_cast<const uint32_t*>(lines + at(cg * 8 + e, d * 4));
+      if constexpr (QT == QWIX_INT8) w[e] ^= 0x80808080u;
+      if constexpr (QT == QWIX_INT4) w[e] ^= 0x88888888u;
     }
-    store8<D>(out, oi + 8 * h, v);
+#pragma unroll
+    for (int k = 0; k < 4 * EPB; ++k) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float x;
+        if constexpr (QT == QWIX_E4M3) {
+          x = e4m3_to_f32(w[e] >> (8 * k));
+          if (zp != nullptr) x = rnd<D>(x - off[e]);
+        } else if constexpr (QT == QWIX_INT8) {
+          x = static_cast<float>((w[e] >> (8 * k)) & 0xFFu) - off[e];
+        } else {
+          x = static_cast<float>((w[e] >> (4 * k)) & 0xFu) - off[e];
+        }
+        v[e] = x * s[e];
+      }
+      const int64_t oi = (o * reduce + r + k) * inner + i;
+      if (vec) {
+        if constexpr (D::kTag == QWIX_BF16)
+          nt_store16(reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + oi),
+                     make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])));
+        else
+          store8<D>(out, oi, v);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e < left) store1<D>(out, oi + e, v[e]);
+      }
+    }
   }
 }
 
@@ -1811,9 +1974,9 @@ int qwix_hip_dequantize(const void* qvalue, int qtype, int q_layout, int64_t out
 #undef QWIX_DEQ_VEC
     return check_launch("dequantize");
   }
-  if (!natural && ptr_ok && inner % 16 == 0 && reduce % (qtype == QWIX_INT4 ? 32 : 16) == 0 && outer <= 65535 &&
-      (inner + 63) / 64 <= 65535) {
-    const dim3 grid(static_cast<unsigned>((reduce + 63) / 64), static_cast<unsigned>((inner + 63) / 64),
+  if (!natural && ptr_ok && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 <= 65535) {
+    const int kt = qtype == QWIX_INT4 ? 256 : 128;
+    const dim3 grid(static_cast<unsigned>((inner + 127) / 128), static_cast<unsigned>((reduce + kt - 1) / kt),
                     static_cast<unsigned>(outer));
 #define QWIX_DEQ_RM(QTT) dequant_rm_kernel<D, QTT><<<grid, 256, 0, st>>>(q, reduce, inner, tile, scale, zp, out)
     QWIX_DISPATCH_D(dtype, {

@@ -468,3 +468,25 @@ def test_int4_with_an_odd_last_axis(shape, how):
     oaq = O.quantize(O.FArr(a_np, O.BF16), O.HowToQuantize(qtype='int8', channelwise_axes=[0]))
     dn = (((1,), (0,)), ((), ()))
     assert np.array_equal(util.f32np(dg.dot_general(aq, q, dn)), O.dot_general(oaq, oq, dn).v)
+
+
+@pytest.mark.parametrize('qtype,method', [('int8', 'absmax'), ('int8', 'minmax'), ('int4', 'absmax'), ('int4', 'minmax'),
+                                          ('float8_e4m3fn', 'absmax'), ('float8_e4m3fn', 'absmax,0.8')])
+@pytest.mark.parametrize('dtype', [O.BF16, O.F32])
+@pytest.mark.parametrize('K,N,tile', [(8, 8, None), (136, 136, None), (264, 200, 8), (520, 120, None), (256, 392, 128),
+                                      (1160, 72, None), (640, 264, 320)])
+def test_weight_columns_and_back_at_tile_edges(K, N, tile, dtype, qtype, method):
+  """Reduce-minor weights around the kernels' blocks (128 rows x 128 or 64 columns, lines of 128 packed bytes, 256-row
+  calibration blocks; widths that are an odd multiple of 8): codes, scales and the dequantized values bit for bit, signed
+  zeros and tiny magnitudes among the inputs, and a calibration factor that lets quotients leave e4m3's range."""
+  from qwix_amd.core import qarray
+  x_np, x_t = util.make((K, N), dtype, seed=K + N, scale=0.02)
+  x_np, x_t = x_np.copy(), x_t.clone()
+  x_np[::3, 1], x_t[::3, 1] = -0.0, -0.0
+  x_np[1::5, 2], x_t[1::5, 2] = -2.0 ** -120, -2.0 ** -120
+  kw = dict(qtype=qtype, channelwise_axes=[1], calibration_method=method)
+  if tile:
+    kw['tiled_axes'] = {0: tile}
+  qa = _check(x_np, x_t, dtype, kw, layout='reduce_minor', what='column blocks')
+  want = O.dequantize(O.quantize(O.FArr(x_np, dtype), O.HowToQuantize(**kw)))
+  assert np.array_equal(util.f32np(qarray.dequantize(qa)), want.v)
