@@ -28,7 +28,7 @@ def sources():
 
 def _compile(src: str, force: bool) -> str:
   obj = os.path.join(OBJ_DIR, src[:-4] + '.o')
-  deps = [os.path.join(HERE, src), os.path.join(HERE, 'common.h'),
+  deps = [os.path.join(HERE, src), os.path.join(HERE, 'common.h'), os.path.join(HERE, 'qgemm_strips.h'),
           os.path.join(os.path.dirname(PKG), 'include', 'qwix_hip.h')]
   if not force and os.path.exists(obj) and all(os.path.getmtime(obj) > os.path.getmtime(d) for d in deps):
     return obj

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "qgemm_strips.h"
 
 namespace qwix {
 namespace {
@@ -2948,6 +2949,18 @@ extern "C" int qwix_hip_qgemm_batched(const void* a, int64_t lda, int64_t a_batc
                 (long long)(M * lda), (long long)(N * ldb));
   const Epilogue ep = make_epilogue(qtype, sa, sa_dtype, sb, sb_dtype, acc_dtype, nullptr, nullptr, out_dtype);
   const Batched bs{a_batch_stride, b_batch_stride, sa_batch_stride, sb_batch_stride, out_batch_stride};
+  // A short contraction: strips of rows instead of tiles (the result's traffic is all there is)
+  const bool all_bf = ep.r0 && ep.r1 && ep.r2 && sa_dtype == QWIX_BF16 && sb_dtype == QWIX_BF16 && out_dtype == QWIX_BF16;
+  const bool all_f32 = !ep.r0 && !ep.r1 && !ep.r2 && sa_dtype == QWIX_F32 && sb_dtype == QWIX_F32 && out_dtype == QWIX_F32;
+  const int64_t piece = out_dtype == QWIX_BF16 ? 8 : 4;
+  if ((K == 64 || K == 128) && sa && sb && (all_bf || all_f32) && N % piece == 0 && ldo % piece == 0 &&
+      out_batch_stride % piece == 0 && sb_batch_stride % 4 == 0 && aligned16(sb) &&
+      (M + 128) * ldo * (out_dtype == QWIX_BF16 ? 2 : 4) < (int64_t{1} << 31)) {
+    const StripArgs p{static_cast<const uint8_t*>(a), lda, a_batch_stride, static_cast<const uint8_t*>(b), ldb, b_batch_stride,
+                      sa, sa_batch_stride, sb, sb_batch_stride, static_cast<uint8_t*>(out), ldo, out_batch_stride,
+                      static_cast<int>(M), static_cast<int>(N)};
+    return qgemm_strips(qtype, K, all_bf, p, batch, stream);
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (qtype == QWIX_INT8) return launch_batched<QWIX_INT8>(a, lda, b, ldb, bs, batch, M, N, K, ep, out, ldo, st);
   return launch_batched<QWIX_E4M3>(a, lda, b, ldb, bs, batch, M, N, K, ep, out, ldo, st);

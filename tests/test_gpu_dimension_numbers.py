@@ -84,6 +84,34 @@ def test_batch_axes_take_one_launch(monkeypatch):
       np.testing.assert_allclose(util.f32np(out), util.f32np(looped), rtol=1e-2, atol=1e-2 * float(looped.abs().max()))
 
 
+@pytest.mark.parametrize('M,N', [(1, 8), (16, 64), (17, 264), (33, 72), (65, 1000), (129, 256), (200, 520), (128, 1032)])
+@pytest.mark.parametrize('K', [64, 128])
+@pytest.mark.parametrize('qtype,dtype', [('int8', O.BF16), ('int8', O.F32), (O.E4M3, O.BF16), (O.E4M3, O.F32)])
+def test_batched_short_contraction(M, N, K, qtype, dtype):
+  """Contractions of 64 and 128 elements run along strips of rows: strips of 16, 32, 64 and 128 rows that end early, column
+  ranges that end inside a wavefront's 64, rows of the result that start inside a 128-byte line.  int8 bit for bit.
+  e4m3: the matrix instruction aligns the exact products of a sum with less than f32 precision (2^-14 of the sum of
+  magnitudes covers it; the 2-D kernels show the same 2^-15.5), and where such a difference crosses a rounding boundary each
+  of the three bf16 roundings of the chain can move the result by one step, 2^-7 of it."""
+  from qwix_amd.core import dot_general as dg
+  from qwix_amd.core import qarray
+  print('case strips', M, N, K, qtype, dtype, flush=True)
+  dn = (((2,), (2,)), ((0,), (0,)))
+  how = dict(qtype=qtype, channelwise_axes=[0, 1])
+  x_np, x_t = util.make((3, M, K), dtype, seed=M + K)
+  w_np, w_t = util.make((3, N, K), dtype, seed=N + K)
+  out = dg.dot_general(qarray.quantize(x_t, qarray.HowToQuantize(**how)), qarray.quantize(w_t, qarray.HowToQuantize(**how)), dn)
+  oxq, owq = (O.quantize(O.FArr(v, dtype), O.HowToQuantize(**how)) for v in (x_np, w_np))
+  want = O.dot_general(oxq, owq, dn)
+  got = util.f32np(out)
+  if qtype == 'int8':
+    assert np.array_equal(got, want.v)
+  else:
+    mags = np.einsum('bmk,bnk->bmn', np.abs(O.dequantize(oxq).v), np.abs(O.dequantize(owq).v))
+    steps = 3 * 2.0 ** -7 if dtype == O.BF16 else 3 * 2.0 ** -23
+    assert np.all(np.abs(got - want.v) <= 2.0 ** -14 * mags + steps * np.abs(want.v))
+
+
 def test_batched_dot_general_on_the_dequantize_path():
   """A float activation against a batched quantized operand takes the dequantize-first path."""
   from qwix_amd.core import dot_general as dg
