@@ -70,6 +70,7 @@ SIGNATURES = {
 }
 
 _lib = None
+recorder_of = None  # thread-local holder of an active plan recorder, once there has been one
 
 
 class QwixHipError(RuntimeError):
@@ -97,12 +98,19 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
   """Calls an int-returning entry point and raises with the library's message on error."""
-  lib = load()
-  status = getattr(lib, name)(*args)
+  status = getattr(load(), name)(*args)
   if status != OK:
-    msg = lib.qwix_hip_last_error().decode('utf-8', 'replace')
-    kind = {1: ValueError, 2: NotImplementedError}.get(status, QwixHipError)
-    raise kind(f'{name}: {msg}')
+    raise_status(name, status)
+  if recorder_of is not None:
+    recorder = getattr(recorder_of, 'recorder', None)
+    if recorder is not None:
+      recorder.note(name, args)
+
+
+def raise_status(name: str, status: int) -> None:
+  msg = load().qwix_hip_last_error().decode('utf-8', 'replace')
+  kind = {1: ValueError, 2: NotImplementedError}.get(status, QwixHipError)
+  raise kind(f'{name}: {msg}')
 
 
 def ptr(t) -> int | None:

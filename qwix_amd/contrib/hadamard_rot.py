@@ -18,6 +18,7 @@ import math
 import torch
 
 from qwix_amd import _lib
+from qwix_amd import plans
 from qwix_amd.core import numerics
 from qwix_amd.core import qarray
 
@@ -134,6 +135,15 @@ def hadamard_quantized_matmul(act: torch.Tensor, weight: qarray.QArray, pre_sign
   act: (M, K) bf16 / f32, K a power of two; weight: a symmetric int8 / int4 QArray of logical shape (K, N) with
   scales per output channel and group of `group` rows (tiles along K only), K-contiguous storage as
   `quantize(..., reduce-minor)` writes it; act_tile: None = one scale per token, else the weight's group."""
+  fixed = ('hadamard_matmul', act_tile, preferred_element_type)
+  out = (plans._native or plans.native()).run(fixed, act, weight, pre_sign, post_sign)
+  if out is not None and out is not True:
+    return out
+  ordinary = lambda: _hadamard_quantized_matmul(act, weight, pre_sign, post_sign, act_tile, preferred_element_type)
+  return ordinary() if out is None else plans.record(fixed, (act, weight, pre_sign, post_sign), ordinary, plans.single)
+
+
+def _hadamard_quantized_matmul(act, weight, pre_sign, post_sign, act_tile, preferred_element_type) -> torch.Tensor:
   from qwix_amd.core import dot_general as dg
   if act.ndim != 2 or not isinstance(weight, qarray.QArray) or weight.zero_point is not None:
     raise NotImplementedError('hadamard_quantized_matmul takes a 2-D activation and a symmetric quantized weight')

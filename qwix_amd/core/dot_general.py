@@ -25,6 +25,7 @@ from typing import Any, Mapping, Sequence
 import torch
 
 from qwix_amd import _lib
+from qwix_amd import plans
 from qwix_amd.core import numerics
 from qwix_amd.core import qarray
 from qwix_amd.core.qarray import Int4Tensor, QArray
@@ -316,6 +317,16 @@ def fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=No
   scratch buffer otherwise.  Bit-identical to quantize(lhs, channelwise over the non-contracting axes)
   followed by dot_general.  Returns None when the operands are not of that kind; the caller then takes the
   two-step route."""
+  fixed = ('fused_act', dimension_numbers, preferred_element_type, act_qtype)
+  out = (plans._native or plans.native()).run(fixed, lhs, rhs)
+  if out is None:
+    return _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype)
+  return out if out is not True else plans.record(
+      fixed, (lhs, rhs), lambda: _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype),
+      plans.single)
+
+
+def _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype):
   if not (_is_float_array(lhs) and lhs.dtype in (torch.bfloat16, torch.float32) and isinstance(rhs, QArray)):
     return None
   if rhs.zero_point is not None or isinstance(rhs.qvalue, Int4Tensor):
@@ -620,6 +631,12 @@ _ZP8_CACHE: dict = {}
 
 def _rhs_zero_point_i8(c: '_Canon', rhs: QArray) -> tuple[torch.Tensor, int]:
   z = rhs.zero_point
+  if z.dtype == torch.int8 and all(z.shape[a] in (1, rhs.shape[a]) for a in c.rfree) and all(z.shape[a] == 1 for a in c.rca[:-1]):
+    # as quantize writes them: already (groups, N) in memory
+    gz = z.shape[c.rca[-1]]
+    p = z.permute(*([c.rca[-1]] + c.rfree + c.rca[:-1]))
+    if p.is_contiguous() and p.numel() == gz * c.N and not (gz > 1 and len(c.rca) > 1):
+      return p.view(gz, c.N), gz
   key = (id(z), tuple(c.rca), tuple(c.rfree))
   hit = _ZP8_CACHE.get(key)
   if hit is not None and hit[0]() is z and hit[1] == z._version:
@@ -948,6 +965,18 @@ def dot_general(lhs: MaybeQ, rhs: MaybeQ, dimension_numbers: DotDimensionNumbers
   values directly.  `precision` and extra keywords (e.g. out_sharding) are accepted and ignored.
   """
   del precision
+  if kwargs and any(v is not None for v in kwargs.values()):
+    return _dot_general(lhs, rhs, dimension_numbers, preferred_element_type, **kwargs)
+  # (which weight-only kernel runs is decided by `fused_wq_min_rows`: another rule, other plans)
+  fixed = ('dot', dimension_numbers, preferred_element_type, fused_wq_min_rows)
+  out = (plans._native or plans.native()).run(fixed, lhs, rhs)
+  if out is None:
+    return _dot_general(lhs, rhs, dimension_numbers, preferred_element_type)
+  return out if out is not True else plans.record(
+      fixed, (lhs, rhs), lambda: _dot_general(lhs, rhs, dimension_numbers, preferred_element_type), plans.single)
+
+
+def _dot_general(lhs: MaybeQ, rhs: MaybeQ, dimension_numbers, preferred_element_type=None, **kwargs) -> torch.Tensor:
   empty = _degenerate(lhs, rhs, dimension_numbers, preferred_element_type)
   if empty is not None:
     return empty

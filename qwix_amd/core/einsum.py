@@ -10,6 +10,7 @@ from typing import Any, Mapping
 
 import torch
 
+from qwix_amd import plans
 from qwix_amd.core import dot_general as _dg
 from qwix_amd.core import einsum_info
 from qwix_amd.core import qarray
@@ -60,6 +61,17 @@ def broadcast_operands(operands: list, subs_list: list[str]) -> list:
 def einsum(*args, _qwix_dot_general=_dg.dot_general, preferred_element_type=None, **kwargs) -> torch.Tensor:
   """Drop-in for jnp.einsum('subscripts', a, b) with QArray operands; the result dtype follows the
   dequantized dtypes unless preferred_element_type is given."""
+  if len(args) == 3 and _qwix_dot_general is _dg.dot_general and not any(v is not None for v in kwargs.values()):
+    fixed = ('einsum', args[0], preferred_element_type, _dg.fused_wq_min_rows)
+    out = (plans._native or plans.native()).run(fixed, args[1], args[2])
+    if out is True:
+      return plans.record(fixed, args[1:], lambda: _einsum(args, _qwix_dot_general, preferred_element_type, kwargs), plans.single)
+    if out is not None:
+      return out
+  return _einsum(args, _qwix_dot_general, preferred_element_type, kwargs)
+
+
+def _einsum(args, _qwix_dot_general, preferred_element_type, kwargs) -> torch.Tensor:
   if not args or not isinstance(args[0], str):
     raise NotImplementedError('einsum expects the subscripts string first')
   einsum_str, operands = args[0], list(args[1:])

@@ -24,6 +24,7 @@ from typing import Any, Callable, Collection, Mapping, Sequence
 import torch
 
 from qwix_amd import _lib
+from qwix_amd import plans
 from qwix_amd.core import numerics
 
 # ------------------------------------------------------------------------------------------
@@ -864,6 +865,37 @@ def quantize_with_scale_zero_point(array: torch.Tensor, qtype, scale: torch.Tens
 def quantize(array: torch.Tensor, how: HowToQuantize, *, layout: str | None = None) -> QArray:
   """Dynamic-range quantization: calibrate, derive scale (and zero point), quantize -- one fused pass.  With a
   `noise_fn` (stochastic rounding) the three steps run one after the other, as the reference's do (qarray.py:638-644)."""
+  if how.noise_fn is not None:
+    return _quantize_any(array, how, layout)
+  fixed = ('quantize', how.qtype, tuple(how.channelwise_axes), tuple(how.tiled_axes.items()), how.calibration_method, layout)
+  out = (plans._native or plans.native()).run(fixed, array)
+  if out is None:
+    return _quantize_any(array, how, layout)
+  return out if out is not True else plans.record(fixed, (array,), lambda: _quantize_any(array, how, layout), _split)
+
+
+def _assemble(qtype: str, q, scale: torch.Tensor, zero_point: torch.Tensor | None = None) -> 'QArray':
+  """A QArray of values whose type and shapes are known to fit (nothing is checked again)."""
+  out = object.__new__(QArray)
+  out.qvalue, out.scale, out.zero_point, out.qtype = q, scale, zero_point, qtype
+  return out
+
+
+def _assemble_int4(shape, packed_axis: int, data, scale, zero_point=None) -> 'QArray':
+  q = object.__new__(Int4Tensor)
+  q.data, q.shape, q.packed_axis = data, shape, packed_axis
+  return _assemble(numerics.INT4, q, scale, zero_point)
+
+
+def _split(qa: 'QArray'):
+  """A QArray's tensors and what puts them together again."""
+  rest = (qa.scale,) if qa.zero_point is None else (qa.scale, qa.zero_point)
+  if isinstance(qa.qvalue, Int4Tensor):
+    return (qa.qvalue.data,) + rest, functools.partial(_assemble_int4, qa.qvalue.shape, qa.qvalue.packed_axis)
+  return (qa.qvalue,) + rest, functools.partial(_assemble, qa.qtype)
+
+
+def _quantize_any(array: torch.Tensor, how: HowToQuantize, layout: str | None) -> QArray:
   if how.noise_fn is not None and numerics.canonical_qtype(how.qtype) in (numerics.INT8, numerics.INT4) and array.numel():
     scale, zp = compute_scale_zero_point(calibrate(array, how), how.qtype)
     return quantize_with_scale_zero_point(array, how.qtype, scale, zp, how.noise_fn, layout='natural')
@@ -960,9 +992,16 @@ def quantize_api(array: torch.Tensor, qtype, *, channelwise_axes: Collection[int
                  scale_dtype: torch.dtype | None = None, layout: str | None = None) -> QArray:
   """Public `qwix.quantize`: like quantize() without building a HowToQuantize; the optional
   scale_dtype cast is applied to the already computed scale."""
-  how = HowToQuantize(qtype=qtype, channelwise_axes=channelwise_axes, tiled_axes=tiled_axes or {},
-                      calibration_method=calibration_method)
-  qa = quantize(array, how, layout=layout)
+  # (the same key as quantize(): without a plan the call goes there)
+  fixed = ('quantize', qtype, tuple(channelwise_axes), tuple(tiled_axes.items()) if tiled_axes else (), calibration_method, layout)
+  qa = (plans._native or plans.native()).run(fixed, array)
+  if qa is None or qa is True:
+    how = HowToQuantize(qtype=qtype, channelwise_axes=channelwise_axes, tiled_axes=tiled_axes or {},
+                        calibration_method=calibration_method)
+    if qa is None:
+      qa = _quantize_any(array, how, layout)
+    else:
+      qa = plans.record(fixed, (array,), lambda: _quantize_any(array, how, layout), _split)
   if scale_dtype is not None:
     qa = dataclasses.replace(qa, scale=qa.scale.to(scale_dtype))
   return qa
@@ -996,6 +1035,13 @@ def physical_layout(qa: QArray) -> tuple[_Plan, int, torch.Tensor]:
 
 def dequantize(array: QArray) -> torch.Tensor:
   """(qvalue - zero_point) * scale in the scale dtype; the reverse of quantize."""
+  out = (plans._native or plans.native()).run('dequantize', array)
+  if out is None:
+    return _dequantize(array)
+  return out if out is not True else plans.record('dequantize', (array,), lambda: _dequantize(array), plans.single)
+
+
+def _dequantize(array: QArray) -> torch.Tensor:
   validate_qarray(array)
   if math.prod(array.shape) == 0:
     return torch.empty(array.shape, dtype=array.scale.dtype, device=array.scale.device)

@@ -22,6 +22,7 @@ from typing import Sequence
 import torch
 
 from qwix_amd import _lib
+from qwix_amd import plans
 from qwix_amd.core import numerics
 from qwix_amd.core import qarray
 from qwix_amd.core import dot_general as _dot_general
@@ -405,5 +406,13 @@ def ragged_dot_general(lhs, rhs, group_sizes: torch.Tensor, dimension_numbers: R
 def ragged_dot(lhs, rhs, group_sizes: torch.Tensor, precision=None, preferred_element_type=None,
                group_offset=None) -> torch.Tensor:
   """Drop-in for lax.ragged_dot: lhs (M, K) . rhs (G, K, N) with the rows of lhs in G groups."""
-  return ragged_dot_general(lhs, rhs, group_sizes, _BASIC_RAGGED_DOT_DIMENSION_NUMBERS, precision=precision,
-                            preferred_element_type=preferred_element_type, group_offset=group_offset)
+  def ordinary():
+    return ragged_dot_general(lhs, rhs, group_sizes, _BASIC_RAGGED_DOT_DIMENSION_NUMBERS, precision=precision,
+                              preferred_element_type=preferred_element_type, group_offset=group_offset)
+  if group_offset is not None:
+    return ordinary()
+  fixed = ('ragged_dot', preferred_element_type)
+  out = (plans._native or plans.native()).run(fixed, lhs, rhs, group_sizes)
+  if out is None:
+    return ordinary()
+  return out if out is not True else plans.record(fixed, (lhs, rhs, group_sizes), ordinary, plans.single)

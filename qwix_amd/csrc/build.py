@@ -1,4 +1,5 @@
-"""Builds libqwix_hip.so (gfx950) from the .hip sources in this directory with hipcc.
+"""Builds libqwix_hip.so (gfx950) from the .hip sources in this directory with hipcc, and the host module _plans.so from
+plans.cpp with g++ against the installed torch.
 
 Run directly (`python qwix_amd/csrc/build.py`) or through `__graft_entry__.build()`.
 Each source is compiled to an object file in `build/`, then everything is linked into
@@ -12,6 +13,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 OUT = os.path.join(PKG, 'libqwix_hip.so')
+PLANS = os.path.join(PKG, '_plans.so')
 OBJ_DIR = os.path.join(HERE, 'build')
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = [
@@ -42,6 +44,25 @@ def _compile(src: str, force: bool) -> str:
   return obj
 
 
+def _build_plans(force: bool) -> None:
+  """The launch plans (host code only): a Python extension linked to libqwix_hip.so next to it."""
+  import sysconfig
+  import torch
+  src = os.path.join(HERE, 'plans.cpp')
+  deps = [src, os.path.join(os.path.dirname(PKG), 'include', 'qwix_hip.h')]
+  if not force and os.path.exists(PLANS) and all(os.path.getmtime(PLANS) > os.path.getmtime(d) for d in deps):
+    return
+  t = os.path.dirname(torch.__file__)
+  cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden',
+         f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', '-I' + os.path.join(t, 'include'),
+         '-I' + os.path.join(t, 'include', 'torch', 'csrc', 'api', 'include'), '-I' + sysconfig.get_paths()['include'], src,
+         '-o', PLANS, '-L' + PKG, '-lqwix_hip', '-L' + os.path.join(t, 'lib'), '-ltorch_python', '-ltorch_cpu', '-lc10',
+         '-Wl,-rpath,$ORIGIN']
+  r = subprocess.run(cmd, capture_output=True, text=True)
+  if r.returncode != 0:
+    raise RuntimeError(f'g++ failed on plans.cpp:\n{r.stderr}')
+
+
 def build(force: bool = True, verbose: bool = True) -> str:
   os.makedirs(OBJ_DIR, exist_ok=True)
   srcs = sources()
@@ -51,6 +72,7 @@ def build(force: bool = True, verbose: bool = True) -> str:
   r = subprocess.run(cmd, capture_output=True, text=True)
   if r.returncode != 0:
     raise RuntimeError(f'link failed:\n{r.stderr}')
+  _build_plans(force)
   if verbose:
     print(f'built {OUT} from {len(srcs)} sources')
   return OUT

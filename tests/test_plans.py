@@ -1,0 +1,222 @@
+"""Launch plans: what the recorder accepts (CPU), and that replayed calls give what the ordinary path gives (GPU)."""
+import threading
+
+import pytest
+import torch
+
+from qwix_amd import _lib
+from qwix_amd import plans
+from tests import util
+
+_DN = (((1,), (0,)), ((), ()))
+
+
+# ---- the recorder, on host memory: addresses are addresses
+
+
+def _recorded(fn, *operands):
+  with plans.Recorder(operands) as rec:
+    out = fn(rec)
+  return rec, out
+
+
+def _note(rec, q, x):
+  rec.note('qwix_hip_ksum_i8', (q.data_ptr(), 64, 4, 64, x.data_ptr(), 7))
+
+
+def test_recorder_tells_operands_buffers_and_constants_apart():
+  q = torch.zeros(8, 64, dtype=torch.int8)
+
+  def fn(rec):
+    out = torch.empty(4, 2, dtype=torch.int32)
+    _note(rec, q[4:], out)
+    return out.t()
+  rec, out = _recorded(fn, q)
+  assert rec.ok and len(rec.buffers) == 1
+  name, args = rec.calls[0]
+  assert name == 'qwix_hip_ksum_i8'
+  assert args == [(plans._OPERAND, 0, 256), (plans._CONST, 0, 64), (plans._CONST, 0, 4), (plans._CONST, 0, 64),
+                  (plans._BUFFER, 0, 0), (plans._STREAM, 0, 0)]
+  assert rec.results((out,)) == [(0, (2, 4), (1, 2), 0)]
+  assert rec.results((torch.zeros(3),)) is None   # not a buffer of the call
+
+
+@pytest.mark.parametrize('what', ['copy', 'fill', 'reduction', 'foreign pointer', 'overlapping operands', 'item'])
+def test_recorder_refuses(what):
+  q = torch.zeros(8, 64, dtype=torch.int8)
+  kept = torch.zeros(64, 8, dtype=torch.int8)
+  second = q[2:] if what == 'overlapping operands' else torch.zeros(1, dtype=torch.int8)
+
+  def fn(rec):
+    out = torch.empty(4, dtype=torch.int32)
+    if what == 'copy':
+      _note(rec, q.t().contiguous(), out)
+    elif what == 'foreign pointer':
+      _note(rec, kept, out)
+    else:
+      _note(rec, q, out)
+      if what == 'fill':
+        out.zero_()
+      elif what == 'reduction':
+        out.sum()
+      elif what == 'item':
+        out[0].item()
+    return out
+  rec, _ = _recorded(fn, q, second)
+  assert not rec.ok
+
+
+# ---- replay
+
+
+def _rand(shape, seed, dtype=torch.bfloat16, std=1.0):
+  g = torch.Generator(device='cpu').manual_seed(seed)
+  return (torch.randn(shape, generator=g) * std).to(dtype).to(util.DEV)
+
+
+def _same(a, b):
+  from qwix_amd.core.qarray import Int4Tensor, QArray
+  if isinstance(a, QArray):
+    assert a.qtype == b.qtype and tuple(a.shape) == tuple(b.shape) and (a.zero_point is None) == (b.zero_point is None)
+    values = lambda q: q.unpack() if isinstance(q, Int4Tensor) else q.view(torch.uint8) if q.dtype == torch.float8_e4m3fn else q
+    assert type(a.qvalue) is type(b.qvalue) and torch.equal(values(a.qvalue), values(b.qvalue))
+    assert torch.equal(a.scale, b.scale) and (a.zero_point is None or torch.equal(a.zero_point, b.zero_point))
+  else:
+    assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype and torch.equal(a, b)
+
+
+def _cases():
+  """name -> (operands of a seed, the operator, its ordinary path)"""
+  import qwix_amd
+  from qwix_amd.contrib import hadamard_rot as hr
+  from qwix_amd.core import dot_general as dg, einsum as es, qarray as qa, ragged_dot as rd
+  def weight(s, qtype, tile=None, method='absmax', k=512, n=200):
+    return qwix_amd.quantize(_rand((k, n), s, std=0.05), qtype, channelwise_axes=[1], tiled_axes={0: tile} if tile else {},
+                             calibration_method=method)
+  act = lambda s, qtype: qwix_amd.quantize(_rand((24, 512), s), qtype, channelwise_axes=[0])
+  how = lambda qtype, **kw: qwix_amd.HowToQuantize(qtype=qtype, **kw)
+  dot = (lambda a, b: qwix_amd.dot_general(a, b, _DN), lambda a, b: dg._dot_general(a, b, _DN))
+  cases = {}
+  for q, method in (('int8', 'absmax'), ('int8', 'minmax'), ('int4', 'absmax'), ('float8_e4m3fn', 'absmax')):
+    rows, cols = how(q, channelwise_axes=[0], calibration_method=method), how(q, channelwise_axes=[1], calibration_method=method)
+    cases[f'rows {q} {method}'] = (lambda s: (_rand((24, 512), s),), lambda x, h=rows: qwix_amd.core.qarray.quantize(x, h),
+                                   lambda x, h=rows: qa._quantize_any(x, h, None))
+    cases[f'columns {q} {method}'] = (lambda s: (_rand((512, 72), s),), lambda x, h=cols: qwix_amd.core.qarray.quantize(x, h),
+                                      lambda x, h=cols: qa._quantize_any(x, h, None))
+    cases[f'dequantize {q} {method}'] = (lambda s, q=q, m=method: (weight(s, q, method=m),), qwix_amd.dequantize, qa._dequantize)
+  for q in ('int8', 'float8_e4m3fn'):
+    cases[f'dot {q}'] = (lambda s, q=q: (act(s, q), weight(s + 1, q)),) + dot
+    cases[f'fused act {q}'] = (lambda s, q=q: (_rand((24, 512), s, torch.float32), weight(s + 1, q)),
+                               lambda a, b, q=q: dg.fused_act_dot_general(a, b, _DN, act_qtype=q),
+                               lambda a, b, q=q: dg._fused_act_dot_general(a, b, _DN, None, q))
+  for tile in (128, 256):
+    cases[f'dot int8 x int4 {tile}'] = (lambda s, t=tile: (act(s, 'int8'), weight(s + 1, 'int4', t)),) + dot
+  for q, method in (('int4', 'absmax'), ('int4', 'minmax'), ('int8', 'minmax')):
+    cases[f'weight only {q} {method}'] = (lambda s, q=q, m=method: (_rand((24, 512), s), weight(s + 1, q, 128, m)),) + dot
+  cases['einsum'] = (lambda s: tuple(qwix_amd.quantize(_rand((3, 40, 64), s + i), 'int8', channelwise_axes=[0, 1]) for i in (0, 1)),
+                     lambda a, b: qwix_amd.einsum('bqd,bkd->bqk', a, b),
+                     lambda a, b: es._einsum(('bqd,bkd->bqk', a, b), dg.dot_general, None, {}))
+  sizes = lambda s: torch.tensor([s % 5, 9, 0, 7], dtype=torch.int32, device=util.DEV)
+  cases['ragged int8'] = (lambda s: (act(s, 'int8'), qwix_amd.quantize(_rand((4, 512, 72), s), 'int8', channelwise_axes=[0, 2]), sizes(s)),
+                          qwix_amd.ragged_dot,
+                          lambda *a: rd.ragged_dot_general(*a, rd._BASIC_RAGGED_DOT_DIMENSION_NUMBERS))
+  cases['hadamard'] = (lambda s: (_rand((24, 512), s), weight(s + 1, 'int4', 128)), hr.hadamard_quantized_matmul,
+                       lambda a, b: hr._hadamard_quantized_matmul(a, b, None, None, None, None))
+  return cases
+
+
+_NAMES = (['%s %s %s' % (w, q, m) for w in ('rows', 'columns', 'dequantize')
+           for q, m in (('int8', 'absmax'), ('int8', 'minmax'), ('int4', 'absmax'), ('float8_e4m3fn', 'absmax'))] +
+          ['%s %s' % (w, q) for w in ('dot', 'fused act') for q in ('int8', 'float8_e4m3fn')] +
+          ['dot int8 x int4 128', 'dot int8 x int4 256', 'weight only int4 absmax', 'weight only int4 minmax',
+           'weight only int8 minmax', 'einsum', 'ragged int8', 'hadamard'])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', _NAMES)
+def test_replay_equals_the_ordinary_path(name):
+  """New operands (other data, other addresses) on every call: the first ones go the ordinary way, the others replay."""
+  make, op, ordinary = _cases()[name]
+  alive = []
+  for seed in range(plans.RECORD_AT + 2):
+    operands = make(10 * seed)
+    alive.append(operands)   # no address comes up twice
+    _same(op(*operands), ordinary(*operands))
+  calls = []
+  call, _lib.call = _lib.call, lambda *a: calls.append(a[0]) or call(*a)
+  try:
+    _same(op(*alive[0]), op(*alive[0]))
+    assert not calls, 'no plan is kept for this kind of call'
+  finally:
+    _lib.call = call
+
+
+@pytest.mark.gpu
+def test_replay_with_other_layouts_options_and_errors():
+  import qwix_amd
+  w = qwix_amd.quantize(_rand((512, 200), 1, std=0.05), 'int8', channelwise_axes=[1])
+  big = _rand((40, 1100), 2)
+  for _ in range(plans.RECORD_AT + 2):
+    for x in (big[:24, :512], big[3:27, 8:520], big[3:27, 3:515], big[:24, :512].contiguous()):   # pitches and alignments
+      got = qwix_amd.quantize(x, 'int8', channelwise_axes=[0])
+      want = qwix_amd.core.qarray._quantize_any(x.contiguous(), qwix_amd.HowToQuantize(qtype='int8', channelwise_axes=[0]), None)
+      _same(got, want)
+      out = qwix_amd.dot_general(got, w, _DN)
+      assert out.dtype == torch.bfloat16
+      assert qwix_amd.dot_general(got, w, _DN, preferred_element_type=torch.float32).dtype == torch.float32
+  with pytest.raises(ValueError, match='differ'):
+    qwix_amd.dot_general(got, qwix_amd.quantize(_rand((256, 200), 1), 'int8', channelwise_axes=[1]), _DN)
+  # one array on both sides: its memory belongs to both operands
+  a = qwix_amd.quantize(_rand((64, 64), 5), 'int8', channelwise_axes=[0])
+  dn = (((1,), (1,)), ((), ()))
+  for _ in range(plans.RECORD_AT + 2):
+    _same(qwix_amd.dot_general(a, a, dn), qwix_amd.core.dot_general._dot_general(a, a, dn))
+
+
+@pytest.mark.gpu
+def test_replay_on_threads_and_streams():
+  import qwix_amd
+  w = qwix_amd.quantize(_rand((512, 200), 1, std=0.05), 'int8', channelwise_axes=[1])
+  xs = [_rand((24, 512), 20 + i) for i in range(4)]
+  step = lambda x: qwix_amd.dot_general(qwix_amd.quantize(x, 'int8', channelwise_axes=[0]), w, _DN)
+  want = [step(x) for x in xs]
+  torch.cuda.synchronize()
+  bad = []
+
+  def work(i):
+    with torch.cuda.stream(torch.cuda.Stream()):
+      for _ in range(50):
+        out = step(xs[i])
+        torch.cuda.current_stream().synchronize()
+        if not torch.equal(out, want[i]):
+          bad.append(i)
+          return
+  threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+  for t in threads:
+    t.start()
+  for t in threads:
+    t.join()
+  assert not bad
+
+
+@pytest.mark.gpu
+def test_replay_inside_a_captured_graph():
+  """Captured calls are replayed plans; every replay of the graph against the eager result."""
+  import qwix_amd
+  w = qwix_amd.quantize(_rand((512, 200), 1, std=0.05), 'int8', channelwise_axes=[1])
+  x = _rand((24, 512), 30)
+  step = lambda: qwix_amd.dot_general(qwix_amd.quantize(x, 'int8', channelwise_axes=[0]), w, _DN)
+  side = torch.cuda.Stream()
+  side.wait_stream(torch.cuda.current_stream())
+  with torch.cuda.stream(side):
+    for _ in range(plans.RECORD_AT + 1):
+      step()
+  torch.cuda.current_stream().wait_stream(side)
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    out = step()
+  for seed in range(31, 35):
+    x.copy_(_rand((24, 512), seed))
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, step())
