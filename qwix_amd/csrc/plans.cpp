@@ -15,6 +15,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <tuple>
 #include <unordered_map>
@@ -100,7 +101,7 @@ struct Plan {
 struct Seen {
   PyObject* fixed;
   std::string signature;
-  Plan* plan = nullptr;
+  std::shared_ptr<const Plan> plan;  // a call holds its own reference: `rebuild` is Python, other threads run meanwhile
   int times = 0;
 };
 struct Cache {
@@ -108,10 +109,7 @@ struct Cache {
   size_t count = 0;
   void clear() {
     for (auto& [h, v] : seen)
-      for (Seen& s : v) {
-        Py_DECREF(s.fixed);
-        delete s.plan;
-      }
+      for (Seen& s : v) Py_DECREF(s.fixed);
     seen.clear();
     count = 0;
   }
@@ -276,11 +274,11 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) try {
   if (s == nullptr) {
     if (c->count >= kMaxSeen) c->clear();
     Py_INCREF(args[0]);
-    c->seen[h].push_back(Seen{args[0], std::move(ops.signature), nullptr, 1});
+    c->seen[h].push_back(Seen{args[0], std::move(ops.signature), {}, 1});
     ++c->count;
     Py_RETURN_NONE;
   }
-  if (s->plan != nullptr) return run_plan(*s->plan, ops);
+  if (const std::shared_ptr<const Plan> p = s->plan) return run_plan(*p, ops);
   if (++s->times == g_record_at) Py_RETURN_TRUE;
   Py_RETURN_NONE;
 } catch (const std::exception&) {  // out of memory and the like: the ordinary path meets it again and raises as torch does
@@ -316,7 +314,7 @@ PyObject* keep(PyObject*, PyObject* args) {
   if (!ok) return nullptr;
   Seen* s = lookup(*c, fixed, ops.signature, h);
   if (s == nullptr || s->plan != nullptr || PyList_GET_SIZE(buffers) > 16 || PyList_GET_SIZE(results) > 8) Py_RETURN_FALSE;
-  auto p = std::make_unique<Plan>();
+  auto p = std::make_shared<Plan>();
   for (Py_ssize_t k = 0; k < PyList_GET_SIZE(buffers); ++k) {
     PyObject *sizes, *strides, *like;
     if (!PyArg_ParseTuple(PyList_GET_ITEM(buffers, k), "OOO", &sizes, &strides, &like)) return nullptr;
@@ -373,7 +371,7 @@ PyObject* keep(PyObject*, PyObject* args) {
   } else if (p->results.size() != 1) {
     Py_RETURN_FALSE;
   }
-  s->plan = p.release();
+  s->plan = std::move(p);
   Py_RETURN_TRUE;
 }
 

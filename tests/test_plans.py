@@ -1,5 +1,7 @@
 """Launch plans: what the recorder accepts (CPU), and that replayed calls give what the ordinary path gives (GPU)."""
+import functools
 import threading
+import weakref
 
 import pytest
 import torch
@@ -64,6 +66,35 @@ def test_recorder_refuses(what):
     return out
   rec, _ = _recorded(fn, q, second)
   assert not rec.ok
+
+
+# ---- the table
+
+
+def test_a_plan_in_use_outlives_a_table_that_starts_anew():
+  """`rebuild` is Python: what it runs, or another thread meanwhile, may fill the table until it is emptied."""
+  n = plans.native()
+  seen = []
+
+  def fill(value):
+    for k in range(9000):   # more signatures than are remembered
+      n.run(('filler', k))
+    seen.append(alive() is not None)
+    return value
+  rebuild = functools.partial(fill, 'done')
+  alive = weakref.ref(rebuild)
+  from qwix_amd.core import qarray
+  n.setup(qarray.QArray, qarray.Int4Tensor, lambda device: 0, _lib.raise_status, 1)
+  try:
+    assert n.run(('outlives',)) is None
+    assert n.keep(('outlives',), (), [], [], [], rebuild)
+    del rebuild   # the table's is the only reference
+    assert n.run(('outlives',)) == 'done'
+    assert seen == [True] and alive() is None   # let go after the call, not under it
+    assert n.run(('outlives',)) is None
+  finally:
+    plans._native = None
+    plans.native()
 
 
 # ---- replay
