@@ -714,6 +714,11 @@ def quantize_with_scale_zero_point(array: torch.Tensor, qtype, scale: torch.Tens
   return QArray(view, scale, zero_point, q)
 
 
+def _tiles_key(tiled_axes) -> tuple:
+  """Tiles by their types too: 1 and 1.0 are one key to a dict, but one element and the whole axis to `_resolve_tile`."""
+  return tuple([(axis, tile, type(tile)) for axis, tile in tiled_axes.items()])
+
+
 def quantize(array: torch.Tensor, how: HowToQuantize, *, layout: str | None = None) -> QArray:
   """Dynamic-range quantization: calibrate, derive scale (and zero point), quantize -- one fused pass.  With a
   `noise_fn` (stochastic rounding) the three steps run one after the other, as the reference's do (qarray.py:638-644)."""
@@ -867,7 +872,7 @@ def quantize(array: torch.Tensor, how: HowToQuantize, *, layout: str | None = No
   `noise_fn` (stochastic rounding) the three steps run one after the other, as the reference's do (qarray.py:638-644)."""
   if how.noise_fn is not None:
     return _quantize_any(array, how, layout)
-  fixed = ('quantize', how.qtype, tuple(how.channelwise_axes), tuple(how.tiled_axes.items()), how.calibration_method, layout)
+  fixed = ('quantize', how.qtype, tuple(how.channelwise_axes), _tiles_key(how.tiled_axes), how.calibration_method, layout)
   out = (plans._native or plans.native()).run(fixed, array)
   if out is None:
     return _quantize_any(array, how, layout)
@@ -993,7 +998,7 @@ def quantize_api(array: torch.Tensor, qtype, *, channelwise_axes: Collection[int
   """Public `qwix.quantize`: like quantize() without building a HowToQuantize; the optional
   scale_dtype cast is applied to the already computed scale."""
   # (the same key as quantize(): without a plan the call goes there)
-  fixed = ('quantize', qtype, tuple(channelwise_axes), tuple(tiled_axes.items()) if tiled_axes else (), calibration_method, layout)
+  fixed = ('quantize', qtype, tuple(channelwise_axes), _tiles_key(tiled_axes) if tiled_axes else (), calibration_method, layout)
   qa = (plans._native or plans.native()).run(fixed, array)
   if qa is None or qa is True:
     how = HowToQuantize(qtype=qtype, channelwise_axes=channelwise_axes, tiled_axes=tiled_axes or {},

@@ -205,6 +205,20 @@ def test_replay_with_other_layouts_options_and_errors():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('first,second', [(1, 1.0), (1.0, 1)])
+def test_a_tile_of_one_element_is_not_the_whole_axis(first, second):
+  """1 == 1.0, but an integer is a size and a float a share of the axis: each has plans of its own."""
+  import qwix_amd
+  x = _rand((64, 72 if isinstance(first, float) else 80), 3)
+  for tile in (first, second):
+    how = qwix_amd.HowToQuantize(qtype='int8', channelwise_axes=[1], tiled_axes={0: tile})
+    want = qwix_amd.core.qarray._quantize_any(x, how, None)
+    for _ in range(plans.RECORD_AT + 2):
+      _same(qwix_amd.quantize(x, 'int8', channelwise_axes=[1], tiled_axes={0: tile}), want)
+      _same(qwix_amd.core.qarray.quantize(x, how), want)
+
+
+@pytest.mark.gpu
 def test_replay_on_threads_and_streams():
   import qwix_amd
   w = qwix_amd.quantize(_rand((512, 200), 1, std=0.05), 'int8', channelwise_axes=[1])
