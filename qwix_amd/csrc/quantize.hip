@@ -1512,6 +1512,12 @@ void launch_rows(const void* x, int64_t nseg, int64_t L, float factor, void* q, 
   constexpr int target = 4;  // 16-byte loads per thread
   int lg = log2_ceil((nvec + target - 1) / target);  // aim at `target` loads per thread, 8 at most
   while ((nvec + (1 << lg) - 1) >> lg > 8) ++lg;
+  // At least eight threads per segment: a group's loads then cover whole 128-byte lines and its nontemporal stores 64 bytes.
+  // With four threads (segments of 128 bf16 elements) a wavefront's stores fell into 32-byte pieces.  bf16 -> int8, at the
+  // operator, 4 / 8 / 16 threads: 65536 x 128 8.9 / 6.2 / 6.4 us, 4096 x 4096 in groups of 128 17.3 / 12.1 / 12.8, 8192 x 8192
+  // in groups of 64 43.3 / 39.1 / 38.7; groups of 256 have eight with `target` and lose with sixteen (10.4 / 11.2), each
+  // thread of a segment works out its scale.
+  while (lg < 3 && (1 << lg) < nvec) ++lg;
   if (lg > 8) lg = 8;
   const int64_t blocks = (nseg + (256 >> lg) - 1) / (256 >> lg);
   const int loads = (nvec + (1 << lg) - 1) >> lg;
@@ -1520,7 +1526,9 @@ void launch_rows(const void* x, int64_t nseg, int64_t L, float factor, void* q, 
   uint8_t* qb = static_cast<uint8_t*>(q);
   int8_t* zb = static_cast<int8_t*>(zp);
   const int sh = (per_scale & (per_scale - 1)) == 0 ? log2_ceil(per_scale) : -1;
-  if (loads <= 2)
+  if (loads <= 1)
+    rows_kernel<D, QT, CAL, MODE, 1><<<grid, 256, 0, st>>>(xb, nseg, nvec, lg, factor, qb, scale, zb, c0, c1, per_scale, sh);
+  else if (loads <= 2)
     rows_kernel<D, QT, CAL, MODE, 2><<<grid, 256, 0, st>>>(xb, nseg, nvec, lg, factor, qb, scale, zb, c0, c1, per_scale, sh);
   else if (loads <= 4)
     rows_kernel<D, QT, CAL, MODE, 4><<<grid, 256, 0, st>>>(xb, nseg, nvec, lg, factor, qb, scale, zb, c0, c1, per_scale, sh);

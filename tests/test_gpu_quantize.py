@@ -39,6 +39,15 @@ def test_rows_subchannel_tiles(dtype, qtype):
     _check(x_np, x_t, dtype, dict(qtype=qtype, channelwise_axes=[0], tiled_axes={1: tile}), what=f'rows tile {tile}')
 
 
+@pytest.mark.parametrize('calibration', ['absmax', 'minmax'])
+@pytest.mark.parametrize('dtype', [O.BF16, O.F32])
+@pytest.mark.parametrize('length', [8, 16, 24, 32, 40, 64, 72, 128, 136, 192, 256])
+def test_short_rows(length, dtype, calibration):
+  """One to eight threads and loads per segment, and rows that end inside a workgroup."""
+  x_np, x_t = util.make((133, length), dtype, seed=length)
+  _check(x_np, x_t, dtype, dict(qtype='int8', channelwise_axes=[0], calibration_method=calibration), what='short rows')
+
+
 @pytest.mark.parametrize('qtype', QTYPES)
 def test_every_bf16_value_rows(qtype):
   """All finite bf16 bit patterns, grouped so that rows span very different magnitudes."""
