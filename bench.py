@@ -860,7 +860,7 @@ class QdotBatched(Workload):
     self.dtype = 'int8'
     self.metric = 'batched int8 qdot GB/s (bqd,bkd->bqk, bf16 out)'
     self.unit = 'GB/s'
-    self.kernel_name = 'qgemm_batched_dma_kernel'
+    self.kernel_name = 'qgemm_strips_kernel'
 
   def setup(self, dev):
     import torch
