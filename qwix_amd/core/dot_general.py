@@ -461,6 +461,7 @@ def _weight_ksums(values_owner, b: torch.Tensor, key_extra: tuple, compute) -> t
   if hit is not None and hit[0]() is store and hit[1] == store._version:
     return hit[2]
   out = compute()
+  plans.kept_aside()
   _KSUM_CACHE[key] = (weakref.ref(store, lambda _, k=key: _KSUM_CACHE.pop(k, None)), store._version, out)
   return out
 
@@ -643,6 +644,7 @@ def _rhs_zero_point_i8(c: '_Canon', rhs: QArray) -> tuple[torch.Tensor, int]:
     return hit[2], hit[3]
   z32, gz = c.rhs_zero_point(rhs)
   zp = z32.to(torch.int8).contiguous()
+  plans.kept_aside()
   _ZP8_CACHE[key] = (weakref.ref(z, lambda _, k=key: _ZP8_CACHE.pop(k, None)), z._version, zp, gz)
   return zp, gz
 
@@ -736,6 +738,9 @@ def _decode_plan(lhs, rhs, dimension_numbers):
     b, b_is4 = c.rhs_values(rhs)
     sb, gb = c.rhs_scale(rhs)
     zp = _rhs_zero_point_i8(c, rhs)[0] if rhs.zero_point is not None else None
+    values = rhs.qvalue.data if b_is4 else rhs.qvalue
+    if any(kept.untyped_storage().data_ptr() != own.untyped_storage().data_ptr() for kept, own in ((b, values), (sb, rhs.scale))):
+      plans.kept_aside()
     plan = (b, numerics.qtype_tag(_qtype_of(rhs)), sb, _lib.float_tag(sb.dtype), zp, c.N, c.K, c.K // gb,
             fused_wq_min_rows(c.N, b_is4, c.K, c.K // gb))
   _DECODE_PLANS[key] = (weakref.ref(rhs, lambda _, k=key: _DECODE_PLANS.pop(k, None)),

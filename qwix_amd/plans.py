@@ -7,8 +7,9 @@ device).  `call` looks the operands' metadata up in a native table and replays t
 A plan is recorded when a kind of call comes up for the `RECORD_AT`-th time: the ordinary path runs once under a `Recorder`, which
 notes every allocation and every entry point call with its constants, and tells operands, buffers and constants apart.  A
 plan is kept only if that is all the path did: any other device operation of torch (a copy, a padding, a reduction), a pointer
-to memory that is neither an operand nor a buffer of this call (a re-laid-out weight kept from earlier), operands that
-overlap, or a result that is not one of the buffers leave the call to the ordinary path for good.
+to memory that is neither an operand nor a buffer of this call (a re-laid-out weight kept from earlier), work whose result
+is kept for later calls (`kept_aside`), operands that overlap, or a result that is not one of the buffers leave the call to
+the ordinary path for good.
 """
 from __future__ import annotations
 
@@ -139,6 +140,14 @@ class Recorder(TorchDispatchMode):
       else:
         return None
     return out
+
+
+def kept_aside() -> None:
+  """Called where an operator has just prepared something from a weight that it keeps and later calls read (a re-laid-out
+  copy, sums): a plan recorded around it would repeat the preparation on every replay."""
+  recorder = getattr(Recorder._active, 'recorder', None)
+  if recorder is not None:
+    recorder.ok = False
 
 
 def record(fixed, operands, fn, split):

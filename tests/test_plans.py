@@ -68,6 +68,78 @@ def test_recorder_refuses(what):
   assert not rec.ok
 
 
+class _StandIn:
+  """In place of the library: every entry point succeeds and writes nothing, no workspace is needed."""
+
+  def __getattr__(self, name):
+    return lambda *args: 0
+
+
+@pytest.fixture
+def stand_in(monkeypatch):
+  from qwix_amd.core import dot_general as dg
+  monkeypatch.setattr(_lib, 'load', _StandIn)
+  monkeypatch.setattr(_lib, 'stream_of', lambda t: 0)
+  yield
+  for cache in (dg._splitk_bytes, dg._dynamic_act_bytes):   # answers of the stand-in
+    cache.cache_clear()
+
+
+def _host_weight(qtype, k, n, layout, zero_point=False):
+  """A (k, n) weight in host memory, one scale per 128 rows and column."""
+  from qwix_amd.core.qarray import Int4Tensor, QArray
+  scale = torch.ones(k // 128, n, dtype=torch.bfloat16)
+  if qtype == 'int4':
+    data = torch.zeros(*((k, n // 2) if layout == 'natural' else (n, k // 2)), dtype=torch.uint8)
+    q = Int4Tensor(data, (k, n), 1) if layout == 'natural' else Int4Tensor(data.t(), (k, n), 0)
+  else:
+    q = torch.zeros(*((k, n) if layout == 'natural' else (n, k)), dtype=torch.int8)
+    q = q if layout == 'natural' else q.t()
+  return QArray(q, scale, torch.zeros(k // 128, n, dtype=torch.int8) if zero_point else None, qtype)
+
+
+def _parts(*operands):
+  from qwix_amd.core.qarray import Int4Tensor, QArray
+  out = []
+  for x in operands:
+    for t in ((x.qvalue, x.scale, x.zero_point) if isinstance(x, QArray) else (x,)):
+      if t is not None:
+        out.append(t.data if isinstance(t, Int4Tensor) else t)
+  return out
+
+
+@pytest.mark.parametrize('qtype', ['int8', 'int4'])
+def test_recorder_refuses_what_is_prepared_once_per_weight(stand_in, qtype):
+  """A weight in the natural layout is transposed at its first use and the copy is kept: a plan recorded at the first use of
+  yet another layer's weight would transpose every layer's weight on every call."""
+  from qwix_amd.core import dot_general as dg
+  x = torch.zeros(3, 256, dtype=torch.bfloat16)
+  for _ in range(4):
+    w = _host_weight(qtype, 256, 64, 'natural')
+    rec, _ = _recorded(lambda rec: dg._dot_general(x, w, _DN), *_parts(x, w))
+    assert not rec.ok
+  ready = _host_weight(qtype, 256, 64, 'reduce_minor')   # nothing to prepare
+  rec, _ = _recorded(lambda rec: dg._dot_general(x, ready, _DN), *_parts(x, ready))
+  assert rec.ok and [name for name, _ in rec.calls] == ['qwix_hip_gemv_wq']
+
+
+def test_recorder_refuses_sums_kept_per_weight(stand_in):
+  """The K-sums of a weight under an asymmetric activation are kept too."""
+  from qwix_amd.core import dot_general as dg
+  from qwix_amd.core.qarray import QArray
+  w = QArray(torch.zeros(64, 256, dtype=torch.int8).t(), torch.ones(1, 64, dtype=torch.bfloat16), None, 'int8')
+  recorded = []
+
+  def fn(rec):
+    def compute():
+      out = torch.empty(64, dtype=torch.int32)
+      _note(rec, w.qvalue, out)
+      return out
+    recorded.append(dg._weight_ksums(w.qvalue, w.qvalue, (), compute))
+  rec, _ = _recorded(fn, *_parts(w))
+  assert not rec.ok and len(rec.calls) == 1 and recorded[0] is not None
+
+
 # ---- the table
 
 
@@ -180,6 +252,27 @@ def test_replay_equals_the_ordinary_path(name):
     assert not calls, 'no plan is kept for this kind of call'
   finally:
     _lib.call = call
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('qtype', ['int8', 'int4'])
+def test_layers_of_one_shape_are_laid_out_once_each(monkeypatch, qtype):
+  """More weights of one shape than calls up to the recorded one, in the natural layout: each is transposed at its first use
+  and never again."""
+  import qwix_amd
+  from qwix_amd.core import dot_general as dg
+  ws = [qwix_amd.quantize(_rand((512, 200), s, std=0.05), qtype, channelwise_axes=[1], tiled_axes={0: 128}, layout='natural')
+        for s in range(plans.RECORD_AT + 2)]
+  names, call = [], _lib.call
+  monkeypatch.setattr(_lib, 'call', lambda *a: names.append(a[0]) or call(*a))
+  for turn in range(4):
+    names.clear()
+    x = _rand((5, 512), turn)
+    outs = [qwix_amd.dot_general(x, w, _DN) for w in ws]
+    assert names.count('qwix_hip_transpose_q') == (len(ws) if turn == 0 else 0), names
+    assert names.count('qwix_hip_gemv_wq') == len(ws)   # (a replayed plan is not seen here)
+    for out, w in zip(outs, ws):
+      _same(out, dg._dot_general(x, w, _DN))
 
 
 @pytest.mark.gpu
