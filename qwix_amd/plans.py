@@ -47,12 +47,21 @@ def native():
   return _native
 
 
-# (and what works on dtypes alone)
-_VIEWS = frozenset((
-    'aten::view', 'aten::_unsafe_view', 'aten::permute', 'aten::transpose.int', 'aten::t', 'aten::expand', 'aten::as_strided',
-    'aten::select.int', 'aten::slice.Tensor', 'aten::unsqueeze', 'aten::squeeze', 'aten::squeeze.dim', 'aten::squeeze.dims',
-    'aten::alias', 'aten::detach', 'aten::promote_types', 'aten::view.dtype', 'aten::_reshape_alias', 'aten::split.Tensor', 'aten::unbind.int'))
 _ALLOCATIONS = frozenset(('aten::empty.memory_format', 'aten::empty_strided', 'aten::empty_like', 'aten::new_empty'))
+
+
+def _storages(values) -> set:
+  return {t.untyped_storage().data_ptr() for v in values for t in (v if isinstance(v, (list, tuple)) else (v,))
+          if isinstance(t, torch.Tensor)}
+
+
+def _is_view(func, args, out) -> bool:
+  """Whether an operation did nothing on the device: it writes to none of its arguments and all it returns are tensors in an
+  argument's memory.  (Told by the effect: `reshape`, `contiguous` and `to` are views or copies, and reach the recorder by
+  these names in inference mode, where torch does not take them apart before.)"""
+  outs = out if isinstance(out, (list, tuple)) else (out,)
+  return (not func._schema.is_mutable and all(isinstance(t, torch.Tensor) for t in outs)
+          and _storages(outs) <= _storages(args))
 
 
 def _extent(t: torch.Tensor) -> tuple[int, int]:
@@ -92,7 +101,7 @@ class Recorder(TorchDispatchMode):
     name = func._schema.name + ('.' + func._schema.overload_name if func._schema.overload_name else '')
     if name in _ALLOCATIONS:
       self.buffers.append(out)
-    elif name not in _VIEWS:
+    elif name != 'aten::promote_types' and not _is_view(func, args, out):   # (that one works on dtypes alone)
       self.ok = False
     return out
 

@@ -43,8 +43,14 @@ def test_recorder_tells_operands_buffers_and_constants_apart():
   assert rec.results((torch.zeros(3),)) is None   # not a buffer of the call
 
 
-@pytest.mark.parametrize('what', ['copy', 'fill', 'reduction', 'foreign pointer', 'overlapping operands', 'item'])
-def test_recorder_refuses(what):
+@pytest.mark.parametrize('inference', [False, True])
+@pytest.mark.parametrize('what', ['copy', 'reshape', 'conversion', 'fill', 'reduction', 'foreign pointer', 'overlapping operands', 'item'])
+def test_recorder_refuses(what, inference):
+  with torch.inference_mode(inference):
+    _check_refused(what)
+
+
+def _check_refused(what):
   q = torch.zeros(8, 64, dtype=torch.int8)
   kept = torch.zeros(64, 8, dtype=torch.int8)
   second = q[2:] if what == 'overlapping operands' else torch.zeros(1, dtype=torch.int8)
@@ -53,6 +59,10 @@ def test_recorder_refuses(what):
     out = torch.empty(4, dtype=torch.int32)
     if what == 'copy':
       _note(rec, q.t().contiguous(), out)
+    elif what == 'reshape':
+      _note(rec, q.t().reshape(-1), out)
+    elif what == 'conversion':
+      _note(rec, q.to(torch.int32), out)
     elif what == 'foreign pointer':
       _note(rec, kept, out)
     else:
@@ -66,6 +76,21 @@ def test_recorder_refuses(what):
     return out
   rec, _ = _recorded(fn, q, second)
   assert not rec.ok
+
+
+@pytest.mark.parametrize('inference', [False, True])
+def test_recorder_takes_views_by_their_effect(inference):
+  """Operations that may copy and do not here; inference mode hands them to the recorder whole."""
+  with torch.inference_mode(inference):
+    q = torch.zeros(8, 64, dtype=torch.int8)
+
+    def fn(rec):
+      out = torch.empty(4, 2, dtype=torch.int32)
+      _note(rec, q.contiguous().to(torch.int8).reshape(4, 128).unbind(0)[1].expand(2, 128).narrow(0, 0, 1).flatten(), out)
+      return out.reshape(8).view(2, 4)
+    rec, out = _recorded(fn, q)
+    assert rec.ok and rec.calls[0][1][0] == (plans._OPERAND, 0, 128)
+    assert rec.results((out,)) == [(0, (2, 4), (4, 1), 0)]
 
 
 class _StandIn:
@@ -143,14 +168,18 @@ def test_recorder_refuses_sums_kept_per_weight(stand_in):
 # ---- the table
 
 
+def _empty_the_table():
+  for k in range(9000):   # more signatures than are remembered
+    plans.native().run(('filler', k))
+
+
 def test_a_plan_in_use_outlives_a_table_that_starts_anew():
   """`rebuild` is Python: what it runs, or another thread meanwhile, may fill the table until it is emptied."""
   n = plans.native()
   seen = []
 
   def fill(value):
-    for k in range(9000):   # more signatures than are remembered
-      n.run(('filler', k))
+    _empty_the_table()
     seen.append(alive() is not None)
     return value
   rebuild = functools.partial(fill, 'done')
@@ -236,19 +265,23 @@ _NAMES = (['%s %s %s' % (w, q, m) for w in ('rows', 'columns', 'dequantize')
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('inference', [False, True])
 @pytest.mark.parametrize('name', _NAMES)
-def test_replay_equals_the_ordinary_path(name):
+def test_replay_equals_the_ordinary_path(name, inference):
   """New operands (other data, other addresses) on every call: the first ones go the ordinary way, the others replay."""
+  _empty_the_table()   # (what the other mode recorded)
   make, op, ordinary = _cases()[name]
   alive = []
   for seed in range(plans.RECORD_AT + 2):
     operands = make(10 * seed)
     alive.append(operands)   # no address comes up twice
-    _same(op(*operands), ordinary(*operands))
+    with torch.inference_mode(inference):   # (the weights are older than a server's inference mode)
+      _same(op(*operands), ordinary(*operands))
   calls = []
   call, _lib.call = _lib.call, lambda *a: calls.append(a[0]) or call(*a)
   try:
-    _same(op(*alive[0]), op(*alive[0]))
+    with torch.inference_mode(inference):
+      _same(op(*alive[0]), op(*alive[0]))
     assert not calls, 'no plan is kept for this kind of call'
   finally:
     _lib.call = call
