@@ -7,7 +7,8 @@
 // nothing here is keyed by the address or the identity of an operand, and nothing outlives a call but the plan.
 //   run(fixed, *operands): the signature is the fixed part (a hashable Python object with the options) and, per
 // operand, dtype, device, shape, strides and the alignment of its memory.
-//   Thread safety: the interpreter lock is held throughout.
+//   Thread safety: the table is only touched under the interpreter lock; allocations and launches run without it, on a plan
+// that the call holds a reference to.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -198,35 +199,52 @@ Seen* lookup(Cache& c, PyObject* fixed, const std::string& signature, uint64_t h
   return nullptr;
 }
 
-PyObject* run_plan(const Plan& p, const Operands& ops) {
-  at::Tensor buffers[16];
-  const size_t nb = p.buffers.size();
-  for (size_t k = 0; k < nb; ++k) {
+// The interpreter lock let go for a scope: allocations can wait for the device and launches for room in its queue, and other
+// threads (a host callback that a stream waits for among them) must be able to run meanwhile.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// Allocates and launches; no Python inside.  Returns a refused call's entry point and status, or {nullptr, 0}.
+std::pair<const EntryPoint*, int> carry_out(const Plan& p, void* const* operands, void* stream, at::Tensor* buffers) {
+  const Unlocked unlocked;
+  for (size_t k = 0; k < p.buffers.size(); ++k) {
     const Buffer& b = p.buffers[k];
     buffers[k] = b.contiguous ? at::empty(b.sizes, b.options) : at::empty_strided(b.sizes, b.strides, b.options);
   }
+  for (const Call& c : p.calls) {
+    Slot slots[kMaxArgs];
+    for (size_t k = 0; k < c.args.size(); ++k) {
+      const Arg& a = c.args[k];
+      switch (a.kind) {
+        case kOperand: slots[k].p = static_cast<char*>(operands[a.index]) + a.value.i; break;
+        case kBuffer: slots[k].p = static_cast<char*>(buffers[a.index].data_ptr()) + a.value.i; break;
+        case kStream: slots[k].p = stream; break;
+        default: slots[k] = a.value;
+      }
+    }
+    if (const int status = c.entry->call(slots)) return {c.entry, status};
+  }
+  return {nullptr, 0};
+}
+
+PyObject* run_plan(const Plan& p, const Operands& ops) {
   PyObject* index = PyLong_FromLong(p.device);
   PyObject* handle = PyObject_CallOneArg(g_stream, index);
   Py_DECREF(index);
   if (handle == nullptr) return nullptr;
   void* stream = reinterpret_cast<void*>(static_cast<intptr_t>(PyLong_AsLongLong(handle)));
   Py_DECREF(handle);
-  for (const Call& c : p.calls) {
-    Slot slots[kMaxArgs];
-    for (size_t k = 0; k < c.args.size(); ++k) {
-      const Arg& a = c.args[k];
-      switch (a.kind) {
-        case kOperand: slots[k].p = static_cast<char*>(ops.tensors[a.index]->data_ptr()) + a.value.i; break;
-        case kBuffer: slots[k].p = static_cast<char*>(buffers[a.index].data_ptr()) + a.value.i; break;
-        case kStream: slots[k].p = stream; break;
-        default: slots[k] = a.value;
-      }
-    }
-    if (const int status = c.entry->call(slots)) {
-      PyObject* r = PyObject_CallFunction(g_fail, "si", c.entry->name, status);  // raises
-      Py_XDECREF(r);
-      return nullptr;
-    }
+  // (the operands' objects are held by the caller and by `ops`; their addresses are read under the lock)
+  std::vector<void*> operands;
+  for (const at::Tensor* t : ops.tensors) operands.push_back(t->data_ptr());
+  at::Tensor buffers[16];
+  const auto [refused, status] = carry_out(p, operands.data(), stream, buffers);
+  if (refused != nullptr) {
+    PyObject* r = PyObject_CallFunction(g_fail, "si", refused->name, status);  // raises
+    Py_XDECREF(r);
+    return nullptr;
   }
   auto result = [&](const Result& r) -> PyObject* {
     at::Tensor& b = buffers[r.buffer];

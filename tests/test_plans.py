@@ -1,5 +1,7 @@
 """Launch plans: what the recorder accepts (CPU), and that replayed calls give what the ordinary path gives (GPU)."""
+import _thread
 import functools
+import sys
 import threading
 import weakref
 
@@ -194,6 +196,29 @@ def test_a_plan_in_use_outlives_a_table_that_starts_anew():
     assert seen == [True] and alive() is None   # let go after the call, not under it
     assert n.run(('outlives',)) is None
   finally:
+    plans._native = None
+    plans.native()
+
+
+def test_a_replay_lets_other_threads_run():
+  """Allocations can wait for the device and launches for room in its queue: a replay does both without the interpreter lock.
+  With a switch interval longer than the test another thread runs only when the lock is let go."""
+  from qwix_amd.core import qarray
+  n = plans.native()
+  n.setup(qarray.QArray, qarray.Int4Tensor, lambda device: 0, _lib.raise_status, 1)
+  interval = sys.getswitchinterval()
+  ran, alive = [], []   # (results stay: torch lets the lock go where a tensor dies)
+  size = 1 << 20   # a mapping of its own, never touched: the allocation takes a while
+  try:
+    assert n.run(('unlocked',)) is None
+    assert n.keep(('unlocked',), (), [((size,), (1,), torch.empty(1, dtype=torch.uint8))], [], [(0, (size,), (1,), 0)], None)
+    sys.setswitchinterval(1000.0)
+    _thread.start_new_thread(ran.append, (True,))   # (does not wait for the thread to run)
+    while not ran and len(alive) < 5000:
+      alive.append(n.run(('unlocked',)))
+    assert ran
+  finally:
+    sys.setswitchinterval(interval)
     plans._native = None
     plans.native()
 
