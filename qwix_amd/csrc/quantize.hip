@@ -1328,12 +1328,12 @@ __global__ void __launch_bounds__(256)
 // bf16 236 -> 154 us (4.6 TB/s), 4096 x 14336 59 -> 31, against tiles of 64 x 64 turned byte by byte.
 template <typename D, int QT>
 __global__ void __launch_bounds__(256)
-    dequant_rm_kernel(const uint8_t* __restrict__ q, int64_t reduce, int64_t inner, int64_t tile,
+    dequant_rm_kernel(const uint8_t* __restrict__ q, int64_t reduce, int64_t inner, int64_t tile, int64_t tile0,
                       const void* __restrict__ scale, const int8_t* __restrict__ zp, void* __restrict__ out) {
   constexpr int EPB = QT == QWIX_INT4 ? 2 : 1, KT = 128 * EPB;  // values per byte, rows of the output per tile
   constexpr int PITCH = 144;
   __shared__ __attribute__((aligned(16))) uint8_t lines[128 * PITCH];
-  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * KT, i0 = static_cast<int64_t>(blockIdx.x) * 128;
+  const int64_t r0 = (tile0 + blockIdx.y) * KT, i0 = static_cast<int64_t>(blockIdx.x) * 128;
   const int64_t o = blockIdx.z;
   const int tid = threadIdx.x;
   const int64_t row_bytes = reduce / EPB, b0 = r0 / EPB;  // reduce % 8 == 0
@@ -1982,17 +1982,21 @@ int qwix_hip_dequantize(const void* qvalue, int qtype, int q_layout, int64_t out
 #undef QWIX_DEQ_VEC
     return check_launch("dequantize");
   }
-  if (!natural && ptr_ok && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 <= 65535) {
+  if (!natural && ptr_ok && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 < (1 << 23)) {
     const int kt = qtype == QWIX_INT4 ? 256 : 128;
-    const dim3 grid(static_cast<unsigned>((inner + 127) / 128), static_cast<unsigned>((reduce + kt - 1) / kt),
-                    static_cast<unsigned>(outer));
-#define QWIX_DEQ_RM(QTT) dequant_rm_kernel<D, QTT><<<grid, 256, 0, st>>>(q, reduce, inner, tile, scale, zp, out)
-    QWIX_DISPATCH_D(dtype, {
-      if (qtype == QWIX_INT8) QWIX_DEQ_RM(QWIX_INT8);
-      else if (qtype == QWIX_INT4) QWIX_DEQ_RM(QWIX_INT4);
-      else if (qtype == QWIX_E4M3) QWIX_DEQ_RM(QWIX_E4M3);
-      else return fail(QWIX_ERR_INVALID_ARGUMENT, "unknown qtype %d", qtype);
-    })
+    const int64_t tiles = (reduce + kt - 1) / kt;
+    // grid y and z end at 65535, x at 2^31 threads: longer reduced axes take several launches
+    for (int64_t t0 = 0; t0 < tiles; t0 += 65535) {
+      const dim3 grid(static_cast<unsigned>((inner + 127) / 128), static_cast<unsigned>(std::min<int64_t>(tiles - t0, 65535)),
+                      static_cast<unsigned>(outer));
+#define QWIX_DEQ_RM(QTT) dequant_rm_kernel<D, QTT><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out)
+      QWIX_DISPATCH_D(dtype, {
+        if (qtype == QWIX_INT8) QWIX_DEQ_RM(QWIX_INT8);
+        else if (qtype == QWIX_INT4) QWIX_DEQ_RM(QWIX_INT4);
+        else if (qtype == QWIX_E4M3) QWIX_DEQ_RM(QWIX_E4M3);
+        else return fail(QWIX_ERR_INVALID_ARGUMENT, "unknown qtype %d", qtype);
+      })
+    }
 #undef QWIX_DEQ_RM
     return check_launch("dequantize");
   }

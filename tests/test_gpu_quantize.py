@@ -499,3 +499,21 @@ def test_weight_columns_and_back_at_tile_edges(K, N, tile, dtype, qtype, method)
   qa = _check(x_np, x_t, dtype, kw, layout='reduce_minor', what='column blocks')
   want = O.dequantize(O.quantize(O.FArr(x_np, dtype), O.HowToQuantize(**kw)))
   assert np.array_equal(util.f32np(qarray.dequantize(qa)), want.v)
+
+
+@pytest.mark.parametrize('qtype,reduce,inner', [('int8', 65535 * 128 + 264, 16), ('int4', 65535 * 256 + 264, 8), ('int8', 24, 65535 * 128 + 264)])
+def test_dequantize_reduce_minor_beyond_one_grid(qtype, reduce, inner):
+  """K-contiguous values with more tiles along the reduced axis than a grid has blocks there, and the same of columns."""
+  from qwix_amd.core import qarray
+  print('case', qtype, reduce, inner, flush=True)
+  g = torch.Generator(device=util.DEV).manual_seed(reduce)
+  codes = torch.randint(0, 256, (inner, reduce // 2 if qtype == 'int4' else reduce), dtype=torch.uint8, device=util.DEV, generator=g)
+  scale = torch.rand(reduce // 24, inner, device=util.DEV, generator=g).to(torch.bfloat16)
+  q = qarray.Int4Tensor(codes.t(), (reduce, inner), 0) if qtype == 'int4' else codes.view(torch.int8).t()
+  got = qarray.dequantize(qarray.QArray(q, scale, None, qtype))
+  for c in range(0, inner, 1 << 20):   # codes and scales are exact in f32, one rounding
+    cols = slice(c, c + (1 << 20))
+    v = codes[cols]
+    v = torch.stack((v << 4, v), dim=2).view(torch.int8).reshape(v.shape[0], reduce) >> 4 if qtype == 'int4' else v.view(torch.int8)
+    want = v.t().float().reshape(reduce // 24, 24, -1) * scale[:, None, cols].float()
+    assert torch.equal(got[:, cols], want.reshape(reduce, -1).to(torch.bfloat16))
