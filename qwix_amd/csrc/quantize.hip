@@ -1318,36 +1318,41 @@ __global__ void __launch_bounds__(256)
   else store1<D>(out, idx, v[0]);
 }
 
-// Reduce-minor layout (values stored (outer, inner, reduce), output (outer, reduce, inner)): tiles of 128 columns (i) x one
-// 128-byte line of packed values per column.  Bound by memory: whole lines come in, 256-byte row pieces leave (bf16), and
-// nothing is turned byte by byte: the lines go to LDS as they are, a thread reads the same dword of eight columns and
-// converts its bytes (nibbles) in place, which yields eight consecutive outputs per row.  Chunk c of column i sits at
+// Reduce-minor layout (values stored (outer, inner, reduce), output (outer, reduce, inner)): tiles of 128 columns (i) x LB
+// bytes of packed values per column.  Bound by memory: whole lines come in (LB 128), 256-byte row pieces leave (bf16), and
+// nothing is turned byte by byte: the lines go to LDS as they are, a thread reads the same dword of CPT columns and
+// converts its bytes (nibbles) in place, which yields CPT consecutive outputs per row.  LB 128: chunk c of column i sits at
 // c ^ ((i >> 4) & 7) at a pitch of 144 bytes, so that those dword reads fall into 64 different banks.  Consecutive blocks
 // take consecutive columns: along the rows instead, blocks that run together write rows a power of two apart for such
 // widths (8192 x 8192, int4 / int8: 32 / 36 us against 45 / 46; 8192 x 28672 e4m3: 154 against 146).  8192 x 28672 e4m3 to
 // bf16 236 -> 154 us (4.6 TB/s), 4096 x 14336 59 -> 31, against tiles of 64 x 64 turned byte by byte.
-template <typename D, int QT>
+//   Small arrays are bound by the latency of one block's load - convert - store chain instead: LB 32 gives each thread a
+// quarter of the work and the chip four times the blocks.  Where the line between the two lies: at the dispatch.
+template <typename D, int QT, int LB>
 __global__ void __launch_bounds__(256)
     dequant_rm_kernel(const uint8_t* __restrict__ q, int64_t reduce, int64_t inner, int64_t tile, int64_t tile0,
                       const void* __restrict__ scale, const int8_t* __restrict__ zp, void* __restrict__ out) {
-  constexpr int EPB = QT == QWIX_INT4 ? 2 : 1, KT = 128 * EPB;  // values per byte, rows of the output per tile
-  constexpr int PITCH = 144;
+  constexpr int EPB = QT == QWIX_INT4 ? 2 : 1, KT = LB * EPB;  // values per byte, rows of the output per tile
+  constexpr int CPT = LB == 128 ? 8 : 4;                       // columns per thread
+  constexpr int CGS = 128 / CPT, DSTEP = 256 / CGS, ITS = LB / 4 / DSTEP;
+  constexpr int PITCH = LB + 16, CHUNKS = LB / 16;
   __shared__ __attribute__((aligned(16))) uint8_t lines[128 * PITCH];
   const int64_t r0 = (tile0 + blockIdx.y) * KT, i0 = static_cast<int64_t>(blockIdx.x) * 128;
   const int64_t o = blockIdx.z;
   const int tid = threadIdx.x;
   const int64_t row_bytes = reduce / EPB, b0 = r0 / EPB;  // reduce % 8 == 0
-  auto at = [](int col, int byte) { return col * PITCH + (((byte >> 4) ^ ((col >> 4) & 7)) << 4) + (byte & 15); };
-  if (i0 + 128 <= inner && b0 + 128 <= row_bytes && row_bytes % 16 == 0) {
-    uint4 v[4];
-    const uint8_t* src = q + (o * inner + i0 + (tid >> 3)) * row_bytes + b0 + (tid & 7) * 16;
+  auto at = [](int col, int byte) { return col * PITCH + (((byte >> 4) ^ ((col >> 4) & (CHUNKS - 1))) << 4) + (byte & 15); };
+  if (i0 + 128 <= inner && b0 + LB <= row_bytes && row_bytes % 16 == 0) {
+    constexpr int LOADS = 128 * CHUNKS / 256, CSTEP = 256 / CHUNKS;
+    uint4 v[LOADS];
+    const uint8_t* src = q + (o * inner + i0 + tid / CHUNKS) * row_bytes + b0 + (tid % CHUNKS) * 16;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const uint4*>(src + j * 32 * row_bytes);
+    for (int j = 0; j < LOADS; ++j) v[j] = *reinterpret_cast<const uint4*>(src + j * CSTEP * row_bytes);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(lines + at((tid >> 3) + j * 32, (tid & 7) * 16)) = v[j];
+    for (int j = 0; j < LOADS; ++j) *reinterpret_cast<uint4*>(lines + at(tid / CHUNKS + j * CSTEP, (tid % CHUNKS) * 16)) = v[j];
   } else {
-    for (int e = tid; e < 128 * 32; e += 256) {  // a dword each
-      const int col = e >> 5, byte = (e & 31) * 4;
+    for (int e = tid; e < 128 * (LB / 4); e += 256) {  // a dword each
+      const int col = e / (LB / 4), byte = (e % (LB / 4)) * 4;
       uint32_t w = 0;
       if (i0 + col < inner && b0 + byte < row_bytes)
         w = *reinterpret_cast<const uint32_t*>(q + (o * inner + i0 + col) * row_bytes + b0 + byte);
@@ -1355,41 +1360,41 @@ __global__ void __launch_bounds__(256)
     }
   }
   __syncthreads();
-  const int cg = tid & 15;                // columns i0 + 8 cg ..
-  const int64_t i = i0 + cg * 8;
+  const int cg = tid % CGS;               // columns i0 + CPT cg ..
+  const int64_t i = i0 + cg * CPT;
   if (i >= inner) return;
-  const int left = static_cast<int>(min(static_cast<int64_t>(8), inner - i));
-  const bool vec = left == 8 && inner % D::kVec == 0;
+  const int left = static_cast<int>(min(static_cast<int64_t>(CPT), inner - i));
+  const bool vec = left == CPT && inner % (CPT < D::kVec ? CPT : D::kVec) == 0;
   int64_t have = -1;
-  float s[8], off[8];
+  float s[CPT], off[CPT];
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int d = (tid >> 4) + it * 16;   // dword of the line: 4 or 8 rows, all in one scale group (tile % 8 == 0)
+  for (int it = 0; it < ITS; ++it) {
+    const int d = tid / CGS + it * DSTEP;  // dword of the line: 4 or 8 rows, all in one scale group (tile % 8 == 0)
     const int64_t r = r0 + d * 4 * EPB;
     if (r >= reduce) break;
     const int64_t si = (o * (reduce / tile) + r / tile) * inner + i;
     if (si != have) {
       have = si;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < CPT; ++e) {
         s[e] = e < left ? load1<D>(scale, si + e) : 0.f;
         // what the offset-binary byte / nibble carries too much, zero point included; integers, exact in every type here
         off[e] = QT == QWIX_INT8 ? 128.f : QT == QWIX_INT4 ? 8.f : 0.f;
         if (zp != nullptr && e < left) off[e] += static_cast<float>(zp[si + e]);
       }
     }
-    uint32_t w[8];
+    uint32_t w[CPT];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      w[e] = *reinterpret_cast<const uint32_t*>(lines + at(cg * 8 + e, d * 4));
+    for (int e = 0; e < CPT; ++e) {
+      w[e] = *reinterpret_cast<const uint32_t*>(lines + at(cg * CPT + e, d * 4));
       if constexpr (QT == QWIX_INT8) w[e] ^= 0x80808080u;
       if constexpr (QT == QWIX_INT4) w[e] ^= 0x88888888u;
     }
 #pragma unroll
     for (int k = 0; k < 4 * EPB; ++k) {
-      float v[8];
+      float v[CPT];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < CPT; ++e) {
         float x;
         if constexpr (QT == QWIX_E4M3) {
           x = e4m3_to_f32(w[e] >> (8 * k));
@@ -1403,14 +1408,18 @@ __global__ void __launch_bounds__(256)
       }
       const int64_t oi = (o * reduce + r + k) * inner + i;
       if (vec) {
-        if constexpr (D::kTag == QWIX_BF16)
+        if constexpr (D::kTag == QWIX_BF16 && CPT == 8)
           nt_store16(reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + oi),
                      make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])));
-        else
+        else if constexpr (D::kTag == QWIX_BF16)
+          *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + oi) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        else if constexpr (CPT == 8)
           store8<D>(out, oi, v);
+        else
+          *reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + oi) = make_float4(v[0], v[1], v[2], v[3]);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < CPT; ++e)
           if (e < left) store1<D>(out, oi + e, v[e]);
       }
     }
@@ -1982,18 +1991,28 @@ int qwix_hip_dequantize(const void* qvalue, int qtype, int q_layout, int64_t out
 #undef QWIX_DEQ_VEC
     return check_launch("dequantize");
   }
-  if (!natural && ptr_ok && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 < (1 << 23)) {
-    const int kt = qtype == QWIX_INT4 ? 256 : 128;
+  // Reduce-minor, bf16 / f32 results of int8 codes in us, tiles of 64 x 64 turned byte by byte (before) / lines of 128 bytes /
+  // lines of 32 bytes / one thread per element:
+  //   256 x 256 3.2 4.2 3.0 2.6 / 3.4 4.8 2.9 2.6, 512 x 512 3.3 4.2 3.1 3.4 / 3.6 4.8 3.1 3.4: an element per thread below that;
+  //   1024 x 1024 3.6 4.4 3.3 6.0 / 4.4 5.6 3.7 6.2, 2048 x 2048 (256 tiles) 6.1 4.8 4.8 / 10.3 9.5 7.3;
+  //   1024 x 8192 (512 tiles) 9.9 5.5 7.3 / 17.1 14.4 11.8, 8192 x 8192 77 36 35 / 169 103 84, 8192 x 28672 235 112 192 /
+  //   381 362 308: lines of 32 bytes up to 256 tiles, and always for f32, whose 4-column pieces are full 16-byte stores.
+  // (int4 and e4m3 cross at the same sizes.)
+  if (!natural && ptr_ok && n >= (1 << 18) && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 < (1 << 23)) {
+    const bool narrow = dtype == QWIX_F32 || outer * ((reduce + 127) / 128) * ((inner + 127) / 128) <= 256;
+    const int kt = (narrow ? 32 : 128) * (qtype == QWIX_INT4 ? 2 : 1);
     const int64_t tiles = (reduce + kt - 1) / kt;
     // grid y and z end at 65535, x at 2^31 threads: longer reduced axes take several launches
     for (int64_t t0 = 0; t0 < tiles; t0 += 65535) {
       const dim3 grid(static_cast<unsigned>((inner + 127) / 128), static_cast<unsigned>(std::min<int64_t>(tiles - t0, 65535)),
                       static_cast<unsigned>(outer));
-#define QWIX_DEQ_RM(QTT) dequant_rm_kernel<D, QTT><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out)
+#define QWIX_DEQ_RM(QTT)                                                                                             \
+  if (narrow) dequant_rm_kernel<D, QTT, 32><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out);      \
+  else dequant_rm_kernel<D, QTT, 128><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out)
       QWIX_DISPATCH_D(dtype, {
-        if (qtype == QWIX_INT8) QWIX_DEQ_RM(QWIX_INT8);
-        else if (qtype == QWIX_INT4) QWIX_DEQ_RM(QWIX_INT4);
-        else if (qtype == QWIX_E4M3) QWIX_DEQ_RM(QWIX_E4M3);
+        if (qtype == QWIX_INT8) { QWIX_DEQ_RM(QWIX_INT8); }
+        else if (qtype == QWIX_INT4) { QWIX_DEQ_RM(QWIX_INT4); }
+        else if (qtype == QWIX_E4M3) { QWIX_DEQ_RM(QWIX_E4M3); }
         else return fail(QWIX_ERR_INVALID_ARGUMENT, "unknown qtype %d", qtype);
       })
     }

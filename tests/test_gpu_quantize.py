@@ -517,3 +517,26 @@ def test_dequantize_reduce_minor_beyond_one_grid(qtype, reduce, inner):
     v = torch.stack((v << 4, v), dim=2).view(torch.int8).reshape(v.shape[0], reduce) >> 4 if qtype == 'int4' else v.view(torch.int8)
     want = v.t().float().reshape(reduce // 24, 24, -1) * scale[:, None, cols].float()
     assert torch.equal(got[:, cols], want.reshape(reduce, -1).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize('qtype,method', [('int8', 'absmax'), ('int8', 'minmax'), ('int4', 'absmax'), ('int4', 'minmax'),
+                                          ('float8_e4m3fn', 'absmax')])
+@pytest.mark.parametrize('dtype', [O.BF16, O.F32])
+@pytest.mark.parametrize('shape', [(504, 520), (512, 512), (1032, 1000), (264, 1030), (2, 520, 304), (2064, 2184)])
+def test_dequantize_reduce_minor_by_size(shape, dtype, qtype, method):
+  """K-contiguous values on both sides of 2^18 elements and of 256 tiles of 128 x 128, with rows, columns and lines that end
+  inside a tile, bit for bit: codes, zero points and products are exact or rounded once."""
+  from qwix_amd.core import qarray
+  print('case', shape, dtype, qtype, method, flush=True)
+  kw = dict(qtype=qtype, channelwise_axes=[a for a in range(len(shape)) if a != len(shape) - 2], tiled_axes={len(shape) - 2: 8},
+            calibration_method=method)
+  if dtype == O.BF16 and shape[-1] % 8 or shape[-1] % 4:   # such widths are quantized in the natural layout
+    x_np, x_t = util.make((shape[1], shape[0]), dtype, seed=sum(shape))
+    kw.update(channelwise_axes=[0], tiled_axes={1: 8})
+    turned = lambda a: a.transpose(1, 0)
+  else:
+    x_np, x_t = util.make(shape, dtype, seed=sum(shape))
+    turned = lambda a: a
+  qa = turned(qarray.quantize(x_t, qarray.HowToQuantize(**kw)))
+  want = turned(O.dequantize(O.quantize(O.FArr(x_np, dtype), O.HowToQuantize(**kw))).v)
+  assert np.array_equal(util.f32np(qarray.dequantize(qa)), want)
