@@ -88,8 +88,17 @@ __device__ __forceinline__ uint8_t q_byte(float v) {  // one value -> one byte (
 // nseg segments of L = nvec * kVec contiguous elements.  log2g: threads per segment; NL: 16-byte
 // loads per thread.  The segment stays in registers in its packed form between the reduction and the
 // quantization (the empty asm keeps the compiler from re-issuing the loads instead), so HBM is read
-// exactly once.  bf16 absmax runs on the packed halves: |x| ordered like its 15 low bits.
+// exactly once.  bf16 absmax runs on the packed halves.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// |x| of a bf16 pair as two signed 16-bit keys that order like the values, NaN below all of them: a maximum of keys leaves NaN
+// out, as fmaxf does.  (|x| has 15 bits and infinity is 0x7F80, so adding 0x7F turns exactly the NaNs negative.)
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+constexpr short kKeyOfZero = 0x7F;
+__device__ __forceinline__ s16x2 abs_keys(uint32_t pair) {
+  return __builtin_bit_cast(s16x2, (pair & 0x7FFF7FFFu) + 0x007F007Fu);
+}
+__device__ __forceinline__ float key_value(short key) { return bf16_bits_to_f32(static_cast<uint16_t>(key - kKeyOfZero)); }
 
 template <typename D, int QT, int CAL, int MODE, int NL>
 __global__ void __launch_bounds__(256)
@@ -121,14 +130,14 @@ __global__ void __launch_bounds__(256)
   if constexpr (MODE != MODE_GIVEN) {
     float mx = 0.f, mn = 0.f;  // minmax clips to include 0; absmax >= 0
     if constexpr (!ASYM && D::kTag == QWIX_BF16) {
-      u16x2 m = {0, 0};
+      s16x2 m = {kKeyOfZero, kKeyOfZero};
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
         const uint32_t w[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[e] & 0x7FFF7FFFu));
+        for (int e = 0; e < 4; ++e) m = __builtin_elementwise_max(m, abs_keys(w[e]));
       }
-      mx = bf16_bits_to_f32(m[0] > m[1] ? m[0] : m[1]);
+      mx = key_value(m[0] > m[1] ? m[0] : m[1]);
     } else {
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
@@ -423,7 +432,7 @@ __global__ void __launch_bounds__(256)
                             uint32_t* __restrict__ ws) {
   constexpr int EV = D::kVec;
   constexpr bool ASYM = (CAL == QWIX_MINMAX);
-  constexpr bool PACKED = !ASYM && D::kTag == QWIX_BF16;  // |x| of a bf16 pair orders like its low 15 bits
+  constexpr bool PACKED = !ASYM && D::kTag == QWIX_BF16;
   __shared__ float red[ASYM ? 2 : 1][4][EV][64];
   unsigned b = blockIdx.x;
   const int64_t cb = b % static_cast<unsigned>(wide_col_blocks);
@@ -437,7 +446,9 @@ __global__ void __launch_bounds__(256)
   const int64_t row_end = (t + 1) * gm.tile;
   const int64_t row0 = t * gm.tile + static_cast<int64_t>(chunk) * kWideRows + w;  // rows row0 + 4 * i
   float mx[EV], mn[EV];
-  u16x2 pm[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  s16x2 pm[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) pm[k] = s16x2{kKeyOfZero, kKeyOfZero};
 #pragma unroll
   for (int e = 0; e < EV; ++e) mx[e] = mn[e] = 0.f;
   const uint8_t* xp = x + ((o * gm.reduce + row0) * gm.inner + c0) * sizeof(typename D::storage);
@@ -462,8 +473,7 @@ __global__ void __launch_bounds__(256)
       if constexpr (PACKED) {
         const uint32_t wd[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-          pm[k] = __builtin_elementwise_max(pm[k], __builtin_bit_cast(u16x2, wd[k] & 0x7FFF7FFFu));
+        for (int k = 0; k < 4; ++k) pm[k] = __builtin_elementwise_max(pm[k], abs_keys(wd[k]));
       } else {
         float f[EV];
         unpack16<D>(raw[j], f);
@@ -482,8 +492,8 @@ __global__ void __launch_bounds__(256)
   if constexpr (PACKED) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      mx[2 * k] = bf16_bits_to_f32(pm[k][0]);
-      mx[2 * k + 1] = bf16_bits_to_f32(pm[k][1]);
+      mx[2 * k] = key_value(pm[k][0]);
+      mx[2 * k + 1] = key_value(pm[k][1]);
     }
   }
 #pragma unroll
@@ -693,21 +703,23 @@ __global__ void __launch_bounds__(256)
   };
   if constexpr (SRC == 2) {
     float mx[EV], mn[EV];
-    if constexpr (!ASYM && D::kTag == QWIX_BF16) {  // |x| of a bf16 pair orders like its low 15 bits
-      u16x2 m[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    if constexpr (!ASYM && D::kTag == QWIX_BF16) {
+      s16x2 m[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) m[k] = s16x2{kKeyOfZero, kKeyOfZero};
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const uint32_t wd[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, wd[k] & 0x7FFF7FFFu));
+        for (int k = 0; k < 4; ++k) m[k] = __builtin_elementwise_max(m[k], abs_keys(wd[k]));
       }
       // lanes l, l^16, l^32 hold the same columns
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 16, 64)));
-        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 32, 64)));
-        mx[2 * k] = bf16_bits_to_f32(m[k][0]);
-        mx[2 * k + 1] = bf16_bits_to_f32(m[k][1]);
+        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(s16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 16, 64)));
+        m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(s16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), 32, 64)));
+        mx[2 * k] = key_value(m[k][0]);
+        mx[2 * k + 1] = key_value(m[k][1]);
       }
     } else {
 #pragma unroll

@@ -540,3 +540,32 @@ def test_dequantize_reduce_minor_by_size(shape, dtype, qtype, method):
   qa = turned(qarray.quantize(x_t, qarray.HowToQuantize(**kw)))
   want = turned(O.dequantize(O.quantize(O.FArr(x_np, dtype), O.HowToQuantize(**kw))).v)
   assert np.array_equal(util.f32np(qarray.dequantize(qa)), want)
+
+
+@pytest.mark.parametrize('qtype', QTYPES)
+@pytest.mark.parametrize('dtype', [O.BF16, O.F32])
+@pytest.mark.parametrize('shape,axis,tile', [
+    ((128, 136), 0, 32), ((256, 136), 0, 128),        # a group inside one block of the strided kernel
+    ((384, 136), 0, 192), ((1024, 136), 0, 512),      # calibrated by a pass of their own: its narrow and its wide kernel
+    ((40, 64), 1, 64), ((40, 256), 1, 128), ((5, 4096), 1, 4096), ((3, 40000), 1, 40000)])   # contiguous groups
+def test_nan_is_left_out_of_the_calibration(shape, axis, tile, dtype, qtype):
+  """A NaN does not hide the magnitudes beside it: scales, and the codes of everything else, are those of the array with
+  zeros in its places."""
+  x_np, x_t = util.make(shape, dtype, seed=shape[0] + tile)
+  at = [(1, 2), (shape[0] // 2, shape[1] // 2), (shape[0] - 1, shape[1] - 1), (0, 2), (2, 2)]
+  rows, cols = [r for r, _ in at], [c for _, c in at]
+  x_np, x_t = x_np.copy(), x_t.clone()
+  for r, c in at:   # the largest of its group, among the elements of the same thread
+    big = (r ^ 4, c) if axis == 0 else (r, c ^ 1)
+    x_np[big] = x_t[big] = 16
+  x_np[rows, cols] = 0
+  x_t[rows, cols] = float('nan')
+  kw = dict(qtype=qtype, channelwise_axes=[1 - axis], tiled_axes={axis: tile})
+  from qwix_amd.core import qarray
+  print('case', shape, axis, tile, dtype, qtype, flush=True)
+  got = qarray.quantize(x_t, qarray.HowToQuantize(**kw))
+  want = O.quantize(O.FArr(x_np, dtype), O.HowToQuantize(**kw))
+  assert np.array_equal(util.f32np(got.scale), want.scale.v)
+  codes, others = util.qvalues_np(got), np.ones(shape, bool)
+  others[rows, cols] = False
+  assert np.array_equal(codes[others], want.qvalue[others])
