@@ -123,13 +123,15 @@ def _group_by_group(fn, lhs, rhs, group_sizes, res_t, **kwargs) -> torch.Tensor:
   return out
 
 
-# Rows per group on average up to which every group streams its weight once per 32 rows (`qwix_hip_gemv_wq_groups`).
+# Rows per group on average up to which every group streams its weight once per 16 or 32 rows (`qwix_hip_gemv_wq_groups`).
+# However the rows are spread: all 3072 rows in one of 64 groups (K 2048, N 4096, int4) take 128 us either way, half of them
+# in one group 144 us here and 2.2 ms group by group, even groups 160 us and 2.2 ms; 6144 rows in one of 128 (N 1536) 104 and 132 us.
 _STREAM_ROWS = 48
 
 
 def _weight_only_groups(lhs, rhs, group_sizes, res_t):
   """All groups of a bf16 activation against int4 / int8 / e4m3 expert weights in one launch, the group sizes read on the
-  device (64 experts x 4 rows, K 2048, N 4096, int4: 2.2 ms group by group, 57 us here).  None when the operands are not of
+  device (64 experts x 4 rows, K 2048, N 4096, int4: 2.2 ms group by group, 50 us here).  None when the operands are not of
   that kind: symmetric K-contiguous weights, scales along the contraction only, in groups that are multiples of 128."""
   if not (_is_float_array(lhs) and lhs.dtype == torch.bfloat16 and isinstance(rhs, QArray) and rhs.zero_point is None):
     return None

@@ -14,6 +14,8 @@
 // A workgroup is 16 wavefronts that split K; each handles NT tiles of 16 output columns with two K
 // blocks of loads in flight (int4 weights by way of a wavefront-private LDS panel, in whole 128-byte lines), and
 // the partial sums meet in LDS.
+#include <algorithm>
+
 #include "common.h"
 
 namespace qwix {
@@ -400,42 +402,116 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_kernel(GemvArgs p) {
   gemv_wq_tile<BQT, NWAVE, NT, SBF, RT, ZP>(p, blockIdx.x * (16 * NT), blockIdx.y * (16 * RT), p.M, red_raw);
 }
 
-// Rows in groups (mixture of experts): blockIdx.y is the group, whose rows every wavefront finds for itself from the group
-// sizes in device memory; the workgroup streams that group's weight columns once per 16 RT rows.  blockIdx.y == G clears
-// the rows that belong to no group.
+// Rows in groups (mixture of experts).  Tiles of TR = 16 RT rows: a row of workgroups (one per 16 NT columns) for the first
+// tile of every group, and rows of them for as many tiles as there can be behind the first ones, in whichever groups they
+// are.  Every wavefront finds its tile for itself from the group sizes in device memory; the workgroup streams that group's
+// weight columns once.  The first row behind the groups also clears the rows that belong to no group.
+//   When one workgroup per group and column tile walked over all rows of its group, a popular group was left to N / 64
+// workgroups (K 2048, int4, N 4096, 64 groups, 256 / 1024 / 3072 rows with half of them in one group: 91 / 260 / 736 us, now 53 /
+// 85 / 144; evenly spread 50 / 76 / 178, now 50 / 75 / 160; int8, N 1408, 1024 rows, half in one group: 184, now 49).
 struct GemvGroups {
   const int32_t* sizes;
   int G;
   int64_t q_stride, s_stride;  // bytes of weights, elements of scales between consecutive groups
+  int unit0;                   // first unit of this launch
 };
+
+struct GroupTile {
+  int group, row, row_end;
+};
+
+// Rows of the groups before g, at most M.
+__device__ __forceinline__ int rows_before(const GemvGroups& gr, int M, int g) {
+  long long before = 0;
+  for (int i = threadIdx.x & 63; i < g; i += 64) before += max(gr.sizes[i], 0);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
+  return __builtin_amdgcn_readfirstlane(static_cast<int>(min(before, static_cast<long long>(M))));
+}
+
+__device__ __forceinline__ int scan_add(int v, int lane) {  // inclusive, over the wavefront
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const int u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  return v;
+}
+
+// The `tile`-th of the tiles that are not the first of their group.  Sizes are clamped so that no group reaches past row M
+// (M < 2^20: 64 clamped sums fit 32 bits).
+template <int TR>
+__device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int tile) {
+  const int lane = threadIdx.x & 63;
+  int g0 = 0, g1 = gr.G, row0 = 0, tile0 = 0;  // rows and later tiles before group g0
+  if (gr.G > 256) {  // a lane each counts a 64th of the groups, so that the search below is within one 64th
+    const int per = (gr.G + 63) / 64;
+    int rows = 0, tiles = 0;
+#pragma unroll 4
+    for (int g = lane * per; g < min((lane + 1) * per, gr.G); ++g) {
+      const int size = min(max(gr.sizes[g], 0), M);
+      rows = min(rows + size, M);
+      tiles = min(tiles + max(size - 1, 0) / TR, 1 << 20);  // more than there are tiles in front of row M
+    }
+    const int last_row = scan_add(rows, lane), last = scan_add(tiles, lane);
+    const unsigned long long here = __ballot(tile >= last - tiles && tile < last);
+    if (here == 0) return {0, 0, 0};
+    const int l = __builtin_ctzll(here);
+    g0 = __builtin_amdgcn_readfirstlane(l * per);
+    g1 = min(g0 + per, gr.G);
+    row0 = __builtin_amdgcn_readfirstlane(__shfl(last_row - rows, l, 64));
+    tile0 = __builtin_amdgcn_readfirstlane(__shfl(last - tiles, l, 64));
+  }
+  for (; g0 < g1 && row0 < M; g0 += 64) {
+    const int size = g0 + lane < g1 ? min(max(gr.sizes[g0 + lane], 0), M) : 0;
+    const int end = min(row0 + scan_add(size, lane), M);
+    const int before = __shfl_up(end, 1, 64);
+    const int start = lane == 0 ? row0 : before;
+    const int tiles = max(end - start - 1, 0) / TR;
+    if (__ballot(tiles > 0) != 0) {
+      const int last = tile0 + scan_add(tiles, lane);  // one past the group's last tile
+      const unsigned long long here = __ballot(tile >= last - tiles && tile < last);
+      if (here != 0) {  // one lane at most
+        const int l = __builtin_ctzll(here);
+        const int first = __shfl(start, l, 64) + (tile - __shfl(last - tiles, l, 64) + 1) * TR;
+        return {__builtin_amdgcn_readfirstlane(g0 + l), __builtin_amdgcn_readfirstlane(first),
+                __builtin_amdgcn_readfirstlane(min(first + TR, __shfl(end, l, 64)))};
+      }
+      tile0 = __builtin_amdgcn_readfirstlane(__shfl(last, 63, 64));
+    }
+    row0 = __builtin_amdgcn_readfirstlane(__shfl(end, 63, 64));
+  }
+  return {0, 0, 0};
+}
 
 template <int BQT, int NWAVE, int NT, bool SBF, int RT>
 __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, GemvGroups gr) {
   extern __shared__ float red_raw[];
-  const int g = blockIdx.y, lane = threadIdx.x & 63;
+  constexpr int TR = 16 * RT;
   const int n_base = blockIdx.x * (16 * NT);
-  long long before = 0;
-  for (int i = lane; i < g; i += 64) before += max(gr.sizes[i], 0);
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
-  // sizes are clamped so that no group reaches past row M
-  const int start = __builtin_amdgcn_readfirstlane(static_cast<int>(min(before, static_cast<long long>(p.M))));
-  if (g == gr.G) {
-    const int cols = min(16 * NT, p.N - n_base);
-    for (int idx = threadIdx.x; idx < (p.M - start) * cols; idx += NWAVE * 64) {
-      const int64_t at = static_cast<int64_t>(start + idx / cols) * p.ldo + n_base + idx % cols;
-      if (p.out_dtype == QWIX_BF16) reinterpret_cast<uint16_t*>(p.out)[at] = 0;
-      else reinterpret_cast<uint32_t*>(p.out)[at] = 0;
+  // Units: the groups' first tiles, then the later tiles.  One per workgroup: in a loop over them the compiler keeps what is the
+  // same in every trip in registers, and the int8 variants lost a tenth to that.
+  const int unit = gr.unit0 + static_cast<int>(blockIdx.y);
+  GroupTile at;
+  if (unit < gr.G) {
+    const int start = rows_before(gr, p.M, unit), size = min(max(gr.sizes[unit], 0), p.M - start);
+    at = {unit, start, start + min(size, TR)};
+  } else {
+    if (unit == gr.G) {
+      const int start = rows_before(gr, p.M, gr.G);
+      const int cols = min(16 * NT, p.N - n_base);
+      for (int idx = threadIdx.x; idx < (p.M - start) * cols; idx += NWAVE * 64) {
+        const int64_t to = static_cast<int64_t>(start + idx / cols) * p.ldo + n_base + idx % cols;
+        if (p.out_dtype == QWIX_BF16) reinterpret_cast<uint16_t*>(p.out)[to] = 0;
+        else reinterpret_cast<uint32_t*>(p.out)[to] = 0;
+      }
     }
-    return;
+    at = later_tile<TR>(gr, p.M, unit - gr.G);
   }
-  const int size = min(max(gr.sizes[g], 0), p.M - start);
-  p.q += g * gr.q_stride;
-  p.s = static_cast<const char*>(p.s) + g * gr.s_stride * (SBF ? 2 : 4);
-  for (int row = 0; row < size; row += 16 * RT) {  // the trip count is the same for the whole workgroup
-    if (row > 0) __syncthreads();  // the partial sums in LDS are read to the end before the next pass writes there
-    gemv_wq_tile<BQT, NWAVE, NT, SBF, RT, false>(p, n_base, start + row, start + size, red_raw);
-  }
+  if (at.row >= at.row_end) return;
+  p.q += at.group * gr.q_stride;
+  p.s = static_cast<const char*>(p.s) + at.group * gr.s_stride * (SBF ? 2 : 4);
+  gemv_wq_tile<BQT, NWAVE, NT, SBF, RT, false>(p, n_base, at.row, at.row_end, red_raw);
 }
 
 }  // namespace
@@ -565,13 +641,18 @@ extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q
   if (q_group_bytes % 16 || q_group_bytes < 0 || s_group_stride < 0)
     return fail(QWIX_ERR_INVALID_ARGUMENT, "bad group strides (weights: %lld bytes, scales: %lld elements)",
                 (long long)q_group_bytes, (long long)s_group_stride);
-  const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride};
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define QWIX_GEMVG_KERNEL(BQT, SBFF, NW, NTT, RTT)                                                         \
   do {                                                                                                     \
     constexpr size_t smem = NW * NTT * (RTT * 1024 > 2048 ? RTT * 1024 : 2048);                            \
-    gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT><<<dim3(static_cast<unsigned>((N + 16 * NTT - 1) / (16 * NTT)),  \
-                                                      static_cast<unsigned>(G + 1)), NW * 64, smem, st>>>(p, gr);   \
+    const unsigned columns = static_cast<unsigned>((N + 16 * NTT - 1) / (16 * NTT));                       \
+    /* at most (M - 1) / TR tiles are not the first of their group; one row clears in any case */          \
+    const int64_t units = G + std::max<int64_t>(1, (M - 1) / (16 * RTT));                                  \
+    for (int64_t u = 0; u < units; u += 65535) { /* a grid's y axis */                                     \
+      const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride, static_cast<int>(u)}; \
+      const dim3 grid(columns, static_cast<unsigned>(std::min<int64_t>(units - u, 65535)));                \
+      gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT><<<grid, NW * 64, smem, st>>>(p, gr);                  \
+    }                                                                                                      \
   } while (0)
 #define QWIX_GEMVG_LAUNCH(NW, NTT, RTT)                                                                    \
   do {                                                                                                     \

@@ -215,6 +215,82 @@ def test_ragged_dot_weight_only_one_launch(G, K, N, M, sizes, wq_type, tiled, dt
   assert np.all(util.f32np(out)[min(sum(sizes), M):] == 0)
 
 
+def _grouped_reference(x, wq, sizes):
+  """Rows of x against the dequantized weight of their own group, in 64 bits."""
+  q = (wq.qvalue.unpack() if wq.qtype == 'int4' else wq.qvalue).to(torch.float64)
+  w = q * wq.scale.to(torch.float64).repeat_interleave(q.shape[1] // wq.scale.shape[1], 1)
+  want, start = torch.zeros(x.shape[0], w.shape[2], dtype=torch.float64, device=x.device), 0
+  for g, size in enumerate(sizes):
+    stop = min(start + max(size, 0), x.shape[0])
+    if stop > start:
+      want[start:stop] = x[start:stop].to(torch.float64) @ w[g]
+    start = stop
+  return want
+
+
+@pytest.mark.parametrize('G,N,M,sizes', [
+    (8, 200, 384, (1, 0, 370, 0, 0, 3, 0, 10)),                   # one group with nearly all rows, two row tiles
+    (64, 72, 600, (0,) * 63 + (600,)),                            # all rows in the last group of a wavefront, one row tile
+    (130, 72, 700, tuple(417 if g == 100 else 2 * (g % 2) for g in range(130))),     # groups past the first 64, rows left over
+    (300, 72, 900, tuple(500 if g == 290 else -1 if g % 5 == 0 else 1 for g in range(300))),   # found in two steps; negative sizes
+    (300, 72, 3500, tuple(2 ** 31 - 1 if g in (200, 250) else 16 + g % 2 for g in range(300))),   # sizes that reach past all rows
+])
+@pytest.mark.parametrize('wq_type', ['int4', 'int8'])
+def test_ragged_dot_weight_only_skewed(G, N, M, sizes, wq_type):
+  """Row tiles spread over workgroups wherever the rows lie (tolerance: f32 sums, as in the test above)."""
+  import qwix_amd
+  _, x = util.make((M, 256), O.BF16, seed=91)
+  _, w = util.make((G, 256, N), O.BF16, seed=92, scale=0.05)
+  wq = qwix_amd.quantize(w, wq_type, channelwise_axes=[0, 2], tiled_axes={1: 128})
+  assert qwix_amd.core.ragged_dot._weight_only_groups(x, wq, _sizes(sizes), torch.float32) is not None
+  out = qwix_amd.ragged_dot(x, wq, _sizes(sizes), preferred_element_type=torch.float32)
+  want = _grouped_reference(x, wq, sizes)
+  assert float((out.to(torch.float64) - want).abs().max()) <= 1e-5 * float(want.abs().max())
+  assert not out[max(0, min(sum(max(s, 0) for s in sizes), M)):].any()
+
+
+def test_ragged_dot_weight_only_more_row_tiles_than_a_grid():
+  """65534 groups of 17 and 3 rows: 98301 row tiles, more than a grid's y axis holds."""
+  import qwix_amd
+  G, M = 65534, 655340
+  g = torch.Generator(device=util.DEV).manual_seed(5)
+  x = torch.randn(M, 128, generator=g, device=util.DEV).to(torch.bfloat16)
+  wq = qwix_amd.quantize((torch.randn(G, 128, 16, generator=g, device=util.DEV) * 0.05).to(torch.bfloat16), 'int8', channelwise_axes=[0, 2])
+  sizes = torch.tensor([17, 3] * (G // 2), dtype=torch.int32, device=util.DEV)
+  out = qwix_amd.core.ragged_dot._weight_only_groups(x, wq, sizes, torch.float32)
+  group = torch.repeat_interleave(torch.arange(G, device=util.DEV), sizes.long())
+  top = 0.0
+  for rows in torch.arange(M, device=util.DEV).split(65536):
+    w = wq.qvalue[group[rows]].double() * wq.scale[group[rows]].double()
+    want = (x[rows].double()[:, :, None] * w).sum(1)
+    top = max(top, float((out[rows].double() - want).abs().max() / want.abs().max()))
+  assert top <= 1e-5   # f32 sums
+
+
+def test_ragged_dot_weight_only_popular_group_is_shared_out():
+  """Half of the rows in one group cost no more than twice what even groups cost (49 us for 41; with one workgroup
+  per group and 64 columns it was 184 for 44)."""
+  import qwix_amd
+  G, M, K, N = 64, 1024, 2048, 1408
+  wq = qwix_amd.quantize((torch.randn(G, K, N, device=util.DEV) * 0.05).to(torch.bfloat16), 'int8', channelwise_axes=[0, 2])
+  x = torch.randn(M, K, device=util.DEV).to(torch.bfloat16)
+  even, skewed = [16] * G, [8] * G
+  skewed[20] = M - 8 * (G - 1)
+
+  def best(sizes):
+    sizes, times = _sizes(sizes), []
+    for _ in range(8):
+      ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+      ev[0].record()
+      for _ in range(5):
+        qwix_amd.ragged_dot(x, wq, sizes)
+      ev[1].record()
+      torch.cuda.synchronize()
+      times.append(ev[0].elapsed_time(ev[1]))
+    return min(times)
+  assert best(skewed) < 2.0 * best(even)
+
+
 def test_ragged_dot_dequantize_first_path():
   """A raw float lhs or a zero point sends the call to the dequantize-first path (ragged_dot.py:278-292)."""
   import qwix_amd
