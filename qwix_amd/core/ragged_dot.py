@@ -141,8 +141,8 @@ def _weight_only_groups(lhs, rhs, group_sizes, res_t):
   M, K = lhs.shape
   G, _, N = rhs.shape
   sg, tiles, sn = rhs.scale.shape
-  if sg not in (1, G) or sn not in (1, N) or K % 128 or (K // tiles) % 128 or M > _STREAM_ROWS * G or G >= 65535:
-    return None
+  if sg not in (1, G) or sn not in (1, N) or K % 128 or (K // tiles) % 128 or M > min(_STREAM_ROWS * G, 65535 * 16) or G >= 65535:
+    return None   # (the kernel counts rows in tiles of 16 and groups in 16 bits)
   if isinstance(rhs.qvalue, Int4Tensor):
     if rhs.qvalue.packed_axis != 1:
       return None

@@ -167,6 +167,18 @@ def test_recorder_refuses_sums_kept_per_weight(stand_in):
   assert not rec.ok and len(rec.calls) == 1 and recorded[0] is not None
 
 
+def test_more_rows_than_one_launch_takes_go_group_by_group(stand_in):
+  """Weight-only experts in one launch end at 65535 * 16 rows; with enough groups even a few rows each come to more."""
+  from qwix_amd.core import ragged_dot as rd
+  from qwix_amd.core.qarray import QArray
+  G = 21846
+  w = QArray(torch.empty(G, 8, 128, dtype=torch.int8).permute(0, 2, 1), torch.empty(1, 1, 8, dtype=torch.bfloat16), None, 'int8')
+  sizes = torch.zeros(G, dtype=torch.int32)
+  for rows, taken in ((65535 * 16, True), (65535 * 16 + 1, False)):
+    out = rd._weight_only_groups(torch.empty(rows, 128, dtype=torch.bfloat16), w, sizes, torch.bfloat16)
+    assert (out is not None) == taken
+
+
 # ---- the table
 
 
