@@ -289,6 +289,14 @@ def _cases():
   cases['ragged int8'] = (lambda s: (act(s, 'int8'), qwix_amd.quantize(_rand((4, 512, 72), s), 'int8', channelwise_axes=[0, 2]), sizes(s)),
                           qwix_amd.ragged_dot,
                           lambda *a: rd.ragged_dot_general(*a, rd._BASIC_RAGGED_DOT_DIMENSION_NUMBERS))
+  for q in ('int4', 'int8'):   # group sizes of their own in every call, empty groups and rows left over among them
+    experts = lambda s, q=q: qwix_amd.quantize(_rand((4, 512, 72), s + 1, std=0.05), q, channelwise_axes=[0, 2], tiled_axes={1: 128})
+    cases[f'experts {q}'] = (lambda s, e=experts: (_rand((40, 512), s), e(s), torch.roll(sizes(s), s // 10)), qwix_amd.ragged_dot,
+                             lambda *a: rd.ragged_dot_general(*a, rd._BASIC_RAGGED_DOT_DIMENSION_NUMBERS))
+    # prompt sizes: the weight dequantized inside the product, its contraction cut into ranges, and dequantized in front of it
+    for rows, k, n in ((200, 512, 8192), (100, 4096, 256), (1100, 512, 200) if q == 'int4' else (520, 512, 11008)):
+      cases[f'weight only {q} {rows} rows'] = (
+          lambda s, q=q, m=rows, k=k, n=n: (_rand((m, k), s), weight(s + 1, q, 128, k=k, n=n)),) + dot
   cases['hadamard'] = (lambda s: (_rand((24, 512), s), weight(s + 1, 'int4', 128)), hr.hadamard_quantized_matmul,
                        lambda a, b: hr._hadamard_quantized_matmul(a, b, None, None, None, None))
   return cases
@@ -299,11 +307,14 @@ _NAMES = (['%s %s %s' % (w, q, m) for w in ('rows', 'columns', 'dequantize')
           ['%s %s' % (w, q) for w in ('dot', 'fused act') for q in ('int8', 'float8_e4m3fn')] +
           ['dot int8 x int4 128', 'dot int8 x int4 256', 'weight only int4 absmax', 'weight only int4 minmax',
            'weight only int8 minmax', 'einsum', 'ragged int8', 'hadamard'])
+_ENTRIES = {f'experts {q}': ['gemv_wq_groups'] for q in ('int4', 'int8')}   # what the ordinary path of a case runs
+_ENTRIES.update({f'weight only {q} {rows} rows': ['gemm_bf16_wq_ws'] for q in ('int4', 'int8') for rows in (200, 100)})
+_ENTRIES.update({f'weight only {q} rows': ['dequantize_rm', 'gemm_bf16'] for q in ('int4 1100', 'int8 520')})
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('inference', [False, True])
-@pytest.mark.parametrize('name', _NAMES)
+@pytest.mark.parametrize('name', _NAMES + list(_ENTRIES))
 def test_replay_equals_the_ordinary_path(name, inference):
   """New operands (other data, other addresses) on every call: the first ones go the ordinary way, the others replay."""
   _empty_the_table()   # (what the other mode recorded)
@@ -318,6 +329,10 @@ def test_replay_equals_the_ordinary_path(name, inference):
   call, _lib.call = _lib.call, lambda *a: calls.append(a[0]) or call(*a)
   try:
     with torch.inference_mode(inference):
+      if name in _ENTRIES:
+        ordinary(*alive[0])
+        assert calls == ['qwix_hip_' + entry for entry in _ENTRIES[name]]
+        calls.clear()
       _same(op(*alive[0]), op(*alive[0]))
     assert not calls, 'no plan is kept for this kind of call'
   finally:
