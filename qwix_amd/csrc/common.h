@@ -241,7 +241,8 @@ struct Divider {
       return x / s;
     }
   }
-  // Divides a pair; the bf16 rounding of both is one convert.  Zero quotients come out as +0.
+  // Divides a pair; the bf16 rounding of both is one convert.  The sign of a zero quotient is that of the f32 quotient or product
+  // (the dividend's: scales are positive); `pair` states it where codes with a -0 are written.
   __device__ __forceinline__ void pair_unsigned(float& a, float& b) const {
     a = raw(a);
     b = raw(b);

@@ -584,8 +584,9 @@ __global__ void cols_finish_cal_kernel(const uint32_t* __restrict__ ws, int64_t 
 
 // One column's eight rows as packed codes (two words, int4: one).  SAFE: the scale was given, not derived from these rows.
 // A quotient carries the sign of its dividend, zero quotients included (the product with the positive reciprocal does).
-// clip (e4m3 from bf16): quotients by a scale that absmax gave stay inside e4m3's range once rounded to bf16 -- |x| / s is at
-// most 448 (1 + 2^-8), which rounds to 448 -- but a calibration factor below one lets them leave it.
+// clip (e4m3 from bf16): quotients by a scale that absmax gave need none.  The scale is absmax / 448 to within 2^-8, so
+// |x| / s is at most 449.8 and the bf16 quotient at most 450 (absmax 230 gives that), which the conversion, rounding to nearest,
+// takes to 448 as it does everything below 464.  A calibration factor below one lets quotients leave that range.
 template <typename D, int QT, bool SAFE, bool ASYM>
 __device__ __forceinline__ void quantize_column(const float (&x)[8], float s, float zf, bool clip, uint32_t (&w)[2]) {
   const Divider<D, SAFE, false> div(s);

@@ -501,6 +501,24 @@ def test_weight_columns_and_back_at_tile_edges(K, N, tile, dtype, qtype, method)
   assert np.array_equal(util.f32np(qarray.dequantize(qa)), want.v)
 
 
+@pytest.mark.parametrize('K,tile', [(96, 32), (512, None)])   # calibrated inside the block, and by a pass of its own
+def test_e4m3_columns_of_every_bf16_maximum(K, tile):
+  """Quotients by a rounded scale reach 450 (for 230, 129 and 8 others of the 128 significands), which has to become 448."""
+  x_np = np.zeros((K, 512), np.float32)
+  tops = np.concatenate([np.arange(128, 256) * 2.0 ** e for e in (0, -9, 40, -40)]).astype(np.float32)
+  x_np[:] = tops * np.linspace(-0.97, 0.97, K, dtype=np.float32)[:, None]
+  x_np = torch.from_numpy(x_np).to(torch.bfloat16).float().numpy()
+  x_np[7::16], x_np[8::16] = tops, -tops
+  scale = torch.from_numpy(tops / 448).to(torch.bfloat16).float().numpy()
+  top_quotients = torch.from_numpy(tops / scale).to(torch.bfloat16)
+  assert float(top_quotients.max()) == 450
+  assert int((top_quotients[:128] > 448).sum()) == 10
+  kw = dict(qtype='float8_e4m3fn', channelwise_axes=[1], tiled_axes={0: tile} if tile else {})
+  x_t = torch.from_numpy(x_np).to(torch.bfloat16).to(util.DEV)
+  q = _check(x_np, x_t, O.BF16, kw, layout='reduce_minor', what='columns of every maximum')
+  assert not ((util.qvalues_np(q) & 0x7F) == 0x7F).any()   # NaN
+
+
 @pytest.mark.parametrize('qtype,reduce,inner', [('int8', 65535 * 128 + 264, 16), ('int4', 65535 * 256 + 264, 8), ('int8', 24, 65535 * 128 + 264)])
 def test_dequantize_reduce_minor_beyond_one_grid(qtype, reduce, inner):
   """K-contiguous values with more tiles along the reduced axis than a grid has blocks there, and the same of columns."""
