@@ -399,7 +399,8 @@ QWIX_API int qwix_hip_gemv_wq_zp(const void* x, int64_t ldx, const void* q, int6
 /* Weight-only product with the rows in groups, one weight per group (ragged_dot.py:229-241 without the dequantized copy,
  * for a few rows per group): rows of x form G consecutive groups of group_sizes[g] rows (device memory, never read on the
  * host; sizes are clamped to the M rows), group g meets the weight at q + g * q_group_bytes with the scales at
- * s + g * s_group_stride elements.  Rows behind the last group come out as zeros.  Otherwise as qwix_hip_gemv_wq. */
+ * s + g * s_group_stride elements.  Rows behind the last group come out as zeros.  G is at most 65534, M 65535 * 16.
+ * Otherwise as qwix_hip_gemv_wq. */
 QWIX_API int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes,
                         int b_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
                         int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out, int out_dtype,

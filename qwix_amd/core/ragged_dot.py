@@ -126,6 +126,9 @@ def _group_by_group(fn, lhs, rhs, group_sizes, res_t, **kwargs) -> torch.Tensor:
 # Rows per group on average up to which every group streams its weight once per 16 or 32 rows (`qwix_hip_gemv_wq_groups`).
 # However the rows are spread: all 3072 rows in one of 64 groups (K 2048, N 4096, int4) take 128 us either way, half of them
 # in one group 144 us here and 2.2 ms group by group, even groups 160 us and 2.2 ms; 6144 rows in one of 128 (N 1536) 104 and 132 us.
+# What group by group is better at are hundreds of rows in very few groups, nearly all others empty: 16 groups, 768 rows, K 4096,
+# N 14336, in one / three of them int8 318 / 314 us here and 191 / 213, int4 201 / 199 and 192 / 262; half of them in one
+# int8 359 and 478, evenly 413 and 759.
 _STREAM_ROWS = 48
 
 
