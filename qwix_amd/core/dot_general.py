@@ -778,7 +778,7 @@ def _decode_plan(lhs, rhs, dimension_numbers):
     if any(kept.untyped_storage().data_ptr() != own.untyped_storage().data_ptr() for kept, own in ((b, values), (sb, rhs.scale))):
       plans.kept_aside()
     plan = (b, numerics.qtype_tag(_qtype_of(rhs)), sb, _lib.float_tag(sb.dtype), zp, c.N, c.K, c.K // gb,
-            fused_wq_min_rows(c.N, b_is4, c.K, c.K // gb))
+            streamed_rows(c.N, b_is4, c.K, c.K // gb))
   _DECODE_PLANS[key] = (weakref.ref(rhs, lambda _, k=key: _DECODE_PLANS.pop(k, None)),
                         _weight_signature(rhs), plan)
   return plan
@@ -794,9 +794,9 @@ def _decode_dot(lhs, rhs, dimension_numbers, preferred_element_type):
   plan = _decode_plan(lhs, rhs, dimension_numbers)
   if plan is None:
     return None
-  b, b_tag, sb, sb_tag, zp, n, k, group, fused_min = plan
+  b, b_tag, sb, sb_tag, zp, n, k, group, most_rows = plan
   m = lhs.shape[0]
-  if lhs.shape[1] != k or len(rhs.shape) != 2 or m > fused_min:
+  if lhs.shape[1] != k or len(rhs.shape) != 2 or m > most_rows:
     return None
   lhs = _aligned_rows(lhs)
   if not _decode_kernel_limits_ok(lhs.stride(0), b.stride(0), n, k, group, b_tag == _lib.INT4, sb.element_size()):
@@ -824,7 +824,7 @@ def _slow_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, 
   if out is not None:
     return out
   c = _weight_only_fit(lhs, rhs, dimension_numbers)
-  if c is not None and (fused_wq_min_rows(c.N, isinstance(rhs.qvalue, Int4Tensor), c.K, c.K // rhs.scale.shape[c.rca[-1]])
+  if c is not None and (streamed_rows(c.N, isinstance(rhs.qvalue, Int4Tensor), c.K, c.K // rhs.scale.shape[c.rca[-1]])
                         < c.M <= WEIGHT_ONLY_MAX_ROWS):
     # one row tile of the dequantizing tile GEMM beats the decode kernel from here on
     out = _dequantize_then_bf16_gemm(lhs, rhs, dimension_numbers, preferred_element_type, fused_only=True)
@@ -896,6 +896,15 @@ def fused_wq_min_rows(n: int, int4: bool = True, k: int = 0, group: int = 0) -> 
   if int4:
     return 64 if n >= 12288 else 80
   return 32 if n >= 12288 else 64
+
+
+def streamed_rows(n: int, int4: bool, k: int, group: int) -> int:
+  """Rows up to which `qwix_hip_gemv_wq` multiplies the weight's codes, exact in bf16, and scales the f32 sums.  What runs beyond
+  them rounds every code x scale to bf16 (`dequantize`'s value where scales are bf16): up to 2^-9 of a weight, where the
+  sums are good to 1e-6.  So the line is drawn by time only where it always was: K in multiples of 256, up to 256 rows."""
+  if k % 256 or not _fused_wq_takes(WEIGHT_ONLY_MAX_ROWS, n, int4):
+    return WEIGHT_ONLY_MAX_ROWS
+  return fused_wq_min_rows(n, int4, k, group)
 
 
 def _dequantize_then_bf16_gemm(lhs, rhs, dimension_numbers, preferred_element_type, fused_only=False):
