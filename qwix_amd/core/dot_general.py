@@ -881,6 +881,14 @@ def _fused_wq_takes(m: int, n: int, int4: bool) -> bool:
 _FUSED_W8_MAX_TILES = 256
 
 
+def _equal_ranges(n: int, k: int, group: int) -> bool:
+  """Whether K can be cut in equal ranges of whole 256-element superslabs and whole scale groups (or equal parts of one), at least
+  1024 elements each, one workgroup of the 128 x 64 tiles per CU."""
+  tiles = -(-n // 64)
+  return tiles <= 128 and any(k % (r * 256) == 0 and ((k // r) % group == 0 or group % (k // r) == 0)
+                              for r in range(2, min(256 // tiles, k // 1024) + 1))
+
+
 def fused_wq_min_rows(n: int, int4: bool = True, k: int = 0, group: int = 0) -> int:
   """Rows above which the dequantizing tile GEMM beats the decode kernel (`qwix_hip_gemv_wq`).  The time of one row
   tile does not depend on the rows (K 4096, up to 128 rows, tiles of 128 x 64: int4 29 / 26 us at N 14336 / 4096, int8
@@ -890,8 +898,9 @@ def fused_wq_min_rows(n: int, int4: bool = True, k: int = 0, group: int = 0) -> 
   Where the tile GEMM cuts K into ranges (given `k` and `group`: few tiles, `qwix_hip_gemm_bf16_wq_ws`) it wins earlier.
   Weights from HBM, decode kernel at 32 / 48 / 64 rows against the tile GEMM's one time up to 128 rows: int4 K 4096,
   N 4096 12 / 15 / 21 against 15 us; K 8192, N 8192 23 / 29 / 40 against 33; K 14336, N 4096 34 / 45 / 64 against 31;
-  int8 13 / 17 / 21 against 15; 25 / 40 / 48 against 34; 35 / 55 / 67 against 32."""
-  if k and group and _lib.load().qwix_hip_gemm_bf16_wq_workspace_bytes(64, n, k, group):
+  int8 13 / 17 / 21 against 15; 25 / 40 / 48 against 34; 35 / 55 / 67 against 32.  Only where the ranges can be equal: for the
+  others, which end in a shorter range, more rows keep their weights unrounded (`streamed_rows`)."""
+  if k and group and _equal_ranges(n, k, group):
     return 48 if int4 else 32
   if int4:
     return 64 if n >= 12288 else 80

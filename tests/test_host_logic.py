@@ -316,3 +316,17 @@ def test_weight_signature_sees_in_place_updates():
   a4 = dg._weight_signature(w4)
   p.data.add_(1)
   assert dg._weight_signature(w4) != a4
+
+
+def test_k_ranges_that_lower_the_streamed_rows():
+  """They are equal ones (the oracle: every number of ranges tried)."""
+  from qwix_amd.core import dot_general as dg
+  for n in (1, 64, 264, 4096, 8192, 8200, 16384):
+    for k in range(256, 16385, 256):
+      for group in (128, 256, 512, k):
+        if k % group:
+          continue
+        tiles = (n + 63) // 64
+        ranges = [r for r in range(2, 257) if tiles <= 128 and r * tiles <= 256 and r * 1024 <= k and k % (r * 256) == 0
+                  and ((k // r) % group == 0 or group % (k // r) == 0)]
+        assert dg.fused_wq_min_rows(n, True, k, group) == (48 if ranges else 64 if n >= 12288 else 80), (n, k, group)
