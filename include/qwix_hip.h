@@ -383,6 +383,13 @@ QWIX_API int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const void
                                  int q_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
                                  int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out, int out_dtype,
                                  int64_t ldo, void* stream);
+/* Both kernels over one array of rows: groups of up to `stream_rows` rows as qwix_hip_gemv_wq_groups computes them (the codes
+ * multiplied as they are, the f32 sums scaled), larger ones as qwix_hip_gemm_bf16_wq_ragged (every code x scale rounded to
+ * bf16 first, up to 2^-9 of a weight).  group % 128 == 0, G at most 65534, M at most 65535 * 16. */
+QWIX_API int qwix_hip_gemm_wq_groups(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int64_t q_group_stride,
+                            int q_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
+                            int64_t s_group_stride, const int32_t* group_sizes, int64_t G, int64_t stream_rows, void* out,
+                            int out_dtype, int64_t ldo, void* stream);
 
 /* dequantize (qarray.py:692-708) of a REDUCE_MINOR qvalue that keeps that layout: out[(o, i, r)] =
  * D(D(q - zp) * scale[o, r / tile, i]) as a row-major (outer, inner, reduce) array, the K-contiguous operand

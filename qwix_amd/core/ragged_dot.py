@@ -7,7 +7,7 @@ array), `_fast_ragged_dot_general` (:123-226) and `_slow_ragged_dot_general` (:2
 lhs is (M, K), rhs is (G, K, N); the rows of lhs form G consecutive groups of `group_sizes` rows
 and group g is multiplied with rhs[g].  `group_sizes` stays in device memory: the kernel reads it,
 so the quantized path never synchronises with the host.  Rows past the last group come out as
-zeros.  Weight-only products of up to 1024 rows per group run in one launch too (`_weight_only_groups`).  int8 activations x
+zeros.  Weight-only products of up to 1024 rows per group run in one launch or two (`_weight_only_groups`).  int8 activations x
 int4 expert weights and the rest of the dequantize-first path run the dense kernels of dot_general group by group (these
 need the group boundaries on the host).  Other dimension numbers with the ragged axis as the only
 free axis of the lhs and one group axis on the rhs (batch axes, several contracting axes, any axis order) run one
@@ -129,7 +129,9 @@ def _group_by_group(fn, lhs, rhs, group_sizes, res_t, **kwargs) -> torch.Tensor:
 # What group by group is better at are hundreds of rows in very few groups, nearly all others empty: 16 groups, 768 rows, K 4096,
 # N 14336, in one / three of them int8 318 / 314 us here and 191 / 213, int4 201 / 199 and 192 / 262; half of them in one
 # int8 359 and 478, evenly 413 and 759.
-# Beyond them the dequantizing tile GEMM takes all groups in one launch (`qwix_hip_gemm_bf16_wq_ragged`).  Streamed / in tiles,
+# Beyond them the dequantizing tile GEMM takes the groups whose rows `dot_general` would not stream (`streamed_rows`: their weights
+# are rounded to bf16 there as well), all of them in one launch, and the streaming kernel the others in another
+# (`qwix_hip_gemm_wq_groups`): no group loses precision to the rows of its neighbours.  All streamed / all in tiles,
 # 48 and 64 rows per group: int4 64 groups, K 2048, N 1024 54 / 66 and 67 / 67 us, 8 groups, K 4096, N 14336 121 / 189 and
 # 153 / 193 us; int8 69 / 72 and 85 / 72 us, 217 / 214 and 255 / 215 us.
 _STREAM_ROWS = 48
@@ -140,7 +142,7 @@ _TILE_ROWS, _TILE_GROUPS = 1024, 1024
 
 
 def _weight_only_groups(lhs, rhs, group_sizes, res_t):
-  """All groups of a bf16 activation against int4 / int8 / e4m3 expert weights in one launch, the group sizes read on the
+  """All groups of a bf16 activation against int4 / int8 / e4m3 expert weights in one launch or two, the group sizes read on the
   device (64 experts x 4 rows, K 2048, N 4096, int4: 2.2 ms group by group, 50 us here).  None when the operands are not of
   that kind: symmetric K-contiguous weights, scales along the contraction only, in groups that are multiples of 128."""
   if not (_is_float_array(lhs) and lhs.dtype == torch.bfloat16 and isinstance(rhs, QArray) and rhs.zero_point is None):
@@ -153,8 +155,11 @@ def _weight_only_groups(lhs, rhs, group_sizes, res_t):
   sg, tiles, sn = rhs.scale.shape
   if sg not in (1, G) or sn not in (1, N) or K % 128 or (K // tiles) % 128:
     return None
+  if M > 65535 * 16 or G >= 65535:   # (the streaming kernel counts rows in tiles of 16, groups in 16 bits)
+    return None
   rows = _STREAM_ROWS_INT4 if q == numerics.INT4 else _STREAM_ROWS
-  stream = M <= min(rows * G, 65535 * 16) and G < 65535   # (that kernel counts rows in tiles of 16, groups in 16 bits)
+  most = _dot_general.streamed_rows(N, q == numerics.INT4, K, K // tiles)
+  stream = M <= max(rows * G, most)
   if not stream and (K < 256 or M > _TILE_ROWS * G or G > _TILE_GROUPS):
     return None
   if isinstance(rhs.qvalue, Int4Tensor):
@@ -165,8 +170,7 @@ def _weight_only_groups(lhs, rhs, group_sizes, res_t):
     b = rhs.qvalue.permute(0, 2, 1)
   if not b.is_contiguous() or rhs.scale.dtype not in (torch.bfloat16, torch.float32):
     return None
-  if stream and not _dot_general._decode_kernel_limits_ok(K, b.stride(1), N, K, K // tiles, q == numerics.INT4,
-                                                          rhs.scale.element_size()):
+  if not _dot_general._decode_kernel_limits_ok(K, b.stride(1), N, K, K // tiles, q == numerics.INT4, rhs.scale.element_size()):
     return None
   x = _dot_general._aligned_rows(lhs)
   if not stream and not _dot_general._bf16_gemm_limits_ok(M, x.stride(0), N, b.stride(1)):
@@ -174,9 +178,10 @@ def _weight_only_groups(lhs, rhs, group_sizes, res_t):
   scale = rhs.scale.expand(sg, tiles, N).contiguous()
   sizes = group_sizes.to(device=x.device, dtype=torch.int32).contiguous()
   out = torch.empty(M, N, dtype=res_t, device=x.device)
-  _lib.call('qwix_hip_gemv_wq_groups' if stream else 'qwix_hip_gemm_bf16_wq_ragged', x.data_ptr(), x.stride(0), b.data_ptr(), b.stride(1), b.stride(0), numerics.qtype_tag(q),
-            M, N, K, K // tiles, scale.data_ptr(), _lib.float_tag(scale.dtype), tiles * N if sg > 1 else 0, sizes.data_ptr(), G,
-            out.data_ptr(), _lib.float_tag(res_t), N, _lib.stream_of(x))
+  _lib.call('qwix_hip_gemv_wq_groups' if stream else 'qwix_hip_gemm_wq_groups', x.data_ptr(), x.stride(0), b.data_ptr(), b.stride(1),
+            b.stride(0), numerics.qtype_tag(q), M, N, K, K // tiles, scale.data_ptr(), _lib.float_tag(scale.dtype),
+            tiles * N if sg > 1 else 0, sizes.data_ptr(), G, *(() if stream else (most,)), out.data_ptr(), _lib.float_tag(res_t), N,
+            _lib.stream_of(x))
   return out
 
 

@@ -327,4 +327,10 @@ __device__ __forceinline__ void buffer_to_lds16(R rsrc, uint8_t* lds, unsigned v
 #endif
 }
 
+// qwix_hip_gemv_wq_groups for the groups of up to `most_rows` rows (gemv_wq.hip): with fewer than M the others and the rows
+// behind the groups are not written.
+int gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes, int b_qtype, int64_t M,
+                   int64_t N, int64_t K, int64_t group, const void* s, int s_dtype, int64_t s_group_stride,
+                   const int32_t* group_sizes, int64_t G, int64_t most_rows, void* out, int out_dtype, int64_t ldo, void* stream);
+
 }  // namespace qwix

@@ -414,6 +414,7 @@ struct GemvGroups {
   int G;
   int64_t q_stride, s_stride;  // bytes of weights, elements of scales between consecutive groups
   int unit0;                   // first unit of this launch
+  int most;                    // groups of more rows, and the rows behind the groups, are left to another launch (INT32_MAX: none are)
 };
 
 struct GroupTile {
@@ -453,7 +454,17 @@ __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int
       rows = min(rows + size, M);
       tiles = min(tiles + max(size - 1, 0) / TR, 1 << 20);  // more than there are tiles in front of row M
     }
-    const int last_row = scan_add(rows, lane), last = scan_add(tiles, lane);
+    const int last_row = scan_add(rows, lane);
+    if (gr.most < M) {  // which groups count is told by the rows that they have in front of row M
+      int start = min(last_row - rows, M);
+      tiles = 0;
+      for (int g = lane * per; g < min((lane + 1) * per, gr.G); ++g) {
+        const int size = min(max(gr.sizes[g], 0), M - start);
+        if (size <= gr.most) tiles += max(size - 1, 0) / TR;
+        start += size;
+      }
+    }
+    const int last = scan_add(tiles, lane);
     const unsigned long long here = __ballot(tile >= last - tiles && tile < last);
     if (here == 0) return {0, 0, 0};
     const int l = __builtin_ctzll(here);
@@ -467,7 +478,7 @@ __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int
     const int end = min(row0 + scan_add(size, lane), M);
     const int before = __shfl_up(end, 1, 64);
     const int start = lane == 0 ? row0 : before;
-    const int tiles = max(end - start - 1, 0) / TR;
+    const int tiles = end - start > gr.most ? 0 : max(end - start - 1, 0) / TR;
     if (__ballot(tiles > 0) != 0) {
       const int last = tile0 + scan_add(tiles, lane);  // one past the group's last tile
       const unsigned long long here = __ballot(tile >= last - tiles && tile < last);
@@ -495,9 +506,9 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, 
   GroupTile at;
   if (unit < gr.G) {
     const int start = rows_before(gr, p.M, unit), size = min(max(gr.sizes[unit], 0), p.M - start);
-    at = {unit, start, start + min(size, TR)};
+    at = {unit, start, size > gr.most ? start : start + min(size, TR)};
   } else {
-    if (unit == gr.G) {
+    if (unit == gr.G && gr.most == INT32_MAX) {
       const int start = rows_before(gr, p.M, gr.G);
       const int cols = min(16 * NT, p.N - n_base);
       for (int idx = threadIdx.x; idx < (p.M - start) * cols; idx += NWAVE * 64) {
@@ -629,10 +640,10 @@ extern "C" int qwix_hip_gemv_wq_zp(const void* x, int64_t ldx, const void* q, in
   return gemv_wq_impl(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, zp, out, out_dtype, ldo, stream);
 }
 
-extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes,
-                                       int b_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
-                                       int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out,
-                                       int out_dtype, int64_t ldo, void* stream) {
+int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes, int b_qtype, int64_t M,
+                         int64_t N, int64_t K, int64_t group, const void* s, int s_dtype, int64_t s_group_stride,
+                         const int32_t* group_sizes, int64_t G, int64_t most_rows, void* out, int out_dtype, int64_t ldo,
+                         void* stream) {
   GemvArgs p;
   if (const int rc = gemv_wq_args(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, nullptr, out, out_dtype, ldo, &p))
     return rc;
@@ -642,14 +653,17 @@ extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q
     return fail(QWIX_ERR_INVALID_ARGUMENT, "bad group strides (weights: %lld bytes, scales: %lld elements)",
                 (long long)q_group_bytes, (long long)s_group_stride);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t most = std::max<int64_t>(1, std::min(most_rows, M));
 #define QWIX_GEMVG_KERNEL(BQT, SBFF, NW, NTT, RTT)                                                         \
   do {                                                                                                     \
     constexpr size_t smem = NW * NTT * (RTT * 1024 > 2048 ? RTT * 1024 : 2048);                            \
     const unsigned columns = static_cast<unsigned>((N + 16 * NTT - 1) / (16 * NTT));                       \
-    /* at most (M - 1) / TR tiles are not the first of their group; one row clears in any case */          \
-    const int64_t units = G + std::max<int64_t>(1, (M - 1) / (16 * RTT));                                  \
+    /* at most (M - 1) / TR tiles are not the first of their group, and no group has more than its rows */ \
+    /* fill; one row clears in any case */                                                                 \
+    const int64_t units = G + std::max<int64_t>(1, std::min((M - 1) / (16 * RTT), G * ((most - 1) / (16 * RTT)))); \
     for (int64_t u = 0; u < units; u += 65535) { /* a grid's y axis */                                     \
-      const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride, static_cast<int>(u)}; \
+      const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride, static_cast<int>(u), \
+                          most_rows < M ? static_cast<int>(most) : INT32_MAX};                             \
       const dim3 grid(columns, static_cast<unsigned>(std::min<int64_t>(units - u, 65535)));                \
       gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT><<<grid, NW * 64, smem, st>>>(p, gr);                  \
     }                                                                                                      \
@@ -685,4 +699,12 @@ extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q
 #undef QWIX_GEMVG_LAUNCH
 #undef QWIX_GEMVG_KERNEL
   return check_launch("gemv_wq (groups)");
+}
+
+extern "C" int qwix_hip_gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes,
+                                       int b_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
+                                       int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out,
+                                       int out_dtype, int64_t ldo, void* stream) {
+  return gemv_wq_groups(x, ldx, q, ldb_bytes, q_group_bytes, b_qtype, M, N, K, group, s, s_dtype, s_group_stride, group_sizes,
+                        G, M, out, out_dtype, ldo, stream);
 }

@@ -1073,6 +1073,7 @@ struct Ragged {
   int G;
   int64_t b_group_stride;   // bytes between consecutive B panels
   int64_t sb_group_stride;  // elements between the rhs scale vectors of consecutive groups (0: one shared vector)
+  int skip;                 // groups of up to this many rows have no tiles here (another launch does them)
 };
 
 constexpr int kRaggedChunk = 16;  // consecutive tile ids that run on one XCD
@@ -1116,7 +1117,7 @@ __device__ __forceinline__ int ragged_tile(const Ragged& rg, int M, int N, int* 
     const int prev = __shfl_up(end, 1, 64);
     start = lane == 0 ? row : prev;
     size = end - start;
-    const int cnt = (size + BM - 1) / BM * tiles_n;
+    const int cnt = size > rg.skip ? (size + BM - 1) / BM * tiles_n : 0;
     const int last = first + static_cast<int>(scan_add(cnt, INT32_MAX));
     before = last - cnt;
     const uint64_t here = __ballot(pid >= before && pid < last);

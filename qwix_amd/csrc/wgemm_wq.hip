@@ -643,11 +643,10 @@ extern "C" int qwix_hip_gemm_bf16_wq_ws(const void* a, int64_t lda, const void* 
                            workspace, workspace_bytes);
 }
 
-extern "C" int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_bytes,
-                                            int64_t q_group_stride, int q_qtype, int64_t M, int64_t N, int64_t K,
-                                            int64_t group, const void* s, int s_dtype, int64_t s_group_stride,
-                                            const int32_t* group_sizes, int64_t G, void* out, int out_dtype, int64_t ldo,
-                                            void* stream) {
+static int wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int64_t q_group_stride, int q_qtype,
+                     int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype, int64_t s_group_stride,
+                     const int32_t* group_sizes, int64_t G, int64_t stream_rows, void* out, int out_dtype, int64_t ldo,
+                     void* stream) {
   if (const int rc = check_wq_args(a, lda, q, ldq_bytes, q_qtype, M, N, K, group, s, s_dtype, nullptr, out, out_dtype, ldo))
     return rc;
   if (!group_sizes || G <= 0 || G > 65536)
@@ -657,7 +656,13 @@ extern "C" int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const vo
                 (long long)q_group_stride, (long long)s_group_stride);
   if ((M / 128 + G + 1) * ((N + 63) / 64) >= (int64_t{1} << 30))
     return fail(QWIX_ERR_UNSUPPORTED, "too many tiles (M=%lld N=%lld G=%lld)", (long long)M, (long long)N, (long long)G);
-  const Ragged rg{group_sizes, static_cast<int>(G), q_group_stride, s_group_stride};
+  if (stream_rows > 0) {
+    if (const int rc = gemv_wq_groups(a, lda, q, ldq_bytes, q_group_stride, q_qtype, M, N, K, group, s, s_dtype, s_group_stride,
+                                      group_sizes, G, stream_rows, out, out_dtype, ldo, stream))
+      return rc;
+    if (stream_rows >= M) return QWIX_OK;
+  }
+  const Ragged rg{group_sizes, static_cast<int>(G), q_group_stride, s_group_stride, static_cast<int>(stream_rows)};
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Up to 80 rows per group on average most groups fit 128 rows; 64-column tiles while 128-column ones would occupy at most
   // half of the CUs.  Tiles of 128 x 64 / 256 x 128, 64 and 96 rows per group on average, some groups up to half as many
@@ -696,4 +701,23 @@ extern "C" int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const vo
 #undef QWIX_WQR_TILE
 #undef QWIX_WQR
   return check_launch("gemm_bf16_wq (ragged)");
+}
+
+extern "C" int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_bytes,
+                                            int64_t q_group_stride, int q_qtype, int64_t M, int64_t N, int64_t K,
+                                            int64_t group, const void* s, int s_dtype, int64_t s_group_stride,
+                                            const int32_t* group_sizes, int64_t G, void* out, int out_dtype, int64_t ldo,
+                                            void* stream) {
+  return wq_ragged(a, lda, q, ldq_bytes, q_group_stride, q_qtype, M, N, K, group, s, s_dtype, s_group_stride, group_sizes, G, 0,
+                   out, out_dtype, ldo, stream);
+}
+
+// Two launches over the same group sizes, each with the groups of its kind.
+extern "C" int qwix_hip_gemm_wq_groups(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int64_t q_group_stride,
+                                       int q_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
+                                       int64_t s_group_stride, const int32_t* group_sizes, int64_t G, int64_t stream_rows,
+                                       void* out, int out_dtype, int64_t ldo, void* stream) {
+  if (stream_rows < 0) return fail(QWIX_ERR_INVALID_ARGUMENT, "stream_rows=%lld is negative", (long long)stream_rows);
+  return wq_ragged(a, lda, q, ldq_bytes, q_group_stride, q_qtype, M, N, K, group, s, s_dtype, s_group_stride, group_sizes, G,
+                   std::min(stream_rows, M), out, out_dtype, ldo, stream);
 }

@@ -4,6 +4,8 @@ int8 x int8: the int32 sums are exact and the epilogue is elementwise, so output
 bit.  e4m3 x e4m3: the matrix instruction's internal accumulation differs from the oracle's single
 rounding of an exact sum (up to 1e-4 of the largest output), so outputs are compared at rtol 1e-2 for
 bf16 results and 1e-3 for f32 results, the tolerances of the dense fp8 GEMM tests."""
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -255,28 +257,58 @@ def test_ragged_dot_weight_only_skewed(G, N, M, sizes, wq_type):
     (2, 640, 264, 600, (256, 300)),                     # ten slabs, 64-column tiles of 256 rows
     (2, 1152, 18440, 514, (257, 257)),                  # 128-column tiles of 256 rows
     (70, 384, 72, 5000, tuple(-3 if g == 5 else 2 ** 31 - 1 if g == 69 else 70 + g % 3 for g in range(70))),  # past 64 groups
+    (300, 256, 72, 20000, tuple(-1 if g == 7 else 0 if g % 50 == 3 else 2 ** 31 - 1 if g == 297 else 60 + g % 140 if g % 3 else 17
+                                for g in range(300))),   # past 256 groups, the last one cut at the last row
 ])
 @pytest.mark.parametrize('wq_type,tiled,dtype', [('int4', {1: 128}, O.BF16), ('int8', {1: 128}, O.BF16), ('int8', None, O.F32),
                                                  ('float8_e4m3fn', {1: 128}, O.F32), ('int4', None, O.F32)])
-def test_ragged_dot_weight_only_tiles(G, K, N, M, sizes, wq_type, tiled, dtype):
-  """Too many rows per group to stream the weights: tiles of 128 and 256 rows that dequantize their group's weights to bf16, as
-  `dequantize` gives them.  f32 results are off by their f32 sums (below 1e-5 of the largest), bf16 results by half a step."""
+@pytest.mark.parametrize('most', [None, 0, 70, 130])
+def test_ragged_dot_weight_only_tiles(G, K, N, M, sizes, wq_type, tiled, dtype, most, monkeypatch):
+  """Too many rows to stream the weights of all groups: those of up to `streamed_rows` rows (and of `most`, also none) are streamed,
+  their weights unrounded; tiles of 128 and 256 rows dequantize the others' to bf16, as `dequantize` gives them.  f32 results
+  are off by their f32 sums (below 1e-5 of the largest), bf16 results by half a step."""
   import qwix_amd
+  from qwix_amd.core import dot_general as dg
+  if most is None:
+    most = dg.streamed_rows(N, wq_type == 'int4', K, 128 if tiled else K)
+  else:
+    monkeypatch.setattr(dg, 'streamed_rows', lambda *a: most)
   _, x = util.make((M, K), O.BF16, seed=93)
   _, w = util.make((G, K, N), dtype, seed=94, scale=0.05)
   wq = qwix_amd.quantize(w, wq_type, channelwise_axes=[0, 2], tiled_axes=tiled or {})
-  d = qwix_amd.dequantize(wq).to(torch.bfloat16).to(torch.float64)
+  rounded = qwix_amd.dequantize(wq).to(torch.bfloat16).to(torch.float64)
+  codes = (wq.qvalue.unpack() if wq_type == 'int4' else wq.qvalue).to(torch.float64)
+  exact = codes * wq.scale.to(torch.float64).repeat_interleave(K // wq.scale.shape[1], 1)
   want, start = torch.zeros(M, N, dtype=torch.float64, device=x.device), 0
   for g, size in enumerate(sizes):
     stop = min(start + max(size, 0), M)
-    want[start:stop] = x[start:stop].to(torch.float64) @ d[g]
+    want[start:stop] = x[start:stop].to(torch.float64) @ (exact if stop - start <= most else rounded)[g]
     start = stop
   largest = float(want.abs().max())
   out = qwix_amd.core.ragged_dot._weight_only_groups(x, wq, _sizes(sizes), torch.float32)
   assert float((out.to(torch.float64) - want).abs().max()) <= 1e-5 * largest
-  low = qwix_amd.ragged_dot(x, wq, _sizes(sizes), preferred_element_type=torch.bfloat16)
+  low = qwix_amd.core.ragged_dot._weight_only_groups(x, wq, _sizes(sizes), torch.bfloat16)
   assert bool(((low.to(torch.float64) - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * largest).all())
   assert not out[start:].any()
+
+
+@pytest.mark.parametrize('K,N,sizes,streamed', [(512, 136, (64, 300, 20, 200), (0, 2)), (384, 72, (256, 17, 257, 0), (0, 1))])
+@pytest.mark.parametrize('wq_type', ['int4', 'int8', 'float8_e4m3fn'])
+def test_small_groups_keep_their_weights_unrounded_beside_large_ones(K, N, sizes, streamed, wq_type):
+  """What a group's weights are rounded to does not depend on the other groups' rows: up to 64 rows (256 with K of 128 mod 256)
+  f32 sums of unrounded weights, (K / 16 + 16) roundings of 2^-24 of the terms' magnitude."""
+  import qwix_amd
+  _, x = util.make((sum(sizes), K), O.BF16, seed=95)
+  _, w = util.make((len(sizes), K, N), O.F32, seed=96, scale=0.05)
+  wq = qwix_amd.quantize(w, wq_type, channelwise_axes=[0, 2], tiled_axes={1: 128})
+  out = qwix_amd.ragged_dot(x, wq, _sizes(sizes), preferred_element_type=torch.float32).to(torch.float64)
+  want = _grouped_reference(x, wq, sizes)
+  codes = wq.qvalue.unpack() if wq_type == 'int4' else wq.qvalue
+  terms = _grouped_reference(x.abs(), types.SimpleNamespace(qtype='int8', qvalue=codes.to(torch.float32).abs(), scale=wq.scale), sizes)
+  bound = (K / 16 + 16) * 2.0 ** -24 * terms
+  for g in streamed:
+    rows = slice(sum(sizes[:g]), sum(sizes[:g + 1]))
+    assert bool(((out - want).abs() <= bound)[rows].all()), (g, float(((out - want).abs() / terms)[rows].max()))
 
 
 @pytest.mark.parametrize('G,K,rows', [(65, 256, 60), (130, 128, 130), (64, 144, 3)])
