@@ -163,7 +163,12 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
 
   def _planned(self, op: str, arg, rule, lhs, rhs, ordinary):
     """One launch plan for the whole of an operation: the quantization of its activations and the contraction.  Only with the
-    stock kernels, dynamic ranges and a weight that is quantized already; `ordinary()` otherwise, and until the plan is kept."""
+    stock kernels and the stock policy (nothing that `ordinary` runs is overridden: plans are shared by all providers), dynamic
+    ranges and a weight that is quantized already; `ordinary()` otherwise, and until the plan is kept."""
+    cls = type(self)
+    if ((cls._prepare, cls._fusable, cls._quantized_dot_general, cls._quantized_einsum) != _STOCK_POLICY
+        or not _POLICY.isdisjoint(self.__dict__)):
+      return ordinary()
     w = rhs.value if isinstance(rhs, Param) else rhs
     boxed = isinstance(w, WithAux)
     if boxed:
@@ -229,6 +234,11 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
                                 ndims=(len(lhs.shape), len(rhs.shape)), tile_size=rule.tile_size)
     lhs, rhs = self._prepare(lhs, rhs, rule, op_id, get_how)
     return self._einsum_fn(einsum_str, lhs, rhs)
+
+
+_POLICY = frozenset(('_prepare', '_fusable', '_quantized_dot_general', '_quantized_einsum'))
+_STOCK_POLICY = (BoxedParamProvider._prepare, BoxedParamProvider._fusable, BoxedParamProvider._quantized_dot_general,
+                 BoxedParamProvider._quantized_einsum)
 
 
 class PtqProvider(BoxedParamProvider):

@@ -386,7 +386,7 @@ def test_a_provider_s_operation_is_one_plan(scheme):
   def attend(params, q, k):
     return nn.ops.einsum('bqd,bkd->bqk', q, k)
   scores = qwix_amd.quantize_model(attend, provider)
-  ordinary, planned = qwix_amd.PtqProvider._planned, []
+  ordinary, calls = qwix_amd.PtqProvider._planned, []
   for i in range(plans.RECORD_AT + 3):
     for rows in (3, 40):
       x, q, k = _rand((rows, 256), 7 * i + rows), _rand((2, rows, 128), 5 * i + rows), _rand((2, 48, 128), 3 * i)
@@ -398,11 +398,64 @@ def test_a_provider_s_operation_is_one_plan(scheme):
         qwix_amd.PtqProvider._planned = ordinary
       for a, b in zip(got, want):
         _same(a, b)
-  prepare, provider._prepare = provider._prepare, lambda *a, **k: planned.append(a) or prepare(*a, **k)
-  mlp.apply(params, x)
-  if act:
-    scores.apply({}, q, k)
-  assert not planned, 'no plan is kept for an operation of the model'
+  call, _lib.call = _lib.call, lambda *a: calls.append(a[0]) or call(*a)
+  try:
+    mlp.apply(params, x)
+    if act:
+      scores.apply({}, q, k)
+  finally:
+    _lib.call = call
+  assert not calls, 'no plan is kept for an operation of the model'
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('first', ['stock', 'subclass', 'instance'])
+@pytest.mark.parametrize('op', ['einsum', 'dot_general'])
+def test_a_provider_s_own_policy_is_not_replaced_by_a_plan(op, first):
+  """Providers that quantize to another type than their rule says beside the stock one, on equal shapes, whichever comes first: each
+  gets its own results on every call."""
+  import dataclasses
+  import qwix_amd
+  from qwix_amd import nn
+  _empty_the_table()
+
+  def another(prepare):
+    return lambda lhs, rhs, rule, *rest, **kw: prepare(lhs, rhs, dataclasses.replace(rule, act_qtype='float8_e4m3fn'), *rest, **kw)
+
+  class Other(qwix_amd.PtqProvider):
+    def _prepare(self, *args, **kw):
+      return another(super()._prepare)(*args, **kw)
+
+    def _fusable(self, rule):
+      return None
+
+  def run(provider, a, b):
+    fn = ((lambda params, q, k: nn.ops.einsum('bqd,bkd->bqk', q, k)) if op == 'einsum' else
+          (lambda params, q, k: nn.ops.dot_general(q[0], k[0], (((1,), (1,)), ((), ())))))
+    return qwix_amd.quantize_model(fn, provider).apply({}, a, b)
+  rule = qwix_amd.QuantizationRule(module_path='.*', weight_qtype='int8', act_qtype='int8')
+  providers = {'stock': qwix_amd.PtqProvider([rule]), 'subclass': Other([rule]), 'instance': qwix_amd.PtqProvider([rule])}
+  own = providers['instance']
+  own._prepare, own._fusable = another(own._prepare), lambda rule: None
+  # the same arithmetic under another identity of the module: no plan of a whole operation is kept for it
+  plain = {name: qwix_amd.PtqProvider([dataclasses.replace(rule, act_qtype='int8' if name == 'stock' else 'float8_e4m3fn')],
+                                      _qarray_module=_OrdinaryModule()) for name in providers}
+  order = [first] + [name for name in providers if name != first]
+  for i in range(plans.RECORD_AT + 3):   # in turn
+    a, b = _rand((2, 24, 128), 3 * i), _rand((2, 40, 128), 3 * i + 1)
+    for name in order:
+      assert torch.equal(run(providers[name], a, b), run(plain[name], a, b)), (name, i)
+  for name in order:   # ... and one after the other
+    for i in range(plans.RECORD_AT + 1):
+      a, b = _rand((2, 56, 128), 3 * i), _rand((2, 72, 128), 3 * i + 1)
+      assert torch.equal(run(providers[name], a, b), run(plain[name], a, b)), (name, i)
+
+
+class _OrdinaryModule:
+
+  def __getattr__(self, name):
+    from qwix_amd.core import qarray
+    return getattr(qarray, name)
 
 
 @pytest.mark.gpu
