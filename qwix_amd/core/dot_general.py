@@ -454,50 +454,105 @@ def _tile_by_tile(lhs, rhs, dimension_numbers, tiled, preferred_element_type, ex
   return total.to(cur).to(res_t)
 
 
+class _Kept:
+  """Tensors made once from a weight and kept for later calls, which may come on other streams: they wait for the work that made the
+  tensors, and a tensor that is let go is not reused under them."""
+
+  __slots__ = ('tensors', 'stream', 'event')
+
+  def __init__(self, *tensors: torch.Tensor):
+    self.tensors = tensors
+    self.stream = self.event = None
+    if tensors[0].is_cuda:
+      self.stream = _lib.stream_of(tensors[0])
+      self.event = torch.cuda.Event()
+      self.event.record(torch.cuda.current_stream(tensors[0].device))
+
+  def ready(self) -> bool:
+    """Whether the current stream can read them now, its wait included.  (A graph that is being captured can wait for nothing
+    outside it, nor ask: False until an ordinary call has seen the work done.)"""
+    if self.stream is None:
+      return True
+    other = _lib.stream_of(self.tensors[0]) != self.stream
+    if self.event is not None:
+      if torch.cuda.is_current_stream_capturing():
+        return False
+      if self.event.query():
+        self.event = None
+      elif other:
+        torch.cuda.current_stream(self.tensors[0].device).wait_event(self.event)
+    if other:
+      for t in self.tensors:
+        t.record_stream(torch.cuda.current_stream(t.device))
+    return True
+
+
+def _may_be_kept(*sources: torch.Tensor) -> bool:
+  """Whether something made from these may serve later calls: not what a graph that is being captured will make at each replay, nor
+  what no version counter watches over."""
+  return not (any(t.is_inference() for t in sources) or (sources[0].is_cuda and torch.cuda.is_current_stream_capturing()))
+
+
+def _state_of(t: torch.Tensor) -> tuple:
+  """Changes when a kept tensor's contents (`copy_`, `neg_`) or memory (`t.data = other`) do.  Writes that torch does not count, through
+  `t.data` or a raw pointer, need `forget_weight`."""
+  return (t._version, t.data_ptr(), t.stride())
+
+
 # K-sums of a weight's quantized values (the zero-point correction of an asymmetric activation, dot_general.py:228-253,
 # multiplies them with the activation's zero points): weights are static, so the sums are kept per values tensor while it
-# is alive and unchanged (identity + torch version counter; entries leave with their tensor).
+# is alive and unchanged (entries leave with their tensor): (id, axes and sizes) -> (weak reference, state, _Kept).  The entry is
+# also found by (id, dimension numbers), for calls that hand the sums to their launch plan as an operand.
 _KSUM_CACHE: dict = {}
 
 
-def _weight_ksums(values_owner, b: torch.Tensor, key_extra: tuple, compute) -> torch.Tensor:
-  """`values_owner`: the tensor object the weight's QArray holds (its identity and version key the entry; `b` may be a
+def _kept_ksums(store: torch.Tensor, key: tuple) -> torch.Tensor | None:
+  hit = _KSUM_CACHE.get(key)
+  if hit is None or hit[0]() is not store or hit[1] != _state_of(store) or not hit[2].ready():
+    return None
+  return hit[2].tensors[0]
+
+
+def _weight_ksums(values_owner, b: torch.Tensor, key_extra: tuple, compute, dimension_numbers=None) -> torch.Tensor:
+  """`values_owner`: the tensor object the weight's QArray holds (its identity and state key the entry; `b` may be a
   re-laid-out copy of it); `compute()` launches the sum kernel and returns the result."""
   store = values_owner.data if isinstance(values_owner, Int4Tensor) else values_owner
   key = (id(store),) + key_extra
-  hit = _KSUM_CACHE.get(key)
-  if hit is not None and hit[0]() is store and hit[1] == store._version:
-    return hit[2]
-  out = compute()
-  plans.kept_aside()
-  _KSUM_CACHE[key] = (weakref.ref(store, lambda _, k=key: _KSUM_CACHE.pop(k, None)), store._version, out)
+  may = _may_be_kept(store)
+  out = None if store.is_inference() else _kept_ksums(store, key)
+  if out is None:
+    out = compute()
+    plans.kept_aside()
+    if may:
+      _KSUM_CACHE[key] = (weakref.ref(store, lambda _, k=key: _KSUM_CACHE.pop(k, None)), _state_of(store), _Kept(out))
+  if may and dimension_numbers is not None:
+    try:
+      name = (id(store), dimension_numbers)
+      _KSUM_CACHE[name] = (weakref.ref(store, lambda _, k=name: _KSUM_CACHE.pop(k, None)),) + _KSUM_CACHE[key][1:]
+    except TypeError:   # dimension numbers as lists: no plan is kept for such a call
+      pass
   return out
 
 
-# The same sums by the weight's values and the call's dimension numbers: a call that finds them hands them to its launch plan as
-# an operand.
-_KSUM_NAMES: dict = {}
-
-
-def _name_ksums(values_owner, dimension_numbers, sums: torch.Tensor) -> None:
-  store = values_owner.data if isinstance(values_owner, Int4Tensor) else values_owner
-  try:
-    key = (id(store), dimension_numbers)
-    _KSUM_NAMES[key] = (weakref.ref(store, lambda _, k=key: _KSUM_NAMES.pop(k, None)), store._version, sums)
-  except TypeError:   # dimension numbers as lists: no plan is kept for such a call
-    pass
-
-
-def _named_ksums(lhs, rhs, dimension_numbers):
+def _named_ksums(rhs, dimension_numbers):
   """The kept K-sums of an asymmetric lhs's weight while that is alive and unchanged, else None."""
-  if not (isinstance(lhs, QArray) and lhs.zero_point is not None and isinstance(rhs, QArray)
-          and type(rhs.qvalue) is torch.Tensor and _KSUM_NAMES):
+  store = rhs.qvalue if isinstance(rhs, QArray) else None
+  if type(store) is not torch.Tensor or store.is_inference():
     return None
   try:
-    hit = _KSUM_NAMES.get((id(rhs.qvalue), dimension_numbers))
+    return _kept_ksums(store, (id(store), dimension_numbers))
   except TypeError:
     return None
-  return hit[2] if hit is not None and hit[0]() is rhs.qvalue and hit[1] == rhs.qvalue._version else None
+
+
+def forget_weight(w: QArray) -> None:
+  """Drops what is kept for a weight.  Needed only after writes to its tensors that torch does not count: through `tensor.data` or a raw
+  pointer (`copy_` and the like, and other memory under `tensor.data = ...`, are noticed)."""
+  stores = [t.data if isinstance(t, Int4Tensor) else t for t in (w.qvalue, w.scale, w.zero_point) if t is not None]
+  ids = {id(w), *map(id, stores)}
+  for table in (_KSUM_CACHE, _ZP8_CACHE, _DECODE_PLANS):
+    for key in [k for k in table if (k[0] if isinstance(k, tuple) else k) in ids]:
+      table.pop(key, None)
 
 
 def _fast_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, *, exact: bool = False,
@@ -586,8 +641,7 @@ def _fast_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, 
           zv = torch.empty(c.N, dtype=torch.int32, device=dev)
           _lib.call('qwix_hip_ksum_i8', b.data_ptr(), b.stride(0), c.N, K, zv.data_ptr(), st)
           return zv
-        zv = _weight_ksums(rhs.qvalue, b, (tuple(c.rca), tuple(c.rfree), K), ksum)
-        _name_ksums(rhs.qvalue, dimension_numbers, zv)
+        zv = _weight_ksums(rhs.qvalue, b, (tuple(c.rca), tuple(c.rfree), K), ksum, dimension_numbers)
       else:
         zv = c.rhs_zero_point(rhs)[0].reshape(c.N)
         zu = torch.empty(c.M, dtype=torch.int32, device=dev)
@@ -1029,16 +1083,14 @@ def dot_general(lhs: MaybeQ, rhs: MaybeQ, dimension_numbers: DotDimensionNumbers
     return _dot_general(lhs, rhs, dimension_numbers, preferred_element_type, **kwargs)
   # (which weight-only kernel runs is decided by `fused_wq_min_rows`: another rule, other plans)
   fixed = ('dot', dimension_numbers, preferred_element_type, fused_wq_min_rows)
-  operands = (lhs, rhs)
-  if type(lhs) is QArray and lhs.zero_point is not None:
-    sums = _named_ksums(lhs, rhs, dimension_numbers)
-    if sums is not None:
-      operands = (lhs, rhs, sums)
-  out = (plans._native or plans.native()).run(fixed, *operands)
+  run = (plans._native or plans.native()).run
+  sums = _named_ksums(rhs, dimension_numbers) if type(lhs) is QArray and lhs.zero_point is not None else None
+  out = run(fixed, lhs, rhs) if sums is None else run(fixed, lhs, rhs, sums)
   if out is None:
     return _dot_general(lhs, rhs, dimension_numbers, preferred_element_type)
   return out if out is not True else plans.record(
-      fixed, operands, lambda: _dot_general(lhs, rhs, dimension_numbers, preferred_element_type), plans.single)
+      fixed, (lhs, rhs) if sums is None else (lhs, rhs, sums),
+      lambda: _dot_general(lhs, rhs, dimension_numbers, preferred_element_type), plans.single)
 
 
 def _dot_general(lhs: MaybeQ, rhs: MaybeQ, dimension_numbers, preferred_element_type=None, **kwargs) -> torch.Tensor:

@@ -48,6 +48,7 @@ def native():
 
 
 _ALLOCATIONS = frozenset(('aten::empty.memory_format', 'aten::empty_strided', 'aten::empty_like', 'aten::new_empty'))
+_ON_THE_HOST = frozenset(('aten::promote_types', 'aten::record_stream'))   # dtypes alone; the allocator's book-keeping
 
 
 def _storages(values) -> set:
@@ -101,7 +102,7 @@ class Recorder(TorchDispatchMode):
     name = func._schema.name + ('.' + func._schema.overload_name if func._schema.overload_name else '')
     if name in _ALLOCATIONS:
       self.buffers.append(out)
-    elif name != 'aten::promote_types' and not _is_view(func, args, out):   # (that one works on dtypes alone)
+    elif name not in _ON_THE_HOST and not _is_view(func, args, out):
       self.ok = False
     return out
 

@@ -369,6 +369,87 @@ def test_asymmetric_rows_replay_with_their_weight_s_sums():
   _same(qwix_amd.dot_general(x, w, dn), dg._dot_general(x, qwix_amd.QArray(w.qvalue.clone(), w.scale, None, w.qtype), dn))
 
 
+def _by_hand(x, w):
+  """dot_general of one asymmetric and one symmetric array in 64 bits, rounded once (bf16 scales: exact products of integers)."""
+  a = (x.qvalue.to(torch.float64) - x.zero_point.to(torch.float64)) * x.scale.to(torch.float64)
+  return a @ (w.qvalue.to(torch.float64) * w.scale.to(torch.float64))
+
+
+def _close(out, want):
+  return bool(((out.to(torch.float64) - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -7 * want.abs().mean()).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('planned', [False, True])
+@pytest.mark.parametrize('change', ['copy_', 'other memory', 'other order', 'forget_weight'])
+def test_a_weight_s_sums_follow_its_changes(planned, change):
+  """Zero points far from 0 multiply the sums: a result with another weight's sums is off by far more than the rounding of its
+  bf16 steps."""
+  import qwix_amd
+  from qwix_amd.core import dot_general as dg
+  _empty_the_table()
+  x = qwix_amd.quantize(_rand((40, 256), 1) + 3, 'int8', channelwise_axes=[0], calibration_method='minmax')
+  w = qwix_amd.quantize(_rand((256, 256), 2) + 1, 'int8', channelwise_axes=[1])
+  for _ in range(plans.RECORD_AT + 2 if planned else 1):
+    assert _close(qwix_amd.dot_general(x, w, _DN), _by_hand(x, w))
+  other = (-w.qvalue).roll(5, 0) // 2
+  if change == 'copy_':
+    w.qvalue.copy_(other)
+  elif change == 'other memory':
+    w.qvalue.data = other.t().contiguous().t()
+  elif change == 'other order':
+    w.qvalue.data = w.qvalue.data.t()
+  else:
+    w.qvalue.data.copy_(other)
+    dg.forget_weight(w)
+  assert _close(qwix_amd.dot_general(x, w, _DN), _by_hand(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('planned', [False, True])
+def test_a_weight_s_sums_are_awaited_on_another_stream(planned):
+  """The first call's stream is still busy when a call on another one wants the sums that it will compute."""
+  import qwix_amd
+  _empty_the_table()
+  x, w = _asymmetric(3, 256, 4096)
+  if planned:
+    for i in range(plans.RECORD_AT + 2):
+      a, b = _asymmetric(30 + i, 256, 4096)
+      for _ in range(2):
+        qwix_amd.dot_general(a, b, _DN)
+  want = _by_hand(x, w)
+  first, second = torch.cuda.Stream(), torch.cuda.Stream()
+  with torch.cuda.stream(first):   # what an allocation for the sums finds there
+    torch.full((4096,), 1 << 20, dtype=torch.int32, device=util.DEV)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(first):
+    torch.cuda._sleep(200_000_000)
+    qwix_amd.dot_general(x, w, _DN)
+  with torch.cuda.stream(second):
+    out = qwix_amd.dot_general(x, w, _DN)
+  torch.cuda.synchronize()
+  assert _close(out, want)
+
+
+@pytest.mark.gpu
+def test_a_weight_s_sums_and_a_captured_graph():
+  """Sums that only the replay computes are no other call's: the first use of a weight is captured, the next one is not."""
+  import qwix_amd
+  _empty_the_table()
+  x, w = _asymmetric(5, 256, 512)
+  warm = _asymmetric(6, 256, 512)
+  qwix_amd.dot_general(*warm, _DN)
+  torch.cuda.synchronize()
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    captured = qwix_amd.dot_general(x, w, _DN)
+  assert _close(qwix_amd.dot_general(x, w, _DN), _by_hand(x, w))
+  for _ in range(3):
+    graph.replay()
+    assert _close(captured, _by_hand(x, w))
+    assert _close(qwix_amd.dot_general(*warm, _DN), _by_hand(*warm))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('scheme', [('int8', 'int8', None), ('float8_e4m3fn', 'float8_e4m3fn', 128), ('int4', None, 128)])
 def test_a_provider_s_operation_is_one_plan(scheme):
