@@ -730,12 +730,13 @@ def _rhs_zero_point_i8(c: '_Canon', rhs: QArray) -> tuple[torch.Tensor, int]:
       return p.view(gz, c.N), gz
   key = (id(z), tuple(c.rca), tuple(c.rfree))
   hit = _ZP8_CACHE.get(key)
-  if hit is not None and hit[0]() is z and hit[1] == z._version:
-    return hit[2], hit[3]
+  if hit is not None and hit[0]() is z and hit[1] == _state_of(z) and hit[2].ready():
+    return hit[2].tensors[0], hit[3]
   z32, gz = c.rhs_zero_point(rhs)
   zp = z32.to(torch.int8).contiguous()
   plans.kept_aside()
-  _ZP8_CACHE[key] = (weakref.ref(z, lambda _, k=key: _ZP8_CACHE.pop(k, None)), z._version, zp, gz)
+  if _may_be_kept(z):
+    _ZP8_CACHE[key] = (weakref.ref(z, lambda _, k=key: _ZP8_CACHE.pop(k, None)), _state_of(z), _Kept(zp), gz)
   return zp, gz
 
 
@@ -807,34 +808,39 @@ _DECODE_PLANS: dict = {}
 
 
 def _weight_signature(rhs: QArray) -> tuple:
-  """Identity and torch version counter of every tensor a kept plan may hold a re-laid-out COPY of: an in-place update
-  (`copy_`, a state reload into existing tensors) keeps the object and bumps the counter."""
+  """Identity and state of every tensor a kept plan may hold a view or a re-laid-out COPY of: an in-place update
+  (`copy_`, a state reload into existing tensors) keeps the object and bumps the version counter, other memory under it moves."""
   def sig(t):
     if t is None:
       return None
     store = t.data if isinstance(t, Int4Tensor) else t
-    return (id(t), id(store), store._version)
+    return (id(t), id(store), *_state_of(store))
   return (sig(rhs.qvalue), sig(rhs.scale), sig(rhs.zero_point))
 
 
 def _decode_plan(lhs, rhs, dimension_numbers):
   key = id(rhs)
   hit = _DECODE_PLANS.get(key)
-  if hit is not None and hit[0]() is rhs and hit[1] == _weight_signature(rhs):
+  if hit is not None and hit[0]() is rhs and hit[1] == _weight_signature(rhs) and (hit[3] is None or hit[3].ready()):
     return hit[2]
-  plan = None
+  plan = copies = None
   c = _weight_only_fit(lhs, rhs, dimension_numbers)
   if c is not None:
     b, b_is4 = c.rhs_values(rhs)
     sb, gb = c.rhs_scale(rhs)
     zp = _rhs_zero_point_i8(c, rhs)[0] if rhs.zero_point is not None else None
     values = rhs.qvalue.data if b_is4 else rhs.qvalue
-    if any(kept.untyped_storage().data_ptr() != own.untyped_storage().data_ptr() for kept, own in ((b, values), (sb, rhs.scale))):
-      plans.kept_aside()
+    made = [t for t, own in ((b, values), (sb, rhs.scale), (zp, rhs.zero_point))
+            if t is not None and t.untyped_storage().data_ptr() != own.untyped_storage().data_ptr()]
     plan = (b, numerics.qtype_tag(_qtype_of(rhs)), sb, _lib.float_tag(sb.dtype), zp, c.N, c.K, c.K // gb,
             streamed_rows(c.N, b_is4, c.K, c.K // gb))
+    if made:
+      plans.kept_aside()
+      if not _may_be_kept(values, rhs.scale):
+        return plan
+      copies = _Kept(*made)
   _DECODE_PLANS[key] = (weakref.ref(rhs, lambda _, k=key: _DECODE_PLANS.pop(k, None)),
-                        _weight_signature(rhs), plan)
+                        _weight_signature(rhs), plan, copies)
   return plan
 
 

@@ -1,5 +1,6 @@
 """Launch plans: what the recorder accepts (CPU), and that replayed calls give what the ordinary path gives (GPU)."""
 import _thread
+import dataclasses
 import functools
 import sys
 import threading
@@ -432,6 +433,39 @@ def test_a_weight_s_sums_are_awaited_on_another_stream(planned):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('inference', [False, True])
+@pytest.mark.parametrize('qtype,layout', [('int8', 'natural'), ('int4', 'natural'), ('int8', 'reduce_minor'), ('int4', 'reduce_minor')])
+def test_a_weight_s_kept_layout_follows_other_memory_and_streams(qtype, layout, inference):
+  """What a weight-only call keeps of its weight (a transposed copy, a view) under 'tensor.data = other', and for a call on another
+  stream while the one that makes the copy is busy."""
+  import qwix_amd
+  from qwix_amd.core import dot_general as dg
+  make = lambda seed: qwix_amd.quantize(_rand((512, 200), seed, std=0.05), qtype, channelwise_axes=[1], tiled_axes={0: 128}, layout=layout)
+  store = lambda w: w.qvalue.data if qtype == 'int4' else w.qvalue
+  x, w, other = _rand((5, 512), 1), make(2), make(3)
+  fresh = lambda w: dg._slow_dot_general(x, dataclasses.replace(w), _DN)   # an object of its own: nothing is kept for it yet
+  with torch.inference_mode(inference):
+    assert torch.equal(dg._dot_general(x, w, _DN), fresh(w))
+  store(w).data = store(other).clone(memory_format=torch.preserve_format)
+  w.scale.data = other.scale.clone()
+  with torch.inference_mode(inference):
+    assert torch.equal(dg._dot_general(x, w, _DN), fresh(other))
+  late = make(4)
+  want = fresh(late)
+  first, second = torch.cuda.Stream(), torch.cuda.Stream()
+  with torch.cuda.stream(first):
+    torch.full((512, 200), 127, dtype=torch.int8, device=util.DEV)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(first):
+    torch.cuda._sleep(200_000_000)
+    dg._dot_general(x, late, _DN)
+  with torch.cuda.stream(second):
+    out = dg._dot_general(x, late, _DN)
+  torch.cuda.synchronize()
+  assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
 def test_a_weight_s_sums_and_a_captured_graph():
   """Sums that only the replay computes are no other call's: the first use of a weight is captured, the next one is not."""
   import qwix_amd
@@ -495,7 +529,6 @@ def test_a_provider_s_operation_is_one_plan(scheme):
 def test_a_provider_s_own_policy_is_not_replaced_by_a_plan(op, first):
   """Providers that quantize to another type than their rule says beside the stock one, on equal shapes, whichever comes first: each
   gets its own results on every call."""
-  import dataclasses
   import qwix_amd
   from qwix_amd import nn
   _empty_the_table()
