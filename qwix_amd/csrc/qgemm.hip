@@ -686,7 +686,7 @@ static int qgemm_impl(const void* a, int64_t lda, const void* b, int64_t ldb, in
                       const int32_t* zv, void* out, int out_dtype, int64_t ldo, void* stream, void* workspace = nullptr,
                       size_t workspace_bytes = 0, bool zu8 = false);
 static int splitk_plan(int64_t M, int64_t N, int64_t K, double other_us, double* model_us = nullptr);
-static bool splits_in_workgroup(int64_t M, int64_t N, int64_t K, bool few_rows, double tiled_us, bool can_split);
+static bool splits_in_workgroup(int64_t M, int64_t N, int64_t K, bool few_rows, double other_us);
 // Problems of up to this many 128 x 128 tiles take 64 x 64 tiles (four times the workgroups).  Measured, int8 and
 // e4m3, bf16 result, weights in the second-level cache / from HBM: 256 x 4096 over K 1024 9.5 -> 5.6 / 12.1 -> 8.4 us,
 // 1024^3 9.3 -> 5.4 / 11.7 -> 8.2, 512 x 4096 over K 4096 23.5 -> 16.2 / 34.9 -> 26.8, 1536 x 2048 over K 2048 (192
@@ -1000,21 +1000,19 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, double other_us, double*
 // 256 x 1024 over K 4096 9.4 us, 59 x 4096 over K 4096 9.5, 33 x 8192 over K 8192 18.3, 100 x 4096 over K 14336 25.3; 200 x 3072 over K
 // 11264 25.3 with 64 rows).  Against several passes of the weight-streaming kernel over weights that do not stay in the
 // caches (33 rows: K 8192, N 8192 25.1 us, K 14336, N 4096 36.2, K 11264, N 3072 28.0) it is ahead from three passes on;
-// smaller weights are streamed faster (59 x 1024 over K 4096 7.0 us); otherwise the models decide, the split-K kernel's with 1.5
-// us on top (100 x 1024 over K 8192: 16.6 us, model 14.5).  Up to 32 rows, and up to 63 where only 64-row tiles are one round, the
+// smaller weights are streamed faster (59 x 1024 over K 4096 7.0 us); otherwise the models decide: `other_us` is the tiled
+// kernels', or where K can be split through a workspace that kernel's with 1.5 us on top (100 x 1024 over K 8192: 16.6 us, model 14.5).  Up to 32 rows, and up to 63 where only 64-row tiles are one round, the
 // one-tile-row kernel is level or ahead (17 rows: N 8192 over K 8192 17.1 against 19.4 us; 33 rows, N 14336 over K 4096 17.1
 // against 18.0).
-static bool splits_in_workgroup(int64_t M, int64_t N, int64_t K, bool few_rows, double tiled_us, bool can_split) {
+static bool splits_in_workgroup(int64_t M, int64_t N, int64_t K, bool few_rows, double other_us) {
   if (M <= 16 || K <= 128) return false;
   const int64_t cols = (N + 63) / 64, low = (M + 31) / 32 * cols, high = (M + 63) / 64 * cols;
   if (K % 128 != 0) return qgemm_long_takes(M, N, K, 1);  // (the other way is the register-staged tile)
   if (M <= 32 || (M < 64 ? low : high) > 256) return false;
   if (few_rows) return N * K >= 12 << 20;
-  double other = tiled_us;
-  if (can_split && splitk_plan(M, N, K, tiled_us, &other) > 0) other += 1.5;
   const double steps = static_cast<double>((K / 128 + 3) / 4), read_us = static_cast<double>(N) * static_cast<double>(K) / 1.0e7;
   const double us = (low > 256 ? 6.2 + 0.75 * steps : 4.6 + 0.53 * steps) + read_us;
-  return us < 0.95 * other;
+  return us < 0.95 * other_us;
 }
 
 template <int QT>
@@ -1065,19 +1063,25 @@ static int qgemm_impl(const void* a, int64_t lda, const void* b, int64_t ldb, in
                       N * K >= (int64_t{8} << 20) && M * lda < (int64_t{1} << 31) && N * ldb < (int64_t{1} << 31);
   const bool few_rows = streams_weights(M, N, K, mid_ok);
   const bool off31 = M * lda < (int64_t{1} << 31) && N * ldb < (int64_t{1} << 31);
-  if (splits_in_workgroup(M, N, K, few_rows, tiled_us, workspace != nullptr) && zu == nullptr && out_dtype != QWIX_I32 && off31 && N % 4 == 0 && ldo % 4 == 0) {
+  // K in ranges through the workspace: only where the caller's holds them (a smaller one is as good as none, whichever kernel
+  // is chosen), and only against the tiled kernels: where the weight-streaming kernel is chosen its own model has spoken
+  double other_us = tiled_us;
+  int splits = 0;
+  if (workspace != nullptr && aligned16(workspace) && zu == nullptr && out_dtype != QWIX_I32 && off31 && !few_rows) {
+    double split_us = 0;
+    splits = splitk_plan(M, N, K, tiled_us, &split_us);
+    if (workspace_bytes < static_cast<size_t>(splits) * M * N * 4) splits = 0;
+    if (splits > 0) other_us = split_us + 1.5;
+  }
+  if (splits_in_workgroup(M, N, K, few_rows, other_us) && zu == nullptr && out_dtype != QWIX_I32 && off31 && N % 4 == 0 && ldo % 4 == 0) {
     const LongArgs p{static_cast<const uint8_t*>(a), lda, 0, static_cast<const uint8_t*>(b), ldb, 0, sa, sa_dtype, 0, sb, sb_dtype, 0,
                      ep.r0, ep.r1, ep.r2, static_cast<uint8_t*>(out), out_dtype, ldo, 0, static_cast<int>(M),
                      static_cast<int>(N), static_cast<int>(K)};
     return qgemm_long(qtype, p, 1, stream);
   }
-  if (workspace != nullptr && zu == nullptr && out_dtype != QWIX_I32 && off31) {
-    // only against the tiled kernels: where the weight-streaming kernel is chosen its own model has spoken
-    const int splits = few_rows ? 0 : splitk_plan(M, N, K, tiled_us);
-    if (splits > 0 && workspace_bytes >= static_cast<size_t>(splits) * M * N * 4 && aligned16(workspace)) {
-      if (qtype == QWIX_INT8) return launch_splitk<QWIX_INT8>(a, lda, b, ldb, M, N, K, splits, ep, out, ldo, workspace, st);
-      return launch_splitk<QWIX_E4M3>(a, lda, b, ldb, M, N, K, splits, ep, out, ldo, workspace, st);
-    }
+  if (splits > 0) {
+    if (qtype == QWIX_INT8) return launch_splitk<QWIX_INT8>(a, lda, b, ldb, M, N, K, splits, ep, out, ldo, workspace, st);
+    return launch_splitk<QWIX_E4M3>(a, lda, b, ldb, M, N, K, splits, ep, out, ldo, workspace, st);
   }
   if (few_rows && K % 128 == 0 && M * lda < (int64_t{1} << 31) && 64 * ldb < (int64_t{1} << 31)) {
     if (qtype == QWIX_INT8) return launch_skinny<QWIX_INT8>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);

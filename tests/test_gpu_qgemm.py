@@ -316,6 +316,27 @@ def test_int8_gemm_split_k_bit_exact(M, K, N, dtype):
   assert torch.equal(again, out)
 
 
+@pytest.mark.parametrize('M,K,N', [(512, 14336, 128), (64, 14336, 4096)])   # wavefronts that split K, unless a workspace splits it
+def test_a_workspace_that_is_too_small_is_as_good_as_none(M, K, N):
+  """Which kernel runs follows from the workspace that can be used: e4m3 sums are added in another order by each."""
+  from qwix_amd import _lib
+  g = torch.Generator(device=util.DEV).manual_seed(K)
+  a, b = (torch.randn(r, K, generator=g, device=util.DEV).to(torch.float8_e4m3fn) for r in (M, N))
+  need = int(_lib.load().qwix_hip_qgemm_workspace_bytes(M, N, K))
+  assert need > 0
+  ws = torch.empty(need + 16, dtype=torch.uint8, device=util.DEV)
+
+  def run(pointer, n):
+    out = torch.empty(M, N, dtype=torch.float32, device=util.DEV)
+    _lib.call('qwix_hip_qgemm_ws', a.data_ptr(), K, b.data_ptr(), K, _lib.E4M3, M, N, K, None, 0, None, 0, _lib.F32,
+              out.data_ptr(), _lib.F32, N, pointer, n, _lib.stream_of(a))
+    return out
+  none = run(None, 0)
+  for pointer, n in ((ws.data_ptr(), 64), (ws.data_ptr(), need - 1), (ws.data_ptr() + 4, need)):
+    assert torch.equal(run(pointer, n), none)
+  assert not torch.equal(run(ws.data_ptr(), need), none)   # (another kernel: the comparison above says something)
+
+
 @pytest.mark.parametrize('dtype', [O.BF16, O.F32])
 def test_fp8_gemm_split_k_close(dtype):
   from qwix_amd.core import dot_general as dg
