@@ -1225,8 +1225,9 @@ int dispatch_grouped_outer(const GroupedArgs& p, hipStream_t st) {
   }
   return launch_grouped_outer<BQT, Fast>(p, st);
 }
+inline bool outer_scales(int sa_dtype, int sb_dtype) { return sb_dtype == QWIX_BF16 && sa_dtype == QWIX_BF16; }
 inline bool takes_outer(const GroupedArgs& p) {
-  return p.sb_dtype == QWIX_BF16 && p.sa_dtype == QWIX_BF16 && p.zu == nullptr && p.acc_out == nullptr && !p.single;
+  return outer_scales(p.sa_dtype, p.sb_dtype) && p.zu == nullptr && p.acc_out == nullptr && !p.single;
 }
 
 // A decode batch against groups of 128: the kernel that splits K over wavefronts, while its N / 32 workgroups (each
@@ -1420,6 +1421,12 @@ static int grouped_ranges(int64_t M, int64_t N, int64_t K, int64_t group) {
   return best > 1 ? best : 0;
 }
 
+// ... of one call: scales per group on both sides (`sag`) only where the fold by outer products takes them.
+static int grouped_ranges_of(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, bool sag, int sa_dtype, int sb_dtype) {
+  if (sag && (b_qtype == QWIX_INT4 || !outer_scales(sa_dtype, sb_dtype))) return 0;
+  return grouped_ranges(M, N, K, group);
+}
+
 // Per-group K-sums of quantized rows: out[row, g] = sum over the g-th group of `group` values of row `row`
 // (int8, or packed int4).  One 16-byte chunk per thread; the chunks of a group that sit in `seg` adjacent
 // lanes (a power of two that divides the chunks per group) are added by shuffles, the rest by integer
@@ -1549,15 +1556,14 @@ static int grouped_impl(const void* a, int64_t lda, const void* b, int64_t ldb_b
     // per-group activation scales ride along in LDS: the tile's scales must fit behind the slab stages
     const bool sag = sa != nullptr && ga > 1;
     // K in ranges with f32 partial sums in the caller's workspace, where the narrow tiles are few
-    // (scales per group on both sides: where the fold by outer products takes them)
-    const int ranges = (workspace && !exact && !zu && !acc_out && aligned16(workspace) && (!sag || takes_outer(p)))
-                           ? grouped_ranges(M, N, K, group) : 0;
+    const int ranges = workspace && !exact && !zu && !acc_out && aligned16(workspace)
+                           ? grouped_ranges_of(M, N, K, group, b_qtype, sag, sa_dtype, sb_dtype) : 0;
     auto run = [&](const GroupedArgs& q) {
       if (b_qtype == QWIX_E4M3) return sag ? dispatch_grouped_f8<true>(q, st) : dispatch_grouped_f8<false>(q, st);
       if (b_qtype == QWIX_INT4) return sag ? dispatch_grouped_dma<QWIX_INT4, true>(q, st) : dispatch_grouped_dma<QWIX_INT4, false>(q, st);
       return sag ? dispatch_grouped_dma<QWIX_INT8, true>(q, st) : dispatch_grouped_dma<QWIX_INT8, false>(q, st);
     };
-    if (ranges > 0 && !(sag && b_qtype == QWIX_INT4) && workspace_bytes >= static_cast<size_t>(ranges) * M * N * 4) {
+    if (ranges > 0 && workspace_bytes >= static_cast<size_t>(ranges) * M * N * 4) {
       GroupedArgs q = p;
       q.ksplit = static_cast<int>(K / ranges);
       if (!sag) q.sa = nullptr;
@@ -1588,10 +1594,15 @@ extern "C" int qwix_hip_qgemm_grouped(const void* a, int64_t lda, const void* b,
                       nullptr, 0, 0, out, out_dtype, ldo, exact, acc_out, stream);
 }
 
-extern "C" size_t qwix_hip_qgemm_grouped_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype) {
+extern "C" size_t qwix_hip_qgemm_grouped_call_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, int sa_dtype,
+                                                    int64_t ga, int sb_dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  (void)b_qtype;
-  return static_cast<size_t>(grouped_ranges(M, N, K, group)) * M * N * 4;
+  return static_cast<size_t>(grouped_ranges_of(M, N, K, group, b_qtype, ga > 1, sa_dtype, sb_dtype)) * M * N * 4;
+}
+
+// (with one activation scale per row, which every weight type splits alike)
+extern "C" size_t qwix_hip_qgemm_grouped_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype) {
+  return qwix_hip_qgemm_grouped_call_bytes(M, N, K, group, b_qtype, QWIX_BF16, 1, QWIX_BF16);
 }
 
 extern "C" int qwix_hip_qgemm_grouped_ws(const void* a, int64_t lda, const void* b, int64_t ldb_bytes, int b_qtype,

@@ -1,5 +1,6 @@
 """Launch plans: what the recorder accepts (CPU), and that replayed calls give what the ordinary path gives (GPU)."""
 import _thread
+import ctypes
 import dataclasses
 import functools
 import sys
@@ -166,6 +167,33 @@ def test_recorder_refuses_sums_kept_per_weight(stand_in):
     recorded.append(dg._weight_ksums(w.qvalue, w.qvalue, (), compute))
   rec, _ = _recorded(fn, *_parts(w))
   assert not rec.ok and len(rec.calls) == 1 and recorded[0] is not None
+
+
+@pytest.mark.parametrize('act,weight,both,dtype,split', [
+    ('int8', 'int8', True, torch.bfloat16, True), ('int8', 'int8', True, torch.float32, False), ('int8', 'int4', True, torch.bfloat16, False),
+    ('int8', 'int4', False, torch.float32, True), ('float8_e4m3fn', 'float8_e4m3fn', True, torch.bfloat16, True),
+    ('float8_e4m3fn', 'float8_e4m3fn', True, torch.float32, False)])
+def test_sub_channel_calls_that_are_not_split_get_no_workspace(stand_in, monkeypatch, act, weight, both, dtype, split):
+  from qwix_amd.core import dot_general as dg
+  from qwix_amd.core.qarray import Int4Tensor, QArray
+  real = ctypes.CDLL(_lib.LIB_PATH)
+
+  class Sizes(_StandIn):
+    def __getattr__(self, name):
+      if not name.endswith('_bytes'):
+        return super().__getattr__(name)
+      fn = getattr(real, name)
+      fn.restype, fn.argtypes = _lib.SIGNATURES[name]
+      return fn
+  monkeypatch.setattr(_lib, 'load', Sizes)
+  M, K, N = 100, 4096, 264
+  values = lambda t, *shape: torch.zeros(*shape, dtype=torch.int8 if t == 'int8' else torch.float8_e4m3fn)
+  wv = Int4Tensor(torch.zeros(N, K // 2, dtype=torch.uint8).t(), (K, N), 0) if weight == 'int4' else values(weight, N, K).t()
+  x = QArray(values(act, M, K), torch.ones(M, K // 128 if both else 1, dtype=dtype), None, act)
+  w = QArray(wv, torch.ones(K // 128, N, dtype=dtype), None, weight)
+  rec, _ = _recorded(lambda rec: dg._dot_general(x, w, _DN), *_parts(x, w))
+  assert [name for name, _ in rec.calls] == ['qwix_hip_qgemm_grouped_ws']
+  assert len(rec.buffers) == (2 if split else 1)
 
 
 def test_more_rows_than_one_launch_takes_go_group_by_group(stand_in):
