@@ -60,7 +60,10 @@ namespace {
 // another round, 512 x 14336 over K 4096, 61 against 104.
 // RAGGED: rows in groups (mixture of experts), found on the device as in the ragged GEMM: the tile's rows end with its
 // group, and weights and scales are the group's.
-template <int OUT, bool SBF, int BM, int BN, int BITS, bool ZP, bool RAGGED = false>
+// HALF: K may be 128 mod 256, the last superslab half of one: another tail behind a branch, clamped loads of the last line of
+// int4 weights and of its scales.  A template parameter because the branch costs registers that all K would pay for (bf16
+// result, 128 x 64 int4 / int8, 256 x 128 int4: 124 / 151 / 248 per lane with it, 86 / 111 / 173 without).
+template <int OUT, bool SBF, int BM, int BN, int BITS, bool ZP, bool HALF, bool RAGGED = false>
 __global__ void __launch_bounds__(512)
     wgemm_wq_kernel(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ Q, int64_t ldq,
                     const void* __restrict__ S, const int8_t* __restrict__ Z, int M, int N, int K, int group,
@@ -140,7 +143,7 @@ __global__ void __launch_bounds__(512)
 
   // ---- loaders: 8 rows x 128 bytes per instruction; the global 16-byte chunk that lands at position lane & 7
   const int lr = lane >> 3;
-  uint32_t goffa[NA], goffq[NQ], back[NQ];
+  uint32_t goffa[NA], goffq[NQ], back[HALF ? NQ : 1];
 #pragma unroll
   for (int j = 0; j < NA; ++j) {
     const int row = (ldw * NA + j) * 8 + lr;
@@ -151,12 +154,11 @@ __global__ void __launch_bounds__(512)
     if constexpr (W8) {  // 16 rows x 64 bytes per instruction (64-column tiles: 8 rows, twice)
       const int row = ldw * RPW + ((lane >> 2) & (RPW - 1));
       goffq[j] = static_cast<uint32_t>(min(n0 + row, N - 1)) * static_cast<uint32_t>(ldq) + ((lane & 3) << 4);
-      back[j] = 0;
     } else {
       const int row = ldw * RPW + j * 8 + lr;
       const uint32_t chunk = (lane & 7) ^ swz8(row);
       goffq[j] = static_cast<uint32_t>(min(n0 + row, N - 1)) * static_cast<uint32_t>(ldq) + (chunk << 4);
-      back[j] = chunk >= 4 ? 64 : 0;
+      if constexpr (HALF) back[j] = chunk >= 4 ? 64 : 0;
     }
   }
   auto issue_a = [&](int kt, int stage) __attribute__((always_inline)) {  // NA loads
@@ -172,9 +174,9 @@ __global__ void __launch_bounds__(512)
       const uint8_t* gq = Q + ss * 128;
       uint8_t* dst = smem + R_BASE + (ss & 1) * R_STAGE + ldw * RPW * 128;
       // the last 128 elements of a K that is no multiple of 256: the line's upper half repeats the lower one
-      const uint32_t half = ss * 256 + 256 > K ? ~0u : 0u;
+      const uint32_t half = HALF && ss * 256 + 256 > K ? ~0u : 0u;
 #pragma unroll
-      for (int j = 0; j < NQ; ++j) QWIX_GLDS16(gq + (goffq[j] - (back[j] & half)), dst + j * 1024);
+      for (int j = 0; j < NQ; ++j) QWIX_GLDS16(gq + (goffq[j] - (HALF ? back[HALF ? j : 0] & half : 0)), dst + j * 1024);
     }
   };
 
@@ -188,7 +190,7 @@ __global__ void __launch_bounds__(512)
   const int slabs_per_group = group >> 6;
   const char* sc_ptr = sptr;
   const int8_t* zp_ptr = ZP ? Z + min(n0 + crow, N - 1) : nullptr;
-  int sc_left = slabs_per_group, sc_groups = K / group;  // (the two slabs past a K of 128 mod 256 read the last group's)
+  int sc_left = slabs_per_group, sc_groups = K / group;  // (HALF: the two slabs past K read the last group's)
   auto request_scales = [&](uint32_t (&dst)[4], int (&dstz)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -199,7 +201,7 @@ __global__ void __launch_bounds__(512)
       if constexpr (ZP) asm volatile("global_load_sbyte %0, %1, off" : "=&v"(dstz[j]) : "v"(zp_ptr) : "memory");
       if (--sc_left == 0) {
         sc_left = slabs_per_group;
-        if (--sc_groups > 0) {
+        if (!HALF || --sc_groups > 0) {
           sc_ptr += s_group_pitch;
           if constexpr (ZP) zp_ptr += N;
         }
@@ -320,7 +322,7 @@ __global__ void __launch_bounds__(512)
   };
   using std::integral_constant;
 
-  const int KT = K / 64;  // a multiple of 2, at least 4
+  const int KT = K / 64;  // a multiple of 4 (HALF: of 2), at least 4
   uint32_t sc_cur[4], sc_next[4] = {0, 0, 0, 0};
   int zp_cur[4] = {0, 0, 0, 0}, zp_next[4] = {0, 0, 0, 0};
   int sta = 0;  // LDS stage of the activations of the slab being multiplied: kt % 3
@@ -393,14 +395,15 @@ __global__ void __launch_bounds__(512)
   };
   auto slabs = [&](auto ROLE) __attribute__((always_inline)) {  // every role passes the same K / 64 barriers
     int kt = 0;
-    for (; kt + 8 <= KT; kt += 4) {
+    // (written as 'kt + 8 <= KT' the same loop takes 102 / 135 / 200 registers in the three tiles named above)
+    for (; kt + (HALF ? 6 : 4) < KT; kt += 4) {
       slab(kt, I0{}, I4{}, ROLE);
       slab(kt + 1, I1{}, I4{}, ROLE);
       slab(kt + 2, I2{}, I4{}, ROLE);
       slab(kt + 3, I3{}, I4{}, ROLE);
       next_scales();
     }
-    if (KT & 2) {  // six left
+    if (HALF && (KT & 2)) {  // six left
       slab(kt, I0{}, I4{}, ROLE);
       slab(kt + 1, I1{}, I4{}, ROLE);
       slab(kt + 2, I2{}, I3{}, ROLE);
@@ -526,6 +529,9 @@ static constexpr size_t wq_lds_bytes(int bm, int bn, int bits) {
   return static_cast<size_t>(bm == 128 ? 4 : 3) * bm * 128 + 2 * bn * 128 + (bits >= 8 ? 4 * (bm == 128 ? 4 : 8) * 1024 : 2 * bn * 128);
 }
 
+// Tiles whose HALF variant keeps its registers: that of 256 x 128 with int4 zero points and f32 scales spills.
+static constexpr bool wq_half_fits(int bm, int bn, int bits, bool zp, bool sbf) { return !(bm == 256 && bn == 128 && bits == 4 && zp && !sbf); }
+
 static int check_wq_args(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int q_qtype, int64_t M, int64_t N,
                          int64_t K, int64_t group, const void* s, int s_dtype, const int8_t* zp, const void* out,
                          int out_dtype, int64_t ldo) {
@@ -564,7 +570,8 @@ static int gemm_bf16_wq_impl(const void* a, int64_t lda, const void* q, int64_t 
   const bool low = plan.low, narrow = plan.narrow;
   // 192-row tiles where they need no more rounds of the CUs than the 256-row ones
   auto rounds = [&](int64_t rows) { return ((M + rows - 1) / rows * ((N + 127) / 128) + 255) / 256; };
-  const bool mid = rounds(192) <= rounds(256);
+  const bool half = K % 256 != 0;
+  const bool mid = rounds(192) <= rounds(256) || (half && !wq_half_fits(256, 128, q_qtype == QWIX_INT4 ? 4 : 8, zp != nullptr, s_dtype == QWIX_BF16));
   hipStream_t st = static_cast<hipStream_t>(stream);
   // with a workspace that holds them: f32 partials of `splits` K ranges, added up (in range order) by a second kernel
   int splits = workspace && plan.range > 0 ? static_cast<int>((K + plan.range - 1) / plan.range) : 0;
@@ -579,12 +586,13 @@ static int gemm_bf16_wq_impl(const void* a, int64_t lda, const void* q, int64_t 
   } while (0)
 #define QWIX_WQ_LAUNCH_Z(OUTT, SBFF, BMM, BNN, BITS, ZPP)                                                            \
   do {                                                                                                               \
-    auto kern = wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, ZPP>;                                                    \
+    auto kern = half ? wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, ZPP, wq_half_fits(BMM, BNN, BITS, ZPP, SBFF)>      \
+                     : wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, ZPP, false>;                                      \
     constexpr size_t smem = wq_lds_bytes(BMM, BNN, BITS);                                                            \
     const dim3 grid(static_cast<unsigned>(((M + BMM - 1) / BMM) * ((N + BNN - 1) / BNN)),                            \
                     static_cast<unsigned>(splits > 0 ? splits : 1));                                                 \
-    static LdsGrant granted;                                                                                         \
-    if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted)) return e_;                           \
+    static LdsGrant granted[2];                                                                                      \
+    if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted[half])) return e_;                     \
     kern<<<grid, 512, smem, st>>>(static_cast<const uint8_t*>(a), 2 * lda, static_cast<const uint8_t*>(q), ldq_bytes, s, \
                                   zp, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),                 \
                                   static_cast<int>(group), kern_dst, kern_ldo, ksplit, Ragged{});                              \
@@ -668,13 +676,15 @@ static int wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_byte
   // half of the CUs.  Tiles of 128 x 64 / 256 x 128, 64 and 96 rows per group on average, some groups up to half as many
   // again: 64 groups, K 2048, N 1024, int8 72 / 71 and 88 / 75 us; 8 groups, K 2176, N 5312 56 / 71 and 73 / 72 us; 8 groups,
   // K 4096, N 14336, int4 193 / 230 and 217 / 233 us; 128 rows 312 / 236 us.
-  const int tile = M <= 80 * G ? 0 : (M / 256 + G) * ((N + 127) / 128) <= 128 ? 1 : 2;
+  const bool half = K % 256 != 0;  // (groups of more than 256 rows, where dot_general's rule says what is streamed)
+  const int tile = M <= 80 * G && !half ? 0 : (M / 256 + G) * ((N + 127) / 128) <= 128 ? 1 : 2;
 #define QWIX_WQR(OUTT, SBFF, BMM, BNN, BITS)                                                                         \
   do {                                                                                                               \
-    auto kern = wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, false, true>;                                            \
+    auto kern = half ? wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, false, (BMM > 128), true>                         \
+                     : wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, false, false, true>;                              \
     constexpr size_t smem = wq_lds_bytes(BMM, BNN, BITS);                                                            \
-    static LdsGrant granted;                                                                                         \
-    if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted)) return e_;                           \
+    static LdsGrant granted[2];                                                                                      \
+    if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted[half])) return e_;                     \
     kern<<<dim3(ragged_grid(M, N, G, BMM, BNN)), 512, smem, st>>>(                                                   \
         static_cast<const uint8_t*>(a), 2 * lda, static_cast<const uint8_t*>(q), ldq_bytes, s, nullptr,              \
         static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), static_cast<int>(group),                      \
