@@ -2161,15 +2161,17 @@ int qwix_hip_dequantize(const void* qvalue, int qtype, int q_layout, int64_t out
   //   1024 x 8192 (512 tiles) 9.9 5.5 7.3 / 17.1 14.4 11.8, 8192 x 8192 77 36 35 / 169 103 84, 8192 x 28672 235 112 192 /
   //   381 362 308 (f32 with eight columns per thread in the long lines: with four, whose 16-byte stores fill whole lines, quantize
   //   and read back 2176 x 3840 24.6 -> 20.4, 7424 x 6288 155.5 -> 145.9, 4096 x 14336 129 -> 126 against lines of 32 bytes): lines of
-  //   32 bytes up to 256 tiles.
-  // (int4 and e4m3 cross at the same sizes; int4 to f32 at twice them: 4224 x 1000 16.2 against 17.2 in long lines.)
+  //   32 bytes up to 256 tiles, of f32 up to 400.
+  // (e4m3 crosses at the same sizes, int4 to bf16 too.  f32, quantized in groups of 128 and read back, lines of 32 bytes / long
+  // ones, 264, 320, 384, 480 and 512 tiles: int8 15.3 / 15.8, 16.9 / 17.1, 18.2 / 18.2, 21.0 / 20.0, 21.3 / 20.2 us; int4, in
+  // tiles of 256 rows, 21.2 / 22.8, 23.4 / 23.9, 25.3 / 25.9, 30.2 / 29.6, 32.6 / 30.8.)
   if (!natural && ptr_ok && n >= (1 << 18) && reduce % 8 == 0 && tile % 8 == 0 && outer <= 65535 && (inner + 127) / 128 < (1 << 23)) {
     // Nontemporal bf16 stores where a 256-byte row piece starts at a 32-byte sector; elsewhere two workgroups write parts of one
     // sector, which have to meet in L2.  Quantize and read back, nontemporal / plain: 4096 x 14344 93.7 / 70.1 us, 4096 x 8200
     // 59.4 / 50.9; 4096 x 8192 43.8 / 58.6, 8192 x 28672 359 / 377, 5120 x 16752 (sectors, not lines) 165 / 167.
     const bool nt = inner % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 32 == 0;
     const int long_rows = dtype == QWIX_F32 && qtype == QWIX_INT4 ? 256 : 128;
-    const bool narrow = outer * ((reduce + long_rows - 1) / long_rows) * ((inner + 127) / 128) <= 256;
+    const bool narrow = outer * ((reduce + long_rows - 1) / long_rows) * ((inner + 127) / 128) <= (dtype == QWIX_F32 ? 400 : 256);
     const int kt = (narrow ? 32 : 128) * (qtype == QWIX_INT4 ? 2 : 1);
     const int64_t tiles = (reduce + kt - 1) / kt;
     // grid y and z end at 65535, x at 2^31 threads: longer reduced axes take several launches

@@ -292,9 +292,10 @@ def test_dequantize(dtype, qtype):
 
 @pytest.mark.parametrize('qtype', QTYPES)
 @pytest.mark.parametrize('dtype', [O.BF16, O.F32])
-@pytest.mark.parametrize('reduce,inner', [(2064, 2048), (2064, 2056), (2048, 2084)])
+@pytest.mark.parametrize('reduce,inner', [(2064, 2048), (2064, 2056), (2048, 2084), (6416, 2048), (6416, 2056), (6400, 2084)])
 def test_dequantize_long_lines(reduce, inner, dtype, qtype):
-  """More than 256 tiles: lines of 128 bytes, with rows that start at sectors, inside one, and without 16-byte pieces (bf16)."""
+  """More than 256 tiles (f32: 400, int4 to f32 of 256 rows): lines of 128 bytes, with rows that start at sectors, inside one, and
+  without 16-byte pieces (bf16)."""
   from qwix_amd.core import qarray
   _, x_t = util.make((reduce, inner), dtype, seed=73)
   qa = qarray.quantize(x_t, qarray.HowToQuantize(qtype=qtype, channelwise_axes=[1], tiled_axes={0: 16}), layout='reduce_minor')
