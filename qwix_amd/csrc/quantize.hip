@@ -864,8 +864,8 @@ __global__ void __launch_bounds__(256)
 // in LDS (64 KB at 4096 rows) and leave as whole columns.
 //   What bounds it: small arrays the launch and one round of loads, large ones memory, read in 32-byte pieces.  The
 // four strips that share the input's 128-byte lines go to one XCD, one after the other, so that three of the four pieces
-// come from its L2.  bf16 to int8, fill + maximum + quantize -> strips: 1920 x 1856 13.9 -> 7.8 us, 14 x 464 x 128 14.6 -> 7.3,
-// 55 x 2784 x 64 22.1 -> 9.6, 640 x 27912 23.6 -> 16.5, 4096 x 14336 48.0 -> 42.1; f32 80.4 -> 63.2.
+// come from its L2.  bf16 to int8 from the caches, fill + maximum + quantize -> strips: 1920 x 1856 13.9 -> 7.8 us, 14 x 464 x 128
+// 14.6 -> 7.3, 55 x 2784 x 64 22.1 -> 9.6; from memory: takes_strips.
 template <typename D, int QT>
 __global__ void __launch_bounds__(1024)
     cols_strip_kernel(const uint8_t* __restrict__ x, ColGeom gm, int pitch, float factor, uint8_t* __restrict__ q,
@@ -1769,6 +1769,17 @@ int run_cols_quantize(const void* x, int dtype, const ColGeom& g, int qtype, int
 // Rows that a strip of 1024 threads holds.  (With sixteen rows per thread a CU has room for one workgroup only and the 32-byte
 // pieces no longer keep up: 8192 x 28672 bf16 286 us in strips, 206 in two passes, 8192 x 1024 15.2 and 14.3.)
 constexpr int64_t kStripRows = 4096;
+// Where one launch that reads the array in 32-byte pieces, once, beats three that read it in rows, twice.  Arrays of up to 32 MB:
+// beyond, memory keeps up with rows only.  From memory, bf16 to int8, strips / two passes, us: 512 x 4096 6.5 / 15.6, 2048 x 2048
+// 11.4 / 16.0, 512 x 28672 20.3 / 21.4, 2048 x 8192 21.7 / 22.9, 1024 x 16384 22.0 / 22.2, 2048 x 9216 28.9 / 24.2, 2048 x 14336
+// 37.8 / 31.9, 4096 x 28672 114.6 / 106.8 (from the caches 64 MB are still ahead: 2048 x 16384 22.8 / 32.3).  The taller the
+// strip, the longer its one round of loads: up to 3072 rows (3072 x 512 15.2 / 15.2, x 2048 15.5 / 17.4), or to 4096 while the strips are
+// a round of the CUs (4096 x 4096 22.3 / 24.0; x 2048, 128 strips, 20.7 / 18.6).
+bool takes_strips(const ColGeom& g, int dtype) {
+  const int64_t strips = g.outer * g.ntiles * ((g.inner + (dtype == QWIX_BF16 ? 15 : 7)) / (dtype == QWIX_BF16 ? 16 : 8));
+  const int64_t bytes = g.outer * g.reduce * g.inner * (dtype == QWIX_BF16 ? 2 : 4);
+  return g.tile <= kStripRows && bytes <= int64_t{32} << 20 && (g.tile <= 3072 || strips >= 256);
+}
 int run_cols_strip(const void* x, int dtype, const ColGeom& g, int qtype, float factor, void* q, void* scale, hipStream_t st) {
   const int nc = dtype == QWIX_BF16 ? 16 : 8;
   int threads = 64;
@@ -1881,8 +1892,7 @@ int qwix_hip_quantize(const void* x, int dtype, int64_t outer, int64_t reduce, i
   const size_t need = qwix_hip_quantize_workspace_bytes(outer, reduce, inner, tile, calibration);
   if (!workspace || workspace_bytes < need)
     return fail(QWIX_ERR_INVALID_ARGUMENT, "workspace of %zu bytes required, got %zu", need, workspace_bytes);
-  if (calibration == QWIX_ABSMAX && q_layout == QWIX_LAYOUT_REDUCE_MINOR && tile <= kStripRows &&
-      outer * g.ntiles * ((inner + 7) / 8) <= INT32_MAX)
+  if (calibration == QWIX_ABSMAX && q_layout == QWIX_LAYOUT_REDUCE_MINOR && takes_strips(g, dtype))
     return run_cols_strip(x, dtype, g, qtype, calib_factor, qvalue, scale, st);
   if (int e = run_cols_absmax(x, dtype, g, calibration, static_cast<uint32_t*>(workspace), st)) return e;
   return run_cols_quantize<0>(x, dtype, g, qtype, calibration, q_layout, static_cast<const uint32_t*>(workspace),

@@ -86,7 +86,7 @@ def test_weight_columns(shape, tile, layout, dtype, qtype):
 @pytest.mark.parametrize('dtype', [O.BF16, O.F32])
 @pytest.mark.parametrize('shape,kw', [
     ((136, 8), {}), ((264, 24), {}), ((1032, 40), {}),                        # one wavefront, an odd column piece, several wavefronts
-    ((4096, 16), {}), ((4104, 24), {}),                                       # the tallest strip; taller goes in two passes
+    ((3072, 16), {}), ((3080, 16), {}), ((4096, 16), {}), ((4104, 24), {}),   # the tallest strips of a few; taller ones go in two passes
     ((3, 520, 40), dict(channelwise_axes=[0, 2])),                            # batches
     ((1024, 72), dict(tiled_axes={0: 256})), ((272, 616), dict(tiled_axes={0: 136})),   # several groups; more strips than a round of XCDs
 ])
@@ -94,6 +94,19 @@ def test_weight_column_strips(shape, kw, dtype, qtype):
   x_np, x_t = util.make(shape, dtype, seed=sum(shape), scale=0.02)
   x_np[..., 1], x_t[..., 1] = 0, 0
   _check(x_np, x_t, dtype, dict(qtype=qtype, channelwise_axes=[1]) | kw, what='strips')
+
+
+@pytest.mark.parametrize('qtype', QTYPES)
+@pytest.mark.parametrize('dtype,shape', [(O.BF16, (4096, 4096)), (O.F32, (4096, 2048)), (O.BF16, (3080, 4096))])
+def test_weight_tall_column_strips(dtype, shape, qtype):
+  """The tallest strips (a round of the CUs of them): the codes and scales of the same columns in an array of two passes."""
+  import qwix_amd
+  _, x = util.make(shape, dtype, seed=11, scale=0.02)
+  whole = qwix_amd.quantize(x, qtype, channelwise_axes=[1])
+  codes = lambda q: q.qvalue.unpack() if qtype == 'int4' else q.qvalue.view(torch.uint8)
+  for first in (0, 1000, shape[1] - 72):
+    part = qwix_amd.quantize(x[:, first:first + 72].contiguous(), qtype, channelwise_axes=[1])
+    assert torch.equal(codes(whole)[:, first:first + 72], codes(part)) and torch.equal(whole.scale[:, first:first + 72], part.scale)
 
 
 @pytest.mark.parametrize('dtype', [O.BF16, O.F32])
