@@ -821,8 +821,19 @@ __global__ void __launch_bounds__(G::kNW * 64) __attribute__((amdgpu_waves_per_e
     const bool first = in_group == 0, last = in_group == tpg - 1;
     if (first && kt + tpg < KT) sb_next = load_sb(g + 1);
     // (groups of several slabs: two loop bodies, the fold after the group's last MFMA)
-    if (first) slab(kt, T{}, F{}, g, sbg, sb_cur, recentre);
-    else slab(kt, F{}, F{}, g, sbg, sb_cur, recentre);
+    // (e4m3 with outer products: one body that starts from cleared sums.  Two of them spill; 16 rows, K 4096, N 4096, groups of 256
+    // 21.1 -> 19.3 us, 4096^3 83.8 / 83.8)
+    if constexpr (OUTER && F8) {
+      if (first) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i] = AccV{0};
+      }
+      slab(kt, F{}, F{}, g, sbg, sb_cur, recentre);
+    } else if (first) {
+      slab(kt, T{}, F{}, g, sbg, sb_cur, recentre);
+    } else {
+      slab(kt, F{}, F{}, g, sbg, sb_cur, recentre);
+    }
     if (last) {
       if constexpr (!AUX) {
 #pragma unroll
