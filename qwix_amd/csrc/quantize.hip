@@ -1460,10 +1460,11 @@ __global__ void __launch_bounds__(256)
 // bf16 236 -> 154 us (4.6 TB/s), 4096 x 14336 59 -> 31, against tiles of 64 x 64 turned byte by byte.
 //   Small arrays are bound by the latency of one block's load - convert - store chain instead: LB 32 gives each thread a
 // quarter of the work and the chip four times the blocks.  Where the line between the two lies: at the dispatch.
-template <typename D, int QT, int LB, int CPT>
+// NT: nontemporal stores (bf16, eight columns per thread), told at compile time: asked per store, 2048 x 8192 9.7 us instead of 9.5.
+template <typename D, int QT, int LB, int CPT, bool NT>
 __global__ void __launch_bounds__(256)
     dequant_rm_kernel(const uint8_t* __restrict__ q, int64_t reduce, int64_t inner, int64_t tile, int64_t tile0,
-                      const void* __restrict__ scale, const int8_t* __restrict__ zp, void* __restrict__ out, bool nt) {
+                      const void* __restrict__ scale, const int8_t* __restrict__ zp, void* __restrict__ out) {
   constexpr int EPB = QT == QWIX_INT4 ? 2 : 1, KT = LB * EPB;  // values per byte, rows of the output per tile
   constexpr int CGS = 128 / CPT, DSTEP = 256 / CGS, ITS = LB / 4 / DSTEP;
   constexpr int PITCH = LB + 16, CHUNKS = LB / 16;
@@ -1473,14 +1474,17 @@ __global__ void __launch_bounds__(256)
   const int tid = threadIdx.x;
   const int64_t row_bytes = reduce / EPB, b0 = r0 / EPB;  // reduce % 8 == 0
   auto at = [](int col, int byte) { return col * PITCH + (((byte >> 4) ^ ((col >> 4) & (CHUNKS - 1))) << 4) + (byte & 15); };
-  if (row_bytes % 16 == 0) {
+  if (row_bytes % 16 == 0 && row_bytes <= UINT32_MAX) {
     // past the last column or the end of a row its last 16 bytes again: what comes of them is not stored
     constexpr int LOADS = 128 * CHUNKS / 256, CSTEP = 256 / CHUNKS;
     uint4 v[LOADS];
     const int last = static_cast<int>(min(static_cast<int64_t>(127), inner - 1 - i0));
     const uint8_t* src = q + (o * inner + i0) * row_bytes + min(b0 + (tid % CHUNKS) * 16, row_bytes - 16);
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j) v[j] = *reinterpret_cast<const uint4*>(src + min(tid / CHUNKS + j * CSTEP, last) * row_bytes);
+    for (int j = 0; j < LOADS; ++j) {
+      const uint32_t col = static_cast<uint32_t>(min(tid / CHUNKS + j * CSTEP, last));
+      v[j] = *reinterpret_cast<const uint4*>(src + static_cast<uint64_t>(col) * static_cast<uint32_t>(row_bytes));
+    }
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) *reinterpret_cast<uint4*>(lines + at(tid / CHUNKS + j * CSTEP, (tid % CHUNKS) * 16)) = v[j];
   } else {
@@ -1544,7 +1548,7 @@ __global__ void __launch_bounds__(256)
         if constexpr (D::kTag == QWIX_BF16 && CPT == 8) {
           uint4* const dst = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + oi);
           const uint4 pk = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-          if (nt) nt_store16(dst, pk);
+          if constexpr (NT) nt_store16(dst, pk);
           else *dst = pk;
         } else if constexpr (D::kTag == QWIX_BF16)
           *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + oi) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
@@ -2189,8 +2193,9 @@ int qwix_hip_dequantize(const void* qvalue, int qtype, int q_layout, int64_t out
       const dim3 grid(static_cast<unsigned>((inner + 127) / 128), static_cast<unsigned>(std::min<int64_t>(tiles - t0, 65535)),
                       static_cast<unsigned>(outer));
 #define QWIX_DEQ_RM(QTT)                                                                                             \
-  if (narrow) dequant_rm_kernel<D, QTT, 32, 4><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out, nt);      \
-  else dequant_rm_kernel<D, QTT, 128, D::kVec><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out, nt)
+  if (narrow) dequant_rm_kernel<D, QTT, 32, 4, false><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out);   \
+  else if (nt) dequant_rm_kernel<D, QTT, 128, D::kVec, D::kVec == 8><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out); \
+  else dequant_rm_kernel<D, QTT, 128, D::kVec, false><<<grid, 256, 0, st>>>(q, reduce, inner, tile, t0, scale, zp, out)
       QWIX_DISPATCH_D(dtype, {
         if (qtype == QWIX_INT8) { QWIX_DEQ_RM(QWIX_INT8); }
         else if (qtype == QWIX_INT4) { QWIX_DEQ_RM(QWIX_INT4); }
