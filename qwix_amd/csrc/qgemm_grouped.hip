@@ -1155,10 +1155,14 @@ __global__ void __launch_bounds__(NWV * 64) qgemm_grouped_decode_kernel(GroupedA
     const int r = wave * (16 / NWV) + q;
     const int m = m0 + 8 * (r >> 2) + 4 * hx + (r & 3);
     if (m >= p.M || n >= p.N) continue;
+    // in double, rounded once: one after the other in f32, the partials of eight or sixteen wavefronts cost more roundings than
+    // the groups that four of them, or a tile's one, would add up by themselves (f32 results, K 1024, against 64 bits: 7.0e-8, with
+    // four or one 5.7e-8, now 4.4e-8)
     const float* part = reinterpret_cast<const float*>(smem) + r * 64 + lane;
-    float v = part[0];
+    double sum = part[0];
 #pragma unroll
-    for (int w = 1; w < NWV; ++w) v += part[w * wstride];
+    for (int w = 1; w < NWV; ++w) sum += static_cast<double>(part[w * wstride]);
+    float v = static_cast<float>(sum);
     if (!SAG && p.sa != nullptr) v *= ld_scale(p.sa, p.sa_dtype, m);
     if (t_bf16) v = round_bf16(v);
     if (p.out_dtype == QWIX_BF16)
