@@ -414,7 +414,7 @@ struct GemvGroups {
   int G;
   int64_t q_stride, s_stride;  // bytes of weights, elements of scales between consecutive groups
   int unit0;                   // first unit of this launch
-  int most;                    // groups of more rows, and the rows behind the groups, are left to another launch (INT32_MAX: none are)
+  int most;                    // BOUND: groups of more rows, and the rows behind the groups, are left to another launch
 };
 
 struct GroupTile {
@@ -441,7 +441,7 @@ __device__ __forceinline__ int scan_add(int v, int lane) {  // inclusive, over t
 
 // The `tile`-th of the tiles that are not the first of their group.  Sizes are clamped so that no group reaches past row M
 // (M < 2^20: 64 clamped sums fit 32 bits).
-template <int TR>
+template <int TR, bool BOUND>
 __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int tile) {
   const int lane = threadIdx.x & 63;
   int g0 = 0, g1 = gr.G, row0 = 0, tile0 = 0;  // rows and later tiles before group g0
@@ -455,7 +455,7 @@ __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int
       tiles = min(tiles + max(size - 1, 0) / TR, 1 << 20);  // more than there are tiles in front of row M
     }
     const int last_row = scan_add(rows, lane);
-    if (gr.most < M) {  // which groups count is told by the rows that they have in front of row M
+    if constexpr (BOUND) {  // which groups count is told by the rows that they have in front of row M
       int start = min(last_row - rows, M);
       tiles = 0;
       for (int g = lane * per; g < min((lane + 1) * per, gr.G); ++g) {
@@ -478,7 +478,7 @@ __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int
     const int end = min(row0 + scan_add(size, lane), M);
     const int before = __shfl_up(end, 1, 64);
     const int start = lane == 0 ? row0 : before;
-    const int tiles = end - start > gr.most ? 0 : max(end - start - 1, 0) / TR;
+    const int tiles = BOUND && end - start > gr.most ? 0 : max(end - start - 1, 0) / TR;
     if (__ballot(tiles > 0) != 0) {
       const int last = tile0 + scan_add(tiles, lane);  // one past the group's last tile
       const unsigned long long here = __ballot(tile >= last - tiles && tile < last);
@@ -495,7 +495,7 @@ __device__ __forceinline__ GroupTile later_tile(const GemvGroups& gr, int M, int
   return {0, 0, 0};
 }
 
-template <int BQT, int NWAVE, int NT, bool SBF, int RT>
+template <int BQT, int NWAVE, int NT, bool SBF, int RT, bool BOUND>
 __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, GemvGroups gr) {
   extern __shared__ float red_raw[];
   constexpr int TR = 16 * RT;
@@ -506,9 +506,9 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, 
   GroupTile at;
   if (unit < gr.G) {
     const int start = rows_before(gr, p.M, unit), size = min(max(gr.sizes[unit], 0), p.M - start);
-    at = {unit, start, size > gr.most ? start : start + min(size, TR)};
+    at = {unit, start, BOUND && size > gr.most ? start : start + min(size, TR)};
   } else {
-    if (unit == gr.G && gr.most == INT32_MAX) {
+    if (!BOUND && unit == gr.G) {
       const int start = rows_before(gr, p.M, gr.G);
       const int cols = min(16 * NT, p.N - n_base);
       for (int idx = threadIdx.x; idx < (p.M - start) * cols; idx += NWAVE * 64) {
@@ -517,7 +517,7 @@ __global__ void __launch_bounds__(NWAVE * 64) gemv_wq_groups_kernel(GemvArgs p, 
         else reinterpret_cast<uint32_t*>(p.out)[to] = 0;
       }
     }
-    at = later_tile<TR>(gr, p.M, unit - gr.G);
+    at = later_tile<TR, BOUND>(gr, p.M, unit - gr.G);
   }
   if (at.row >= at.row_end) return;
   p.q += at.group * gr.q_stride;
@@ -663,9 +663,10 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
     const int64_t units = G + std::max<int64_t>(1, std::min((M - 1) / (16 * RTT), G * ((most - 1) / (16 * RTT)))); \
     for (int64_t u = 0; u < units; u += 65535) { /* a grid's y axis */                                     \
       const GemvGroups gr{group_sizes, static_cast<int>(G), q_group_bytes, s_group_stride, static_cast<int>(u), \
-                          most_rows < M ? static_cast<int>(most) : INT32_MAX};                             \
+                          static_cast<int>(most)};                                                         \
       const dim3 grid(columns, static_cast<unsigned>(std::min<int64_t>(units - u, 65535)));                \
-      gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT><<<grid, NW * 64, smem, st>>>(p, gr);                  \
+      if (most_rows < M) gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT, true><<<grid, NW * 64, smem, st>>>(p, gr); \
+      else gemv_wq_groups_kernel<BQT, NW, NTT, SBFF, RTT, false><<<grid, NW * 64, smem, st>>>(p, gr);      \
     }                                                                                                      \
   } while (0)
 #define QWIX_GEMVG_LAUNCH(NW, NTT, RTT)                                                                    \
