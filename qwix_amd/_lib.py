@@ -133,6 +133,11 @@ def stream_of(t: torch.Tensor) -> int:
   return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def stream_on(index: int) -> int:
+  """The same for a device by its index."""
+  return _raw_stream(index) if _raw_stream is not None else torch.cuda.current_stream(index).cuda_stream
+
+
 def float_tag(dtype: torch.dtype) -> int:
   if dtype == torch.float32:
     return F32

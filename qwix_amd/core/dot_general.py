@@ -458,13 +458,13 @@ class _Kept:
   """Tensors made once from a weight and kept for later calls, which may come on other streams: they wait for the work that made the
   tensors, and a tensor that is let go is not reused under them."""
 
-  __slots__ = ('tensors', 'stream', 'event')
+  __slots__ = ('tensors', 'device', 'stream', 'event')
 
   def __init__(self, *tensors: torch.Tensor):
     self.tensors = tensors
-    self.stream = self.event = None
+    self.device = self.stream = self.event = None
     if tensors[0].is_cuda:
-      self.stream = _lib.stream_of(tensors[0])
+      self.device, self.stream = tensors[0].device.index, _lib.stream_of(tensors[0])
       self.event = torch.cuda.Event()
       self.event.record(torch.cuda.current_stream(tensors[0].device))
 
@@ -473,7 +473,7 @@ class _Kept:
     outside it, nor ask: False until an ordinary call has seen the work done.)"""
     if self.stream is None:
       return True
-    other = _lib.stream_of(self.tensors[0]) != self.stream
+    other = _lib.stream_on(self.device) != self.stream
     if self.event is not None:
       if torch.cuda.is_current_stream_capturing():
         return False
@@ -537,10 +537,8 @@ def _weight_ksums(values_owner, b: torch.Tensor, key_extra: tuple, compute, dime
 def _named_ksums(rhs, dimension_numbers):
   """The kept K-sums of an asymmetric lhs's weight while that is alive and unchanged, else None."""
   store = rhs.qvalue if isinstance(rhs, QArray) else None
-  if type(store) is not torch.Tensor or store.is_inference():
-    return None
   try:
-    return _kept_ksums(store, (id(store), dimension_numbers))
+    return _kept_ksums(store, (id(store), dimension_numbers)) if type(store) is torch.Tensor else None
   except TypeError:
     return None
 
