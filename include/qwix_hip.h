@@ -365,13 +365,16 @@ QWIX_API int qwix_hip_gemm_bf16_wq(const void* a, int64_t lda, const void* q, in
                           int64_t N, int64_t K, int64_t group, const void* s, int s_dtype, const int8_t* zp,
                           void* out, int out_dtype, int64_t ldo, void* stream);
 
-/* qwix_hip_gemm_bf16_wq with K cut into ranges while its tiles would cover at most half of the CUs (the same call in
- * the reference: _slow_dot_general, qwix/_src/core/dot_general.py:264-275): every range's workgroups write f32
+/* qwix_hip_gemm_bf16_wq for any K that is a multiple of 128 from 256 on, cut into ranges while its tiles would cover at
+ * most half of the CUs (the same call in the reference: _slow_dot_general, qwix/_src/core/dot_general.py:264-275): every range's workgroups write f32
  * partials into `workspace` (qwix_hip_gemm_bf16_wq_workspace_bytes(M, N, K, group) bytes, 16-byte aligned; 0 = this
  * shape is not split) and a second kernel adds them in range order and rounds once to out_dtype.  The f32 sums are
  * then formed in another order than the unsplit kernel's, so results agree with qwix_hip_gemm_bf16_wq to f32
- * rounding of the accumulation, not bit for bit.  With workspace NULL or too small: exactly qwix_hip_gemm_bf16_wq.  K is any
- * multiple of 128 from 256 on. */
+ * rounding of the accumulation, not bit for bit.  With workspace NULL or too small nothing is split: for K % 256 == 0 the bits
+ * of qwix_hip_gemm_bf16_wq, which refuses the other K, and for those still the bits of qwix_hip_dequantize_rm (to bf16)
+ * followed by qwix_hip_gemm_bf16.  Every code x scale is rounded to bf16 before it is multiplied, split or not (up to 2^-9 of a
+ * weight; the reference's own dequantize rounds so where scales are bf16); qwix_hip_gemv_wq multiplies the codes as they are
+ * and scales the f32 sums. */
 QWIX_API size_t qwix_hip_gemm_bf16_wq_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group);
 QWIX_API int qwix_hip_gemm_bf16_wq_ws(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int q_qtype, int64_t M,
                              int64_t N, int64_t K, int64_t group, const void* s, int s_dtype, const int8_t* zp,
@@ -381,7 +384,8 @@ QWIX_API int qwix_hip_gemm_bf16_wq_ws(const void* a, int64_t lda, const void* q,
 /* The same product with the rows of `a` in G consecutive groups (mixture of experts, _slow_ragged_dot_general,
  * qwix/_src/core/ragged_dot.py:229-241): rows of group g meet weights q + g * q_group_stride bytes and scales
  * s + g * s_group_stride elements (0: shared).  group_sizes: G int32 in device memory, read by the kernel; sizes are clamped
- * to the rows that exist, rows past the last group come out as zeros.  K % 128 == 0, K >= 256; symmetric weights. */
+ * to the rows that exist, rows past the last group come out as zeros.  K % 128 == 0, K >= 256; symmetric weights.  Weights are
+ * rounded to bf16 as in qwix_hip_gemm_bf16_wq, those of small groups too: qwix_hip_gemm_wq_groups streams these. */
 QWIX_API int qwix_hip_gemm_bf16_wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_bytes, int64_t q_group_stride,
                                  int q_qtype, int64_t M, int64_t N, int64_t K, int64_t group, const void* s, int s_dtype,
                                  int64_t s_group_stride, const int32_t* group_sizes, int64_t G, void* out, int out_dtype,

@@ -822,7 +822,7 @@ __global__ void __launch_bounds__(G::kNW * 64) __attribute__((amdgpu_waves_per_e
     if (first && kt + tpg < KT) sb_next = load_sb(g + 1);
     // (groups of several slabs: two loop bodies, the fold after the group's last MFMA)
     // (e4m3 with outer products: one body that starts from cleared sums.  Two of them spill; 16 rows, K 4096, N 4096, groups of 256
-    // 21.1 -> 19.3 us, 4096^3 83.8 / 83.8)
+    // 21.1 -> 19.3 us, 4096^3 83.8 -> 83.6)
     if constexpr (OUTER && F8) {
       if (first) {
 #pragma unroll

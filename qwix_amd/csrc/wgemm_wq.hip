@@ -675,7 +675,9 @@ static int wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_byte
   // Up to 80 rows per group on average most groups fit 128 rows; 64-column tiles while 128-column ones would occupy at most
   // half of the CUs.  Tiles of 128 x 64 / 256 x 128, 64 and 96 rows per group on average, some groups up to half as many
   // again: 64 groups, K 2048, N 1024, int8 72 / 71 and 88 / 75 us; 8 groups, K 2176, N 5312 56 / 71 and 73 / 72 us; 8 groups,
-  // K 4096, N 14336, int4 193 / 230 and 217 / 233 us; 128 rows 312 / 236 us.
+  // K 4096, N 14336, int4 193 / 230 and 217 / 233 us; 128 rows 312 / 236 us.  A group with nearly all rows has its weight converted
+  // once per row tile; sizes are not known here.  Such calls group by group / here, 640 rows in 8 groups, all but 28 in one, K 4096,
+  // N 14336: int4 324 / 177 us, int8 334 / 215; 1280 rows int4 353 / 229, int8 398 / 280; 140 rows in 2 groups int8 119 / 74.
   const bool half = K % 256 != 0;  // (groups of more than 256 rows, where dot_general's rule says what is streamed)
   const int tile = M <= 80 * G && !half ? 0 : (M / 256 + G) * ((N + 127) / 128) <= 128 ? 1 : 2;
 #define QWIX_WQR(OUTT, SBFF, BMM, BNN, BITS)                                                                         \
