@@ -231,7 +231,7 @@ extern "C" int qwix_hip_qgemm_ragged(const void* a, int64_t lda, const void* b, 
     return fail(QWIX_ERR_UNSUPPORTED, "ragged qgemm: operand too large for 32-bit offsets (M*lda=%lld N*ldb=%lld)",
                 (long long)(M * lda), (long long)(N * ldb));
   const Epilogue ep = make_epilogue(qtype, sa, sa_dtype, sb, sb_dtype, acc_dtype, nullptr, nullptr, out_dtype);
-  const Ragged rg{group_sizes, static_cast<int>(G), b_group_stride, sb_group_stride};
+  const Ragged rg{group_sizes, static_cast<int>(G), 0, b_group_stride, sb_group_stride};
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (K % 128 == 0 && M <= 16 * G && G + 1 <= 65535 && 64 * ldb < (int64_t{1} << 31)) {
     // at most 16 rows per group on average (decode): stream every group's weight once instead of tiling

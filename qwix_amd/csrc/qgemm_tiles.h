@@ -1071,9 +1071,9 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
 struct Ragged {
   const int32_t* group_sizes;  // G entries
   int G;
+  int skip;                 // groups of up to this many rows have no tiles here (another launch does them)
   int64_t b_group_stride;   // bytes between consecutive B panels
   int64_t sb_group_stride;  // elements between the rhs scale vectors of consecutive groups (0: one shared vector)
-  int skip;                 // groups of up to this many rows have no tiles here (another launch does them)
 };
 
 constexpr int kRaggedChunk = 16;  // consecutive tile ids that run on one XCD

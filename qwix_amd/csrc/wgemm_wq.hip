@@ -63,11 +63,13 @@ namespace {
 // HALF: K may be 128 mod 256, the last superslab half of one: another tail behind a branch, clamped loads of the last line of
 // int4 weights and of its scales.  A template parameter because the branch costs registers that all K would pay for (bf16
 // result, 128 x 64 int4 / int8, 256 x 128 int4: 124 / 151 / 248 per lane with it, 86 / 111 / 173 without).
+struct NoGroups {};  // (unused arguments would move the ones behind them into another line of the argument block)
 template <int OUT, bool SBF, int BM, int BN, int BITS, bool ZP, bool HALF, bool RAGGED = false>
 __global__ void __launch_bounds__(512)
     wgemm_wq_kernel(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ Q, int64_t ldq,
                     const void* __restrict__ S, const int8_t* __restrict__ Z, int M, int N, int K, int group,
-                    uint8_t* __restrict__ out, int64_t ldo, int ksplit, Ragged rg) {
+                    uint8_t* __restrict__ out, int64_t ldo, int ksplit,
+                    typename std::conditional<RAGGED, Ragged, NoGroups>::type rg) {
   static_assert((BM == 256 && (BN == 128 || BN == 64)) || (BM == 192 && BN == 128) || (BM == 128 && BN == 64),
                 "tiles of 256 x 128, 192 x 128, 256 x 64, 128 x 64");
   if (ksplit > 0) {
@@ -595,7 +597,7 @@ static int gemm_bf16_wq_impl(const void* a, int64_t lda, const void* q, int64_t 
     if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted[half])) return e_;                     \
     kern<<<grid, 512, smem, st>>>(static_cast<const uint8_t*>(a), 2 * lda, static_cast<const uint8_t*>(q), ldq_bytes, s, \
                                   zp, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),                 \
-                                  static_cast<int>(group), kern_dst, kern_ldo, ksplit, Ragged{});                              \
+                                  static_cast<int>(group), kern_dst, kern_ldo, ksplit, NoGroups{});                            \
   } while (0)
 #define QWIX_WQ_TILE(OUTT, SBFF, BITS)                                                                               \
   do {                                                                                                               \
@@ -670,7 +672,7 @@ static int wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_byte
       return rc;
     if (stream_rows >= M) return QWIX_OK;
   }
-  const Ragged rg{group_sizes, static_cast<int>(G), q_group_stride, s_group_stride, static_cast<int>(stream_rows)};
+  const Ragged rg{group_sizes, static_cast<int>(G), static_cast<int>(stream_rows), q_group_stride, s_group_stride};
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Up to 80 rows per group on average most groups fit 128 rows; 64-column tiles while 128-column ones would occupy at most
   // half of the CUs.  Tiles of 128 x 64 / 256 x 128, 64 and 96 rows per group on average, some groups up to half as many
