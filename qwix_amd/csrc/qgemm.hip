@@ -798,7 +798,7 @@ extern "C" int qwix_hip_gemm_bf16(const void* a, int64_t lda, const void* b, int
   const int64_t ldab = 2 * lda, ldbb = 2 * ldb, kb = 2 * K;  // the tile bodies count bytes
   if (M * ldab >= (int64_t{1} << 31) || N * ldbb >= (int64_t{1} << 31))
     return fail(QWIX_ERR_UNSUPPORTED, "operands beyond 2 GiB are not supported by the bf16 GEMM");
-  const Epilogue ep{nullptr, nullptr, 0, 0, out_dtype, 0, 0, 0, nullptr, nullptr};
+  const Epilogue ep{nullptr, nullptr, 0, 0, out_dtype, 0, 0, 0, 0, nullptr, nullptr};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool big = ((M + 255) / 256) * ((N + 255) / 256) >= 192;
   // Below that the rules of the quantized GEMM, which walks slabs of the same bytes: 64 x 64 tiles up to kSmallTiles tiles
@@ -922,7 +922,7 @@ __global__ void __launch_bounds__(256)
   tile_coords((M + 127) / 128, (N + 127) / 128, &tile_m, &tile_n);
   const int k0 = blockIdx.y * slabs_per_split * 128;
   const int klen = min(K - k0, slabs_per_split * 128);  // > 0: the host sizes the grid that way
-  const Epilogue raw{nullptr, nullptr, 0, 0, QT == QWIX_INT8 ? QWIX_I32 : QWIX_F32, 0, 0, 0, nullptr, nullptr};
+  const Epilogue raw{nullptr, nullptr, 0, 0, QT == QWIX_INT8 ? QWIX_I32 : QWIX_F32, 0, 0, 0, 0, nullptr, nullptr};
   uint8_t* part = ws + static_cast<int64_t>(blockIdx.y) * M * N * 4;
   qgemm_dma_tile<QT, 128, 128, 2, 2, (QT == QWIX_INT8 ? QWIX_I32 : QWIX_F32), 0>(A + k0, lda, B + k0, ldb, tile_m * 128,
                                                                                 tile_n * 128, M, N, klen, raw, part, N);

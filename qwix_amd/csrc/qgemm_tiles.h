@@ -47,13 +47,14 @@ struct Epilogue {
   const void* sa;  // per m, or null
   const void* sb;  // per n, or null
   int sa_dtype, sb_dtype, out_dtype;
-  int r0, r1, r2;
+  int r0, r1;
+  int16_t r2, zu8;  // (16 bits: a word more moves the kernels' last arguments into a third line, which every workgroup waits for)
   // Zero-point correction of an asymmetric operand (int8 only): acc[m,n] -= zu[m] * zv[n], where one
   // vector holds the zero points and the other the K-sums of the opposite operand's quantized values.
   const void* zu;  // int32, or int8 with zu8 (zero points as quantize writes them)
   const int32_t* zv;
-  int zu8;
 };
+static_assert(sizeof(Epilogue) == 56, "the argument blocks of the GEMM kernels");
 __device__ __forceinline__ int zu_at(const Epilogue& ep, int m) {
   return ep.zu8 ? static_cast<int>(static_cast<const int8_t*>(ep.zu)[m]) : static_cast<const int32_t*>(ep.zu)[m];
 }
@@ -1294,18 +1295,18 @@ __device__ __forceinline__ void skinny_block(const uint8_t* __restrict__ A, int6
 // float accumulator starts in acc_dtype; each multiply happens in the promotion of both sides.
 static Epilogue make_epilogue(int qtype, const void* sa, int sa_dtype, const void* sb, int sb_dtype, int acc_dtype,
                               const void* zu, const int32_t* zv, int out_dtype, bool zu8 = false) {
-  Epilogue ep{sa, sb, sa_dtype, sb_dtype, out_dtype, 0, 0, 0, zu, zv, zu8};
+  Epilogue ep{sa, sb, sa_dtype, sb_dtype, out_dtype, 0, 0, 0, zu8, zu, zv};
   int cur = (qtype == QWIX_INT8) ? QWIX_I32 : acc_dtype;
   if (cur == QWIX_BF16) ep.r0 = 1;
-  auto step = [&](const void* s, int s_dtype, int* r_after) {
+  auto step = [&](const void* s, int s_dtype, auto& r_after) {
     if (!s) return;
     const int t = (cur == QWIX_I32) ? s_dtype : ((cur == QWIX_F32 || s_dtype == QWIX_F32) ? QWIX_F32 : QWIX_BF16);
     if (cur == QWIX_I32 && t == QWIX_BF16) ep.r0 = 1;
-    *r_after = (t == QWIX_BF16);
+    r_after = (t == QWIX_BF16);
     cur = t;
   };
-  step(sa, sa_dtype, &ep.r1);
-  step(sb, sb_dtype, &ep.r2);
+  step(sa, sa_dtype, ep.r1);
+  step(sb, sb_dtype, ep.r2);
   return ep;
 }
 

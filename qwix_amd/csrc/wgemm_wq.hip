@@ -466,7 +466,7 @@ __global__ void __launch_bounds__(512)
     for (int qd = 0; qd < 4; ++qd)
 #pragma unroll
       for (int r = 0; r < 4; ++r) sbv[j][qd][r] = 1.f;
-  const Epilogue ep{nullptr, nullptr, 0, 0, OUT, 0, 0, 0, nullptr, nullptr};
+  const Epilogue ep{nullptr, nullptr, 0, 0, OUT, 0, 0, 0, 0, nullptr, nullptr};
   staged_epilogue<OUT, 0, TM, TN, NWAVES, LDS_BYTES, false>(acc, sav, sbv, ep, m0 + wm * WM, n0 + wn * WN, M, N, out, ldo,
                                                             smem, wave, lane);
 }
@@ -623,7 +623,7 @@ static int gemm_bf16_wq_impl(const void* a, int64_t lda, const void* q, int64_t 
 #undef QWIX_WQ_LAUNCH_Z
   if (int e = check_launch("gemm_bf16_wq")) return e;
   if (splits > 0) {
-    const Epilogue ep{nullptr, nullptr, 0, 0, out_dtype, 0, 0, 0, nullptr, nullptr};
+    const Epilogue ep{nullptr, nullptr, 0, 0, out_dtype, 0, 0, 0, 0, nullptr, nullptr};
     const int64_t threads = (M * N + 3) / 4;
     splitk_reduce_kernel<false><<<dim3(static_cast<unsigned>((threads + 255) / 256)), 256, 0, st>>>(
         static_cast<const uint8_t*>(workspace), splits, static_cast<int>(M), static_cast<int>(N), ep,
