@@ -30,7 +30,7 @@ def sources():
 
 def _compile(src: str, force: bool) -> str:
   obj = os.path.join(OBJ_DIR, src[:-4] + '.o')
-  deps = [os.path.join(HERE, f) for f in (src, 'common.h', 'qgemm_strips.h', 'qgemm_tiles.h')]
+  deps = [os.path.join(HERE, f) for f in (src, 'common.h', 'qgemm_grouped.h', 'qgemm_strips.h', 'qgemm_tiles.h')]
   deps.append(os.path.join(os.path.dirname(PKG), 'include', 'qwix_hip.h'))
   if not force and os.path.exists(obj) and all(os.path.getmtime(obj) > os.path.getmtime(d) for d in deps):
     return obj

@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "qgemm_grouped.h"
 
 namespace qwix {
 namespace {
@@ -32,30 +33,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 128, BK = 128, TM = 2, TN = 2, kPad = 16;
-
-struct GroupedArgs {
-  const uint8_t* A; int64_t lda;
-  const uint8_t* B; int64_t ldb;
-  int M, N, K, group;
-  const void* sa; int sa_dtype; int ga;
-  const void* sb; int sb_dtype;
-  int t_dtype;      // dtype of the scaled partials (promotion of the scale dtypes, and of acc_dtype for e4m3)
-  int acc_dtype;    // e4m3 operands: the dtype each group's f32 dot is rounded to before it is scaled
-  uint8_t* out; int out_dtype; int64_t ldo;
-  int32_t* acc_out;
-  // Zero-point correction of an asymmetric operand, per group: acc_g[m,n] -= zu[m,g] * zv[g,n].  One array
-  // holds zero points, the other the per-group K-sums of the opposite operand; element strides, 0 along the
-  // group axis for an array that is the same for all groups.  Both null: symmetric operands.
-  const int32_t* zu; int64_t zu_sm, zu_sg;
-  const int32_t* zv; int64_t zv_sn, zv_sg;
-  // One group spans all of K (int4 weights with per-channel scales): the fast kernel then scales like the untiled
-  // contraction, ((T(acc) * sx) * sy) with a rounding per step (dot_general.py:255-261), not like a sum of partials.
-  int single;
-  // K in ranges (0: none): workgroups with blockIdx.y = y contract elements [y ksplit, (y + 1) ksplit) -- whole groups --
-  // and write the f32 sums of their scaled partials, without the activation scale and the final rounding, as the y-th
-  // M x N array at `out` (the host passes f32, ldo = N, sa = null); grouped_reduce_kernel finishes.
-  int ksplit;
-};
 
 __device__ __forceinline__ float ld_scale(const void* p, int dtype, int64_t i) {
   return dtype == QWIX_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p)[i])
@@ -1367,6 +1344,29 @@ int dispatch_grouped_f8(const GroupedArgs& p, hipStream_t st) {
              : launch_grouped_dma<Q, false, SAG, false, false, 2, false>(p, st);
 }
 
+// Groups of 128 with bf16 scales, where 128 x 256 tiles are many enough for them: tiles of 64, 96 or 128 rows per wavefront
+// (qgemm_grouped_wide.hip; 2, 3 or 4 tiles of 32, the result) or 0, the 128 x 256 tiles of this file.  What counts is the rounds of the
+// CUs: one of 256 rows takes 1.67 times one of 128 rows, one of 192 rows 1.2 times (4096^3, 1 / 2 / 2 rounds, us: one scale per row, int8
+// 71 / 100 / 86, int4 68 / 100 / 81, e4m3 62 / 89 / 76; scales on both sides, int8 86 / 117 / 95, e4m3 77 / 106 / 86; 6000 x 3000 over K
+// 2048, 2 / 2 / 3 rounds, int8 75 / 60 / 69).  For 128 rows the kernel with eight
+// wavefronts of 64 x 64 is ahead while K is short (128 x 28672 over K 1024 16.9 -> 15.4 us, 300 x 20480 over K 1536 21.7 -> 19.8) and with
+// scales on both sides from two rounds on (4096^3 100 -> 95); with a long K and weights that come from HBM this file's is, whose
+// loads are a slab further ahead (500 x 14336 over K 4096 53 against 44).
+static int wide_rows(const GroupedArgs& p, int b_qtype, bool sag) {
+  if (p.group != Fast::kBK || p.single || p.zu || p.acc_out || p.ksplit || p.sb_dtype != QWIX_BF16 || p.K < 2 * Fast::kBK) return 0;
+  if (sag ? b_qtype == QWIX_INT4 || p.sa_dtype != QWIX_BF16 : b_qtype != QWIX_E4M3 && p.t_dtype != QWIX_BF16) return 0;
+  if (takes_narrow(p, sag)) return 0;
+  const int64_t groups = p.K / Fast::kBK;  // 32-bit byte offsets over a tile's rows and over the scales
+  if (256 * p.lda + p.K > INT32_MAX || 256 * p.ldb + p.K > INT32_MAX || groups * p.N * 2 > INT32_MAX || (sag && p.M * groups * 2 > INT32_MAX))
+    return 0;
+  auto rounds = [&](int64_t rows) { return ((p.M + rows - 1) / rows * ((p.N + 255) / 256) + 255) / 256; };
+  const int64_t r2 = rounds(128);
+  const double t4 = 1.67 * rounds(256), t3 = 1.2 * rounds(192), t2 = static_cast<double>(r2);
+  if (t4 < t2 && t4 <= t3) return 4;
+  if (t3 < t2) return 3;
+  return p.K <= 2048 || (sag && r2 > 1) ? 2 : 0;
+}
+
 // out[m, n] = cast(T(sa[m] * sum over ranges of ws[r][m][n])): what the tile kernel's epilogue does with its f32 sums,
 // after the K ranges' partial sums are added in range order.  Four consecutive elements of (m, n) per thread.
 __global__ void __launch_bounds__(256)
@@ -1574,6 +1574,7 @@ static int grouped_impl(const void* a, int64_t lda, const void* b, int64_t ldb_b
     const int ranges = workspace && !exact && !zu && !acc_out && aligned16(workspace)
                            ? grouped_ranges_of(M, N, K, group, b_qtype, sag, sa_dtype, sb_dtype) : 0;
     auto run = [&](const GroupedArgs& q) {
+      if (const int tm = wide_rows(q, b_qtype, sag)) return qgemm_grouped_wide(q, b_qtype, sag, tm, st);
       if (b_qtype == QWIX_E4M3) return sag ? dispatch_grouped_f8<true>(q, st) : dispatch_grouped_f8<false>(q, st);
       if (b_qtype == QWIX_INT4) return sag ? dispatch_grouped_dma<QWIX_INT4, true>(q, st) : dispatch_grouped_dma<QWIX_INT4, false>(q, st);
       return sag ? dispatch_grouped_dma<QWIX_INT8, true>(q, st) : dispatch_grouped_dma<QWIX_INT8, false>(q, st);
