@@ -229,6 +229,16 @@ QWIX_API int qwix_hip_qgemm_batched(const void* a, int64_t lda, int64_t a_batch_
                            void* out, int out_dtype, int64_t ldo, int64_t out_batch_stride,
                            void* stream);
 
+/* Batched contraction of two floating operands, both quantized on the way (the 'bqd,bkd->bqk' scores of attention under a rule
+ * with act_qtype; providers/boxed_param.py:173-236 quantizes each operand, then _fast_dot_general): x (batch, M, K) and
+ * y (batch, N, K), dense bf16 rows, each row with its own absmax scale, to int8 or e4m3; out (batch, M, N) bf16.  Bit-identical to
+ * qwix_hip_quantize of both and qwix_hip_qgemm_batched.  K is 64 or 128, N a multiple of 8.  Up to 64 rows of x one launch, and no
+ * workspace; else both are quantized first, in one launch, into a workspace of qwix_hip_qgemm_batched_act_workspace_bytes bytes (16-byte aligned, used
+ * by this call until it has finished on `stream`). */
+QWIX_API size_t qwix_hip_qgemm_batched_act_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K);
+QWIX_API int qwix_hip_qgemm_batched_act(const void* x, const void* y, int qtype, int64_t batch, int64_t M, int64_t N,
+                               int64_t K, void* out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Decode-size w8a8 with the activation quantization folded into the GEMM: per-token absmax int8
  * quantization of x (quantize, qwix/_src/core/qarray.py:638-644, as PtqProvider applies it to the
  * lhs of dot_general, providers/boxed_param.py:416-455) followed by _fast_dot_general

@@ -44,6 +44,13 @@ def _binary(lhs, rhs, einsum_str: str, dot_general_fn, preferred_element_type, *
   return out
 
 
+def fused_act_einsum(einsum_str: str, lhs, rhs, act_qtype):
+  """Two floating operands quantized on the way (dot_general.fused_act_batched); None when it does not take them."""
+  info = einsum_info.EinsumInfo.parse(einsum_str, ndims=(len(lhs.shape), len(rhs.shape)))
+  out = _dg.fused_act_batched(lhs, rhs, info.dimension_numbers, act_qtype)
+  return out if out is None or info.output_perm is None else out.permute(*info.output_perm)
+
+
 def broadcast_operands(operands: list, subs_list: list[str]) -> list:
   """einsum_info.py:197-241: operands that share a subscript with different sizes are brought to the
   largest one when it is a multiple of the others (size 1 included), values repeated tile-wise."""

@@ -327,6 +327,11 @@ __device__ __forceinline__ void buffer_to_lds16(R rsrc, uint8_t* lds, unsigned v
 #endif
 }
 
+// Dense bf16 rows of K = 64 or 128 elements of two arrays, 16-byte aligned, to int8 or e4m3 with a scale per row, in one launch
+// (quantize.hip); fewer than 2^36 rows.
+int quantize_two_rows(const void* x, int64_t nx, void* qx, void* sx, const void* y, int64_t ny, void* qy, void* sy, int64_t K,
+                      int qtype, void* stream);
+
 // qwix_hip_gemv_wq_groups for the groups of up to `most_rows` rows (gemv_wq.hip): with fewer than M the others and the rows
 // behind the groups are not written.
 int gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes, int b_qtype, int64_t M,

@@ -24,6 +24,9 @@ struct StripArgs {
 // out, and 32-bit byte offsets over b and over M + 128 rows of out.
 int qgemm_strips(int qtype, int64_t K, bool bf16, const StripArgs& p, int64_t batch, void* stream);
 
+// The same from bf16 rows of both, quantized in the kernel, for up to 64 rows of a (strides in bytes of them, sa and sb unused).
+int qgemm_strips_act(int qtype, int64_t K, const StripArgs& p, int64_t batch, void* stream);
+
 struct LongArgs {
   const uint8_t* a;
   int64_t lda, a_stride;  // bytes; strides between consecutive problems

@@ -25,7 +25,8 @@ enum { MODE_QUANT = 0, MODE_CALIB = 1, MODE_GIVEN = 2 };
 
 // Quantize N consecutive values (already divided / shifted) and store them packed.  BOUNDED selects
 // the two-op clamp-and-round converter (vector paths); the scalar paths keep NaN -> 0.
-template <int QT, int N, bool BOUNDED = false>
+// NT: eight bytes as a nontemporal store.
+template <int QT, int N, bool BOUNDED = false, bool NT = true>
 __device__ __forceinline__ void store_q(const float* v, uint8_t* q, int64_t elem, const uint32_t* bf16_signs = nullptr) {
   if constexpr (QT == QWIX_INT8) {
     uint32_t w[N / 4];
@@ -38,8 +39,10 @@ __device__ __forceinline__ void store_q(const float* v, uint8_t* q, int64_t elem
         w[i] = pack4_i8(to_int_q<QT>(v[4 * i]), to_int_q<QT>(v[4 * i + 1]), to_int_q<QT>(v[4 * i + 2]),
                         to_int_q<QT>(v[4 * i + 3]));
     }
-    if constexpr (N == 8)
+    if constexpr (N == 8 && NT)
       nt_store8(reinterpret_cast<uint2*>(q + elem), make_uint2(w[0], w[1]));
+    else if constexpr (N == 8)
+      *reinterpret_cast<uint2*>(q + elem) = make_uint2(w[0], w[1]);
     else
       *reinterpret_cast<uint32_t*>(q + elem) = w[0];
   } else if constexpr (QT == QWIX_E4M3) {
@@ -56,8 +59,10 @@ __device__ __forceinline__ void store_q(const float* v, uint8_t* q, int64_t elem
         w[i] = (__builtin_amdgcn_perm(bf16_signs[2 * i + 1], bf16_signs[2 * i], 0x07050301u) & 0x80808080u) |
                (w[i] & 0x7F7F7F7Fu);
     }
-    if constexpr (N == 8)
+    if constexpr (N == 8 && NT)
       nt_store8(reinterpret_cast<uint2*>(q + elem), make_uint2(w[0], w[1]));
+    else if constexpr (N == 8)
+      *reinterpret_cast<uint2*>(q + elem) = make_uint2(w[0], w[1]);
     else
       *reinterpret_cast<uint32_t*>(q + elem) = w[0];
   } else {  // INT4: element `elem` is even; low nibble = even element.
@@ -100,9 +105,8 @@ __device__ __forceinline__ s16x2 abs_keys(uint32_t pair) {
 }
 __device__ __forceinline__ float key_value(short key) { return bf16_bits_to_f32(static_cast<uint16_t>(key - kKeyOfZero)); }
 
-template <typename D, int QT, int CAL, int MODE, int NL>
-__global__ void __launch_bounds__(256)
-    rows_kernel(const uint8_t* __restrict__ x, int64_t nseg, int nvec, int log2g, float factor,
+template <typename D, int QT, int CAL, int MODE, int NL, bool NT = true>
+__device__ __forceinline__ void rows_block(unsigned block, const uint8_t* __restrict__ x, int64_t nseg, int nvec, int log2g, float factor,
                 uint8_t* __restrict__ q, void* __restrict__ scale, int8_t* __restrict__ zp,
                 void* __restrict__ cal0, void* __restrict__ cal1, int per_scale, int per_shift) {
   constexpr int EV = D::kVec;
@@ -110,7 +114,7 @@ __global__ void __launch_bounds__(256)
   __shared__ float red[2][4];
   const int tid = threadIdx.x;
   const int g = 1 << log2g;
-  const int64_t seg = (static_cast<int64_t>(blockIdx.x) << (8 - log2g)) + (tid >> log2g);
+  const int64_t seg = (static_cast<int64_t>(block) << (8 - log2g)) + (tid >> log2g);
   const int lane = tid & (g - 1);
   const bool seg_ok = seg < nseg;
   const uint4* xv = reinterpret_cast<const uint4*>(x) + seg * nvec;
@@ -226,9 +230,9 @@ __global__ void __launch_bounds__(256)
         }
         if constexpr (QT == QWIX_E4M3 && D::kTag == QWIX_BF16) {
           const uint32_t signs[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-          store_q<QT, EV, kBounded>(t, q, (seg * nvec + v) * EV, signs);
+          store_q<QT, EV, kBounded, NT>(t, q, (seg * nvec + v) * EV, signs);
         } else {
-          store_q<QT, EV, kBounded>(t, q, (seg * nvec + v) * EV);
+          store_q<QT, EV, kBounded, NT>(t, q, (seg * nvec + v) * EV);
         }
       }
     }
@@ -253,6 +257,30 @@ __global__ void __launch_bounds__(256)
   } else {
     quantize_all(std::integral_constant<bool, MODE == MODE_GIVEN>{});
   }
+}
+
+template <typename D, int QT, int CAL, int MODE, int NL>
+__global__ void __launch_bounds__(256)
+    rows_kernel(const uint8_t* __restrict__ x, int64_t nseg, int nvec, int log2g, float factor,
+                uint8_t* __restrict__ q, void* __restrict__ scale, int8_t* __restrict__ zp,
+                void* __restrict__ cal0, void* __restrict__ cal1, int per_scale, int per_shift) {
+  rows_block<D, QT, CAL, MODE, NL>(blockIdx.x, x, nseg, nvec, log2g, factor, q, scale, zp, cal0, cal1, per_scale, per_shift);
+}
+
+// The rows of two arrays in one launch, the first `split` blocks the first one's.  Plain stores: the product behind this launch reads the
+// codes several times, and from the caches (32 x 2048 x 2048 x 128: nontemporal 10.0 us and 82 us of the product, plain 11.2 and 68).
+struct Rows {
+  const uint8_t* x;
+  int64_t nseg;
+  uint8_t* q;
+  void* scale;
+};
+template <int QT, int NL>
+__global__ void __launch_bounds__(256) two_rows_kernel(Rows a, Rows b, unsigned split, int nvec, int log2g) {
+  const bool first = blockIdx.x < split;
+  const Rows r = first ? a : b;
+  rows_block<BF16, QT, QWIX_ABSMAX, MODE_QUANT, NL, false>(first ? blockIdx.x : blockIdx.x - split, r.x, r.nseg, nvec, log2g, 0.f, r.q, r.scale,
+                                                    nullptr, nullptr, nullptr, 1, 0);
 }
 
 // Any segment length (also odd ones): one workgroup per segment, two strided scalar passes; the
@@ -1825,6 +1853,24 @@ int check_cols(const void* x, int dtype, int64_t reduce, int64_t inner, int64_t 
 }
 
 }  // namespace
+
+int quantize_two_rows(const void* x, int64_t nx, void* qx, void* sx, const void* y, int64_t ny, void* qy, void* sy, int64_t K,
+                      int qtype, void* stream) {
+  const int nvec = static_cast<int>(K / 8), lg = 3;
+  const int64_t bx = (nx + 31) / 32, by = (ny + 31) / 32;
+  const Rows a{static_cast<const uint8_t*>(x), nx, static_cast<uint8_t*>(qx), sx}, b{static_cast<const uint8_t*>(y), ny, static_cast<uint8_t*>(qy), sy};
+  const dim3 grid(static_cast<unsigned>(bx + by));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const unsigned split = static_cast<unsigned>(bx);
+  if (qtype == QWIX_INT8) {
+    if (K == 64) two_rows_kernel<QWIX_INT8, 1><<<grid, 256, 0, st>>>(a, b, split, nvec, lg);
+    else two_rows_kernel<QWIX_INT8, 2><<<grid, 256, 0, st>>>(a, b, split, nvec, lg);
+  } else {
+    if (K == 64) two_rows_kernel<QWIX_E4M3, 1><<<grid, 256, 0, st>>>(a, b, split, nvec, lg);
+    else two_rows_kernel<QWIX_E4M3, 2><<<grid, 256, 0, st>>>(a, b, split, nvec, lg);
+  }
+  return check_launch("quantize (two arrays)");
+}
 }  // namespace qwix
 
 using namespace qwix;

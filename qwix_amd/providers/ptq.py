@@ -232,6 +232,12 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
   def _quantized_einsum(self, rule, op_id, einsum_str, lhs, rhs):
     get_how = functools.partial(_einsum.get_how_to_quantize, einsum_str=einsum_str,
                                 ndims=(len(lhs.shape), len(rhs.shape)), tile_size=rule.tile_size)
+    fused_qtype = self._fusable(rule)
+    if (fused_qtype is not None and self._einsum_fn is _einsum.einsum and type(lhs) is torch.Tensor and type(rhs) is torch.Tensor
+        and type(self)._prepare is BoxedParamProvider._prepare and '_prepare' not in self.__dict__):
+      out = _einsum.fused_act_einsum(einsum_str, lhs, rhs, fused_qtype)
+      if out is not None:
+        return out
     lhs, rhs = self._prepare(lhs, rhs, rule, op_id, get_how)
     return self._einsum_fn(einsum_str, lhs, rhs)
 

@@ -142,6 +142,47 @@ def test_batched_long_contraction(B, M, N, K, qtype, dtype):
   assert bool(((out.to(torch.float64) - want).abs() <= 2.0 ** -14 * terms + steps * want.abs()).all())
 
 
+@pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('K', [64, 128])
+@pytest.mark.parametrize('shape', [(1, 8), (16, 264), (17, 24), (33, 520), (64, 1000), (65, 72), (130, 2056), (3, 96, 2, 40)])
+def test_scores_quantized_inside_the_product(shape, K, qtype):
+  """Both operands of a scores product under a rule with act_qtype: quantized rows inside the kernel (the second operand too up to 64
+  rows), against quantize() of each and the contraction, bit for bit; rows of zeros, of signed zeros and with infinities and NaN among
+  them.  What the fused call does not take (f32, other layouts) gives the same results by the ordinary path."""
+  import qwix_amd
+  from qwix_amd import nn
+  print('case scores', shape, K, qtype, flush=True)
+  gen = torch.Generator(device=util.DEV).manual_seed(sum(shape) + K)
+  if len(shape) == 2:
+    spec, ls, rs = 'bqd,bkd->bqk', (3, shape[0], K), (3, shape[1], K)
+  else:  # two batch axes, two free axes on the left, the result in another order
+    spec, ls, rs = 'abqhd,abkd->abkqh', (2, shape[0], shape[1], shape[2], K), (2, shape[0], shape[3], K)
+  lhs = torch.randn(*ls, generator=gen, device=util.DEV).to(torch.bfloat16)
+  rhs = torch.randn(*rs, generator=gen, device=util.DEV).to(torch.bfloat16)
+  for t in (lhs, rhs):
+    rows = t.view(-1, K)
+    rows[0] = 0
+    rows[-1, ::2] = -0.0
+    if rows.shape[0] > 4:
+      rows[2, 5] = float('inf')
+      rows[3, 7] = float('nan')
+      rows[4] *= 1e-38
+  rule = qwix_amd.QuantizationRule(module_path='.*', weight_qtype=qtype, act_qtype=qtype)
+  model = qwix_amd.quantize_model(lambda params, a, b: nn.ops.einsum(spec, a, b), qwix_amd.PtqProvider([rule]))
+
+  def want(a, b):
+    q = [qwix_amd.quantize(t, qtype, channelwise_axes=list(range(t.ndim - 1))) for t in (a, b)]
+    return qwix_amd.einsum(spec, *q)
+  for _ in range(6):  # the ordinary path, then its plan
+    got = model.apply({}, lhs, rhs)
+    assert torch.equal(got.view(torch.int16), want(lhs, rhs).view(torch.int16))
+  strided = torch.cat([rhs, rhs], -1)[..., :K]
+  assert not strided.is_contiguous()
+  assert torch.equal(model.apply({}, lhs, strided).view(torch.int16), got.view(torch.int16))
+  f32 = model.apply({}, lhs.float(), rhs.float())
+  assert f32.dtype == torch.float32 and torch.equal(f32.view(torch.int32), want(lhs.float(), rhs.float()).view(torch.int32))
+
+
 def test_batched_dot_general_on_the_dequantize_path():
   """A float activation against a batched quantized operand takes the dequantize-first path."""
   from qwix_amd.core import dot_general as dg
