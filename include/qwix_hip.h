@@ -269,6 +269,12 @@ QWIX_API int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ldx,
                                int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
                                void* out, int out_dtype, int64_t ldo, void* workspace,
                                size_t workspace_bytes, void* stream);
+/* The same of max(x, 0), where a ReLU stands in front: rows of at most 32 KB.  Bit-identical to the ReLU and
+ * qwix_hip_qgemm_dynamic_act (a negative NaN counts as 0). */
+QWIX_API int qwix_hip_qgemm_dynamic_relu(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype,
+                                int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
+                                void* out, int out_dtype, int64_t ldo, void* workspace,
+                                size_t workspace_bytes, void* stream);
 
 /* out[r] = sum_k q[r*ld + k] for int8 rows (K % 16 == 0): the K-sums qwix_hip_qgemm_zp needs
  * (the reference obtains them as a dot_general against the broadcast zero point,

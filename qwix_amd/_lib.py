@@ -50,6 +50,7 @@ SIGNATURES = {
     'qwix_hip_qgemm_fused_act': (_int, [_vp, _int, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _int, _vp, _int, _i64, _vp]),
     'qwix_hip_qgemm_dynamic_act_workspace_bytes': (_sz, [_i64, _i64, _i64, _int]),
     'qwix_hip_qgemm_dynamic_act': (_int, [_vp, _int, _i64, _vp, _i64, _int, _i64, _i64, _i64, _vp, _int, _int, _vp, _int, _i64, _vp, _sz, _vp]),
+    'qwix_hip_qgemm_dynamic_relu': (_int, [_vp, _int, _i64, _vp, _i64, _int, _i64, _i64, _i64, _vp, _int, _int, _vp, _int, _i64, _vp, _sz, _vp]),
     'qwix_hip_qgemm_hadamard_act_workspace_bytes': (_sz, [_i64, _i64, _i64, _int]),
     'qwix_hip_qgemm_hadamard_act': (_int, [_vp, _int, _i64, _i64, _i64, _vp, _vp, _f32, _i64, _vp, _i64, _int, _i64, _vp, _int, _vp, _int, _i64, _vp, _sz, _vp]),
     'qwix_hip_ksum_i8': (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),

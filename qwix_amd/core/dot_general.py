@@ -345,23 +345,23 @@ def fused_act_batched(lhs, rhs, dimension_numbers, act_qtype):
   return out.reshape(*bshape, *lhs.shape[nb:-1], *rhs.shape[nb:-1])
 
 
-def fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, act_qtype=numerics.INT8):
+def fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, act_qtype=numerics.INT8, relu=False):
   """Dynamic per-token quantization of a float lhs (absmax over the whole contraction, to the weight's own
   qtype: int8 or e4m3) and the quantized contraction against a per-channel weight in one library call
   (qwix_hip_qgemm_dynamic_act): one launch at decode sizes, the quantize kernel and the GEMM back to back on a
   scratch buffer otherwise.  Bit-identical to quantize(lhs, channelwise over the non-contracting axes)
   followed by dot_general.  Returns None when the operands are not of that kind; the caller then takes the
-  two-step route."""
-  fixed = ('fused_act', dimension_numbers, preferred_element_type, act_qtype)
+  two-step route.  `relu`: of max(lhs, 0), read from lhs itself."""
+  fixed = ('fused_act', dimension_numbers, preferred_element_type, act_qtype, relu)
   out = (plans._native or plans.native()).run(fixed, lhs, rhs)
   if out is None:
-    return _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype)
+    return _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype, relu)
   return out if out is not True else plans.record(
-      fixed, (lhs, rhs), lambda: _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype),
+      fixed, (lhs, rhs), lambda: _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype, relu),
       plans.single)
 
 
-def _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype):
+def _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, act_qtype, relu=False):
   if not (_is_float_array(lhs) and lhs.dtype in (torch.bfloat16, torch.float32) and isinstance(rhs, QArray)):
     return None
   if rhs.zero_point is not None or isinstance(rhs.qvalue, Int4Tensor):
@@ -386,12 +386,14 @@ def _fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type, 
   x = c.lhs_values(lhs)
   if x.stride(1) != 1 or x.stride(0) != c.K:
     x = x.contiguous()
+  if relu and (c.K * x.element_size() > 16 * 2048 or x.data_ptr() % 16):
+    return None
   b, _ = c.rhs_values(rhs)
   sb, _ = c.rhs_scale(rhs)
   out = torch.empty(c.M, c.N, dtype=res_t, device=x.device)
   nws = _dynamic_act_bytes(c.M, c.N, c.K, _lib.float_tag(x.dtype))
   ws = torch.empty(nws, dtype=torch.uint8, device=x.device) if nws else None
-  _lib.call('qwix_hip_qgemm_dynamic_act', x.data_ptr(), _lib.float_tag(x.dtype), x.stride(0), b.data_ptr(), b.stride(0),
+  _lib.call('qwix_hip_qgemm_dynamic_relu' if relu else 'qwix_hip_qgemm_dynamic_act', x.data_ptr(), _lib.float_tag(x.dtype), x.stride(0), b.data_ptr(), b.stride(0),
             _lib.INT8 if act_qtype == numerics.INT8 else _lib.E4M3, c.M, c.N, c.K, sb.data_ptr(),
             _lib.float_tag(sb.dtype), _tag_of(acc_t) if acc_t != torch.int32 else 0, out.data_ptr(),
             _lib.float_tag(res_t), c.N, _lib.ptr(ws), nws, _lib.stream_of(x))

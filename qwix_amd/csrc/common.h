@@ -143,6 +143,17 @@ __device__ __forceinline__ void unpack16(const uint4& v, float* f) {
   }
 }
 
+// max(x, 0) of a 16-byte vector of D, as integers: the encoding of a negative value, -0 and a negative NaN included, is a negative integer.
+template <typename D>
+__device__ __forceinline__ uint4 relu16(const uint4& v) {
+  typedef short s16x2 __attribute__((ext_vector_type(2)));
+  auto one = [](uint32_t w) -> uint32_t {
+    if constexpr (D::kTag == QWIX_BF16) return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, w), s16x2{0, 0}));
+    return static_cast<uint32_t>(max(static_cast<int>(w), 0));
+  };
+  return make_uint4(one(v.x), one(v.y), one(v.z), one(v.w));
+}
+
 // ------------------------------------------------------------------ qtype traits
 template <int QT>
 struct QTraits;
@@ -326,6 +337,10 @@ __device__ __forceinline__ void buffer_to_lds16(R rsrc, uint8_t* lds, unsigned v
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(lds), 16, voffset, soffset, 0, 0);
 #endif
 }
+
+// max(x, 0) of dense rows of K elements, 16-byte aligned, at most 2048 whole 16-byte vectors each, to int8 or e4m3 with a scale per row
+// (quantize.hip).
+int quantize_relu_rows(const void* x, int dtype, int64_t rows, int64_t K, int qtype, void* q, void* scale, void* stream);
 
 // Dense bf16 rows of K = 64 or 128 elements of two arrays, 16-byte aligned, to int8 or e4m3 with a scale per row, in one launch
 // (quantize.hip); fewer than 2^36 rows.

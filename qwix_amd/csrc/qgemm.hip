@@ -510,7 +510,7 @@ int launch_skinny(const void* a, int64_t lda, const void* b, int64_t ldb, int64_
 template <typename D, int NT, int KB>
 __global__ void __launch_bounds__(kSkinnyWaves * 64)
     qgemm_skinny_fused_kernel(const uint8_t* __restrict__ X, int64_t ldx, const uint8_t* __restrict__ B, int64_t ldb,
-                              int M, int N, int K, Epilogue ep, uint8_t* __restrict__ out, int64_t ldo) {
+                              int M, int N, int K, int relu, Epilogue ep, uint8_t* __restrict__ out, int64_t ldo) {
   constexpr int ES = D::kTag == QWIX_BF16 ? 2 : 4;   // bytes per activation
   constexpr int XV = 32 * ES / 16;                    // 16-byte loads per lane and K block (32 elements)
   __shared__ v4i red[kSkinnyWaves][NT][64];
@@ -551,6 +551,12 @@ __global__ void __launch_bounds__(kSkinnyWaves * 64)
     }
   }
 
+  if (relu) {
+#pragma unroll
+    for (int j = 0; j < KB; ++j)
+#pragma unroll
+      for (int v = 0; v < XV; ++v) xr[j][v] = relu16<D>(xr[j][v]);
+  }
   // ---- absmax of the 16 rows
   float mx = 0.f;
 #pragma unroll
@@ -633,7 +639,7 @@ __global__ void __launch_bounds__(kSkinnyWaves * 64)
 }
 
 template <typename D, int KB>
-int launch_skinny_fused(const void* x, int64_t ldx, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+int launch_skinny_fused(const void* x, int64_t ldx, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K, bool relu,
                         const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
   const unsigned gy = static_cast<unsigned>((M + 15) / 16);
 #define QWIX_FUSED(NTT)                                                                                              \
@@ -641,7 +647,7 @@ int launch_skinny_fused(const void* x, int64_t ldx, const void* b, int64_t ldb, 
                                           kSkinnyWaves * 64, 0, st>>>(static_cast<const uint8_t*>(x), ldx,           \
                                                                       static_cast<const uint8_t*>(b), ldb,           \
                                                                       static_cast<int>(M), static_cast<int>(N),      \
-                                                                      static_cast<int>(K), ep, static_cast<uint8_t*>(out), ldo)
+                                                                      static_cast<int>(K), relu ? 1 : 0, ep, static_cast<uint8_t*>(out), ldo)
   if (N >= 192 * 32)
     QWIX_FUSED(2);
   else
@@ -712,9 +718,8 @@ static double tiled_model_us(int64_t M, int64_t N, int64_t K) {
 
 static bool streams_weights(int64_t M, int64_t N, int64_t K, bool one_tile_row = false);
 
-extern "C" int qwix_hip_qgemm_fused_act(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb,
-                                        int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, void* out,
-                                        int out_dtype, int64_t ldo, void* stream) {
+static int fused_act_impl(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                          bool relu, const void* sb, int sb_dtype, void* out, int out_dtype, int64_t ldo, void* stream) {
   if (!x || !b || !out) return fail(QWIX_ERR_INVALID_ARGUMENT, "null x/b/out");
   if (x_dtype != QWIX_BF16 && x_dtype != QWIX_F32) return fail(QWIX_ERR_INVALID_ARGUMENT, "activations must be bf16 or f32");
   if ((sb && sb_dtype != QWIX_BF16 && sb_dtype != QWIX_F32) || (out_dtype != QWIX_BF16 && out_dtype != QWIX_F32))
@@ -734,8 +739,14 @@ extern "C" int qwix_hip_qgemm_fused_act(const void* x, int x_dtype, int64_t ldx,
   // the activation scale is computed in the activations' dtype, like the stand-alone quantize does
   const Epilogue ep = make_epilogue(QWIX_INT8, x, x_dtype, sb, sb_dtype, 0, nullptr, nullptr, out_dtype);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (x_dtype == QWIX_BF16) return launch_skinny_fused<BF16, 1>(x, ldx, b, ldb, M, N, K, ep, out, ldo, st);
-  return launch_skinny_fused<F32, 1>(x, ldx, b, ldb, M, N, K, ep, out, ldo, st);
+  if (x_dtype == QWIX_BF16) return launch_skinny_fused<BF16, 1>(x, ldx, b, ldb, M, N, K, relu, ep, out, ldo, st);
+  return launch_skinny_fused<F32, 1>(x, ldx, b, ldb, M, N, K, relu, ep, out, ldo, st);
+}
+
+extern "C" int qwix_hip_qgemm_fused_act(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb,
+                                        int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, void* out,
+                                        int out_dtype, int64_t ldo, void* stream) {
+  return fused_act_impl(x, x_dtype, ldx, b, ldb, M, N, K, false, sb, sb_dtype, out, out_dtype, ldo, stream);
 }
 
 // Workspace of qwix_hip_qgemm_dynamic_act: the quantized rows, their scales, what the quantize kernel itself needs
@@ -749,10 +760,9 @@ extern "C" size_t qwix_hip_qgemm_dynamic_act_workspace_bytes(int64_t M, int64_t 
          dyn_align(qwix_hip_qgemm_workspace_bytes(M, N, K));
 }
 
-extern "C" int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype,
-                                          int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
-                                          void* out, int out_dtype, int64_t ldo, void* workspace,
-                                          size_t workspace_bytes, void* stream) {
+static int dynamic_act_impl(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype, int64_t M, int64_t N,
+                            int64_t K, bool relu, const void* sb, int sb_dtype, int acc_dtype, void* out, int out_dtype,
+                            int64_t ldo, void* workspace, size_t workspace_bytes, void* stream) {
   if (!x || !b || !out) return fail(QWIX_ERR_INVALID_ARGUMENT, "null x/b/out");
   if (x_dtype != QWIX_BF16 && x_dtype != QWIX_F32) return fail(QWIX_ERR_INVALID_ARGUMENT, "activations must be bf16 or f32");
   if (qtype != QWIX_INT8 && qtype != QWIX_E4M3)
@@ -761,7 +771,7 @@ extern "C" int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ld
                                              (long long)N, (long long)K);
   // decode-size int8 calls: one launch (the rows are quantized in the GEMM's prologue)
   if (qtype == QWIX_INT8 && M <= 32 && K % 128 == 0 && K <= 128 * kSkinnyWaves && sb != nullptr)
-    return qwix_hip_qgemm_fused_act(x, x_dtype, ldx, b, ldb, M, N, K, sb, sb_dtype, out, out_dtype, ldo, stream);
+    return fused_act_impl(x, x_dtype, ldx, b, ldb, M, N, K, relu, sb, sb_dtype, out, out_dtype, ldo, stream);
   // otherwise: the quantize kernel, then the GEMM, on the caller's scratch memory
   if (ldx != K) return fail(QWIX_ERR_UNSUPPORTED, "the two-launch route needs dense activation rows (ldx=%lld K=%lld)",
                             (long long)ldx, (long long)K);
@@ -775,11 +785,30 @@ extern "C" int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ld
   const size_t qws_bytes = qwix_hip_quantize_workspace_bytes(M, K, 1, K, QWIX_ABSMAX);
   uint8_t* gws = qws + dyn_align(qws_bytes);
   const size_t gws_bytes = qwix_hip_qgemm_workspace_bytes(M, N, K);
-  if (int e = qwix_hip_quantize(x, x_dtype, M, K, 1, K, qtype, QWIX_ABSMAX, 0.f, QWIX_LAYOUT_NATURAL, q, sa, nullptr,
-                                qws_bytes ? qws : nullptr, qws_bytes, stream))
+  if (relu && (K % 8 || K * static_cast<int64_t>(es) > 16 * 2048 || !aligned16(x)))
+    return fail(QWIX_ERR_UNSUPPORTED, "a ReLU in front needs 16-byte aligned rows of at most 32 KB (K=%lld)", (long long)K);
+  if (int e = relu ? quantize_relu_rows(x, x_dtype, M, K, qtype, q, sa, stream)
+                   : qwix_hip_quantize(x, x_dtype, M, K, 1, K, qtype, QWIX_ABSMAX, 0.f, QWIX_LAYOUT_NATURAL, q, sa, nullptr,
+                                       qws_bytes ? qws : nullptr, qws_bytes, stream))
     return e;
   return qgemm_impl(q, K, b, ldb, qtype, M, N, K, sa, x_dtype, sb, sb_dtype, acc_dtype, nullptr, nullptr, out, out_dtype,
                     ldo, stream, gws_bytes ? gws : nullptr, gws_bytes);
+}
+
+extern "C" int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype,
+                                          int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
+                                          void* out, int out_dtype, int64_t ldo, void* workspace,
+                                          size_t workspace_bytes, void* stream) {
+  return dynamic_act_impl(x, x_dtype, ldx, b, ldb, qtype, M, N, K, false, sb, sb_dtype, acc_dtype, out, out_dtype, ldo, workspace,
+                          workspace_bytes, stream);
+}
+
+extern "C" int qwix_hip_qgemm_dynamic_relu(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype,
+                                           int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
+                                           void* out, int out_dtype, int64_t ldo, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+  return dynamic_act_impl(x, x_dtype, ldx, b, ldb, qtype, M, N, K, true, sb, sb_dtype, acc_dtype, out, out_dtype, ldo, workspace,
+                          workspace_bytes, stream);
 }
 
 extern "C" int qwix_hip_gemm_bf16(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,

@@ -12,6 +12,7 @@ import threading
 import torch
 
 from qwix_amd import qconfig
+from qwix_amd.providers.ptq import BoxedParamProvider
 from qwix_amd.providers.ptq import Param
 
 _tls = threading.local()
@@ -25,8 +26,13 @@ class _Ops:
   """Interception points: the two functions the provider overrides."""
 
   @staticmethod
-  def dot_general(lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None):
+  def dot_general(lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, lhs_relu=False):
+    """lhs_relu: of max(lhs, 0), which a provider may take together with the contraction."""
     p = current_provider()
+    if lhs_relu and p is not None and type(p).dot_general is BoxedParamProvider.dot_general and 'dot_general' not in p.__dict__:
+      return p.dot_general(lhs, rhs, dimension_numbers, precision, preferred_element_type, lhs_relu=True)
+    if lhs_relu:
+      lhs = torch.relu(lhs)
     if p is not None:
       return p.dot_general(lhs, rhs, dimension_numbers, precision, preferred_element_type)
     rhs = rhs.value if isinstance(rhs, Param) else rhs
@@ -56,9 +62,14 @@ class Dense:
       p['bias'] = torch.zeros(self.features, dtype=dtype, device=device)
     return p
 
-  def __call__(self, params: dict, x: torch.Tensor) -> torch.Tensor:
+  def __call__(self, params: dict, x: torch.Tensor, *, relu: bool = False) -> torch.Tensor:
+    """relu: of max(x, 0)."""
+    numbers = (((x.ndim - 1,), (0,)), ((), ()))
     with qconfig.module_scope(self.name):
-      y = ops.dot_general(x, Param(params, 'kernel'), (((x.ndim - 1,), (0,)), ((), ())))
+      if relu:
+        y = ops.dot_general(x, Param(params, 'kernel'), numbers, lhs_relu=True)
+      else:
+        y = ops.dot_general(x, Param(params, 'kernel'), numbers)
     if self.use_bias:
       y = y + params['bias'].to(y.dtype)
     return y
@@ -91,5 +102,4 @@ class MLP:
 
   def __call__(self, params: dict, x: torch.Tensor) -> torch.Tensor:
     h = self.layers[0](params['Dense_0'], x)
-    h = torch.relu(h)
-    return self.layers[1](params['Dense_1'], h)
+    return self.layers[1](params['Dense_1'], h, relu=True)

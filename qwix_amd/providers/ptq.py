@@ -161,13 +161,17 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
     qt = str(rule.act_qtype).replace('torch.', '')
     return qt if qt in ('int8', 'float8_e4m3fn') else None
 
+  def _stock(self) -> bool:
+    """Whether nothing that decides how an operation runs is overridden, in the class or in this object."""
+    cls = type(self)
+    return ((cls._prepare, cls._fusable, cls._quantized_dot_general, cls._quantized_einsum) == _STOCK_POLICY
+            and _POLICY.isdisjoint(self.__dict__))
+
   def _planned(self, op: str, arg, rule, lhs, rhs, ordinary):
     """One launch plan for the whole of an operation: the quantization of its activations and the contraction.  Only with the
     stock kernels and the stock policy (nothing that `ordinary` runs is overridden: plans are shared by all providers), dynamic
     ranges and a weight that is quantized already; `ordinary()` otherwise, and until the plan is kept."""
-    cls = type(self)
-    if ((cls._prepare, cls._fusable, cls._quantized_dot_general, cls._quantized_einsum) != _STOCK_POLICY
-        or not _POLICY.isdisjoint(self.__dict__)):
+    if not self._stock():
       return ordinary()
     w = rhs.value if isinstance(rhs, Param) else rhs
     boxed = isinstance(w, WithAux)
@@ -193,8 +197,16 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
     return _qarray.dequantize(x) if isinstance(x, _qarray.QArray) else x
 
   # -- ops
-  def dot_general(self, lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, out_sharding=None):
+  def dot_general(self, lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, out_sharding=None,
+                  lhs_relu=False):
+    """lhs_relu: of max(lhs, 0); where the activations are quantized on the way, without an array of its own."""
     rule, op_id = self._get_current_rule_and_op_id('dot_general')
+    if lhs_relu:
+      out = (None if rule is None or rule.act_qtype is None or rule.weight_qtype is None or out_sharding is not None else
+             self._relu_dot_general(rule, lhs, rhs, dimension_numbers))
+      if out is not None:
+        return out
+      lhs = torch.relu(lhs)
     if rule is None or rule.weight_qtype is None:
       # no rule for this op: the float contraction, batch axes included (boxed_param.py:119-127)
       return _dot_general.float_dot_general(self._unbox_float(lhs), self._unbox_float(rhs), dimension_numbers,
@@ -203,6 +215,16 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
       return self._quantized_dot_general(rule, op_id, lhs, rhs, dimension_numbers, out_sharding)
     return self._planned('dot_general', dimension_numbers, rule, lhs, rhs,
                          lambda: self._quantized_dot_general(rule, op_id, lhs, rhs, dimension_numbers, None))
+
+  def _relu_dot_general(self, rule, lhs, rhs, dimension_numbers):
+    """The contraction of max(lhs, 0) as one operation, under the stock policy and with a weight that is quantized already; else None."""
+    w = rhs.value if isinstance(rhs, Param) else rhs
+    if isinstance(w, WithAux):
+      w = w.array
+    if not self._stock() or type(lhs) is not torch.Tensor or not lhs.is_cuda or not isinstance(w, _qarray.QArray):
+      return None
+    qtype = self._fusable(rule)
+    return None if qtype is None else _dot_general.fused_act_dot_general(lhs, w, dimension_numbers, act_qtype=qtype, relu=True)
 
   def _quantized_dot_general(self, rule, op_id, lhs, rhs, dimension_numbers, out_sharding):
     get_how = functools.partial(_dot_general.get_how_to_quantize, dimension_numbers=dimension_numbers,
@@ -234,7 +256,7 @@ class BoxedParamProvider(qconfig.QuantizationProvider):
                                 ndims=(len(lhs.shape), len(rhs.shape)), tile_size=rule.tile_size)
     fused_qtype = self._fusable(rule)
     if (fused_qtype is not None and self._einsum_fn is _einsum.einsum and type(lhs) is torch.Tensor and type(rhs) is torch.Tensor
-        and type(self)._prepare is BoxedParamProvider._prepare and '_prepare' not in self.__dict__):
+        and self._stock()):
       out = _einsum.fused_act_einsum(einsum_str, lhs, rhs, fused_qtype)
       if out is not None:
         return out

@@ -39,15 +39,21 @@ def current_module_path() -> tuple[str, ...]:
   return tuple(getattr(_tls, 'path', ()))
 
 
-@contextlib.contextmanager
-def module_scope(name: str):
-  """Pushes `name` on this thread's module path for the duration of the block."""
-  old = current_module_path()
-  _tls.path = old + (name,)
-  try:
-    yield
-  finally:
-    _tls.path = old
+class module_scope(contextlib.ContextDecorator):
+  """Pushes `name` on this thread's module path for the duration of the block (or of the decorated function's calls)."""
+
+  def __init__(self, name: str):
+    self._name = name
+
+  def _recreate_cm(self) -> 'module_scope':
+    return module_scope(self._name)  # calls may nest
+
+  def __enter__(self) -> None:
+    self._old = current_module_path()
+    _tls.path = self._old + (self._name,)
+
+  def __exit__(self, *exc) -> None:
+    _tls.path = self._old
 
 
 class QuantizationProvider:
@@ -56,6 +62,7 @@ class QuantizationProvider:
   def __init__(self, rules: Sequence[QuantizationRule], *, disable_jit: bool = False):
     self._rules = [self._init_rule(rule) for rule in rules]
     self._rule_matches = [False] * len(self._rules)
+    self._rule_of: dict[tuple[tuple[str, ...], str], int] = {}  # (module path, op) -> the rule that applies, -1: none
     self._op_counts: dict[tuple[tuple[str, ...], str], int] = {}
     self._initial_run_complete = False  # set by the model wrapper once the model has run under this provider
     self.disable_jit = disable_jit
@@ -79,17 +86,22 @@ class QuantizationProvider:
 
   def _get_current_rule_and_op_id(self, op_name: str, *, only_rule: bool = False):
     path = current_module_path()
-    path_str = '/'.join(path)
+    key = (path, op_name)
+    i = self._rule_of.get(key)
+    if i is None:
+      path_str = '/'.join(path)
+      i = next((i for i, r in enumerate(self._rules)
+                if re.fullmatch(r.module_path, path_str) and (not r.op_names or op_name in r.op_names)), -1)
+      if len(self._rule_of) < 4096:
+        self._rule_of[key] = i
     rule = None
-    for i, r in enumerate(self._rules):
-      if re.fullmatch(r.module_path, path_str) and (not r.op_names or op_name in r.op_names):
-        rule = r
-        self._rule_matches[i] = True
-        break
+    if i >= 0:
+      rule = self._rules[i]
+      self._rule_matches[i] = True
     if only_rule:
       return rule, None
-    n = self._op_counts.get((path, op_name), 0)
-    self._op_counts[(path, op_name)] = n + 1
+    n = self._op_counts.get(key, 0)
+    self._op_counts[key] = n + 1
     return rule, f'{op_name}{n}'
 
   def get_unused_rules(self) -> list[QuantizationRule]:

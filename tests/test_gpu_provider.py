@@ -291,3 +291,36 @@ def test_decode_size_calls_fold_the_activation_quantization_into_the_gemm(monkey
   assert len(calls) == 4                                                   # 64 tokens: the same entry point, two launches
   monkeypatch.setattr(dg, 'fused_act_dot_general', lambda *a, **k: None)
   assert torch.equal(fused, ptq_model.apply(qparams, big))
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('rows,hidden', [(1, 256), (20, 2048), (33, 2048), (32, 2176), (300, 4096), (65, 8320), (9, 16512)])
+def test_relu_inside_the_quantization_of_the_next_layer(rows, hidden, qtype, dtype):
+  """The MLP's second layer takes max(h, 0) from h itself: against a ReLU of its own in front of the plain operation, bit for bit,
+  with rows that are negative throughout and with the kernel that quantizes in the product (up to 32 rows, K up to 2048); rows of
+  more than 32 KB keep the ReLU of their own."""
+  import qwix_amd
+  from qwix_amd import nn
+  print('case relu', rows, hidden, qtype, dtype, flush=True)
+  g = torch.Generator(device=util.DEV).manual_seed(rows + hidden)
+
+  class Plain(nn.MLP):
+    def __call__(self, params, x):
+      return self.layers[1](params['Dense_1'], torch.relu(self.layers[0](params['Dense_0'], x)))
+  rule = qwix_amd.QuantizationRule(module_path='.*', weight_qtype=qtype, act_qtype=qtype)
+  params = {'Dense_0': {'kernel': torch.randn(128, hidden, generator=g, device=util.DEV).to(dtype)},
+            'Dense_1': {'kernel': torch.randn(hidden, 136, generator=g, device=util.DEV).to(dtype)}}
+  x = torch.randn(rows, 128, generator=g, device=util.DEV).to(dtype)
+  models = [qwix_amd.quantize_model(m(hidden, 136), qwix_amd.PtqProvider([rule])) for m in (nn.MLP, Plain)]
+  params = qwix_amd.quantize_params(params, models[0].init(params, x))
+  for _ in range(6):  # the ordinary path, then its plan
+    got, want = (m.apply(params, x) for m in models)
+    assert got.dtype == dtype and torch.equal(got, want)
+  negative = {'Dense_0': params['Dense_0'], 'Dense_1': params['Dense_1']}
+  assert torch.equal(models[0].apply(negative, torch.zeros_like(x)), models[1].apply(negative, torch.zeros_like(x)))
+  # a provider with a dot_general of its own never sees the option
+  class Own(qwix_amd.PtqProvider):
+    def dot_general(self, lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, out_sharding=None):
+      return super().dot_general(lhs, rhs, dimension_numbers, precision, preferred_element_type, out_sharding=out_sharding)
+  assert torch.equal(qwix_amd.quantize_model(nn.MLP(hidden, 136), Own([rule])).apply(params, x), want)
