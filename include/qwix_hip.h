@@ -327,7 +327,8 @@ QWIX_API int qwix_hip_qgemm_hadamard_act(const void* x, int x_dtype, int64_t M, 
  * (qwix_hip_qgemm_grouped_call_bytes of the same arguments, ga == 1 without activation scales; 16-byte aligned; 0 = this call is
  * not split; qwix_hip_qgemm_grouped_workspace_bytes: the same for ga == 1); a second kernel adds them in range order, applies the
  * activation scale and rounds as the unsplit kernel's epilogue does.  The groups' f32 partials are then added in
- * another order than in qwix_hip_qgemm_grouped with exact == 0 (which itself is free in that order).  With workspace
+ * another order than in qwix_hip_qgemm_grouped with exact == 0 (which itself is free in that order).  Calls that run faster on
+ * the kernel for few tiles, whose wavefronts share K, leave the workspace alone: the same result with and without one.  With workspace
  * NULL or too small, with exact != 0, zero points or acc_out: exactly qwix_hip_qgemm_grouped. */
 QWIX_API size_t qwix_hip_qgemm_grouped_call_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, int sa_dtype,
                                          int64_t ga, int sb_dtype);

@@ -1222,6 +1222,36 @@ inline bool takes_outer(const GroupedArgs& p) {
   return outer_scales(p.sa_dtype, p.sb_dtype) && p.zu == nullptr && p.acc_out == nullptr && !p.single;
 }
 
+// us of the narrow tiles (128 x 64, two workgroups per CU; symmetric operands) with K in `sp` ranges (1: not split).  A tile walks its
+// slabs at about 0.78 us each (0.51 us up to 64 rows) after 3 us, however few tiles there are (weights from HBM); the ranges cost a
+// second launch and their partial arrays written and read.
+inline double narrow_us(int64_t M, int64_t N, int64_t K, int64_t sp) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64);
+  const double rounds = static_cast<double>((sp * tiles + 511) / 512);
+  const double walk = 3.0 + static_cast<double>(K / 128 / sp) * (M <= 64 ? 0.51 : 0.78) * rounds;
+  return sp == 1 ? walk : walk + 3.5 + static_cast<double>(sp * M * N) * 8.0 / 4.0e6;
+}
+constexpr int kMaxRanges = 8;  // what grouped_reduce_kernel reads in one batch
+// ... with the best number of ranges (0: one).
+inline int narrow_ranges(int64_t M, int64_t N, int64_t K, int64_t group, double* best_us) {
+  int best = 1;
+  *best_us = narrow_us(M, N, K, 1);
+  for (int64_t sp = 2; sp <= kMaxRanges && sp * 1024 <= K; ++sp) {
+    if (K % (sp * group)) continue;
+    const double us = narrow_us(M, N, K, sp);
+    if (us < (best == 1 ? 0.85 : 0.93) * *best_us) { best = static_cast<int>(sp); *best_us = us; }
+  }
+  return best > 1 ? best : 0;
+}
+
+// us of the decode kernel: a CU holds one workgroup of eight (byte weights: of four) wavefronts, which share the slabs.
+inline double decode_us(int64_t M, int64_t N, int64_t K, int b_qtype, bool sag) {
+  const double t = static_cast<double>(((M + 31) / 32) * ((N + 31) / 32)) / 256.0;
+  const double rounds = t <= 1.0 ? 1.0 : 0.5 * (t + static_cast<double>(static_cast<int64_t>(t + 0.999)));
+  const int64_t waves = b_qtype == QWIX_INT4 ? 8 : 4;
+  return 1.5 + rounds * (2.3 + static_cast<double>((K / 128 + waves - 1) / waves) * (b_qtype == QWIX_INT4 ? 0.8 : 0.62) * (sag ? 1.1 : 1.0));
+}
+
 // A decode batch against groups of 128: the kernel that splits K over wavefronts, while its N / 32 workgroups (each
 // reads all the activation rows) are a few hundred.  Weights from HBM, 16 rows, int8 x int4, one scale per token: K 4096,
 // N 4096 15.5 -> 8.6 us, N 14336 16.0 -> 12.3, K 14336, N 4096 76.6 -> 19.9, K 8192, N 8192 27.2 -> 13.8; at N 28672 the
@@ -1231,7 +1261,21 @@ inline bool takes_outer(const GroupedArgs& p) {
 // stages are smaller, weights of up to 80 MB are the decode kernel's at any N (K from 2048 on; int4 12 rows, N 28672 over K 1024 11.6 -> 12.1): int8 N 14336 over K 4096 19.5 -> 16.9, N 9088
 // over K 8192 31.5 -> 29.0, int4 N 28672 over K 4096 22.0 -> 18.3, e4m3 N 14336 over K 2048 12.0 -> 10.3 (4 rows; 16 rows 19.7 ->
 // 17.1, 32.1 -> 29.4, 22.2 -> 20.7, 12.2 -> 10.6); int8 N 18176 over K 8192 (149 MB) 49.3 against 50.5.
+// More rows, where the narrow tiles are few: a workgroup's wavefronts then share K where a tile walks it alone, or in ranges with a second
+// launch.  Weights from HBM, narrow tiles -> this, us: int4 51 x 2048 over K 5376 14.8 -> 7.8, 89 x 2880 over K 2048 16.4 -> 8.5, 128 x 2048
+// over K 8192 17.9 -> 9.6, 300 x 1024 over K 2048 17.4 -> 8.2; int8 17.6 -> 12.4 and 17.7 -> 9.4 for the last two, e4m3 with scales on both
+// sides 18.2 -> 13.2, 18.0 -> 9.6; int8 600 x 2048 over K 1024 12.6 against 17.7.  f32 weight scales keep the tiles' order of the groups,
+// in which the run that dumps its partials gives equal bits.
 inline bool takes_decode(const GroupedArgs& p, int b_qtype) {
+  if (p.M > 32) {
+    const bool sag = p.sa != nullptr && p.ga > 1;
+    if (p.ksplit || p.zu || p.acc_out || p.single || p.sb_dtype != QWIX_BF16 || p.group != Fast::kBK || p.K / Fast::kBK < 4 || (sag && b_qtype == QWIX_INT4) ||
+        !takes_narrow(p, sag) || 32 * p.lda >= (int64_t{1} << 31) || 32 * p.ldb >= (int64_t{1} << 31) || p.K > 16384)
+      return false;
+    double us;
+    narrow_ranges(p.M, p.N, p.K, p.group, &us);
+    return decode_us(p.M, p.N, p.K, b_qtype, sag) < 0.95 * us;
+  }
   const int64_t halves = static_cast<int64_t>(p.N) * (b_qtype == QWIX_INT4 ? 1 : 2);  // half bytes of a weight row
   const bool few = halves <= 16384 || (p.M <= 16 && p.K >= 2048 && halves * p.K <= int64_t{160} << 20);
   return p.ksplit == 0 && p.zu == nullptr && p.acc_out == nullptr && p.M <= 32 && p.group == Fast::kBK && !p.single &&
@@ -1407,12 +1451,8 @@ __global__ void __launch_bounds__(256)
       reinterpret_cast<float*>(out)[static_cast<int64_t>(m) * ldo + n] = t;
   }
 }
-constexpr int kMaxRanges = 8;  // what grouped_reduce_kernel reads in one batch
 
-// The K ranges of qwix_hip_qgemm_grouped_ws (0: none): for the narrow tiles (128 x 64, two workgroups per CU) of the
-// fast kernel, symmetric operands, above the decode kernel's 32 rows.  A tile walks its slabs at about 0.78 us each
-// (0.51 us up to 64 rows) after 3 us, however few tiles there are (weights from HBM); the ranges cost a second launch and
-// their partial arrays written and read.  int8, one scale per row / scales per group on both sides, 128 rows: N 1280 over K
+// The K ranges of qwix_hip_qgemm_grouped_ws (0: none): for the narrow tiles of the fast kernel, symmetric operands, above 32 rows.  int8, one scale per row / scales per group on both sides, 128 rows: N 1280 over K
 // 4096 28.3 / 33.9 us in one, 20.5 / 23.1, 15.5 / 18.0 and 13.6 / 14.3 in 2, 4 and 8 ranges; N 3072 over K 8192 50.5 / 61.2 and
 // 31.5 / 37.2, 21.4 / 23.8, 19.7 / 21.1; 768 rows, N 1280 29.2 / 34.4 and 22.5 / 25.7, 21.2 / 22.7, 28.6 / 30.0; 512 rows, N
 // 3072 52.5 / 64.2 and 42.7 / 49.6, 43.8 / 48.7, 52.1 / 55.6; e4m3 within 15 % of these.
@@ -1420,20 +1460,8 @@ static int grouped_ranges(int64_t M, int64_t N, int64_t K, int64_t group) {
   if (M <= 32 || group <= 0 || group % 128 || K % group || group == K) return 0;
   const int64_t wide = ((M + Fast::kBM - 1) / Fast::kBM) * ((N + Fast::kBN - 1) / Fast::kBN);
   if (!(wide <= kNarrowTiles || M <= 64)) return 0;
-  const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64);
-  auto model = [&](int64_t sp) {
-    const double rounds = static_cast<double>((sp * tiles + 511) / 512);
-    const double walk = 3.0 + static_cast<double>(K / 128 / sp) * (M <= 64 ? 0.51 : 0.78) * rounds;
-    return sp == 1 ? walk : walk + 3.5 + static_cast<double>(sp * M * N) * 8.0 / 4.0e6;
-  };
-  int best = 1;
-  double best_us = model(1);
-  for (int64_t sp = 2; sp <= kMaxRanges && sp * 1024 <= K; ++sp) {
-    if (K % (sp * group)) continue;
-    const double us = model(sp);
-    if (us < (best == 1 ? 0.85 : 0.93) * best_us) { best = static_cast<int>(sp); best_us = us; }
-  }
-  return best > 1 ? best : 0;
+  double us;
+  return narrow_ranges(M, N, K, group, &us);
 }
 
 // ... of one call: scales per group on both sides (`sag`) only where the fold by outer products takes them.
@@ -1571,7 +1599,7 @@ static int grouped_impl(const void* a, int64_t lda, const void* b, int64_t ldb_b
     // per-group activation scales ride along in LDS: the tile's scales must fit behind the slab stages
     const bool sag = sa != nullptr && ga > 1;
     // K in ranges with f32 partial sums in the caller's workspace, where the narrow tiles are few
-    const int ranges = workspace && !exact && !zu && !acc_out && aligned16(workspace)
+    const int ranges = workspace && !exact && !zu && !acc_out && aligned16(workspace) && !takes_decode(p, b_qtype)
                            ? grouped_ranges_of(M, N, K, group, b_qtype, sag, sa_dtype, sb_dtype) : 0;
     auto run = [&](const GroupedArgs& q) {
       if (const int tm = wide_rows(q, b_qtype, sag)) return qgemm_grouped_wide(q, b_qtype, sag, tm, st);
