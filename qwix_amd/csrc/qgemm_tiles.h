@@ -976,13 +976,13 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
     const int m_base = m0 + wm * 128, n_base = n0 + wn * 64;
     if (ep.sa != nullptr) {
       const int64_t es = ep.sa_dtype == QWIX_BF16 ? 2 : 4;
-      const int64_t want = (static_cast<int64_t>(m_base) * es + lane * 8) & ~int64_t{3}, last = (M * es - 4) & ~int64_t{3};
+      const int64_t want = (static_cast<int64_t>(m_base) * es + lane * 8) & ~int64_t{3}, last = M * es < 4 ? 0 : (M * es - 4) & ~int64_t{3};
       const int64_t off = want < last ? want : last;
       warm_a = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(ep.sa) + off);
     }
     if (ep.sb != nullptr) {
       const int64_t es = ep.sb_dtype == QWIX_BF16 ? 2 : 4;
-      const int64_t want = (static_cast<int64_t>(n_base) * es + lane * 4) & ~int64_t{3}, last = (N * es - 4) & ~int64_t{3};
+      const int64_t want = (static_cast<int64_t>(n_base) * es + lane * 4) & ~int64_t{3}, last = N * es < 4 ? 0 : (N * es - 4) & ~int64_t{3};
       const int64_t off = want < last ? want : last;
       warm_b = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(ep.sb) + off);
     }
