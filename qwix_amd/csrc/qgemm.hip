@@ -292,47 +292,75 @@ int launch_mid(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M
   return check_launch("qgemm (one tile row)");
 }
 
-template <int QT, int OUT, int EPI>
+// Rows of the ping-pong tiles / 64 of a dense product (0: 128 x 128 tiles or less).  Up to one 128 x 128 tile per CU those have three slab
+// stages and start sooner (1024 x 4096 over K 4096 24.8 against 27.8 us with 128 rows, 1500 x 1500 over K 8192 41.3 against 51.1), and
+// up to two per CU they overlap a short K's start with the other tile's end (4096 x 2048 over K 1024, e4m3 15.0 against 17.4).  Beyond:
+// int8 / e4m3, weights from HBM, 128 x 128 or (fifth on) 256 x 256 tiles -> these: 2048 x 4096 over K 4096 39.5 -> 35.9 / 36.3 -> 34.7
+// (128 rows), 512 x 14336 over K 4096 43.6 -> 38.8 / 44.5 -> 39.0 (128), 5224 x 1776 over K 3584 53.7 -> 37.3 (192), 2186 x 4992 over
+// K 9984 168 -> 100 (192); 3000 x 4096 over K 4096 50.6 -> 48.4 / 49.4 -> 44.6 (192), 2304 x 8192 over K 512 28.3 -> 23.9 / 32.7 -> 27.1.
+inline int pp_rows(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles_n = (N + 255) / 256;
+  const bool big = ((M + 255) / 256) * tiles_n >= 192;
+  if (!big && (tiles128 <= 256 || (tiles128 <= 512 && K < 1536))) return 0;
+  int best = 4;
+  double best_us = 0;
+  for (int tm = 4; tm >= 2; --tm) {
+    const double us = pp_us(tm, static_cast<double>((M + 64 * tm - 1) / (64 * tm) * tiles_n), K);
+    if (tm == 4 || us < best_us) { best = tm; best_us = us; }
+  }
+  return best;
+}
+
+template <int QT, int OUT, int EPI, int TM>
 __global__ void __launch_bounds__(512)
     qgemm_pp_kernel(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B, int64_t ldb, int M,
                     int N, int K, Epilogue ep, uint8_t* __restrict__ out, int64_t ldo) {
+  constexpr int BM = 64 * TM;
   int tile_m, tile_n;
-  tile_coords((M + 255) / 256, (N + 255) / 256, &tile_m, &tile_n);
-  qgemm_pp_tile<QT, OUT, EPI>(A, lda, B, ldb, tile_m * 256, tile_n * 256, M, N, K, ep, out, ldo);
+  tile_coords((M + BM - 1) / BM, (N + 255) / 256, &tile_m, &tile_n);
+  qgemm_pp_tile<QT, OUT, EPI, TM>(A, lda, B, ldb, tile_m * BM, tile_n * 256, M, N, K, ep, out, ldo);
 }
 
-template <int QT, int OUT, int EPI>
-int launch_pp(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-              const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
-  constexpr size_t smem = 5 * 256 * 128;
-  auto kern = qgemm_pp_kernel<QT, OUT, EPI>;
+template <int QT, int OUT, int EPI, int TM>
+int launch_pp_tile(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                   const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
+  constexpr int BM = 64 * TM;
+  constexpr size_t smem = (2 * BM + 3 * 256) * 128;
+  auto kern = qgemm_pp_kernel<QT, OUT, EPI, TM>;
   static LdsGrant granted;
   if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted)) return e_;
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + 255) / 256);
   kern<<<dim3(static_cast<unsigned>(tiles)), 512, smem, st>>>(
       static_cast<const uint8_t*>(a), lda, static_cast<const uint8_t*>(b), ldb, static_cast<int>(M),
       static_cast<int>(N), static_cast<int>(K), ep, static_cast<uint8_t*>(out), ldo);
   return check_launch("qgemm (ping-pong)");
 }
+template <int QT, int OUT, int EPI>
+int launch_pp(int tm, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+              const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
+  if (tm == 2) return launch_pp_tile<QT, OUT, EPI, 2>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+  if (tm == 3) return launch_pp_tile<QT, OUT, EPI, 3>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+  return launch_pp_tile<QT, OUT, EPI, 4>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+}
 
 template <int QT>
-int dispatch_pp(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+int dispatch_pp(int tm, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
                 const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
   const bool all = ep.r0 && ep.r1 && ep.r2, none = !ep.r0 && !ep.r1 && !ep.r2;
   if (ep.zu != nullptr) {
     if constexpr (QT == QWIX_INT8) {
-      if (ep.out_dtype == QWIX_BF16 && all) return launch_pp<QT, QWIX_BF16, 4>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
-      if (ep.out_dtype == QWIX_BF16) return launch_pp<QT, QWIX_BF16, 3>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
-      return launch_pp<QT, QWIX_F32, 3>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+      if (ep.out_dtype == QWIX_BF16 && all) return launch_pp<QT, QWIX_BF16, 4>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+      if (ep.out_dtype == QWIX_BF16) return launch_pp<QT, QWIX_BF16, 3>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+      return launch_pp<QT, QWIX_F32, 3>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
     }
     return fail(QWIX_ERR_UNSUPPORTED, "zero-point correction needs int8 operands");
   }
   if (ep.out_dtype == QWIX_BF16) {
-    if (all) return launch_pp<QT, QWIX_BF16, 1>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
-    return launch_pp<QT, QWIX_BF16, 2>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+    if (all) return launch_pp<QT, QWIX_BF16, 1>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+    return launch_pp<QT, QWIX_BF16, 2>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
   }
-  if (none) return launch_pp<QT, QWIX_F32, 0>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
-  return launch_pp<QT, QWIX_F32, 2>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+  if (none) return launch_pp<QT, QWIX_F32, 0>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+  return launch_pp<QT, QWIX_F32, 2>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
 }
 
 template <int QT, int BM, int BN, int BK>
@@ -830,6 +858,7 @@ extern "C" int qwix_hip_gemm_bf16(const void* a, int64_t lda, const void* b, int
   const Epilogue ep{nullptr, nullptr, 0, 0, out_dtype, 0, 0, 0, 0, nullptr, nullptr};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool big = ((M + 255) / 256) * ((N + 255) / 256) >= 192;
+  const int tm = pp_rows(M, N, kb);
   // Below that the rules of the quantized GEMM, which walks slabs of the same bytes: 64 x 64 tiles up to kSmallTiles tiles
   // of 128 x 128, four slab stages while they are at most two per CU; three stages for 128 x 128 tiles that are at
   // most one per CU.  With the dequantization in front, int4: 1300 x 1024 over K 1024 18.3 -> 12.6 us, 3000 x 1024 over K 7168
@@ -837,7 +866,7 @@ extern "C" int qwix_hip_gemm_bf16(const void* a, int64_t lda, const void* b, int
   const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
   auto run = [&](auto out_tag) {
     constexpr int OUT = decltype(out_tag)::value;
-    if (big && kb >= 256) return launch_pp<kOpBf16, OUT, 0>(a, ldab, b, ldbb, M, N, kb, ep, out, ldo, st);
+    if (tm && kb >= 256) return launch_pp<kOpBf16, OUT, 0>(tm, a, ldab, b, ldbb, M, N, kb, ep, out, ldo, st);
     if (big) return launch_dma<kOpBf16, 256, 256, 2, 4, OUT, 0>(a, ldab, b, ldbb, M, N, kb, ep, out, ldo, st);
     if (tiles128 <= kSmallTiles && tiles64 <= 512) return launch_dma<kOpBf16, 64, 64, 2, 2, OUT, 0, 4>(a, ldab, b, ldbb, M, N, kb, ep, out, ldo, st);
     if (tiles128 <= kSmallTiles) return launch_dma<kOpBf16, 64, 64, 2, 2, OUT, 0>(a, ldab, b, ldbb, M, N, kb, ep, out, ldo, st);
@@ -1161,14 +1190,15 @@ static int qgemm_impl(const void* a, int64_t lda, const void* b, int64_t ldb, in
     if (qtype == QWIX_INT8) return launch_skinny<QWIX_INT8>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
     return launch_skinny<QWIX_E4M3>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
   }
-  // 256 x 256 tiles once they fill most of the chip's 256 CUs; smaller problems use 128 x 128 tiles.
+  // 256 x 256 tiles once they fill most of the chip's 256 CUs; smaller problems use the tiles of pp_rows, or 128 x 128 and less.
   const bool big = ((M + 255) / 256) * ((N + 255) / 256) >= 192;
+  const int tm = big || !mid_ok ? pp_rows(M, N, K) : 0;
   const bool off32 = M * lda < (int64_t{1} << 31) && N * ldb < (int64_t{1} << 31);  // 32-bit lane offsets
   if (K % 128 == 0 && off32) {  // direct-to-LDS pipeline
-    // long K on a full chip: the ping-pong schedule (no raw-accumulator variant of it exists)
-    if (big && K >= 256 && out_dtype != QWIX_I32) {
-      if (qtype == QWIX_INT8) return dispatch_pp<QWIX_INT8>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
-      return dispatch_pp<QWIX_E4M3>(a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+    // the ping-pong schedule with 128, 192 or 256 rows (no raw-accumulator variant of it exists)
+    if (tm && K >= 256 && out_dtype != QWIX_I32) {
+      if (qtype == QWIX_INT8) return dispatch_pp<QWIX_INT8>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
+      return dispatch_pp<QWIX_E4M3>(tm, a, lda, b, ldb, M, N, K, ep, out, ldo, st);
     }
     // 64 x 64 tiles with four slab stages, at most two per CU
     const bool small_deep = ((M + 127) / 128) * ((N + 127) / 128) <= kSmallTiles && ((M + 63) / 64) * ((N + 63) / 64) <= 512;

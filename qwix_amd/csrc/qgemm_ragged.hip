@@ -22,43 +22,71 @@ __global__ void __launch_bounds__(WGM * WGN * 64)
                                                                         m_lim, N, K, e, out, ldo);
 }
 
-template <int QT, int OUT, int EPI>
+template <int QT, int OUT, int EPI, int TM>
 __global__ void __launch_bounds__(512)
     qgemm_ragged_pp_kernel(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B, int64_t ldb,
                            Ragged rg, int M, int N, int K, Epilogue ep, uint8_t* __restrict__ out, int64_t ldo) {
   int g, m0, m_lim, n0;
-  const int kind = ragged_tile<256, 256>(rg, M, N, &g, &m0, &m_lim, &n0);
+  const int kind = ragged_tile<64 * TM, 256>(rg, M, N, &g, &m0, &m_lim, &n0);
   if (kind == 0) return;
   using OutT = typename std::conditional<OUT == QWIX_BF16, uint16_t, uint32_t>::type;
   if (kind == 2) {
-    zero_tile<256, 256, OutT>(out, ldo, m0, m_lim, n0, N, 512);
+    zero_tile<64 * TM, 256, OutT>(out, ldo, m0, m_lim, n0, N, 512);
     return;
   }
   const Epilogue e = group_epilogue(ep, rg, g);
-  qgemm_pp_tile<QT, OUT, EPI>(A, lda, B + g * rg.b_group_stride, ldb, m0, n0, m_lim, N, K, e, out, ldo);
+  qgemm_pp_tile<QT, OUT, EPI, TM>(A, lda, B + g * rg.b_group_stride, ldb, m0, n0, m_lim, N, K, e, out, ldo);
 }
 
-template <int QT, int OUT, int EPI>
-int launch_ragged_pp_epi(const void* a, int64_t lda, const void* b, int64_t ldb, const Ragged& rg, int64_t M, int64_t N,
+template <int QT, int OUT, int EPI, int TM>
+int launch_ragged_pp_tile(const void* a, int64_t lda, const void* b, int64_t ldb, const Ragged& rg, int64_t M, int64_t N,
                          int64_t K, const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
-  constexpr size_t smem = 5 * 256 * 128;
-  auto kern = qgemm_ragged_pp_kernel<QT, OUT, EPI>;
+  constexpr size_t smem = (2 * 64 * TM + 3 * 256) * 128;
+  auto kern = qgemm_ragged_pp_kernel<QT, OUT, EPI, TM>;
   static LdsGrant granted;
   if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted)) return e_;
-  kern<<<dim3(ragged_grid(M, N, rg.G, 256, 256)), 512, smem, st>>>(
+  kern<<<dim3(ragged_grid(M, N, rg.G, 64 * TM, 256)), 512, smem, st>>>(
       static_cast<const uint8_t*>(a), lda, static_cast<const uint8_t*>(b), ldb, rg, static_cast<int>(M),
       static_cast<int>(N), static_cast<int>(K), ep, static_cast<uint8_t*>(out), ldo);
   return check_launch("ragged qgemm (ping-pong)");
 }
+template <int QT, int OUT, int EPI>
+int launch_ragged_pp_epi(int tm, const void* a, int64_t lda, const void* b, int64_t ldb, const Ragged& rg, int64_t M, int64_t N,
+                         int64_t K, const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
+  if (tm == 2) return launch_ragged_pp_tile<QT, OUT, EPI, 2>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+  if (tm == 3) return launch_ragged_pp_tile<QT, OUT, EPI, 3>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+  return launch_ragged_pp_tile<QT, OUT, EPI, 4>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+}
+// Ping-pong tiles of 64 * tm rows for a ragged product of more than 48 rows per group (0: 128 x 128 tiles).  The sizes are on the device:
+// each group is taken to end 0.45 of a tile early, and to have at least one.  Where 128 x 128 tiles are about one per CU and K is short
+// their two small workgroups per CU start and finish sooner.  int8 / e4m3, 8 to 64 groups of uneven sizes, weights from HBM, 128 x 128
+// tiles -> these, us: 4000 rows, 16 groups, N 4096 over K 2048 74.7 -> 58.9 / 72.4 -> 59.6 (192 rows); 4656, 16, N 1472, K 2816
+// 57.7 -> 35.6 (192); 3096, 16, N 2688, K 2176 50.8 -> 47.3 (128; 36.1 with 256, which no average shows); 6000, 16, N 2048, K 1024
+// 31.5 -> 22.9 / 29.2 -> 25.1 (256); 930, 8, N 1280, K 1152 12.5 against 13.0 (128).
+inline int ragged_pp_rows(int64_t M, int64_t N, int64_t K, int64_t G, bool big) {
+  auto tile_rows = [&](int64_t rows) {
+    const double per_group = static_cast<double>(M) / static_cast<double>(G * rows) + 0.45;
+    return static_cast<double>(G) * (per_group > 1.0 ? per_group : 1.0);
+  };
+  if (!big && K < 1536 && tile_rows(128) * static_cast<double>((N + 127) / 128) <= 256.0) return 0;
+  int best = 4;
+  double best_us = 0;
+  for (int tm = 4; tm >= 2; --tm) {
+    const double us = pp_us(tm, tile_rows(64 * tm) * static_cast<double>((N + 255) / 256), K);
+    if (tm == 4 || us < best_us) { best = tm; best_us = us; }
+  }
+  return best;
+}
+
 // The epilogue's rounding flags at compile time when every step rounds to bf16 (bf16 scales, bf16 result) or none
 // does (f32 throughout), as the dense dispatch does; at run time otherwise.
 template <int QT, int OUT>
-int launch_ragged_pp(const void* a, int64_t lda, const void* b, int64_t ldb, const Ragged& rg, int64_t M, int64_t N,
+int launch_ragged_pp(int tm, const void* a, int64_t lda, const void* b, int64_t ldb, const Ragged& rg, int64_t M, int64_t N,
                      int64_t K, const Epilogue& ep, void* out, int64_t ldo, hipStream_t st) {
   const bool all = ep.r0 && ep.r1 && ep.r2, none = !ep.r0 && !ep.r1 && !ep.r2;
-  if (OUT == QWIX_BF16 && all) return launch_ragged_pp_epi<QT, OUT, 1>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
-  if (OUT == QWIX_F32 && none) return launch_ragged_pp_epi<QT, OUT, 0>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
-  return launch_ragged_pp_epi<QT, OUT, 2>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+  if (OUT == QWIX_BF16 && all) return launch_ragged_pp_epi<QT, OUT, 1>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+  if (OUT == QWIX_F32 && none) return launch_ragged_pp_epi<QT, OUT, 0>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+  return launch_ragged_pp_epi<QT, OUT, 2>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
 }
 
 template <int QT, int BM, int BN, int BK>
@@ -240,9 +268,8 @@ extern "C" int qwix_hip_qgemm_ragged(const void* a, int64_t lda, const void* b, 
     return launch_ragged_skinny<QWIX_E4M3>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
   }
   if (K % 128 == 0) {
-    // 256-row tiles pay off once the average group is several tiles tall; 128-row tiles waste fewer rows
-    // at the ragged end of each group.
     const bool big = M / G >= 768 && ((M + 255) / 256) * ((N + 255) / 256) >= 192;
+    const int tm = ragged_pp_rows(M, N, K, G, big);
     // 17 to 48 rows per group on average: 64-row tiles with the deep weight prefetch (64 groups x 32 rows, K 2048,
     // N 4096: 131.7 against 144.8 us; from 64 rows per group on the 128-row tile wins again, 174 against 160 us)
     if (M <= 48 * G && out_dtype != QWIX_I32 &&
@@ -254,13 +281,13 @@ extern "C" int qwix_hip_qgemm_ragged(const void* a, int64_t lda, const void* b, 
       if (out_dtype == QWIX_BF16) return launch_ragged_mid<QWIX_E4M3, QWIX_BF16>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
       return launch_ragged_mid<QWIX_E4M3, QWIX_F32>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
     }
-    if (big && K >= 256 && out_dtype != QWIX_I32) {
+    if (tm && K >= 256 && out_dtype != QWIX_I32) {
       if (qtype == QWIX_INT8) {
-        if (out_dtype == QWIX_BF16) return launch_ragged_pp<QWIX_INT8, QWIX_BF16>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
-        return launch_ragged_pp<QWIX_INT8, QWIX_F32>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+        if (out_dtype == QWIX_BF16) return launch_ragged_pp<QWIX_INT8, QWIX_BF16>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+        return launch_ragged_pp<QWIX_INT8, QWIX_F32>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
       }
-      if (out_dtype == QWIX_BF16) return launch_ragged_pp<QWIX_E4M3, QWIX_BF16>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
-      return launch_ragged_pp<QWIX_E4M3, QWIX_F32>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+      if (out_dtype == QWIX_BF16) return launch_ragged_pp<QWIX_E4M3, QWIX_BF16>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
+      return launch_ragged_pp<QWIX_E4M3, QWIX_F32>(tm, a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);
     }
     if (qtype == QWIX_INT8) {
       if (big) return dispatch_ragged_dma<QWIX_INT8, 256, 256, 2, 4>(a, lda, b, ldb, rg, M, N, K, ep, out, ldo, st);

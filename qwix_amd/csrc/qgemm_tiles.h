@@ -4,7 +4,7 @@
 //   qgemm_tile      register-staged 128 x 128 tile, any K that is a multiple of 16
 //   qgemm_dma_tile  K % 128 == 0: 128-byte K slabs go global -> LDS directly, two stages (three or four where a
 //                   problem's tiles are so few per CU that nothing else covers the latency of the loads)
-//   qgemm_pp_tile   256 x 256, long K: two wavefront groups half a slab out of phase (ping-pong)
+//   qgemm_pp_tile   128, 192 or 256 x 256, long K: two wavefront groups half a slab out of phase (ping-pong)
 //   qgemm_mid_tile  one tile row, weights straight into registers
 //   skinny_block    up to 16 rows, K split over the wavefronts
 // Each is a device function of a tile origin and a row limit.  K is walked in slabs through LDS; rows are stored so that
@@ -872,15 +872,18 @@ __device__ __forceinline__ void qgemm_mid_tile(const uint8_t* __restrict__ A, in
 // what makes room for loading B two slabs ahead, which gives those loads three phases to land and
 // lets them be issued from the compute phase without a wait behind them.  Every load is waited for
 // by the wavefront that issued it (vmcnt, oldest first) before the barrier that publishes it.
-template <int QT, int OUT, int EPI>
+//   TM: the tile has 64 * TM rows (128, 192 or 256).  Per slab the LDS moves 176, 216 or 256 KB at 128 bytes a clock against 1024, 1536
+// or 2048 clocks of MFMAs per SIMD, so lower tiles are bound by the LDS and cost more per row; they pay where they leave less of the
+// chip idle in the last round, or less of a tile empty (pp_us).
+template <int QT, int OUT, int EPI, int TM = 4>
 __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B,
                                               int64_t ldb, int m0, int n0, int M, int N, int K, const Epilogue& ep,
                                               uint8_t* __restrict__ out, int64_t ldo) {
   constexpr bool IS_INT = (QT == QWIX_INT8);
   constexpr bool IS_BF = (QT == kOpBf16);
   constexpr bool B16 = IS_INT || IS_BF;  // 16 bytes per lane and k-step
-  constexpr int BM = 256, BN = 256, BK = 128, WGN = 4;
-  constexpr int TM = 4, TN = 2;                 // wave tile 128 x 64
+  constexpr int BM = 64 * TM, BN = 256, BK = 128, WGN = 4;
+  constexpr int TN = 2;                         // wave tile 32 * TM x 64
   constexpr int KSTEP = B16 ? 32 : 64, NK = BK / KSTEP;
   constexpr int A_STAGE = BM * BK, B_STAGE = BN * BK, B_BASE = 2 * A_STAGE;
   constexpr int LDS_BYTES = 2 * A_STAGE + 3 * B_STAGE;
@@ -900,21 +903,25 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-  // ---- loader: this wavefront brings rows [wm*128 + wn*32, +32) of A and of B, 8 rows per instruction
+  // ---- loader: this wavefront brings 8 * TM rows of its group's half of A and rows [wm*128 + wn*32, +32) of B, 8 rows per
+  // instruction
   const int lr = lane >> 3;
   const int lrow0 = wm * 128 + wn * 32;
-  uint32_t goffa[4], goffb[4];
+  const int arow0 = wm * (32 * TM) + wn * (8 * TM);
+  uint32_t goffa[TM], goffb[4];
+  const uint32_t lc = static_cast<uint32_t>((lane & 7) ^ swz8(lr));  // the row groups start at multiples of 8
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+    goffa[j] = static_cast<uint32_t>(min(m0 + arow0 + j * 8 + lr, M - 1)) * static_cast<uint32_t>(lda) + lc * 16;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const uint32_t lc = static_cast<uint32_t>((lane & 7) ^ swz8(lrow0 + j * 8 + lr));
-    goffa[j] = static_cast<uint32_t>(min(m0 + lrow0 + j * 8 + lr, M - 1)) * static_cast<uint32_t>(lda) + lc * 16;
     goffb[j] = static_cast<uint32_t>(min(n0 + lrow0 + j * 8 + lr, N - 1)) * static_cast<uint32_t>(ldb) + lc * 16;
   }
   auto load_a = [&](int kt) {  // own half of the A rows of slab kt
     const uint8_t* gk = A + kt * BK;
-    uint8_t* dst = smem + (kt & 1) * A_STAGE + lrow0 * BK;
+    uint8_t* dst = smem + (kt & 1) * A_STAGE + arow0 * BK;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) QWIX_GLDS16_AT_INPLACE(gk, goffa[j], dst + j * 1024);
+    for (int j = 0; j < TM; ++j) QWIX_GLDS16_AT_INPLACE(gk, goffa[j], dst + j * 1024);
   };
   auto load_b = [&](int kt, int stage) {  // own half of the B rows of slab kt
     const uint8_t* gk = B + kt * BK;
@@ -924,7 +931,7 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   };
 
   // ---- fragments of a whole slab
-  const int a_row = (wm * 128 + (lane & 31)) * BK;
+  const int a_row = (wm * (32 * TM) + (lane & 31)) * BK;
   const int b_row = B_BASE + (wn * 64 + (lane & 31)) * BK;
   const int hx = lane >> 5, x7 = swz8(lane & 31);
   FragT fa[NK][TM], fb[NK][TN];
@@ -958,9 +965,10 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   };
   // s_waitcnt on vmcnt only (expcnt 7, lgkmcnt 15 stay open): all but the newest `left` direct-to-LDS
   // loads of this wavefront have landed
-  auto wait_loads = [&](int left) {  // left: 0 or 4
-    if (left == 0) __builtin_amdgcn_s_waitcnt(0x0F70); else __builtin_amdgcn_s_waitcnt(0x0F74);
-  };
+  auto wait_loads = [&](auto left) { __builtin_amdgcn_s_waitcnt(0x0F70 | decltype(left)::value); };
+  using None = std::integral_constant<int, 0>;
+  using NewA = std::integral_constant<int, TM>;
+  using NewB = std::integral_constant<int, 4>;
   auto barrier = [&]() {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -973,7 +981,7 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   // now, under the equally cold first slab loads: 128 row scales and 64 column scales, 8 / 4 bytes per lane.
   uint32_t warm_a = 0, warm_b = 0;
   if constexpr (OUT != QWIX_I32) {
-    const int m_base = m0 + wm * 128, n_base = n0 + wn * 64;
+    const int m_base = m0 + wm * (32 * TM), n_base = n0 + wn * 64;
     if (ep.sa != nullptr) {
       const int64_t es = ep.sa_dtype == QWIX_BF16 ? 2 : 4;
       const int64_t want = (static_cast<int64_t>(m_base) * es + lane * 8) & ~int64_t{3}, last = M * es < 4 ? 0 : (M * es - 4) & ~int64_t{3};
@@ -991,14 +999,14 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   load_a(0);
   load_b(0, 0);
   load_b(1, 1);
-  wait_loads(0);
+  wait_loads(None{});
   asm volatile("" ::"v"(warm_a), "v"(warm_b));  // the touches above have landed too; their values are not used
   barrier();
   if (wm == 1) barrier();  // the lower group starts half a slab late
 
   // B is loaded two slabs ahead, during the compute phase, one load after each k-step's MFMAs (those
   // loads have three phases to land); A one slab ahead, in the memory phase.  The waits before the
-  // barriers leave the four loads just issued in flight and cover the four issued one phase earlier.
+  // barriers leave the loads just issued in flight and cover those issued one phase earlier.
   int bst = 0;  // B stage of slab kt = kt % 3
   // One slab; whether A of the next slab and B of the one after it are still to be requested is known at compile time,
   // so that the steady state is one basic block (a branch would end the scheduling regions that the fences below
@@ -1010,9 +1018,9 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
     __builtin_amdgcn_sched_barrier(0);  // fragment reads first: the loads below may not slip in front of them
     if constexpr (more_a) {
       load_a(kt + 1);
-      wait_loads(4);
+      wait_loads(NewA{});
     } else {
-      wait_loads(0);
+      wait_loads(None{});
     }
     barrier();
     // compute phase
@@ -1041,7 +1049,7 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
       __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_s_setprio(0);
-    if constexpr (more_b) wait_loads(4); else wait_loads(0);
+    if constexpr (more_b) wait_loads(NewB{}); else wait_loads(None{});
     barrier();
     bst = bst == 2 ? 0 : bst + 1;
   };
@@ -1056,11 +1064,21 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   slab(kt, F_{}, F_{});
   if (wm == 0) barrier();
 
-  const int m_base = m0 + wm * 128, n_base = n0 + wn * 64;
+  const int m_base = m0 + wm * (32 * TM), n_base = n0 + wn * 64;
   float sav[TM];
   float sbv[TN][4][4];
   fetch_scales<OUT, TM, TN>(ep, m_base, n_base, M, N, lane, sav, sbv);
   staged_epilogue<OUT, EPI, TM, TN, 8, LDS_BYTES>(acc, sav, sbv, ep, m_base, n_base, M, N, out, ldo, smem, wave, lane);
+}
+
+// us that `tiles` ping-pong tiles of 64 * tm rows take over K, one tile per CU at a time: a round's start and end, and its slabs, which
+// cost more the more CUs are at work (clock, L2).  Fitted to 130 dense and 130 ragged shapes, int8 and e4m3, weights from HBM: the
+// choice it makes is within 1 % (dense) and 2 % (ragged, sizes unknown) of the best of the three on average.
+inline double pp_us(int tm, double tiles, int64_t K) {
+  const double ends = 3.0 + tm, fixed = tm == 2 ? 0.44 : tm == 3 ? 0.55 : 0.64, busy = tm == 2 ? 0.5 : tm == 3 ? 0.65 : 0.8;
+  const double slabs = static_cast<double>(K / 128), rounds = tiles / 256.0;
+  const double full = static_cast<double>(static_cast<int64_t>(rounds + 1e-9)), rest = rounds - full;
+  return full * (ends + slabs * (fixed + busy)) + (rest > 1e-6 ? ends + slabs * (fixed + busy * rest) : 0.0);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -363,6 +363,36 @@ def test_int8_gemm_split_over_wavefronts_bit_exact(M, K, N, dtype):
   assert torch.equal(out, acc.to(torch.float32).to(out.dtype) * xq.scale * wq.scale)
 
 
+@pytest.mark.parametrize('kind', ['int8', 'e4m3', 'bf16'])
+@pytest.mark.parametrize('M,K,N', [(3087, 256, 4900), (1290, 1536, 3201),       # 128 rows: a remainder of 15 and of 10 rows, of 36 and 129 columns
+                                   (1417, 256, 5382), (5224, 1536, 1776), (129, 1536, 33000),     # 192 rows
+                                   (2306, 640, 4868)])                           # 256 rows
+def test_tiles_of_128_to_256_rows(M, K, N, kind):
+  """Ping-pong tiles of every height with partial tiles in both directions, from two slabs on: small integers, whose sums are exact in f32
+  in any order, equal a product in 64 bits; scaled by powers of two they equal its bf16."""
+  from qwix_amd import _lib
+  g = torch.Generator().manual_seed(M)
+  torch_dt = {'int8': torch.int8, 'e4m3': torch.float8_e4m3fn, 'bf16': torch.bfloat16}[kind]
+  a_i, b_i = (torch.randint(-7, 8, shape, generator=g, dtype=torch.int8).to(util.DEV) for shape in ((M, K), (N, K)))
+  a, b = a_i.to(torch.float32).to(torch_dt), b_i.to(torch.float32).to(torch_dt)
+  want = a_i.to(torch.float64) @ b_i.to(torch.float64).T
+  print('case tile rows', M, K, N, kind, flush=True)
+  out = torch.full((M, N), 7.0, dtype=torch.float32, device=util.DEV)
+  if kind == 'bf16':
+    _lib.call('qwix_hip_gemm_bf16', a.data_ptr(), K, b.data_ptr(), K, M, N, K, out.data_ptr(), _lib.F32, N, _lib.stream_of(a))
+    assert torch.equal(out.to(torch.float64), want)
+    return
+  qt, acc = (_lib.INT8, _lib.I32) if kind == 'int8' else (_lib.E4M3, _lib.F32)
+  _lib.call('qwix_hip_qgemm', a.data_ptr(), K, b.data_ptr(), K, qt, M, N, K, None, 0, None, 0, acc, out.data_ptr(), _lib.F32, N,
+            _lib.stream_of(a))
+  assert torch.equal(out.to(torch.float64), want)
+  sa, sb = ((2.0 ** torch.randint(-3, 3, (n,), generator=g)).to(torch.bfloat16).to(util.DEV) for n in (M, N))
+  scaled = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=util.DEV)
+  _lib.call('qwix_hip_qgemm', a.data_ptr(), K, b.data_ptr(), K, qt, M, N, K, sa.data_ptr(), _lib.BF16, sb.data_ptr(), _lib.BF16, acc,
+            scaled.data_ptr(), _lib.BF16, N, _lib.stream_of(a))
+  assert torch.equal(scaled, want.to(torch.float32).to(torch.bfloat16) * sa[:, None] * sb[None, :])
+
+
 def test_split_k_is_not_offered_where_it_cannot_pay():
   from qwix_amd import _lib
   f = _lib.load().qwix_hip_qgemm_workspace_bytes

@@ -330,6 +330,37 @@ def test_ragged_dot_looks_at_64_groups_at_a_time(G, K, rows):
   assert start == M
 
 
+@pytest.mark.parametrize('kind', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('M,K,N,sizes', [
+    (400, 1536, 317, (1, 0, 127, 129, 65)),                                    # 128 rows
+    (2499, 384, 2076, (1, 192, 193, 0) + (120,) * 15 + (300,)),                # 192
+    (3973, 640, 2565, (1, 256, 257, 0, 1500, 1900, 2 ** 31 - 1)),              # 256
+    (3329, 256, 4100, (3300, 0, 1)),                                           # 256: a group of many tiles
+])
+def test_ragged_dot_tiles_of_128_to_256_rows(M, K, N, sizes, kind):
+  """Tile heights are chosen from the average size: groups of one row at the front, a tile and a row more, none; the last rows in no group.
+  Small integers under scales that are powers of two: every step of the rounding chain is applied to exact values."""
+  import qwix_amd
+  g = torch.Generator().manual_seed(K + N)
+  dt = torch.int8 if kind == 'int8' else torch.float8_e4m3fn
+  G = len(sizes)
+  a_i = torch.randint(-7, 8, (M, K), generator=g, dtype=torch.int8).to(util.DEV)
+  b_i = torch.randint(-7, 8, (G, K, N), generator=g, dtype=torch.int8).to(util.DEV)
+  sa = 2.0 ** torch.randint(-3, 3, (M, 1), generator=g).to(util.DEV)
+  sb = 2.0 ** torch.randint(-3, 3, (G, 1, N), generator=g).to(util.DEV)
+  print('case ragged tile rows', M, K, N, kind, flush=True)
+  x = qwix_amd.QArray(a_i.to(torch.float32).to(dt), sa.to(torch.bfloat16), None, kind)
+  w = qwix_amd.QArray(b_i.to(torch.float32).to(dt), sb.to(torch.bfloat16), None, kind)
+  out = qwix_amd.ragged_dot(x, w, _sizes(sizes))
+  start = 0
+  for i, size in enumerate(sizes):
+    stop = min(start + size, M)
+    want = (a_i[start:stop].to(torch.float64) @ b_i[i].to(torch.float64)).to(torch.float32).to(torch.bfloat16)
+    assert torch.equal(out[start:stop], want * sa[start:stop].to(torch.bfloat16) * sb[i].to(torch.bfloat16)), i
+    start = stop
+  assert torch.count_nonzero(out[start:]).item() == 0
+
+
 def test_ragged_dot_weight_only_more_row_tiles_than_a_grid():
   """65534 groups of 17 and 3 rows: 98301 row tiles, more than a grid's y axis holds."""
   import qwix_amd
