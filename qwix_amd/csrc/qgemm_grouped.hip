@@ -329,21 +329,24 @@ int launch_grouped(const GroupedArgs& p, hipStream_t st) {
                                    (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
 
 struct Fast {
-  static constexpr int kBM = 128, kBN = 256, kBK = 128, kNW = 8, kTM = 4;
+  static constexpr int kBM = 128, kBN = 256, kBK = 128, kNW = 8, kTM = 4, kWR = 1;
 };
-// The same kernel with two wavefronts and 64 columns per workgroup: four times the workgroups, for problems whose
-// 128 x 256 tiles would leave most of the chip idle (a few hundred rows, or decode batches, against a weight of a few
-// thousand columns).
+// The same kernel with 64 columns per workgroup: four times the workgroups, for problems whose 128 x 256 tiles would leave most
+// of the chip idle (a few hundred rows, or decode batches, against a weight of a few thousand columns).  Bound by what a wavefront does
+// one after the other in a slab: four wavefronts of 64 x 32, two on every SIMD where two workgroups share a CU, halve it against two
+// of 128 x 32 (us, weights from HBM, int4 / int8 with one scale per row / int8 with scales on both sides: 600 x 2048 over K 1024 12.5 /
+// 12.7 / 12.9 -> 9.5 / 9.4 / 9.5, 256 x 4096 over K 2048 17.7 / 17.9 / 19.6 -> 13.8 / 13.3 / 14.5, 512 x 3072 over K 8192 41.1 / 41.6 / 47.6 ->
+// 33.4 / 33.1 / 37.2; equal bits).
 struct Narrow {
-  static constexpr int kBM = 128, kBN = 64, kBK = 128, kNW = 2, kTM = 4;
+  static constexpr int kBM = 128, kBN = 64, kBK = 128, kNW = 4, kTM = 2, kWR = 2;
 };
 // ... and with 64 or 32 rows for decode batches: a quarter of the MFMAs and folds per slab where the other rows of a
 // 128-row tile would be padding.
 struct Narrow64 {
-  static constexpr int kBM = 64, kBN = 64, kBK = 128, kNW = 2, kTM = 2;
+  static constexpr int kBM = 64, kBN = 64, kBK = 128, kNW = 4, kTM = 1, kWR = 2;
 };
 struct Narrow32 {
-  static constexpr int kBM = 32, kBN = 64, kBK = 128, kNW = 2, kTM = 1;
+  static constexpr int kBM = 32, kBN = 64, kBK = 128, kNW = 2, kTM = 1, kWR = 1;
 };
 
 // SAG: the activations carry one scale per row and group as well (both operands tiled along K): the
@@ -376,7 +379,8 @@ template <int BQT, bool SBF, bool SAG, bool AUX, bool MAGIC = false, int ST = 2,
 __global__ void __launch_bounds__(G::kNW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     qgemm_grouped_dma_kernel(GroupedArgs p) {
   constexpr int BM = G::kBM, BN = G::kBN, BK = G::kBK, NW = G::kNW, TM = G::kTM;
-  constexpr int WR = 1;  // every wavefront owns all rows of its 32 columns
+  constexpr int WR = G::kWR;  // wavefronts one below the other; each owns BM / WR rows of its 32 columns
+  static_assert(BM == 32 * TM * WR);
   constexpr bool W4 = (BQT == QWIX_INT4);
   if (p.ksplit > 0) {  // this workgroup's range of K: every operand moves to its first element
     const int y = blockIdx.y, k0 = y * p.ksplit;
@@ -944,9 +948,7 @@ size_t grouped_dma_lds(bool sag, int64_t K, int64_t group, int st, int64_t zu_gr
 // rows of zero-point side values that ride along in LDS: one per group, one in all, or none
 inline int64_t zu_groups_of(const GroupedArgs& p) { return p.zu == nullptr ? 0 : (p.zu_sg != 0 ? p.K / p.group : 1); }
 constexpr size_t kLdsMax = 160 * 1024;
-// Up to this many 128 x 256 tiles the narrow geometries run instead (from about 128 tiles on the wide tile's reuse of
-// a weight fragment over four MFMAs wins: 512 x 14336 over K 4096, 224 tiles, 42.6 against 71.5 us).
-constexpr int64_t kNarrowTiles = 80;
+constexpr int64_t kNarrowTiles = 512;  // of 128 x 64, two per CU
 
 template <int BQT, bool SBF, bool SAG, bool AUX, bool MAGIC, int ST, bool ONE, bool DUMP = false, typename G = Fast,
           bool OUTER = false>
@@ -1189,12 +1191,15 @@ int launch_grouped_decode(const GroupedArgs& p, hipStream_t st) {
   return launch_grouped_decode_rows<BQT, SBF, SAG, 32>(p, st);
 }
 
-// The narrow geometries: few 128 x 256 tiles (under a third of the CUs), or a decode batch.  With scales per group on both
-// sides while the 128 x 64 tiles are one round of the CUs (768 x 3072 over K 8192, 72 wide tiles: 121 us narrow, 101 wide),
-// or with K in ranges.  Scales on both sides, int8, weights from HBM, wide -> narrow: 256 x 1280 over K 4096 52 -> 33 us.
+// The narrow geometries: a decode batch, or 128 x 64 tiles that are one round of the CUs.  Two of their workgroups share a CU while
+// the LDS holds both: always, except with scales per group on both sides and a K of more than 4096.  128 x 256 tiles -> 128 x 64, us,
+// int8 with one scale per row / scales on both sides, weights from HBM: 384 tiles, 512 x 6144 over K 4096 39.2 / 46.7 -> 27.0 / 31.5; 352,
+// 1960 x 1408 over K 4096 39.3 / 46.7 -> 26.5 / 30.9; 512, 2048 x 2048 over K 4096 40.2 / 46.8 -> 32.9 / 35.1, 1000 x 4096 over K 2048
+// 23.0 / 24.5 -> 18.4 / 21.9; 640, 1200 x 4096 over K 8192 73.4 / 87.8 against 86.0 / 126; 768, 767 x 8192 over K 4096 42.6 / 48.2
+// against 49.7 / 56.6.
 inline bool takes_narrow(const GroupedArgs& p, bool sag) {
-  const int64_t wide = static_cast<int64_t>((p.M + Fast::kBM - 1) / Fast::kBM) * ((p.N + Fast::kBN - 1) / Fast::kBN);
-  return wide <= (sag && p.ksplit == 0 ? 64 : kNarrowTiles) || p.M <= 64;
+  const int64_t tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 63) / 64);
+  return tiles <= (sag && p.ksplit == 0 && p.K > 4096 ? 256 : kNarrowTiles) || p.M <= 64;
 }
 
 // Both operands with bf16 scales per group: the fold by outer products (see OUTER).  -1: the scales do not fit in LDS.
@@ -1222,24 +1227,32 @@ inline bool takes_outer(const GroupedArgs& p) {
   return outer_scales(p.sa_dtype, p.sb_dtype) && p.zu == nullptr && p.acc_out == nullptr && !p.single;
 }
 
-// us of the narrow tiles (128 x 64, two workgroups per CU; symmetric operands) with K in `sp` ranges (1: not split).  A tile walks its
-// slabs at about 0.78 us each (0.51 us up to 64 rows) after 3 us, however few tiles there are (weights from HBM); the ranges cost a
-// second launch and their partial arrays written and read.
-inline double narrow_us(int64_t M, int64_t N, int64_t K, int64_t sp) {
+// us of the narrow tiles (128 x 64; symmetric operands) with K in `sp` ranges (1: not split).  A tile walks its slabs at about 0.5 us
+// each after 3 us, however few tiles there are (weights from HBM), at 0.7 to 0.85 where two share a CU (64 rows: 0.38 to 0.5, and 0.6);
+// scales on both sides (`sag`) leave room for one where a range has more than 4096 of K.  The ranges cost a second launch and their
+// partial arrays written and read.  Fitted to 90 shapes of 33 to 2048 rows.
+inline double narrow_us(int64_t M, int64_t N, int64_t K, int64_t sp, bool sag) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64);
-  const double rounds = static_cast<double>((sp * tiles + 511) / 512);
-  const double walk = 3.0 + static_cast<double>(K / 128 / sp) * (M <= 64 ? 0.51 : 0.78) * rounds;
+  const double load = static_cast<double>(sp * tiles) / 256.0;
+  const bool low = M <= 64, two = low || !(sag && K / sp > 4096);
+  const double one_us = low ? 0.38 + 0.12 * (load < 1.0 ? load : 1.0) : 0.5, full_us = low ? 0.6 : 0.85;
+  double slab;
+  if (load <= 1.0) slab = one_us;
+  else if (!two) slab = one_us * static_cast<double>(static_cast<int64_t>(load + 0.999));
+  else if (load <= 2.0) slab = low ? full_us : 0.69 + 0.16 * (load - 1.0);
+  else slab = full_us * static_cast<double>(static_cast<int64_t>(0.5 * load + 0.999));
+  const double walk = 3.0 + static_cast<double>(K / 128 / sp) * slab;
   return sp == 1 ? walk : walk + 3.5 + static_cast<double>(sp * M * N) * 8.0 / 4.0e6;
 }
 constexpr int kMaxRanges = 8;  // what grouped_reduce_kernel reads in one batch
 // ... with the best number of ranges (0: one).
-inline int narrow_ranges(int64_t M, int64_t N, int64_t K, int64_t group, double* best_us) {
+inline int narrow_ranges(int64_t M, int64_t N, int64_t K, int64_t group, bool sag, double* best_us) {
   int best = 1;
-  *best_us = narrow_us(M, N, K, 1);
+  *best_us = narrow_us(M, N, K, 1, sag);
   for (int64_t sp = 2; sp <= kMaxRanges && sp * 1024 <= K; ++sp) {
     if (K % (sp * group)) continue;
-    const double us = narrow_us(M, N, K, sp);
-    if (us < (best == 1 ? 0.85 : 0.93) * *best_us) { best = static_cast<int>(sp); *best_us = us; }
+    const double us = narrow_us(M, N, K, sp, sag);
+    if (us < 0.93 * *best_us) { best = static_cast<int>(sp); *best_us = us; }
   }
   return best > 1 ? best : 0;
 }
@@ -1262,10 +1275,10 @@ inline double decode_us(int64_t M, int64_t N, int64_t K, int b_qtype, bool sag) 
 // over K 8192 31.5 -> 29.0, int4 N 28672 over K 4096 22.0 -> 18.3, e4m3 N 14336 over K 2048 12.0 -> 10.3 (4 rows; 16 rows 19.7 ->
 // 17.1, 32.1 -> 29.4, 22.2 -> 20.7, 12.2 -> 10.6); int8 N 18176 over K 8192 (149 MB) 49.3 against 50.5.
 // More rows, where the narrow tiles are few: a workgroup's wavefronts then share K where a tile walks it alone, or in ranges with a second
-// launch.  Weights from HBM, narrow tiles -> this, us: int4 51 x 2048 over K 5376 14.8 -> 7.8, 89 x 2880 over K 2048 16.4 -> 8.5, 128 x 2048
-// over K 8192 17.9 -> 9.6, 300 x 1024 over K 2048 17.4 -> 8.2; int8 17.6 -> 12.4 and 17.7 -> 9.4 for the last two, e4m3 with scales on both
-// sides 18.2 -> 13.2, 18.0 -> 9.6; int8 600 x 2048 over K 1024 12.6 against 17.7.  f32 weight scales keep the tiles' order of the groups,
-// in which the run that dumps its partials gives equal bits.
+// launch.  Weights from HBM, the best of these -> this, us: int4 71 x 2048 over K 3584 16.1 -> 8.2, 71 x 1088 over K 4352 17.6 -> 7.9;
+// int8 84 x 2304 over K 6912 14.3 -> 10.9; scales on both sides, int8 318 x 1280 over K 3328 16.6 -> 15.1, e4m3 178 x 1312 over K 2560
+// 14.1 -> 7.9; int8 238 x 4008 over K 2048 13.7 against 20.2.  f32 weight scales keep the tiles' order of the groups, in which the run that
+// dumps its partials gives equal bits.
 inline bool takes_decode(const GroupedArgs& p, int b_qtype) {
   if (p.M > 32) {
     const bool sag = p.sa != nullptr && p.ga > 1;
@@ -1273,7 +1286,7 @@ inline bool takes_decode(const GroupedArgs& p, int b_qtype) {
         !takes_narrow(p, sag) || 32 * p.lda >= (int64_t{1} << 31) || 32 * p.ldb >= (int64_t{1} << 31) || p.K > 16384)
       return false;
     double us;
-    narrow_ranges(p.M, p.N, p.K, p.group, &us);
+    narrow_ranges(p.M, p.N, p.K, p.group, sag, &us);
     return decode_us(p.M, p.N, p.K, b_qtype, sag) < 0.95 * us;
   }
   const int64_t halves = static_cast<int64_t>(p.N) * (b_qtype == QWIX_INT4 ? 1 : 2);  // half bytes of a weight row
@@ -1310,10 +1323,7 @@ int dispatch_grouped_dma(const GroupedArgs& p, hipStream_t st) {
       const int rc = sbf ? launch_grouped_decode<BQT, true, false>(p, st) : launch_grouped_decode<BQT, false, false>(p, st);
       if (rc >= 0) return rc;
     }
-    // Few 128 x 256 tiles (under a third of the CUs), or a decode batch: 128 x 64 tiles of two wavefronts, four times
-    // the workgroups; 32 or 64 rows per tile up to 64 rows.  int8 x int4 in groups of 128, weights from HBM, K 4096,
-    // N 4096, 16 / 64 / 128 / 512 rows: 35.7 / 36.5 / 38.4 / 39.0 us with the wide tile, 15.5 / 19.6 / 28.3 / 29.5 us now
-    // (K 8192, N 8192: 64.1 / 65.0 / 67.7 / 69.9 -> 27.2 / 34.7 / 49.1 / 70.0 us).
+    // (a kernel for 32 or 64 rows per tile up to 64 rows)
     if (takes_narrow(p, false)) {
       if (p.group == Fast::kBK && p.M <= 64) {  // decode batches: tiles of 32 or 64 rows
         if (sbf && p.t_dtype == QWIX_BF16)
@@ -1452,22 +1462,22 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The K ranges of qwix_hip_qgemm_grouped_ws (0: none): for the narrow tiles of the fast kernel, symmetric operands, above 32 rows.  int8, one scale per row / scales per group on both sides, 128 rows: N 1280 over K
-// 4096 28.3 / 33.9 us in one, 20.5 / 23.1, 15.5 / 18.0 and 13.6 / 14.3 in 2, 4 and 8 ranges; N 3072 over K 8192 50.5 / 61.2 and
-// 31.5 / 37.2, 21.4 / 23.8, 19.7 / 21.1; 768 rows, N 1280 29.2 / 34.4 and 22.5 / 25.7, 21.2 / 22.7, 28.6 / 30.0; 512 rows, N
-// 3072 52.5 / 64.2 and 42.7 / 49.6, 43.8 / 48.7, 52.1 / 55.6; e4m3 within 15 % of these.
-static int grouped_ranges(int64_t M, int64_t N, int64_t K, int64_t group) {
+// The K ranges of qwix_hip_qgemm_grouped_ws (0: none): for the narrow tiles of the fast kernel, symmetric operands, above 32 rows.  In one /
+// 2 / 4 / 8 ranges, us, weights from HBM: int8, one scale per row, 95 x 1912 over K 10240 45.0 / 28.8 / 19.4 / 15.6, 607 x 1408 over K 4608
+// 23.2 / 20.0 / 19.8 / -; scales on both sides, int8 93 x 1216 over K 4096 23.3 / 17.7 / 13.5 / -, e4m3 212 x 1168 over K 5120 26.2 / 19.2 /
+// 14.7 / -, 370 x 4744 over K 4096 23.7 / 24.6 / 30.6 / -.
+static int grouped_ranges(int64_t M, int64_t N, int64_t K, int64_t group, bool sag) {
   if (M <= 32 || group <= 0 || group % 128 || K % group || group == K) return 0;
-  const int64_t wide = ((M + Fast::kBM - 1) / Fast::kBM) * ((N + Fast::kBN - 1) / Fast::kBN);
-  if (!(wide <= kNarrowTiles || M <= 64)) return 0;
+  const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64);
+  if (!(tiles <= (sag && K > 4096 ? kNarrowTiles / 2 : kNarrowTiles) || M <= 64)) return 0;
   double us;
-  return narrow_ranges(M, N, K, group, &us);
+  return narrow_ranges(M, N, K, group, sag, &us);
 }
 
 // ... of one call: scales per group on both sides (`sag`) only where the fold by outer products takes them.
 static int grouped_ranges_of(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, bool sag, int sa_dtype, int sb_dtype) {
   if (sag && (b_qtype == QWIX_INT4 || !outer_scales(sa_dtype, sb_dtype))) return 0;
-  return grouped_ranges(M, N, K, group);
+  return grouped_ranges(M, N, K, group, sag);
 }
 
 // Per-group K-sums of quantized rows: out[row, g] = sum over the g-th group of `group` values of row `row`
