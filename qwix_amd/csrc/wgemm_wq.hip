@@ -58,11 +58,19 @@ namespace {
 // per tile: int4 333 x 14336 over K 4096 64.9 -> 56.2 us, 181 x 28288 over K 1792 29.0 -> 26.7, 160 x 28672 over K 8192 122 -> 109,
 // 700 x 14336 over K 4096 118 -> 107; int8 333 x 14336 62.3 -> 54.5; e4m3 380 x 10240 over K 2048 31.0 -> 27.3; where it takes
 // another round, 512 x 14336 over K 4096, 61 against 104.
+//   With int4 weights it splits the work as the 128-row tile does: four wavefronts of 96 x 64 multiply (80 KB of fragment reads per
+// slab instead of 128), four request and dequantize, and the LDS (160 KB) holds a fourth stage of activations.  333 x 14336 over K 4096
+// 59.5 -> 56.5 us, 700 x 14336 over K 4096 105 -> 101, 160 x 28672 over K 8192 102 -> 95.5, 181 x 28288 over K 1792 27.5 -> 27.3; no part
+// of a slab bounds it alone (without MFMAs 43, without activation loads 46, without conversion 52).  A 256-row tile has no room for that
+// stage and loses (512 x 14336 over K 4096 63.7 -> 66.9); a HALF one spills.
 // RAGGED: rows in groups (mixture of experts), found on the device as in the ragged GEMM: the tile's rows end with its
 // group, and weights and scales are the group's.
 // HALF: K may be 128 mod 256, the last superslab half of one: another tail behind a branch, clamped loads of the last line of
 // int4 weights and of its scales.  A template parameter because the branch costs registers that all K would pay for (bf16
 // result, 128 x 64 int4 / int8, 256 x 128 int4: 124 / 151 / 248 per lane with it, 86 / 111 / 173 without).
+// Whether a tile's wavefronts split the work (see above), and its stages of activations.
+constexpr bool wq_spec(int bm, int bn, int bits, bool half) { return bm == 128 || (bits == 4 && bm == 192 && !half); }
+constexpr int wq_stages(int bm, int bn, int bits, bool half) { return wq_spec(bm, bn, bits, half) ? 4 : 3; }
 struct NoGroups {};  // (unused arguments would move the ones behind them into another line of the argument block)
 template <int OUT, bool SBF, int BM, int BN, int BITS, bool ZP, bool HALF, bool RAGGED = false>
 __global__ void __launch_bounds__(512)
@@ -86,8 +94,10 @@ __global__ void __launch_bounds__(512)
     out += static_cast<int64_t>(blockIdx.y) * M * N * 4;
     K = min(ksplit, K - k0);
   }
-  constexpr int NWAVES = BM == 128 ? 4 : 8, NTHREADS = NWAVES * 64, NA = BM / 8 / NWAVES;  // NA: activation loads per wavefront and slab
-  constexpr int WGN = BM == 192 ? 4 : 2, WN = BN / WGN, WM = BM / (NWAVES / WGN), TM = WM / 32, TN = WN / 32;
+  // SPEC: as many wavefronts again that only request the operands (rows and weight rows of wavefront wave - NWAVES)
+  constexpr bool SPEC = wq_spec(BM, BN, BITS, HALF);
+  constexpr int NWAVES = SPEC ? 4 : 8, NTHREADS = NWAVES * 64, NA = BM / 8 / NWAVES;  // NA: activation loads per wavefront and slab
+  constexpr int WGN = BM == 192 && !SPEC ? 4 : 2, WN = BN / WGN, WM = BM / (NWAVES / WGN), TM = WM / 32, TN = WN / 32;
   constexpr int BK = 128, NK = 4;  // bytes of an activation row per slab (64 elements); k-steps of 16 elements
   static_assert(BITS == 4 || BITS == 8 || BITS == 9, "int4, int8 or (9) e4m3 weights");
   constexpr bool W8 = BITS >= 8;   // one byte per weight
@@ -95,21 +105,19 @@ __global__ void __launch_bounds__(512)
   static_assert(!(F8 && ZP), "float weights have no zero point");
   // raw weights: int4 two buffers of a superslab (BN x 128 bytes), int8 four of a slab (1 KB per wavefront)
   constexpr int A_STAGE = BM * BK, C_STAGE = BN * BK, R_STAGE = W8 ? NWAVES * 1024 : BN * 128;
-  // slabs between the request of activations and their use; the 128-row tile has the LDS for one more
-  constexpr int AL = BM == 128 ? 3 : 2, AST = AL + 1;
+  // slabs between the request of activations and their use; where the LDS holds it one more
+  constexpr int AST = wq_stages(BM, BN, BITS, HALF), AL = AST - 1;
   static_assert(AL == 2 || AL == 3, "the last four slabs are the only special ones");
   constexpr int C_BASE = AST * A_STAGE, R_BASE = C_BASE + 2 * C_STAGE, LDS_BYTES = R_BASE + (W8 ? 4 : 2) * R_STAGE;  // <= 160 KB
-  constexpr int RPW = BN / NWAVES;  // weight rows per wavefront: 16 or 8
+  constexpr int RPW = BN / NWAVES;  // weight rows per wavefront: 16, 8 or 32
   constexpr int NQ = W8 ? 1 : RPW / 8;  // direct-to-LDS loads of weights per wavefront and request
-  constexpr int TPR = NTHREADS / BN;    // converter threads per weight row: 4 or 8
-  constexpr int NPT = 64 / TPR;     // elements per thread and slab: 16 or 8
-  constexpr int NCQ = NPT / 4;      // conversion steps of four elements: 4 or 2
+  constexpr int TPR = NTHREADS / BN;    // converter threads per weight row: 4, 8 or 2
+  constexpr int NPT = 64 / TPR;     // elements per thread and slab: 16, 8 or 32
+  constexpr int NCQ = NPT / 4;      // conversion steps of four elements: 4, 2 or 8
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
-  // SPEC: as many wavefronts again that only request the operands (rows and weight rows of wavefront wave - NWAVES)
-  constexpr bool SPEC = BM == 128;
   const bool loader = SPEC && wave >= NWAVES;
   // who dequantizes: the requesting wavefronts for int4 (measured 32.6 -> 30.2 us at 128 x 14336 x 4096), the multiplying
   // ones for bytes (30.4 against 32.8 us)
@@ -363,7 +371,7 @@ __global__ void __launch_bounds__(512)
     }
     if constexpr (role == 2 && converts && more) {  // the whole conversion while the requests are under way
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) convert_quarter(q4, sc, zc);
+      for (int q4 = 0; q4 < (NCQ > 4 ? NCQ : 4); ++q4) convert_quarter(q4, sc, zc);
     }
     if constexpr (multiplies) {
 #pragma unroll
@@ -440,7 +448,7 @@ __global__ void __launch_bounds__(512)
   if (converter) {
     convert_read(0);
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) convert_quarter(q4, scale_value(sc_cur[0]), zp_cur[0]);
+    for (int q4 = 0; q4 < (NCQ > 4 ? NCQ : 4); ++q4) convert_quarter(q4, scale_value(sc_cur[0]), zp_cur[0]);
     convert_write(0);
   }
   end_of_slab(integral_constant<int, 0>{});
@@ -525,10 +533,10 @@ static int wq_splits(int64_t M, int64_t N, int64_t K, int64_t group) {
   return len == 0 ? 0 : static_cast<int>((K + len - 1) / len);
 }
 
-// LDS of a workgroup: activations in three stages (128-row tile: four), converted weights 2 x BN x 128, raw weights
+// LDS of a workgroup: activations in three stages (where the wavefronts split the work: four), converted weights 2 x BN x 128, raw weights
 // 2 x BN x 128 (bytes: 4 KB per 32 rows): at most 160 KB.
-static constexpr size_t wq_lds_bytes(int bm, int bn, int bits) {
-  return static_cast<size_t>(bm == 128 ? 4 : 3) * bm * 128 + 2 * bn * 128 + (bits >= 8 ? 4 * (bm == 128 ? 4 : 8) * 1024 : 2 * bn * 128);
+static constexpr size_t wq_lds_bytes(int bm, int bn, int bits, bool half) {
+  return static_cast<size_t>(wq_stages(bm, bn, bits, half)) * bm * 128 + 2 * bn * 128 + (bits >= 8 ? 4 * (bm == 128 ? 4 : 8) * 1024 : 2 * bn * 128);
 }
 
 // Tiles whose HALF variant keeps its registers: that of 256 x 128 with int4 zero points and f32 scales spills.
@@ -590,7 +598,7 @@ static int gemm_bf16_wq_impl(const void* a, int64_t lda, const void* q, int64_t 
   do {                                                                                                               \
     auto kern = half ? wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, ZPP, wq_half_fits(BMM, BNN, BITS, ZPP, SBFF)>      \
                      : wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, ZPP, false>;                                      \
-    constexpr size_t smem = wq_lds_bytes(BMM, BNN, BITS);                                                            \
+    const size_t smem = wq_lds_bytes(BMM, BNN, BITS, half && wq_half_fits(BMM, BNN, BITS, ZPP, SBFF));                \
     const dim3 grid(static_cast<unsigned>(((M + BMM - 1) / BMM) * ((N + BNN - 1) / BNN)),                            \
                     static_cast<unsigned>(splits > 0 ? splits : 1));                                                 \
     static LdsGrant granted[2];                                                                                      \
@@ -686,7 +694,7 @@ static int wq_ragged(const void* a, int64_t lda, const void* q, int64_t ldq_byte
   do {                                                                                                               \
     auto kern = half ? wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, false, (BMM > 128), true>                         \
                      : wgemm_wq_kernel<OUTT, SBFF, BMM, BNN, BITS, false, false, true>;                              \
-    constexpr size_t smem = wq_lds_bytes(BMM, BNN, BITS);                                                            \
+    const size_t smem = wq_lds_bytes(BMM, BNN, BITS, half && (BMM > 128));                                            \
     static LdsGrant granted[2];                                                                                      \
     if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted[half])) return e_;                     \
     kern<<<dim3(ragged_grid(M, N, G, BMM, BNN)), 512, smem, st>>>(                                                   \
