@@ -35,7 +35,14 @@ __global__ void __launch_bounds__(512)
     return;
   }
   const Epilogue e = group_epilogue(ep, rg, g);
-  qgemm_pp_tile<QT, OUT, EPI, TM>(A, lda, B + g * rg.b_group_stride, ldb, m0, n0, m_lim, N, K, e, out, ldo);
+  // The last tile of a group is no higher than its rows need: 64, 128 or 192 rows cost 0.4, 0.6 and 0.8 of 256.  8192 rows in 8 groups, N 14336
+  // over K 4096, int8 507 -> 470 us; 2843 in 32, N 1984 over K 1792 37.6 -> 29.2; 2097 in 8, N 13248 over K 1536 85.7 -> 72.1.
+  const uint8_t* bg = B + g * rg.b_group_stride;
+  const int rows = m_lim - m0;
+  if (rows <= 64) qgemm_pp_tile<QT, OUT, EPI, 1>(A, lda, bg, ldb, m0, n0, m_lim, N, K, e, out, ldo);
+  else if (TM > 2 && rows <= 128) qgemm_pp_tile<QT, OUT, EPI, 2>(A, lda, bg, ldb, m0, n0, m_lim, N, K, e, out, ldo);
+  else if (TM > 3 && rows <= 192) qgemm_pp_tile<QT, OUT, EPI, 3>(A, lda, bg, ldb, m0, n0, m_lim, N, K, e, out, ldo);
+  else qgemm_pp_tile<QT, OUT, EPI, TM>(A, lda, bg, ldb, m0, n0, m_lim, N, K, e, out, ldo);
 }
 
 template <int QT, int OUT, int EPI, int TM>
@@ -60,9 +67,9 @@ int launch_ragged_pp_epi(int tm, const void* a, int64_t lda, const void* b, int6
 // Ping-pong tiles of 64 * tm rows for a ragged product of more than 48 rows per group (0: 128 x 128 tiles).  The sizes are on the device:
 // each group is taken to end 0.45 of a tile early, and to have at least one.  Where 128 x 128 tiles are about one per CU and K is short
 // their two small workgroups per CU start and finish sooner.  int8 / e4m3, 8 to 64 groups of uneven sizes, weights from HBM, 128 x 128
-// tiles -> these, us: 4000 rows, 16 groups, N 4096 over K 2048 74.7 -> 58.9 / 72.4 -> 59.6 (192 rows); 4656, 16, N 1472, K 2816
-// 57.7 -> 35.6 (192); 3096, 16, N 2688, K 2176 50.8 -> 47.3 (128; 36.1 with 256, which no average shows); 6000, 16, N 2048, K 1024
-// 31.5 -> 22.9 / 29.2 -> 25.1 (256); 930, 8, N 1280, K 1152 12.5 against 13.0 (128).
+// tiles -> these, us: 4000 rows, 16 groups, N 4096 over K 2048 74.7 -> 56.0 / 72.4 -> 57.6 (192 rows); 4656, 16, N 1472, K 2816
+// 57.7 -> 36.0 (192); 7974, 32, N 1088, K 2048 47.4 -> 34.7 (256); 930, 8, N 1280, K 1152 12.5 against 13.0 (128).  The choice is
+// within 2 % of the best of the three on average; what it misses lies in the sizes (2871 rows, 16, N 3392, K 2688 57.1, 45.3 with 256).
 inline int ragged_pp_rows(int64_t M, int64_t N, int64_t K, int64_t G, bool big) {
   auto tile_rows = [&](int64_t rows) {
     const double per_group = static_cast<double>(M) / static_cast<double>(G * rows) + 0.45;

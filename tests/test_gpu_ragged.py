@@ -334,7 +334,7 @@ def test_ragged_dot_looks_at_64_groups_at_a_time(G, K, rows):
 @pytest.mark.parametrize('M,K,N,sizes', [
     (400, 1536, 317, (1, 0, 127, 129, 65)),                                    # 128 rows
     (2499, 384, 2076, (1, 192, 193, 0) + (120,) * 15 + (300,)),                # 192
-    (3973, 640, 2565, (1, 256, 257, 0, 1500, 1900, 2 ** 31 - 1)),              # 256
+    (3973, 640, 2565, (1, 256, 257, 0, 1460, 1900, 2 ** 31 - 1)),              # 256; last tiles of 1, 180, 108 and 98 rows
     (3329, 256, 4100, (3300, 0, 1)),                                           # 256: a group of many tiles
 ])
 def test_ragged_dot_tiles_of_128_to_256_rows(M, K, N, sizes, kind):
