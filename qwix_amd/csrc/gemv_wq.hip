@@ -571,8 +571,8 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
   if (const int rc = gemv_wq_args(x, ldx, q, ldb_bytes, b_qtype, M, N, K, group, s, s_dtype, zp, out, out_dtype, ldo, &p))
     return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // Byte weights of 32 MB and more stream faster through the smallest workgroups (4 wavefronts, two row tiles, several
-  // workgroups per CU) whatever the rows, even when the second row tile is empty: K 4096, N 14336, int8, 1 / 16 / 32
+  // Up to 16 rows, byte weights of 32 MB and more stream faster through the smallest workgroups (4 wavefronts, two row tiles, several
+  // workgroups per CU), even though the second row tile is empty: K 4096, N 14336, int8, 1 / 16 / 32
   // rows 25.5 / 26.9 / 21.9 -> 16.2 / 17.5 / 21.0 us (8 wavefronts: 16.5 / 18.2), e4m3 21.9 / 23.8 -> 15.5 / 17.8;
   // K = N = 8192: 20.0 / 24.4 / 29.4 -> 17.8 / 20.0 / 26.9; at 16 MB (K = N = 4096) 9.3 against 10.2 us the other way
   // round, and int4 gains nothing at any size.
@@ -606,20 +606,39 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
   do {                                                                                                     \
     if (zp) QWIX_GEMV_LAUNCH_ZP(NW, NTT, RTT, true); else QWIX_GEMV_LAUNCH_ZP(NW, NTT, RTT, false);        \
   } while (0)
-#define QWIX_GEMV_LAUNCH(NW, NTT)                                                                          \
+  // More than 16 rows, 32 in a pass: eight wavefronts that share K, one workgroup per CU.  The narrower its columns the sooner it is done
+  // (64 / 32 / 16 columns 1.7 / 1.2 / 1), but a second round of the CUs takes as long as the first; 64 columns that are more than a round
+  // run on four wavefronts, two workgroups per CU.  Weights from HBM, 16 / 32 / 64 columns: int4 19 x 5136 over K 3968 14.0 / 9.1 / 12.0,
+  // 20 x 8960 over K 3968 20.2 / 16.8 / 12.4, 64 x 4096 over K 4096 18.4 / 12.4 / -; int8 39 x 2752 over K 3456 14.1 / 12.6 / 16.6, 77 x 4336
+  // over K 4992 35.2 / 31.6 / 22.4, 113 x 3224 over K 9600 74.6 / 54.4 / 37.7 (columns by N alone, four wavefronts: 78.7); on four / eight
+  // wavefronts of 64 columns 206 x 5696 over K 8832 98.3 / 103, int4 130 x 14720 over K 9856 113 / 132.
+  if (M > 16) {
+    int64_t wgs = 0;
+    double best = 0;
+    int nt = 1;
+    for (int t = 1; t <= 4; t *= 2) {
+      const int64_t w = ((N + 16 * t - 1) / (16 * t)) * ((M + 31) / 32);
+      const double cost = static_cast<double>((w + 255) / 256) * (t == 1 ? 1.0 : t == 2 ? 1.2 : 1.7);
+      if (t == 1 || cost < best) { best = cost; nt = t; wgs = w; }
+    }
+    if (nt == 1) QWIX_GEMV_LAUNCH_RT(8, 1, 2);
+    else if (nt == 2) QWIX_GEMV_LAUNCH_RT(8, 2, 2);
+    else if (wgs <= 256) QWIX_GEMV_LAUNCH_RT(8, 4, 2);
+    else QWIX_GEMV_LAUNCH_RT(4, 4, 2);
+    return check_launch("gemv_wq");
+  }
+#define QWIX_GEMV_LAUNCH(NTT)                                                                              \
   do {                                                                                                     \
-    if (M <= 16 && !small_groups) QWIX_GEMV_LAUNCH_RT(NW, NTT, 1);                                         \
-    else if (M <= 32 && !small_groups) QWIX_GEMV_LAUNCH_RT(8, NTT, 2);                                     \
-    else QWIX_GEMV_LAUNCH_RT(4, NTT, 2); /* several passes side by side: smaller workgroups, two per CU */  \
+    if (small_groups) QWIX_GEMV_LAUNCH_RT(4, NTT, 2); else QWIX_GEMV_LAUNCH_RT(16, NTT, 1);                \
   } while (0)
   // Wider column tiles reuse each activation fragment more often; narrower ones keep every CU busy
   // when the weight matrix has few columns.
   if (N >= 192 * 64)
-    QWIX_GEMV_LAUNCH(16, 4);
+    QWIX_GEMV_LAUNCH(4);
   else if (N >= 192 * 32)
-    QWIX_GEMV_LAUNCH(16, 2);
+    QWIX_GEMV_LAUNCH(2);
   else
-    QWIX_GEMV_LAUNCH(16, 1);
+    QWIX_GEMV_LAUNCH(1);
 #undef QWIX_GEMV_LAUNCH
 #undef QWIX_GEMV_LAUNCH_RT
 #undef QWIX_GEMV_LAUNCH_ZP
