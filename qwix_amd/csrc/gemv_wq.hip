@@ -15,6 +15,7 @@
 // blocks of loads in flight (int4 weights by way of a wavefront-private LDS panel, in whole 128-byte lines), and
 // the partial sums meet in LDS.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 
@@ -705,16 +706,31 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
   //   8 groups x 2 rows, K 2048, N 3072 (384): 4 x 64 8.3, 8 x 32 9.2, 2 x 64 11.6
   //   8 groups x 2 rows, K 4096, N 1024 (128): 8 x 32 6.6 / 9.9, 4 x 64 10.4 / 15.8, 2 x 64 15.8 / 20.4
   // Two row tiles pay for themselves where groups of more than 16 rows are common (64 groups of 8 / 12 / 16 / 30 rows on
-  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4); bytes take them always (64 x 4
-  // rows 96.5 against 97.5, 64 x 16 rows 157 against 119).
-  const int64_t wgs = G * ((N + 63) / 64);
-  const bool two = M > 10 * G;
-  if (wgs < 320) {
-    if (two) QWIX_GEMVG_LAUNCH(8, 2, 2); else QWIX_GEMVG_LAUNCH(8, 2, 1);
-  } else if (b_qtype == QWIX_INT4 && wgs >= 1024) {
-    if (two) QWIX_GEMVG_LAUNCH(2, 4, 2); else QWIX_GEMVG_LAUNCH(2, 4, 1);
+  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4); bytes take them also where thousands of
+  // workgroups stream (64 x 4 rows 96.5 against 97.5).
+  //   What counts is the workgroups that have rows: with a few rows over many groups most groups are empty (rows that fall
+  // anywhere: exp(-M / G) of them).  One row tile, 2 x 64 / 4 x 64 / 8 x 32 / 4 x 32 columns: int4 64 groups x 0.4 rows, K 3840, N 1024 (320)
+  // 18.1 / 15.1 / 13.6 / 13.8; 32 x 4.3, K 3968, N 1728 (852) 26.7 / 27.9 / 27.6 / 27.7; int8 32 x 0.3, K 2816, N 1984 (243) 18.3 / 16.3 / 13.3 /
+  // 16.0, two tiles 4 x 64 17.1; 16 x 2.5, K 3072, N 1600 (367) 22.5 / 20.0 / 19.6 / 18.8, 20.7; 8 x 1.9, K 2176, N 7488 (792) 27.3 / 29.2 /
+  // 29.3 / 27.6, 31.0.  Two row tiles, by the tiles there are: 8 x 15.5, K 2432, N 2048 (256) 8 x 32 columns 16.7, 8 x 64 13.0, 4 x 64 14.2.
+  const double per_group = static_cast<double>(M) / static_cast<double>(G), cols = static_cast<double>((N + 63) / 64);
+  if (M > 10 * G) {
+    const double tiles = static_cast<double>(G) * std::max(1.0, per_group / 32 + 0.5) * cols;
+    if (2 * tiles <= 256) QWIX_GEMVG_LAUNCH(8, 2, 2);
+    else if (tiles <= 256) QWIX_GEMVG_LAUNCH(8, 4, 2);
+    else if (b_qtype == QWIX_INT4 && tiles >= 1024) QWIX_GEMVG_LAUNCH(2, 4, 2);
+    else QWIX_GEMVG_LAUNCH(4, 4, 2);
   } else {
-    if (two || b_qtype != QWIX_INT4) QWIX_GEMVG_LAUNCH(4, 4, 2); else QWIX_GEMVG_LAUNCH(4, 4, 1);
+    const double wgs = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
+    if (b_qtype == QWIX_INT4) {
+      if (wgs < (K >= 2048 ? 320 : 200)) QWIX_GEMVG_LAUNCH(8, 2, 1);  // (16 x 0.6, K 1664, N 2816: 9.3 against 8.3)
+      else if (wgs < 800) QWIX_GEMVG_LAUNCH(4, 4, 1);
+      else QWIX_GEMVG_LAUNCH(2, 4, 1);
+    } else {
+      if (wgs < 300) QWIX_GEMVG_LAUNCH(8, 2, 1);
+      else if (wgs < 1500) QWIX_GEMVG_LAUNCH(4, 2, 1);
+      else QWIX_GEMVG_LAUNCH(4, 4, 2);
+    }
   }
 #undef QWIX_GEMVG_LAUNCH
 #undef QWIX_GEMVG_KERNEL
