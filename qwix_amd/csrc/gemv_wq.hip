@@ -723,7 +723,7 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
   } else {
     const double wgs = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
     if (b_qtype == QWIX_INT4) {
-      if (wgs < (K >= 2048 ? 320 : 200)) QWIX_GEMVG_LAUNCH(8, 2, 1);  // (16 x 0.6, K 1664, N 2816: 9.3 against 8.3)
+      if (wgs < (K >= 2048 ? 320 : 260)) QWIX_GEMVG_LAUNCH(8, 2, 1);  // (4 x 64 over K 1664, 303: 8.3 against 9.3; over K 1408, 217: 6.4 against 5.7)
       else if (wgs < 800) QWIX_GEMVG_LAUNCH(4, 4, 1);
       else QWIX_GEMVG_LAUNCH(2, 4, 1);
     } else {
