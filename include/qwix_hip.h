@@ -239,6 +239,14 @@ QWIX_API size_t qwix_hip_qgemm_batched_act_workspace_bytes(int64_t batch, int64_
 QWIX_API int qwix_hip_qgemm_batched_act(const void* x, const void* y, int qtype, int64_t batch, int64_t M, int64_t N,
                                int64_t K, void* out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* ... with the contracted axis of the second operand in front ('bqk,bkd->bqd', probabilities and values): y (batch, K, N), each of its columns
+ * with its own absmax scale.  Bit-identical to qwix_hip_quantize of both and qwix_hip_qgemm_batched; both are quantized in one
+ * launch, into a workspace of qwix_hip_qgemm_batched_act_kn_workspace_bytes bytes (0: this shape is not taken; K a multiple of 16
+ * up to 4096, N of 8, y up to 32 MB). */
+QWIX_API size_t qwix_hip_qgemm_batched_act_kn_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K);
+QWIX_API int qwix_hip_qgemm_batched_act_kn(const void* x, const void* y, int qtype, int64_t batch, int64_t M, int64_t N,
+                                  int64_t K, void* out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Decode-size w8a8 with the activation quantization folded into the GEMM: per-token absmax int8
  * quantization of x (quantize, qwix/_src/core/qarray.py:638-644, as PtqProvider applies it to the
  * lhs of dot_general, providers/boxed_param.py:416-455) followed by _fast_dot_general

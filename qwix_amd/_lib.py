@@ -47,6 +47,8 @@ SIGNATURES = {
     'qwix_hip_qgemm_batched': (_int, [_vp, _i64, _i64, _vp, _i64, _i64, _int, _i64, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _i64, _int, _vp, _int, _i64, _i64, _vp]),
     'qwix_hip_qgemm_batched_act_workspace_bytes': (_sz, [_i64, _i64, _i64, _i64]),
     'qwix_hip_qgemm_batched_act': (_int, [_vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
+    'qwix_hip_qgemm_batched_act_kn': (_int, [_vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
+    'qwix_hip_qgemm_batched_act_kn_workspace_bytes': (_sz, [_i64, _i64, _i64, _i64]),
     'qwix_hip_qgemm_fused_act': (_int, [_vp, _int, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _int, _vp, _int, _i64, _vp]),
     'qwix_hip_qgemm_dynamic_act_workspace_bytes': (_sz, [_i64, _i64, _i64, _int]),
     'qwix_hip_qgemm_dynamic_act': (_int, [_vp, _int, _i64, _vp, _i64, _int, _i64, _i64, _i64, _vp, _int, _int, _vp, _int, _i64, _vp, _sz, _vp]),

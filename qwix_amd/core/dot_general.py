@@ -320,20 +320,33 @@ def _batched_qgemm(lhs, rhs, dimension_numbers, preferred_element_type):
 
 def fused_act_batched(lhs, rhs, dimension_numbers, act_qtype):
   """Dynamic absmax quantization of two floating operands, one scale per row of each, and their batched contraction in one
-  library call (qwix_hip_qgemm_batched_act): attention scores.  Bit-identical to quantize() of both, channelwise over all axes but the
-  contracted one, followed by dot_general.  Returns None for operands of another kind: anything but dense bf16 arrays of equal batch
-  axes in front and one contracted axis of 64 or 128 elements at the end."""
+  library call (qwix_hip_qgemm_batched_act, _act_kn): attention scores, and probabilities with values.  Bit-identical to quantize() of
+  both, channelwise over all axes but the contracted one, followed by dot_general.  Returns None for operands of another kind: anything but
+  dense bf16 arrays of equal batch axes in front and one contracted axis, of 64 or 128 elements at the end of both, or at the end of
+  the first and behind the batch axes of the second."""
   for t in (lhs, rhs):
     if (type(t) is not torch.Tensor or t.dtype != torch.bfloat16 or not t.is_cuda or not t.is_contiguous() or t.is_neg()
         or t.data_ptr() % 16):
       return None
   (lca, rca), (lba, rba) = dimension_numbers
   nb = len(lba)
-  if (list(lca) != [lhs.ndim - 1] or list(rca) != [rhs.ndim - 1] or list(lba) != list(range(nb)) or list(rba) != list(range(nb))
-      or nb == 0 or lhs.device != rhs.device or lhs.shape[:nb] != rhs.shape[:nb] or lhs.shape[-1] != rhs.shape[-1]):
+  turned = list(rca) == [nb] and rhs.ndim > nb + 1
+  if (list(lca) != [lhs.ndim - 1] or not (turned or list(rca) == [rhs.ndim - 1]) or list(lba) != list(range(nb))
+      or list(rba) != list(range(nb)) or nb == 0 or lhs.device != rhs.device or lhs.shape[:nb] != rhs.shape[:nb]
+      or lhs.shape[-1] != rhs.shape[rca[0]]):
     return None
   bshape, K = tuple(lhs.shape[:nb]), int(lhs.shape[-1])
-  Bt, M, N = math.prod(bshape), math.prod(lhs.shape[nb:-1]), math.prod(rhs.shape[nb:-1])
+  rfree = rhs.shape[nb + 1:] if turned else rhs.shape[nb:-1]
+  Bt, M, N = math.prod(bshape), math.prod(lhs.shape[nb:-1]), math.prod(rfree)
+  if turned:
+    nws = int(_lib.load().qwix_hip_qgemm_batched_act_kn_workspace_bytes(Bt, M, N, K))
+    if nws == 0:
+      return None
+    out = torch.empty(Bt, M, N, dtype=torch.bfloat16, device=lhs.device)
+    ws = torch.empty(nws, dtype=torch.uint8, device=lhs.device)
+    _lib.call('qwix_hip_qgemm_batched_act_kn', lhs.data_ptr(), rhs.data_ptr(), _lib.INT8 if act_qtype == numerics.INT8 else _lib.E4M3,
+              Bt, M, N, K, out.data_ptr(), ws.data_ptr(), nws, _lib.stream_of(lhs))
+    return out.reshape(*bshape, *lhs.shape[nb:-1], *rfree)
   if (K not in (64, 128) or not 0 < Bt <= 65535 or M == 0 or N == 0 or N % 8 or 2 * (M + 128) * N >= 1 << 31
       or 2 * max(M, N) * K >= 1 << 31):
     return None
@@ -342,7 +355,7 @@ def fused_act_batched(lhs, rhs, dimension_numbers, act_qtype):
   ws = torch.empty(nws, dtype=torch.uint8, device=lhs.device) if nws else None
   _lib.call('qwix_hip_qgemm_batched_act', lhs.data_ptr(), rhs.data_ptr(), _lib.INT8 if act_qtype == numerics.INT8 else _lib.E4M3,
             Bt, M, N, K, out.data_ptr(), _lib.ptr(ws), nws, _lib.stream_of(lhs))
-  return out.reshape(*bshape, *lhs.shape[nb:-1], *rhs.shape[nb:-1])
+  return out.reshape(*bshape, *lhs.shape[nb:-1], *rfree)
 
 
 def fused_act_dot_general(lhs, rhs, dimension_numbers, preferred_element_type=None, act_qtype=numerics.INT8, relu=False):

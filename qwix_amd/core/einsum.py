@@ -6,6 +6,7 @@ qwix_amd dot_general).  N-ary einsums are contracted pairwise left to right.
 """
 from __future__ import annotations
 
+import functools
 from typing import Any, Mapping
 
 import torch
@@ -44,11 +45,18 @@ def _binary(lhs, rhs, einsum_str: str, dot_general_fn, preferred_element_type, *
   return out
 
 
+@functools.lru_cache(maxsize=256)
+def _contraction(einsum_str: str, ndims: tuple[int, int]):
+  """Dimension numbers and output order of an einsum string (12 us to work out: as much as a small product takes)."""
+  info = einsum_info.EinsumInfo.parse(einsum_str, ndims=ndims)
+  return info.dimension_numbers, info.output_perm
+
+
 def fused_act_einsum(einsum_str: str, lhs, rhs, act_qtype):
   """Two floating operands quantized on the way (dot_general.fused_act_batched); None when it does not take them."""
-  info = einsum_info.EinsumInfo.parse(einsum_str, ndims=(len(lhs.shape), len(rhs.shape)))
-  out = _dg.fused_act_batched(lhs, rhs, info.dimension_numbers, act_qtype)
-  return out if out is None or info.output_perm is None else out.permute(*info.output_perm)
+  dimension_numbers, perm = _contraction(einsum_str, (len(lhs.shape), len(rhs.shape)))
+  out = _dg.fused_act_batched(lhs, rhs, dimension_numbers, act_qtype)
+  return out if out is None or perm is None else out.permute(*perm)
 
 
 def broadcast_operands(operands: list, subs_list: list[str]) -> list:

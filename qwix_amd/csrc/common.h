@@ -347,6 +347,12 @@ int quantize_relu_rows(const void* x, int dtype, int64_t rows, int64_t K, int qt
 int quantize_two_rows(const void* x, int64_t nx, void* qx, void* sx, const void* y, int64_t ny, void* qy, void* sy, int64_t K,
                       int qtype, void* stream);
 
+// x (batch, M, K), a scale per row, and y (batch, K, N), a scale per column and its codes as (batch, N, K), both dense bf16, 16-byte
+// aligned, to int8 or e4m3 in one launch (quantize.hip), where takes_rows_and_cols.
+bool takes_rows_and_cols(int64_t batch, int64_t M, int64_t N, int64_t K);
+int quantize_rows_and_cols(const void* x, void* qx, void* sx, const void* y, void* qy, void* sy, int64_t batch, int64_t M, int64_t N,
+                           int64_t K, int qtype, void* stream);
+
 // qwix_hip_gemv_wq_groups for the groups of up to `most_rows` rows (gemv_wq.hip): with fewer than M the others and the rows
 // behind the groups are not written.
 int gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_bytes, int64_t q_group_bytes, int b_qtype, int64_t M,

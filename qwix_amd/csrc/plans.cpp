@@ -66,7 +66,7 @@ const EntryPoint kEntries[] = {
     QWIX_ENTRY(qwix_hip_qgemm_grouped_zp),  QWIX_ENTRY(qwix_hip_gemm_bf16),           QWIX_ENTRY(qwix_hip_gemm_bf16_wq_ws),
     QWIX_ENTRY(qwix_hip_gemv_wq),           QWIX_ENTRY(qwix_hip_gemv_wq_zp),          QWIX_ENTRY(qwix_hip_gemv_wq_groups),
     QWIX_ENTRY(qwix_hip_gemm_wq_groups),    QWIX_ENTRY(qwix_hip_qgemm_zp_i8),
-    QWIX_ENTRY(qwix_hip_qgemm_batched_act),  QWIX_ENTRY(qwix_hip_qgemm_dynamic_relu),  QWIX_ENTRY(qwix_hip_fwht),              QWIX_ENTRY(qwix_hip_fwht_quantize),
+    QWIX_ENTRY(qwix_hip_qgemm_batched_act),  QWIX_ENTRY(qwix_hip_qgemm_batched_act_kn),  QWIX_ENTRY(qwix_hip_qgemm_dynamic_relu),  QWIX_ENTRY(qwix_hip_fwht),              QWIX_ENTRY(qwix_hip_fwht_quantize),
 };
 constexpr int kMaxArgs = 32;
 

@@ -1011,6 +1011,38 @@ extern "C" int qwix_hip_qgemm_batched_act(const void* x, const void* y, int qtyp
   return qgemm_strips(qtype, K, true, p, batch, stream);
 }
 
+// The product of probabilities and values: as above with the second operand's contracted axis in front (codes turned while they are
+// quantized).  Quantization of both in one launch, then the batched GEMM.
+static bool batched_act_kn_shape(int64_t batch, int64_t M, int64_t N, int64_t K) {
+  return batch > 0 && batch <= 65535 && M > 0 && N > 0 && K > 0 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX &&
+         M * K < (int64_t{1} << 30) && N * K < (int64_t{1} << 30) && M * N < (int64_t{1} << 30) && takes_rows_and_cols(batch, M, N, K);
+}
+extern "C" size_t qwix_hip_qgemm_batched_act_kn_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K) {
+  if (!batched_act_kn_shape(batch, M, N, K)) return 0;
+  return dyn_align(static_cast<size_t>(batch) * M * K) + dyn_align(static_cast<size_t>(batch) * N * K) +
+         dyn_align(static_cast<size_t>(batch) * M * 2) + dyn_align(static_cast<size_t>(batch) * N * 2);
+}
+
+extern "C" int qwix_hip_qgemm_batched_act_kn(const void* x, const void* y, int qtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                                             void* out, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!x || !y || !out) return fail(QWIX_ERR_INVALID_ARGUMENT, "null x/y/out");
+  if (qtype != QWIX_INT8 && qtype != QWIX_E4M3) return fail(QWIX_ERR_UNSUPPORTED, "int8 or e4m3 (got qtype %d)", qtype);
+  const size_t need = qwix_hip_qgemm_batched_act_kn_workspace_bytes(batch, M, N, K);
+  if (need == 0)
+    return fail(QWIX_ERR_UNSUPPORTED, "K a multiple of 16, N of 8, columns short enough for strips (batch=%lld M=%lld N=%lld K=%lld)",
+                (long long)batch, (long long)M, (long long)N, (long long)K);
+  if (!aligned16(x) || !aligned16(y) || !aligned16(out)) return fail(QWIX_ERR_INVALID_ARGUMENT, "x, y and out must be 16-byte aligned");
+  if (!workspace || workspace_bytes < need || !aligned16(workspace))
+    return fail(QWIX_ERR_INVALID_ARGUMENT, "workspace of %zu bytes required, got %zu", need, workspace_bytes);
+  uint8_t* qx = static_cast<uint8_t*>(workspace);
+  uint8_t* qy = qx + dyn_align(static_cast<size_t>(batch) * M * K);
+  uint8_t* sx = qy + dyn_align(static_cast<size_t>(batch) * N * K);
+  uint8_t* sy = sx + dyn_align(static_cast<size_t>(batch) * M * 2);
+  if (int e = quantize_rows_and_cols(x, qx, sx, y, qy, sy, batch, M, N, K, qtype, stream)) return e;
+  return qwix_hip_qgemm_batched(qx, K, M * K, qy, K, N * K, qtype, batch, M, N, K, sx, QWIX_BF16, M, sy, QWIX_BF16, N,
+                                qtype == QWIX_INT8 ? 0 : QWIX_BF16, out, QWIX_BF16, N, M * N, stream);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Split-K for problems whose 128 x 128 tiles occupy a fraction of the chip while K is long (a few hundred
 // rows against a narrow weight): the grid gets a second dimension over ranges of K slabs, every workgroup

@@ -105,15 +105,16 @@ __device__ __forceinline__ s16x2 abs_keys(uint32_t pair) {
 }
 __device__ __forceinline__ float key_value(short key) { return bf16_bits_to_f32(static_cast<uint16_t>(key - kKeyOfZero)); }
 
-// RELU: the rows' values are max(x, 0).
-template <typename D, int QT, int CAL, int MODE, int NL, bool NT = true, bool RELU = false>
+// RELU: the rows' values are max(x, 0).  PARTS: workgroups of up to 1024 threads, every 256 of them a block by themselves.
+template <typename D, int QT, int CAL, int MODE, int NL, bool NT = true, bool RELU = false, bool PARTS = false>
 __device__ __forceinline__ void rows_block(unsigned block, const uint8_t* __restrict__ x, int64_t nseg, int nvec, int log2g, float factor,
                 uint8_t* __restrict__ q, void* __restrict__ scale, int8_t* __restrict__ zp,
                 void* __restrict__ cal0, void* __restrict__ cal1, int per_scale, int per_shift) {
   constexpr int EV = D::kVec;
   constexpr bool ASYM = (CAL == QWIX_MINMAX);
-  __shared__ float red[2][4];
-  const int tid = threadIdx.x;
+  __shared__ float reds[PARTS ? 4 : 1][2][4];
+  auto& red = reds[PARTS ? threadIdx.x >> 8 : 0];
+  const int tid = PARTS ? threadIdx.x & 255 : threadIdx.x;
   const int g = 1 << log2g;
   const int64_t seg = (static_cast<int64_t>(block) << (8 - log2g)) + (tid >> log2g);
   const int lane = tid & (g - 1);
@@ -907,16 +908,14 @@ __global__ void __launch_bounds__(256)
 // come from its L2.  bf16 to int8 from the caches, fill + maximum + quantize -> strips: 1920 x 1856 13.9 -> 7.8 us, 14 x 464 x 128
 // 14.6 -> 7.3, 55 x 2784 x 64 22.1 -> 9.6; from memory: takes_strips.
 template <typename D, int QT>
-__global__ void __launch_bounds__(1024)
-    cols_strip_kernel(const uint8_t* __restrict__ x, ColGeom gm, int pitch, float factor, uint8_t* __restrict__ q,
-                      void* __restrict__ scale) {
+__device__ __forceinline__ void strip_block(unsigned b, unsigned strips, const uint8_t* __restrict__ x, const ColGeom& gm, int pitch,
+                                            float factor, uint8_t* __restrict__ q, void* __restrict__ scale) {
   constexpr int EV = D::kVec, NC = 2 * EV, EPB = (QT == QWIX_INT4) ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) uint8_t stage[];  // [column][rows]
   const int tid = threadIdx.x, tc = tid & 1, rb = tid >> 1, waves = blockDim.x >> 6;
   float* red = reinterpret_cast<float*>(stage + NC * pitch);  // [wavefront][column]
   float* sh_s = red + waves * NC;
-  unsigned b = blockIdx.x;
-  if (b < (gridDim.x & ~31u)) b = (b & ~31u) + (b & 7) * 4 + ((b >> 3) & 3);
+  if (b < (strips & ~31u)) b = (b & ~31u) + (b & 7) * 4 + ((b >> 3) & 3);
   const unsigned cbs = static_cast<unsigned>((gm.inner + NC - 1) / NC);
   const unsigned cb = b % cbs;
   b /= cbs;
@@ -1014,6 +1013,27 @@ __global__ void __launch_bounds__(1024)
       for (int k = 0; k < nb; ++k) dst[k] = src[k];
     }
   }
+}
+template <typename D, int QT>
+__global__ void __launch_bounds__(1024)
+    cols_strip_kernel(const uint8_t* __restrict__ x, ColGeom gm, int pitch, float factor, uint8_t* __restrict__ q,
+                      void* __restrict__ scale) {
+  strip_block<D, QT>(blockIdx.x, gridDim.x, x, gm, pitch, factor, q, scale);
+}
+
+// Rows of one array and strips of columns of another in one launch, the first `strips` workgroups the strips: neither waits for the
+// other, and most of the time of both is their launch and one round of loads (a whole product of probabilities and values, quantized in two launches / here, us:
+// 7 x 1 x 192 x 64 14.9 / 10.5, 4 x 512 x 1024 x 128 16.4 / 13.2, 8 x 986 x 2512 x 128 39.4 / 33.2).  Plain stores, as in two_rows_kernel.
+template <int QT, int NL>
+__global__ void __launch_bounds__(1024) rows_and_strips_kernel(Rows r, int nvec, int log2g, unsigned strips, const uint8_t* __restrict__ y,
+                                                               ColGeom gm, int pitch, uint8_t* __restrict__ qy, void* __restrict__ sy) {
+  if (blockIdx.x < strips) {
+    strip_block<BF16, QT>(blockIdx.x, strips, y, gm, pitch, 0.f, qy, sy);
+    return;
+  }
+  const unsigned block = (blockIdx.x - strips) * (blockDim.x >> 8) + (threadIdx.x >> 8);
+  rows_block<BF16, QT, QWIX_ABSMAX, MODE_QUANT, NL, false, false, true>(block, r.x, r.nseg, nvec, log2g, 0.f, r.q, r.scale, nullptr, nullptr,
+                                                                        nullptr, 1, 0);
 }
 
 // ------------------------------------------------------------------------------------ generic 5-D
@@ -1907,6 +1927,43 @@ int quantize_two_rows(const void* x, int64_t nx, void* qx, void* sx, const void*
     else two_rows_kernel<QWIX_E4M3, 2><<<grid, 256, 0, st>>>(a, b, split, nvec, lg);
   }
   return check_launch("quantize (two arrays)");
+}
+
+bool takes_rows_and_cols(int64_t batch, int64_t M, int64_t N, int64_t K) {
+  const ColGeom g = make_col_geom(batch, K, N, K, 8);
+  return K % 16 == 0 && K / 8 <= 2048 && N % 8 == 0 && batch * M < (int64_t{1} << 31) && takes_strips(g, QWIX_BF16);
+}
+int quantize_rows_and_cols(const void* x, void* qx, void* sx, const void* y, void* qy, void* sy, int64_t batch, int64_t M, int64_t N,
+                           int64_t K, int qtype, void* stream) {
+  const ColGeom g = make_col_geom(batch, K, N, K, 8);
+  int threads = 256;
+  while (threads < 1024 && 4 * threads < K) threads *= 2;
+  const int pitch = static_cast<int>((K + 15) / 16 * 16 + 16);
+  const size_t smem = static_cast<size_t>(16) * pitch + (threads / 64 + 1) * 16 * sizeof(float);
+  const unsigned strips = static_cast<unsigned>(batch * ((N + 15) / 16));
+  const int nvec = static_cast<int>(K / 8), lg = rows_log2g(nvec), loads = (nvec + (1 << lg) - 1) >> lg;
+  const int64_t per = static_cast<int64_t>(256 >> lg) * (threads / 256);  // rows per workgroup
+  const dim3 grid(strips + static_cast<unsigned>((batch * M + per - 1) / per));
+  const Rows r{static_cast<const uint8_t*>(x), batch * M, static_cast<uint8_t*>(qx), sx};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define QWIX_MIX(QTT, NLL)                                                                                              \
+  do {                                                                                                                 \
+    auto kern = rows_and_strips_kernel<QTT, NLL>;                                                                      \
+    static LdsGrant granted;                                                                                           \
+    if (int e_ = grant_lds(reinterpret_cast<const void*>(kern), smem, granted)) return e_;                             \
+    kern<<<grid, threads, smem, st>>>(r, nvec, lg, strips, static_cast<const uint8_t*>(y), g, pitch, static_cast<uint8_t*>(qy), sy); \
+  } while (0)
+#define QWIX_MIX_NL(QTT)            \
+  do {                              \
+    if (loads <= 1) QWIX_MIX(QTT, 1); \
+    else if (loads <= 2) QWIX_MIX(QTT, 2); \
+    else if (loads <= 4) QWIX_MIX(QTT, 4); \
+    else QWIX_MIX(QTT, 8);          \
+  } while (0)
+  if (qtype == QWIX_INT8) QWIX_MIX_NL(QWIX_INT8); else QWIX_MIX_NL(QWIX_E4M3);
+#undef QWIX_MIX_NL
+#undef QWIX_MIX
+  return check_launch("quantize (rows and columns)");
 }
 }  // namespace qwix
 

@@ -183,6 +183,38 @@ def test_scores_quantized_inside_the_product(shape, K, qtype):
   assert f32.dtype == torch.float32 and torch.equal(f32.view(torch.int32), want(lhs.float(), rhs.float()).view(torch.int32))
 
 
+@pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('batch,M,K,N', [(3, 1, 16, 8), (2, 24, 192, 64), (3, 130, 464, 136), (1, 70, 1040, 24), (2, 33, 2512, 128), (4, 9, 3072, 64),
+                                         (32, 3, 4096, 128), (5, 300, 2064, 40)])
+def test_probabilities_and_values_quantized_in_one_launch(batch, M, K, N, qtype):
+  """Rows of the first and columns of the second operand under a rule with act_qtype, against quantize() of each and the contraction, bit
+  for bit: workgroups of 256 to 1024 threads, rows of one to eight loads per thread, the last strip partly empty; zeros, signed zeros,
+  infinities and NaN among them.  Other layouts give the same results by the ordinary path."""
+  import qwix_amd
+  from qwix_amd import _lib, nn
+  print('case values', batch, M, K, N, qtype, flush=True)
+  assert _lib.load().qwix_hip_qgemm_batched_act_kn_workspace_bytes(batch, M, N, K) > 0
+  gen = torch.Generator(device=util.DEV).manual_seed(M + K + N)
+  lhs = torch.softmax(torch.randn(batch, M, K, generator=gen, device=util.DEV) * 2, -1).to(torch.bfloat16)
+  rhs = torch.randn(batch, K, N, generator=gen, device=util.DEV).to(torch.bfloat16)
+  lhs[0, 0] = 0
+  rhs[0, :, 0] = 0
+  rhs[-1, ::2, 1] = -0.0
+  if M > 2:
+    lhs[-1, 1, 3], lhs[-1, 2, 5] = float('inf'), float('nan')
+    rhs[-1, 2, 3], rhs[-1, 3, 4] = float('nan'), float('-inf')
+  rule = qwix_amd.QuantizationRule(module_path='.*', weight_qtype=qtype, act_qtype=qtype)
+  model = qwix_amd.quantize_model(lambda params, a, b: nn.ops.einsum('bqk,bkd->bqd', a, b), qwix_amd.PtqProvider([rule]))
+  ql = qwix_amd.quantize(lhs, qtype, channelwise_axes=[0, 1])
+  qr = qwix_amd.quantize(rhs, qtype, channelwise_axes=[0, 2])
+  want = qwix_amd.einsum('bqk,bkd->bqd', ql, qr)
+  for _ in range(6):  # the ordinary path, then its plan
+    assert torch.equal(model.apply({}, lhs, rhs).view(torch.int16), want.view(torch.int16))
+  strided = torch.cat([rhs, rhs], -1)[..., :N]
+  assert not strided.is_contiguous()
+  assert torch.equal(model.apply({}, lhs, strided).view(torch.int16), want.view(torch.int16))
+
+
 def test_batched_dot_general_on_the_dequantize_path():
   """A float activation against a batched quantized operand takes the dequantize-first path."""
   from qwix_amd.core import dot_general as dg
