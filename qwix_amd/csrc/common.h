@@ -143,13 +143,20 @@ __device__ __forceinline__ void unpack16(const uint4& v, float* f) {
   }
 }
 
-// max(x, 0) of a 16-byte vector of D, as integers: the encoding of a negative value, -0 and a negative NaN included, is a negative integer.
+// max(x, 0) of a 16-byte vector of D, NaN kept as it is, as integers: the encoding of a negative value, -0 included, is a negative integer,
+// and above that of -infinity as an unsigned one stand exactly the negative NaNs.
 template <typename D>
 __device__ __forceinline__ uint4 relu16(const uint4& v) {
   typedef short s16x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
   auto one = [](uint32_t w) -> uint32_t {
-    if constexpr (D::kTag == QWIX_BF16) return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, w), s16x2{0, 0}));
-    return static_cast<uint32_t>(max(static_cast<int>(w), 0));
+    if constexpr (D::kTag == QWIX_BF16) {
+      const uint32_t positive = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, w), s16x2{0, 0}));
+      const u16x2 beyond = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w), u16x2{0xFF80, 0xFF80});
+      const u16x2 nan = u16x2{0, 0} - __builtin_elementwise_min(beyond, u16x2{1, 1});  // all bits of a negative NaN's half
+      return positive | (w & __builtin_bit_cast(uint32_t, nan));
+    }
+    return w > 0xFF800000u ? w : static_cast<uint32_t>(max(static_cast<int>(w), 0));
   };
   return make_uint4(one(v.x), one(v.y), one(v.z), one(v.w));
 }

@@ -324,3 +324,34 @@ def test_relu_inside_the_quantization_of_the_next_layer(rows, hidden, qtype, dty
     def dot_general(self, lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, out_sharding=None):
       return super().dot_general(lhs, rhs, dimension_numbers, precision, preferred_element_type, out_sharding=out_sharding)
   assert torch.equal(qwix_amd.quantize_model(nn.MLP(hidden, 136), Own([rule])).apply(params, x), want)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('rows,k', [(3, 256), (70, 1032)])
+def test_relu_inside_the_quantization_keeps_nan(rows, k, qtype, dtype):
+  """NaN of either sign, the smallest and the largest of each, and infinities pass max(x, 0) as torch.relu passes them: in the product
+  (3 rows, int8) and in a launch of its own."""
+  import qwix_amd
+  from qwix_amd import nn
+  print('case relu of NaN', rows, k, qtype, dtype, flush=True)
+  g = torch.Generator(device=util.DEV).manual_seed(rows + k)
+
+  class Layer:
+    def __init__(self, inside):
+      self.inside, self.dense = inside, nn.Dense(136)
+
+    def __call__(self, params, x):
+      return self.dense(params['Dense_0'], x, relu=True) if self.inside else self.dense(params['Dense_0'], torch.relu(x))
+  rule = qwix_amd.QuantizationRule(module_path='.*', weight_qtype=qtype, act_qtype=qtype)
+  x = torch.randn(rows, k, generator=g, device=util.DEV).to(dtype)
+  bits = x.view(torch.int16 if dtype == torch.bfloat16 else torch.int32)
+  inf = 0x7F80 if dtype == torch.bfloat16 else 0x7F800000
+  low = -0x8000 if dtype == torch.bfloat16 else -0x80000000
+  for i, v in enumerate((inf + 1, low + inf + 1, low + (-low - 1), -low - 1, low + inf, low)):
+    bits[i % 2, 5 * i] = v  # NaN, -NaN (the smallest, the largest), NaN, -infinity, -0
+  params = {'Dense_0': {'kernel': torch.randn(k, 136, generator=g, device=util.DEV).to(dtype)}}
+  models = [qwix_amd.quantize_model(Layer(inside), qwix_amd.PtqProvider([rule])) for inside in (True, False)]
+  params = qwix_amd.quantize_params(params, models[0].init(params, x))
+  got, want = (m.apply(params, x) for m in models)
+  assert torch.equal(got.nan_to_num(nan=12345.0), want.nan_to_num(nan=12345.0))
