@@ -330,3 +330,28 @@ def test_k_ranges_that_lower_the_streamed_rows():
         ranges = [r for r in range(2, 257) if tiles <= 128 and r * tiles <= 256 and r * 1024 <= k and k % (r * 256) == 0
                   and ((k // r) % group == 0 or group % (k // r) == 0)]
         assert dg.fused_wq_min_rows(n, True, k, group) == (48 if ranges else 64 if n >= 12288 else 80), (n, k, group)
+
+
+def test_relu_with_a_layer_or_an_operation_of_the_users():
+  """MLP and Dense pass the option of a ReLU only to code that knows it: a layer or a dot_general put in their place runs as before."""
+  from qwix_amd import nn
+  mlp = nn.MLP(8, 4)
+  g = torch.Generator().manual_seed(0)
+  params, x = mlp.init(g, 6), torch.randn(3, 6, generator=g)
+  want = torch.relu(x @ params['Dense_0']['kernel']) @ params['Dense_1']['kernel']
+  assert torch.equal(mlp(params, x), want)
+
+  class Scaled(nn.Dense):
+    def __call__(self, params, x):
+      return 2 * super().__call__(params, x)
+  mlp.layers[1] = Scaled(4, name='Dense_1')
+  assert torch.equal(mlp(params, x), 2 * want)
+  mlp.layers[1] = lambda params, x: x @ params['kernel']
+  assert torch.equal(mlp(params, x), want)
+  stock, seen = nn.ops.dot_general, []
+  nn.ops.dot_general = lambda lhs, rhs, dimension_numbers: (seen.append(lhs.min()), stock(lhs, rhs, dimension_numbers))[1]
+  try:
+    assert torch.equal(nn.MLP(8, 4)(params, x), want)
+  finally:
+    del nn.ops.dot_general
+  assert nn.ops.dot_general is stock and len(seen) == 2 and seen[1] >= 0
