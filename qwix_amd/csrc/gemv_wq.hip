@@ -706,8 +706,7 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
   //   8 groups x 2 rows, K 2048, N 3072 (384): 4 x 64 8.3, 8 x 32 9.2, 2 x 64 11.6
   //   8 groups x 2 rows, K 4096, N 1024 (128): 8 x 32 6.6 / 9.9, 4 x 64 10.4 / 15.8, 2 x 64 15.8 / 20.4
   // Two row tiles pay for themselves where groups of more than 16 rows are common (64 groups of 8 / 12 / 16 / 30 rows on
-  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4); bytes take them also where thousands of
-  // workgroups stream (64 x 4 rows 96.5 against 97.5).
+  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4).
   //   What counts is the workgroups that have rows: with a few rows over many groups most groups are empty (rows that fall
   // anywhere: exp(-M / G) of them).  One row tile, 2 x 64 / 4 x 64 / 8 x 32 / 4 x 32 columns: int4 64 groups x 0.4 rows, K 3840, N 1024 (320)
   // 18.1 / 15.1 / 13.6 / 13.8; 32 x 4.3, K 3968, N 1728 (852) 26.7 / 27.9 / 27.6 / 27.7; int8 32 x 0.3, K 2816, N 1984 (243) 18.3 / 16.3 / 13.3 /
@@ -727,9 +726,15 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
       else if (wgs < 800) QWIX_GEMVG_LAUNCH(4, 4, 1);
       else QWIX_GEMVG_LAUNCH(2, 4, 1);
     } else {
+      // Bytes, four wavefronts, 32 columns / 64 / 64 and two row tiles, uneven groups: 64 columns read an activation half as often, which
+      // counts the more rows there are (16 groups, K 1024, N 8192, 3 / 7 rows 29.0 / 26.7 / 32.2, 33.5 / 30.1 / 35.2; 64, 1920, 1024, 2.5 / 8
+      // rows 25.3 / 26.6 / 28.7, 31.4 / 30.1 / 30.0) and the more rounds of the CUs stream (64, 2048, 4096, 1 row 63.1 / 61.5 / 67.7); 32 fill
+      // a chip that 64 leave idle (32, 3072, 1216, 2.5 / 8 rows 26.9 / 28.7 / 33.6, 30.8 / 31.3 / 33.2).  Second passes over a long K cost more
+      // than the empty tile of most groups once some groups have them (64, 4096, 1024, 8 / 10 rows 58.1 / 57.5 / 56.3, 63.8 / 60.8 / 57.5).
       if (wgs < 300) QWIX_GEMVG_LAUNCH(8, 2, 1);
-      else if (wgs < 1500) QWIX_GEMVG_LAUNCH(4, 2, 1);
-      else QWIX_GEMVG_LAUNCH(4, 4, 2);
+      else if (per_group >= 9.25 && K > 3072) QWIX_GEMVG_LAUNCH(4, 4, 2);
+      else if (wgs >= 1750 || (wgs >= 690 && per_group >= 4.5) || (wgs >= 500 && per_group >= 7.5)) QWIX_GEMVG_LAUNCH(4, 4, 1);
+      else QWIX_GEMVG_LAUNCH(4, 2, 1);
     }
   }
 #undef QWIX_GEMVG_LAUNCH
