@@ -713,18 +713,27 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
   // 16.0, two tiles 4 x 64 17.1; 16 x 2.5, K 3072, N 1600 (367) 22.5 / 20.0 / 19.6 / 18.8, 20.7; 8 x 1.9, K 2176, N 7488 (792) 27.3 / 29.2 /
   // 29.3 / 27.6, 31.0.  Two row tiles, by the tiles there are: 8 x 15.5, K 2432, N 2048 (256) 8 x 32 columns 16.7, 8 x 64 13.0, 4 x 64 14.2.
   const double per_group = static_cast<double>(M) / static_cast<double>(G), cols = static_cast<double>((N + 63) / 64);
-  if (M > 10 * G) {
-    const double tiles = static_cast<double>(G) * std::max(1.0, per_group / 32 + 0.5) * cols;
+  const double wgs = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
+  const double tiles = static_cast<double>(G) * std::max(1.0, per_group / 32 + 0.5) * cols;
+  // int4, uneven groups, 4 x 64 / 2 x 64 columns with one row tile, 4 x 64 / 2 x 64 with two: second passes over some groups cost less than an
+  // empty tile in most (64 groups of 12 / 16 rows, K 2048, N 4096 73.0 / 70.2 / 81.0 / 74.8, 85.9 / 81.2 / 85.8 / 78.4; 64, 1024, 2048 21.4 / 20.6 /
+  // 26.3 / 24.9, 25.7 / 24.1 / 28.0 / 26.2; 64, 1920, 1024 20.8 / 23.1 / 23.4 / 23.6, 24.6 / 26.3 / 25.6 / 26.6; 16, 1408, 3072 14.8 / 13.3 / 18.1 /
+  // 15.0, 16.7 / 15.3 / 19.4 / 16.1; 8, 4096, 4096 19.0 / 21.1 / 20.5 / 27.3, 22.0 / 22.0 / 22.1 / 28.1).
+  const bool one = M <= 10 * G || (b_qtype == QWIX_INT4 && tiles >= 320 && per_group <= (wgs >= 3000 ? 14 : 16));
+  if (!one) {
     if (2 * tiles <= 256) QWIX_GEMVG_LAUNCH(8, 2, 2);
     else if (tiles <= 256) QWIX_GEMVG_LAUNCH(8, 4, 2);
     else if (b_qtype == QWIX_INT4 && tiles >= 1024) QWIX_GEMVG_LAUNCH(2, 4, 2);
     else QWIX_GEMVG_LAUNCH(4, 4, 2);
   } else {
-    const double wgs = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
     if (b_qtype == QWIX_INT4) {
+      // Two wavefronts or four, one row tile: 64 groups of 1 / 6 rows, K 4096, N 1024 2 x 64 columns 22.6 / 31.7, 4 x 64 20.5 / 32.9; 32, 2048, 2048
+      // 6 / 9.8 rows 15.6 / 19.0, 16.9 / 18.8; 64, 1920, 1024 9.8 rows 22.0, 19.7; 16, 2048, 8192 3 / 8 rows 30.4 / 34.5, 28.2 / 33.4; 8, 2048, 14336
+      // 29.1 / 30.1, 26.4 / 29.3; 64, 2048, 4096 8 rows 58.7, 60.4.
+      const bool two_waves = per_group > 10 ? wgs >= 1500 : wgs >= 3000 || (wgs >= 800 && wgs < 1500 && per_group < 7.5);
       if (wgs < (K >= 2048 ? 320 : 260)) QWIX_GEMVG_LAUNCH(8, 2, 1);  // (4 x 64 over K 1664, 303: 8.3 against 9.3; over K 1408, 217: 6.4 against 5.7)
-      else if (wgs < 800) QWIX_GEMVG_LAUNCH(4, 4, 1);
-      else QWIX_GEMVG_LAUNCH(2, 4, 1);
+      else if (two_waves) QWIX_GEMVG_LAUNCH(2, 4, 1);
+      else QWIX_GEMVG_LAUNCH(4, 4, 1);
     } else {
       // Bytes, four wavefronts, 32 columns / 64 / 64 and two row tiles, uneven groups: 64 columns read an activation half as often, which
       // counts the more rows there are (16 groups, K 1024, N 8192, 3 / 7 rows 29.0 / 26.7 / 32.2, 33.5 / 30.1 / 35.2; 64, 1920, 1024, 2.5 / 8

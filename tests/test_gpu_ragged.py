@@ -196,6 +196,8 @@ def test_ragged_dot_weight_only_experts(sizes, wq_type, tiled):
     (8, 640, 1032, 120, (40, 0, 33, 16, 1, 17, 2, 3)),             # two row tiles, 64 columns on eight wavefronts
     (32, 640, 1032, 12, (3, 0, 1) + (0,) * 20 + (5, 2) + (0,) * 7),   # most groups empty
     (64, 384, 1000, 420, tuple((5 * i) % 18 for i in range(64))),  # bytes: 4 wavefronts x 64 columns, second passes of one row
+    (64, 384, 2000, 800, tuple((11 * i) % 26 for i in range(64))),  # int4: 2 wavefronts, one row tile, second passes of up to 9 rows
+    (64, 384, 1000, 770, tuple((11 * i) % 25 for i in range(64))),  # int4: 4 wavefronts
 ])
 @pytest.mark.parametrize('wq_type,tiled,dtype', [('int4', {1: 128}, O.BF16), ('int8', {1: 128}, O.BF16), ('int8', None, O.F32),
                                                  ('float8_e4m3fn', {1: 128}, O.BF16), ('int4', None, O.F32)])
