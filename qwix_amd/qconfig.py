@@ -44,11 +44,14 @@ class module_scope(contextlib.ContextDecorator):
 
   def __init__(self, name: str):
     self._name = name
+    self._old = None
 
   def _recreate_cm(self) -> 'module_scope':
     return module_scope(self._name)  # calls may nest
 
   def __enter__(self) -> None:
+    if self._old is not None:  # it holds one path to go back to
+      raise RuntimeError('a module_scope is entered once: make another one')
     self._old = current_module_path()
     _tls.path = self._old + (self._name,)
 

@@ -181,6 +181,25 @@ def test_rule_lookup_first_full_match_wins_and_op_ids():
   assert (r.module_path, r.weight_qtype, r.act_qtype, r.tile_size, r.weight_calibration_method, tuple(r.act_batch_axes)) == ('.*', None, None, None, 'absmax', (0,))
 
 
+def test_a_module_scope_is_entered_once():
+  """A second entry of one object, inside its block or behind it, is refused and leaves the path as it is; a decorated function's
+  calls get an object each."""
+  scope = qconfig.module_scope('a')
+  with scope:
+    with pytest.raises(RuntimeError):
+      scope.__enter__()
+    assert qconfig.current_module_path() == ('a',)
+  assert qconfig.current_module_path() == ()
+  with pytest.raises(RuntimeError):
+    scope.__enter__()
+  assert qconfig.current_module_path() == ()
+
+  @qconfig.module_scope('f')
+  def nested(n):
+    return nested(n - 1) if n else qconfig.current_module_path()
+  assert nested(2) == ('f', 'f', 'f') and nested(0) == ('f',) and qconfig.current_module_path() == ()
+
+
 def test_qarray_array_methods_follow_the_reference_table():
   """qarray_test.py:228-302: scale shapes under reshape / transpose / slicing of a (2, 2, 6) array quantized
   channelwise on axis 0 with tiles of 2 on axis 2 (scale (2, 1, 3))."""
