@@ -858,6 +858,13 @@ __device__ __forceinline__ void qgemm_mid_tile(const uint8_t* __restrict__ A, in
                                                          lane);
 }
 
+// Byte offset of the scale that a lane touches: element `i` of `count`, `es` bytes each, or the last one.  What is read there is the
+// element's first two bytes: a wider load would reach behind a vector of one bf16, and is misaligned where a group's scales start at an
+// odd element.
+constexpr int64_t scale_touch(int64_t i, int64_t count, int64_t es) { return (i < count ? i : count - 1) * es; }
+static_assert(scale_touch(0, 1, 2) == 0 && scale_touch(127, 1, 2) == 0 && scale_touch(126, 3, 2) + 2 == 3 * 2 && scale_touch(2, 3, 4) + 4 == 3 * 4 &&
+              scale_touch(int64_t{1} << 30, int64_t{1} << 31, 4) == int64_t{1} << 32, "every touch lies in its vector");
+
 // ------------------------------------------------------------------------------------------------
 // Ping-pong variant of the 256 x 256 kernel for long K.  The eight wavefronts form two groups (the
 // upper and the lower 128 rows of the tile; the two wavefronts that share a SIMD are in different
@@ -978,22 +985,15 @@ __device__ __forceinline__ void qgemm_pp_tile(const uint8_t* __restrict__ A, int
   const int KT = K / BK;  // >= 2
   // The scale vectors are first needed in the epilogue, where a cold fetch (address translation plus a trip
   // to HBM) would stall every wavefront with nothing to hide behind.  Touch this wavefront's pieces of them
-  // now, under the equally cold first slab loads: 128 row scales and 64 column scales, 8 / 4 bytes per lane.
+  // now, under the equally cold first slab loads: every second of up to 128 row scales, each of 64 column scales.
   uint32_t warm_a = 0, warm_b = 0;
   if constexpr (OUT != QWIX_I32) {
-    const int m_base = m0 + wm * (32 * TM), n_base = n0 + wn * 64;
-    if (ep.sa != nullptr) {
-      const int64_t es = ep.sa_dtype == QWIX_BF16 ? 2 : 4;
-      const int64_t want = (static_cast<int64_t>(m_base) * es + lane * 8) & ~int64_t{3}, last = M * es < 4 ? 0 : (M * es - 4) & ~int64_t{3};
-      const int64_t off = want < last ? want : last;
-      warm_a = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(ep.sa) + off);
-    }
-    if (ep.sb != nullptr) {
-      const int64_t es = ep.sb_dtype == QWIX_BF16 ? 2 : 4;
-      const int64_t want = (static_cast<int64_t>(n_base) * es + lane * 4) & ~int64_t{3}, last = N * es < 4 ? 0 : (N * es - 4) & ~int64_t{3};
-      const int64_t off = want < last ? want : last;
-      warm_b = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(ep.sb) + off);
-    }
+    if (ep.sa != nullptr)
+      warm_a = *reinterpret_cast<const uint16_t*>(static_cast<const uint8_t*>(ep.sa) +
+                                                  scale_touch(m0 + wm * (32 * TM) + 2 * lane, M, ep.sa_dtype == QWIX_BF16 ? 2 : 4));
+    if (ep.sb != nullptr)
+      warm_b = *reinterpret_cast<const uint16_t*>(static_cast<const uint8_t*>(ep.sb) +
+                                                  scale_touch(n0 + wn * 64 + lane, N, ep.sb_dtype == QWIX_BF16 ? 2 : 4));
   }
   // ---- prologue: A of slab 0, B of slabs 0 and 1 (each wavefront its rows)
   load_a(0);

@@ -393,6 +393,29 @@ def test_tiles_of_128_to_256_rows(M, K, N, kind):
   assert torch.equal(scaled, want.to(torch.float32).to(torch.bfloat16) * sa[:, None] * sb[None, :])
 
 
+@pytest.mark.parametrize('scale', [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('kind', ['int8', 'e4m3'])
+@pytest.mark.parametrize('N', [1, 2, 3])
+def test_ping_pong_tiles_with_the_shortest_scale_vectors(N, kind, scale):
+  """A weight of one to three columns under rows enough for ping-pong tiles, which touch their scales in front of the loop: each
+  touch lies in its vector (checked where it is worked out, at compile time), and the products are exact."""
+  from qwix_amd import _lib
+  M, K = 33000, 1536
+  g = torch.Generator().manual_seed(N)
+  dt, qt, acc = (torch.int8, _lib.INT8, _lib.I32) if kind == 'int8' else (torch.float8_e4m3fn, _lib.E4M3, _lib.F32)
+  a_i, b_i = (torch.randint(-7, 8, shape, generator=g, dtype=torch.int8).to(util.DEV) for shape in ((M, K), (N, K)))
+  a, b = a_i.to(torch.float32).to(dt), b_i.to(torch.float32).to(dt)
+  sa, sb = ((2.0 ** torch.randint(-3, 3, (n,), generator=g)).to(scale).to(util.DEV) for n in (M, N))
+  out = torch.full((M, N), 7.0, dtype=torch.float32, device=util.DEV)
+  print('case shortest scales', N, kind, scale, flush=True)
+  _lib.call('qwix_hip_qgemm', a.data_ptr(), K, b.data_ptr(), K, qt, M, N, K, sa.data_ptr(), _lib.float_tag(scale), sb.data_ptr(),
+            _lib.float_tag(scale), acc, out.data_ptr(), _lib.F32, N, _lib.stream_of(a))
+  want = (a_i.to(torch.float64) @ b_i.to(torch.float64).T).to(torch.float32)
+  if kind == 'int8':  # (integer sums are rounded to the scales' type first)
+    want = want.to(scale).to(torch.float32)
+  assert torch.equal(out, want * sa[:, None].to(torch.float32) * sb[None, :].to(torch.float32))
+
+
 def test_split_k_is_not_offered_where_it_cannot_pay():
   from qwix_amd import _lib
   f = _lib.load().qwix_hip_qgemm_workspace_bytes
