@@ -573,9 +573,9 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
     return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Up to 16 rows, byte weights of 32 MB and more stream faster through the smallest workgroups (4 wavefronts, two row tiles, several
-  // workgroups per CU), even though the second row tile is empty: K 4096, N 14336, int8, 1 / 16 / 32
-  // rows 25.5 / 26.9 / 21.9 -> 16.2 / 17.5 / 21.0 us (8 wavefronts: 16.5 / 18.2), e4m3 21.9 / 23.8 -> 15.5 / 17.8;
-  // K = N = 8192: 20.0 / 24.4 / 29.4 -> 17.8 / 20.0 / 26.9; at 16 MB (K = N = 4096) 9.3 against 10.2 us the other way
+  // workgroups per CU), even though the second row tile is empty: K 4096, N 14336, int8, 1 / 16
+  // rows 25.5 / 26.9 -> 16.2 / 17.5 us (8 wavefronts: 16.5 / 18.2), e4m3 21.9 / 23.8 -> 15.5 / 17.8;
+  // K = N = 8192: 20.0 / 24.4 -> 17.8 / 20.0; at 16 MB (K = N = 4096) 9.3 against 10.2 us the other way
   // round, and int4 gains nothing at any size.
   const bool small_groups = b_qtype != QWIX_INT4 && N * K >= (int64_t{32} << 20);
 #define QWIX_GEMV_KERNEL(KERN, NW, NTT, RTT)                                                                \
@@ -610,9 +610,15 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
   // More than 16 rows, 32 in a pass: eight wavefronts that share K, one workgroup per CU.  The narrower its columns the sooner it is done
   // (64 / 32 / 16 columns 1.7 / 1.2 / 1), but a second round of the CUs takes as long as the first; 64 columns that are more than a round
   // run on four wavefronts, two workgroups per CU.  Weights from HBM, 16 / 32 / 64 columns: int4 19 x 5136 over K 3968 14.0 / 9.1 / 12.0,
-  // 20 x 8960 over K 3968 20.2 / 16.8 / 12.4, 64 x 4096 over K 4096 18.4 / 12.4 / -; int8 39 x 2752 over K 3456 14.1 / 12.6 / 16.6, 77 x 4336
+  // 20 x 8960 over K 3968 20.2 / 16.8 / 12.4, 64 x 4096 over K 4096 18.9 / 12.9 / 14.9; int8 39 x 2752 over K 3456 14.1 / 12.6 / 16.6, 77 x 4336
   // over K 4992 35.2 / 31.6 / 22.4, 113 x 3224 over K 9600 74.6 / 54.4 / 37.7 (columns by N alone, four wavefronts: 78.7); on four / eight
   // wavefronts of 64 columns 206 x 5696 over K 8832 98.3 / 103, int4 130 x 14720 over K 9856 113 / 132.
+  //   Bytes whose workgroups nearly fill a round stream as fast with four wavefronts, which have half as many partial sums to add; that takes
+  // a K of some length, and with 32 columns e4m3, whose conversion is the cheaper one.  Eight / four wavefronts, 32 rows, 64 columns: int8
+  // 14336 over K 4096 22.6 / 21.3, 16384 over K 8192 40.1 / 38.4, e4m3 16384 over K 4096 23.7 / 21.6; over K 2048 int8 12288 11.9 / 12.6, e4m3
+  // 14336 11.8 / 12.4; 163 workgroups, int8 18 x 10432 over K 5376 21.6 / 22.5.  32 columns, N 8192 over K 8192 / 3072 / 2048: e4m3 28.2 / 26.1,
+  // 12.7 / 12.1, 8.8 / 9.2, int8 27.4 / 27.5, 13.3 / 13.3, 9.2 / 10.0.  Of 273 shapes of 17 to 64 rows the rule's choice is 0.3 % behind the best
+  // of the six variants on average.
   if (M > 16) {
     int64_t wgs = 0;
     double best = 0;
@@ -622,10 +628,12 @@ static int gemv_wq_impl(const void* x, int64_t ldx, const void* q, int64_t ldb_b
       const double cost = static_cast<double>((w + 255) / 256) * (t == 1 ? 1.0 : t == 2 ? 1.2 : 1.7);
       if (t == 1 || cost < best) { best = cost; nt = t; wgs = w; }
     }
+    const bool full = b_qtype != QWIX_INT4 && K >= 3072;
     if (nt == 1) QWIX_GEMV_LAUNCH_RT(8, 1, 2);
+    else if (nt == 2 && full && b_qtype == QWIX_E4M3 && wgs >= 224) QWIX_GEMV_LAUNCH_RT(4, 2, 2);
     else if (nt == 2) QWIX_GEMV_LAUNCH_RT(8, 2, 2);
-    else if (wgs <= 256) QWIX_GEMV_LAUNCH_RT(8, 4, 2);
-    else QWIX_GEMV_LAUNCH_RT(4, 4, 2);
+    else if (wgs > 256 || (full && wgs >= 192)) QWIX_GEMV_LAUNCH_RT(4, 4, 2);
+    else QWIX_GEMV_LAUNCH_RT(8, 4, 2);
     return check_launch("gemv_wq");
   }
 #define QWIX_GEMV_LAUNCH(NTT)                                                                              \
