@@ -333,8 +333,8 @@ QWIX_API int qwix_hip_qgemm_hadamard_act(const void* x, int x_dtype, int64_t M, 
  * scale per row (ga == 1), or with bf16 scales per group on both sides of int8 x int8 and e4m3 x e4m3; more than 32 rows,
  * exact == 0.  Every range's workgroups write the f32 sums of their groups' scaled partials into `workspace`
  * (qwix_hip_qgemm_grouped_call_bytes of the same arguments, ga == 1 without activation scales; 16-byte aligned; 0 = this call is
- * not split; qwix_hip_qgemm_grouped_workspace_bytes: the same for ga == 1); a second kernel adds them in range order, applies the
- * activation scale and rounds as the unsplit kernel's epilogue does.  The groups' f32 partials are then added in
+ * not split, or runs on the kernel for few tiles; qwix_hip_qgemm_grouped_workspace_bytes: as much as any call of the shape with ga == 1
+ * uses, whatever its scales' types); a second kernel adds them in range order, applies the activation scale and rounds as the unsplit kernel's epilogue does.  The groups' f32 partials are then added in
  * another order than in qwix_hip_qgemm_grouped with exact == 0 (which itself is free in that order).  Calls that run faster on
  * the kernel for few tiles, whose wavefronts share K, leave the workspace alone: the same result with and without one.  With workspace
  * NULL or too small, with exact != 0, zero points or acc_out: exactly qwix_hip_qgemm_grouped. */

@@ -158,7 +158,8 @@ def _hadamard_quantized_matmul(act, weight, pre_sign, post_sign, act_tile, prefe
   bq = _lib.INT4 if b_is4 else _lib.INT8
   need = int(_lib.load().qwix_hip_qgemm_hadamard_act_workspace_bytes(c.M, c.K, tile, _lib.float_tag(x.dtype)))
   # room behind it for the GEMM's K ranges (few tiles, one scale per token; 0 bytes otherwise)
-  need += int(_lib.load().qwix_hip_qgemm_grouped_workspace_bytes(c.M, c.N, c.K, group, bq)) if tile == c.K else 0
+  need += int(_lib.load().qwix_hip_qgemm_grouped_call_bytes(c.M, c.N, c.K, group, bq, _lib.float_tag(x.dtype), 1,
+                                                            _lib.float_tag(sb.dtype))) if tile == c.K else 0
   ws = torch.empty(max(int(need), 16), dtype=torch.uint8, device=x.device)
   out = torch.empty(c.M, c.N, dtype=res_t, device=x.device)
   _lib.call('qwix_hip_qgemm_hadamard_act', x.data_ptr(), _lib.float_tag(x.dtype), c.M, c.N, c.K, _lib.ptr(pre_sign),

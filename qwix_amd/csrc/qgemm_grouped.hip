@@ -1197,10 +1197,11 @@ int launch_grouped_decode(const GroupedArgs& p, hipStream_t st) {
 // 1960 x 1408 over K 4096 39.3 / 46.7 -> 26.5 / 30.9; 512, 2048 x 2048 over K 4096 40.2 / 46.8 -> 32.9 / 35.1, 1000 x 4096 over K 2048
 // 23.0 / 24.5 -> 18.4 / 21.9; 640, 1200 x 4096 over K 8192 73.4 / 87.8 against 86.0 / 126; 768, 767 x 8192 over K 4096 42.6 / 48.2
 // against 49.7 / 56.6.
-inline bool takes_narrow(const GroupedArgs& p, bool sag) {
-  const int64_t tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 63) / 64);
-  return tiles <= (sag && p.ksplit == 0 && p.K > 4096 ? 256 : kNarrowTiles) || p.M <= 64;
+inline bool narrow_tiles(int64_t M, int64_t N, int64_t K, bool sag_whole) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64);
+  return tiles <= (sag_whole && K > 4096 ? 256 : kNarrowTiles) || M <= 64;
 }
+inline bool takes_narrow(const GroupedArgs& p, bool sag) { return narrow_tiles(p.M, p.N, p.K, sag && p.ksplit == 0); }
 
 // Both operands with bf16 scales per group: the fold by outer products (see OUTER).  -1: the scales do not fit in LDS.
 template <int BQT, typename G>
@@ -1279,16 +1280,19 @@ inline double decode_us(int64_t M, int64_t N, int64_t K, int b_qtype, bool sag) 
 // int8 84 x 2304 over K 6912 14.3 -> 10.9; scales on both sides, int8 318 x 1280 over K 3328 16.6 -> 15.1, e4m3 178 x 1312 over K 2560
 // 14.1 -> 7.9; int8 238 x 4008 over K 2048 13.7 against 20.2.  f32 weight scales keep the tiles' order of the groups, in which the run that
 // dumps its partials gives equal bits.
+inline bool rows_share_k(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, bool sag, int sb_dtype) {
+  if (M <= 32 || sb_dtype != QWIX_BF16 || group != Fast::kBK || K / Fast::kBK < 4 || K > 16384 || (sag && b_qtype == QWIX_INT4) ||
+      !narrow_tiles(M, N, K, sag))
+    return false;
+  double us;
+  narrow_ranges(M, N, K, group, sag, &us);
+  return decode_us(M, N, K, b_qtype, sag) < 0.95 * us;
+}
+
 inline bool takes_decode(const GroupedArgs& p, int b_qtype) {
-  if (p.M > 32) {
-    const bool sag = p.sa != nullptr && p.ga > 1;
-    if (p.ksplit || p.zu || p.acc_out || p.single || p.sb_dtype != QWIX_BF16 || p.group != Fast::kBK || p.K / Fast::kBK < 4 || (sag && b_qtype == QWIX_INT4) ||
-        !takes_narrow(p, sag) || 32 * p.lda >= (int64_t{1} << 31) || 32 * p.ldb >= (int64_t{1} << 31) || p.K > 16384)
-      return false;
-    double us;
-    narrow_ranges(p.M, p.N, p.K, p.group, sag, &us);
-    return decode_us(p.M, p.N, p.K, b_qtype, sag) < 0.95 * us;
-  }
+  if (p.M > 32)  // (rows of a pitch beyond 32-bit offsets never come here: grouped_impl)
+    return !p.ksplit && !p.zu && !p.acc_out && !p.single &&
+           rows_share_k(p.M, p.N, p.K, p.group, b_qtype, p.sa != nullptr && p.ga > 1, p.sb_dtype);
   const int64_t halves = static_cast<int64_t>(p.N) * (b_qtype == QWIX_INT4 ? 1 : 2);  // half bytes of a weight row
   const bool few = halves <= 16384 || (p.M <= 16 && p.K >= 2048 && halves * p.K <= int64_t{160} << 20);
   return p.ksplit == 0 && p.zu == nullptr && p.acc_out == nullptr && p.M <= 32 && p.group == Fast::kBK && !p.single &&
@@ -1650,13 +1654,14 @@ extern "C" int qwix_hip_qgemm_grouped(const void* a, int64_t lda, const void* b,
 
 extern "C" size_t qwix_hip_qgemm_grouped_call_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, int sa_dtype,
                                                     int64_t ga, int sb_dtype) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || rows_share_k(M, N, K, group, b_qtype, ga > 1, sb_dtype)) return 0;
   return static_cast<size_t>(grouped_ranges_of(M, N, K, group, b_qtype, ga > 1, sa_dtype, sb_dtype)) * M * N * 4;
 }
 
-// (with one activation scale per row, which every weight type splits alike)
+// (with one activation scale per row, which every weight type splits alike, and scales of any dtype)
 extern "C" size_t qwix_hip_qgemm_grouped_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype) {
-  return qwix_hip_qgemm_grouped_call_bytes(M, N, K, group, b_qtype, QWIX_BF16, 1, QWIX_BF16);
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return static_cast<size_t>(grouped_ranges_of(M, N, K, group, b_qtype, false, QWIX_BF16, QWIX_BF16)) * M * N * 4;
 }
 
 extern "C" int qwix_hip_qgemm_grouped_ws(const void* a, int64_t lda, const void* b, int64_t ldb_bytes, int b_qtype,

@@ -42,6 +42,21 @@ def test_argument_validation_happens_before_any_launch():
     qarray.quantize(torch.zeros(4, 8), qarray.HowToQuantize(qtype='int8'))
 
 
+@pytest.mark.parametrize('M,N,K,qtype,ga,decode', [
+    (71, 2048, 3584, _lib.INT4, 1, True), (84, 2304, 6912, _lib.INT8, 1, True), (100, 1280, 4096, _lib.INT8, 32, True),
+    (200, 1280, 3328, _lib.E4M3, 26, True), (607, 1408, 4608, _lib.INT8, 1, False), (512, 1024, 8192, _lib.INT8, 1, False)])
+def test_sub_channel_calls_that_no_range_of_k_serves_need_no_scratch(M, N, K, qtype, ga, decode):
+  """Calls of the kernel whose wavefronts share K ask for no workspace; f32 weight scales keep the tiles, and what serves every
+  type of scales stays what the ranges take."""
+  lib = _lib.load()
+  size = lambda sb: lib.qwix_hip_qgemm_grouped_call_bytes(M, N, K, 128, qtype, _lib.BF16, ga, sb)
+  assert (size(_lib.BF16) == 0) == decode
+  if ga == 1:
+    any_scales = lib.qwix_hip_qgemm_grouped_workspace_bytes(M, N, K, 128, qtype)
+    assert any_scales >= 2 * M * N * 4 and any_scales % (M * N * 4) == 0
+    assert size(_lib.F32) == any_scales and (decode or size(_lib.BF16) == any_scales)
+
+
 def test_bounds_and_eligibility():
   assert numerics.get_symmetric_bound('int8') == 127.5 and numerics.get_symmetric_bound(torch.int8) == 127.5
   assert numerics.get_symmetric_bound('int4') == 7.5 and numerics.get_symmetric_bound(torch.float8_e4m3fn) == 448.0
