@@ -277,8 +277,8 @@ QWIX_API int qwix_hip_qgemm_dynamic_act(const void* x, int x_dtype, int64_t ldx,
                                int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
                                void* out, int out_dtype, int64_t ldo, void* workspace,
                                size_t workspace_bytes, void* stream);
-/* The same of max(x, 0), where a ReLU stands in front: rows of at most 32 KB.  Bit-identical to the ReLU and
- * qwix_hip_qgemm_dynamic_act (a negative NaN counts as 0). */
+/* The same of max(x, 0), where a ReLU stands in front (NaN of either sign stays NaN): x 16-byte aligned, K a multiple of 8, rows of at
+ * most 32 KB.  Bit-identical to the ReLU and qwix_hip_qgemm_dynamic_act. */
 QWIX_API int qwix_hip_qgemm_dynamic_relu(const void* x, int x_dtype, int64_t ldx, const void* b, int64_t ldb, int qtype,
                                 int64_t M, int64_t N, int64_t K, const void* sb, int sb_dtype, int acc_dtype,
                                 void* out, int out_dtype, int64_t ldo, void* workspace,
