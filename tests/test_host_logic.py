@@ -42,6 +42,49 @@ def test_argument_validation_happens_before_any_launch():
     qarray.quantize(torch.zeros(4, 8), qarray.HowToQuantize(qtype='int8'))
 
 
+def test_products_that_quantize_on_the_way_refuse_what_they_do_not_take():
+  """Scores, probabilities with values, and a ReLU in front: every refusal with its message, in front of any launch."""
+  lib = _lib.load()
+  at = lambda v: ctypes.c_void_p(v)
+  x, y, out, ws, off = at(1 << 20), at(2 << 20), at(3 << 20), at(4 << 20), at((4 << 20) + 8)
+
+  def scores(M=65, N=72, K=64, batch=2, qt=_lib.INT8, x=x, y=y, out=out, ws=ws, less=0):
+    n = lib.qwix_hip_qgemm_batched_act_workspace_bytes(batch, M, N, K)
+    return lib.qwix_hip_qgemm_batched_act(x, y, qt, batch, M, N, K, out, ws, max(0, n - less), None), lib.qwix_hip_last_error()
+
+  def values(M=65, N=72, K=64, batch=2, qt=_lib.INT8, x=x, y=y, out=out, ws=ws, less=0):
+    n = lib.qwix_hip_qgemm_batched_act_kn_workspace_bytes(batch, M, N, K)
+    return lib.qwix_hip_qgemm_batched_act_kn(x, y, qt, batch, M, N, K, out, ws, max(0, n - less), None), lib.qwix_hip_last_error()
+
+  def relu(M=33, N=72, K=256, x_dtype=_lib.BF16, qt=_lib.INT8, ldx=None, x=x, y=y, out=out, ws=ws, less=0):
+    n = lib.qwix_hip_qgemm_dynamic_act_workspace_bytes(M, N, K, x_dtype)
+    return lib.qwix_hip_qgemm_dynamic_relu(x, x_dtype, ldx or K, y, (K + 15) // 16 * 16, qt, M, N, K, None, 0, 0, out, x_dtype, N, ws,
+                                           max(0, n - less), None), lib.qwix_hip_last_error()
+  for f in (scores, values, relu):
+    for bad, message in ((dict(x=None), b'null'), (dict(y=None), b'null'), (dict(out=None), b'null'), (dict(qt=_lib.INT4), b'int8 or e4m3'),
+                         (dict(ws=None), b'workspace'), (dict(less=1), b'workspace'), (dict(ws=off), b'workspace')):
+      rc, said = f(**bad)
+      assert rc != 0 and message in said, (f.__name__, bad, rc, said)
+  for f in (scores, values):
+    for bad in (dict(x=off), dict(y=off), dict(out=off)):
+      rc, said = f(**bad)
+      assert rc != 0 and b'aligned' in said, (f.__name__, bad, rc, said)
+  for bad, message in ((dict(K=96), b'K 64 or 128'), (dict(N=12), b'multiple of 8'), (dict(M=1 << 24), b'32-bit'), (dict(batch=65536), b'bad shape'),
+                       (dict(batch=0), b'bad shape'), (dict(M=0), b'bad shape'), (dict(M=64, N=12), b'multiple of 8')):
+    rc, said = scores(**bad)
+    assert rc != 0 and message in said, (bad, rc, said)
+  assert lib.qwix_hip_qgemm_batched_act_workspace_bytes(2, 64, 72, 64) == 0  # one launch
+  for bad in (dict(K=72), dict(N=12), dict(K=4112), dict(batch=65536), dict(M=0), dict(K=4096, N=8192)):  # (y of more than 32 MB)
+    shape = {**dict(M=65, N=72, K=64, batch=2), **bad}
+    assert lib.qwix_hip_qgemm_batched_act_kn_workspace_bytes(shape['batch'], shape['M'], shape['N'], shape['K']) == 0
+    rc, said = values(**bad)
+    assert rc != 0 and b'multiple of 16' in said, (bad, rc, said)
+  for bad, message in ((dict(x=off), b'aligned'), (dict(K=16512), b'32 KB'), (dict(K=8320, x_dtype=_lib.F32), b'32 KB'), (dict(K=260), b'32 KB'),
+                       (dict(ldx=264), b'dense')):
+    rc, said = relu(**bad)
+    assert rc != 0 and message in said, (bad, rc, said)
+
+
 @pytest.mark.parametrize('M,N,K,qtype,ga,decode', [
     (71, 2048, 3584, _lib.INT4, 1, True), (84, 2304, 6912, _lib.INT8, 1, True), (100, 1280, 4096, _lib.INT8, 32, True),
     (200, 1280, 3328, _lib.E4M3, 26, True), (607, 1408, 4608, _lib.INT8, 1, False), (512, 1024, 8192, _lib.INT8, 1, False)])
