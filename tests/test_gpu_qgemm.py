@@ -393,6 +393,30 @@ def test_tiles_of_128_to_256_rows(M, K, N, kind):
   assert torch.equal(scaled, want.to(torch.float32).to(torch.bfloat16) * sa[:, None] * sb[None, :])
 
 
+@pytest.mark.parametrize('kind', ['int8', 'e4m3'])
+@pytest.mark.parametrize('M,K,N', [(1290, 1536, 3201), (1417, 256, 5382), (2306, 640, 4868)])  # 128, 192 and 256 rows per tile
+def test_ping_pong_tiles_with_a_pitch(M, K, N, kind):
+  """Rows of both operands and of the result in wider arrays: small integers, exact as above; what lies between the operands' rows is not
+  multiplied, and what lies between the result's rows stays."""
+  from qwix_amd import _lib
+  g = torch.Generator().manual_seed(M + 1)
+  dt, qt, acc = (torch.int8, _lib.INT8, _lib.I32) if kind == 'int8' else (torch.float8_e4m3fn, _lib.E4M3, _lib.F32)
+  a_i, b_i = (torch.randint(-7, 8, shape, generator=g, dtype=torch.int8).to(util.DEV) for shape in ((M, K), (N, K)))
+  want = a_i.to(torch.float64) @ b_i.to(torch.float64).T
+
+  def wide(t, pad):
+    w = torch.full((t.shape[0], K + pad), 0x7F, dtype=torch.uint8, device=util.DEV)  # (a NaN of e4m3)
+    w[:, :K] = t.to(torch.float32).to(dt).view(torch.uint8)
+    return w
+  for a_pad, b_pad in ((16, 272), (144, 0)):
+    a, b = wide(a_i, a_pad), wide(b_i, b_pad)
+    out = torch.full((M, N + 24), 7.0, dtype=torch.float32, device=util.DEV)
+    print('case tile pitch', M, K, N, kind, a_pad, b_pad, flush=True)
+    _lib.call('qwix_hip_qgemm', a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), qt, M, N, K, None, 0, None, 0, acc, out.data_ptr(), _lib.F32,
+              N + 24, _lib.stream_of(a))
+    assert torch.equal(out[:, :N].to(torch.float64), want) and bool((out[:, N:] == 7.0).all())
+
+
 @pytest.mark.parametrize('scale', [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize('kind', ['int8', 'e4m3'])
 @pytest.mark.parametrize('N', [1, 2, 3])

@@ -366,6 +366,33 @@ def test_ragged_dot_tiles_of_128_to_256_rows(M, K, N, sizes, kind):
   assert torch.count_nonzero(out[start:]).item() == 0
 
 
+@pytest.mark.parametrize('kind', ['int8', 'float8_e4m3fn'])
+@pytest.mark.parametrize('M,K,N,sizes', [(400, 1536, 317, (1, 0, 127, 129, 65)), (2499, 384, 2076, (1, 192, 193, 0) + (120,) * 15 + (300,)),
+                                         (3973, 640, 2565, (1, 256, 257, 0, 1460, 1900, 2 ** 31 - 1))])  # as above: 64 to 256 rows
+def test_ragged_product_with_a_pitch(M, K, N, sizes, kind):
+  """Rows of both operands, and the groups' weights, further apart than they are long, through the C ABI: exact as above."""
+  from qwix_amd import _lib
+  g = torch.Generator().manual_seed(K + N)
+  dt, qt, acc = (torch.int8, _lib.INT8, _lib.I32) if kind == 'int8' else (torch.float8_e4m3fn, _lib.E4M3, _lib.F32)
+  G = len(sizes)
+  a_i = torch.randint(-7, 8, (M, K), generator=g, dtype=torch.int8).to(util.DEV)
+  b_i = torch.randint(-7, 8, (G, N, K), generator=g, dtype=torch.int8).to(util.DEV)
+  a = torch.full((M, K + 48), 0x7F, dtype=torch.uint8, device=util.DEV)  # (0x7F: a NaN of e4m3)
+  b = torch.full((G, N + 3, K + 16), 0x7F, dtype=torch.uint8, device=util.DEV)
+  a[:, :K], b[:, :N, :K] = a_i.to(torch.float32).to(dt).view(torch.uint8), b_i.to(torch.float32).to(dt).view(torch.uint8)
+  out = torch.full((M, N + 8), 7.0, dtype=torch.float32, device=util.DEV)
+  counts = _sizes(sizes)
+  print('case ragged pitch', M, K, N, kind, flush=True)
+  _lib.call('qwix_hip_qgemm_ragged', a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(1), b.stride(0), qt, M, N, K, counts.data_ptr(), G, None, 0,
+            None, 0, 0, acc, out.data_ptr(), _lib.F32, N + 8, _lib.stream_of(a))
+  start = 0
+  for i, size in enumerate(sizes):
+    stop = min(start + size, M)
+    assert torch.equal(out[start:stop, :N].to(torch.float64), a_i[start:stop].to(torch.float64) @ b_i[i].to(torch.float64).T), i
+    start = stop
+  assert torch.count_nonzero(out[start:, :N]).item() == 0 and bool((out[:, N:] == 7.0).all())
+
+
 def test_ragged_dot_weight_only_more_row_tiles_than_a_grid():
   """65534 groups of 17 and 3 rows: 98301 row tiles, more than a grid's y axis holds."""
   import qwix_amd
