@@ -145,12 +145,12 @@ def test_batched_long_contraction(B, M, N, K, qtype, dtype):
 @pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
 @pytest.mark.parametrize('K', [64, 128])
 @pytest.mark.parametrize('shape', [(1, 8), (16, 264), (17, 24), (33, 520), (64, 1000), (65, 72), (130, 2056), (3, 96, 2, 40)])
-def test_scores_quantized_inside_the_product(shape, K, qtype):
+def test_scores_quantized_inside_the_product(shape, K, qtype, monkeypatch):
   """Both operands of a scores product under a rule with act_qtype: quantized rows inside the kernel (the second operand too up to 64
   rows), against quantize() of each and the contraction, bit for bit; rows of zeros, of signed zeros and with infinities and NaN among
   them.  What the fused call does not take (f32, other layouts) gives the same results by the ordinary path."""
   import qwix_amd
-  from qwix_amd import nn
+  from qwix_amd import _lib, nn
   print('case scores', shape, K, qtype, flush=True)
   gen = torch.Generator(device=util.DEV).manual_seed(sum(shape) + K)
   if len(shape) == 2:
@@ -173,6 +173,10 @@ def test_scores_quantized_inside_the_product(shape, K, qtype):
   def want(a, b):
     q = [qwix_amd.quantize(t, qtype, channelwise_axes=list(range(t.ndim - 1))) for t in (a, b)]
     return qwix_amd.einsum(spec, *q)
+  names, call = [], _lib.call
+  monkeypatch.setattr(_lib, 'call', lambda *a: names.append(a[0]) or call(*a))
+  model.apply({}, lhs, rhs)
+  assert names == ['qwix_hip_qgemm_batched_act']
   for _ in range(6):  # the ordinary path, then its plan
     got = model.apply({}, lhs, rhs)
     assert torch.equal(got.view(torch.int16), want(lhs, rhs).view(torch.int16))
@@ -186,7 +190,7 @@ def test_scores_quantized_inside_the_product(shape, K, qtype):
 @pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
 @pytest.mark.parametrize('batch,M,K,N', [(3, 1, 16, 8), (2, 24, 192, 64), (3, 130, 464, 136), (1, 70, 1040, 24), (2, 33, 2512, 128), (4, 9, 3072, 64),
                                          (32, 3, 4096, 128), (5, 300, 2064, 40)])
-def test_probabilities_and_values_quantized_in_one_launch(batch, M, K, N, qtype):
+def test_probabilities_and_values_quantized_in_one_launch(batch, M, K, N, qtype, monkeypatch):
   """Rows of the first and columns of the second operand under a rule with act_qtype, against quantize() of each and the contraction, bit
   for bit: workgroups of 256 to 1024 threads, rows of one to eight loads per thread, the last strip partly empty; zeros, signed zeros,
   infinities and NaN among them.  Other layouts give the same results by the ordinary path."""
@@ -208,6 +212,10 @@ def test_probabilities_and_values_quantized_in_one_launch(batch, M, K, N, qtype)
   ql = qwix_amd.quantize(lhs, qtype, channelwise_axes=[0, 1])
   qr = qwix_amd.quantize(rhs, qtype, channelwise_axes=[0, 2])
   want = qwix_amd.einsum('bqk,bkd->bqd', ql, qr)
+  names, call = [], _lib.call
+  monkeypatch.setattr(_lib, 'call', lambda *a: names.append(a[0]) or call(*a))
+  model.apply({}, lhs, rhs)
+  assert names == ['qwix_hip_qgemm_batched_act_kn']
   for _ in range(6):  # the ordinary path, then its plan
     assert torch.equal(model.apply({}, lhs, rhs).view(torch.int16), want.view(torch.int16))
   strided = torch.cat([rhs, rhs], -1)[..., :N]

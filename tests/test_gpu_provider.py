@@ -296,12 +296,12 @@ def test_decode_size_calls_fold_the_activation_quantization_into_the_gemm(monkey
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize('qtype', ['int8', 'float8_e4m3fn'])
 @pytest.mark.parametrize('rows,hidden', [(1, 256), (20, 2048), (33, 2048), (32, 2176), (300, 4096), (65, 8320), (9, 16512)])
-def test_relu_inside_the_quantization_of_the_next_layer(rows, hidden, qtype, dtype):
+def test_relu_inside_the_quantization_of_the_next_layer(rows, hidden, qtype, dtype, monkeypatch):
   """The MLP's second layer takes max(h, 0) from h itself: against a ReLU of its own in front of the plain operation, bit for bit,
   with rows that are negative throughout and with the kernel that quantizes in the product (up to 32 rows, K up to 2048); rows of
   more than 32 KB keep the ReLU of their own."""
   import qwix_amd
-  from qwix_amd import nn
+  from qwix_amd import _lib, nn
   print('case relu', rows, hidden, qtype, dtype, flush=True)
   g = torch.Generator(device=util.DEV).manual_seed(rows + hidden)
 
@@ -313,12 +313,22 @@ def test_relu_inside_the_quantization_of_the_next_layer(rows, hidden, qtype, dty
             'Dense_1': {'kernel': torch.randn(hidden, 136, generator=g, device=util.DEV).to(dtype)}}
   x = torch.randn(rows, 128, generator=g, device=util.DEV).to(dtype)
   models = [qwix_amd.quantize_model(m(hidden, 136), qwix_amd.PtqProvider([rule])) for m in (nn.MLP, Plain)]
+  negative = {'Dense_0': {'kernel': -params['Dense_0']['kernel'].abs() - 1}, 'Dense_1': params['Dense_1']}
   params = qwix_amd.quantize_params(params, models[0].init(params, x))
+  names, call = [], _lib.call
+  monkeypatch.setattr(_lib, 'call', lambda *a: names.append(a[0]) or call(*a))
   for _ in range(6):  # the ordinary path, then its plan
     got, want = (m.apply(params, x) for m in models)
     assert got.dtype == dtype and torch.equal(got, want)
-  negative = {'Dense_0': params['Dense_0'], 'Dense_1': params['Dense_1']}
-  assert torch.equal(models[0].apply(negative, torch.zeros_like(x)), models[1].apply(negative, torch.zeros_like(x)))
+  assert ('qwix_hip_qgemm_dynamic_relu' in names) == (hidden * x.element_size() <= 32768)
+  negative = qwix_amd.quantize_params(negative, models[0].init(negative, x))
+  x = x.abs() + 1
+  x[1::2] *= -1  # every second row of h positive throughout, the others negative
+  got, want = (m.apply(negative, x) for m in models)
+  assert torch.equal(got, want)
+  assert torch.count_nonzero(got[::2]).item() == 0 and bool((got[1::2] != 0).any(-1).all())
+  assert torch.equal(models[0].apply(params, torch.zeros_like(x)), models[1].apply(params, torch.zeros_like(x)))
+  want = models[1].apply(params, x)
   # a provider with a dot_general of its own never sees the option
   class Own(qwix_amd.PtqProvider):
     def dot_general(self, lhs, rhs, dimension_numbers, precision=None, preferred_element_type=None, *, out_sharding=None):
