@@ -707,52 +707,39 @@ int qwix::gemv_wq_groups(const void* x, int64_t ldx, const void* q, int64_t ldb_
     else if (sbf) QWIX_GEMVG_KERNEL(QWIX_INT8, true, NW, NTT, RTT);                                        \
     else QWIX_GEMVG_KERNEL(QWIX_INT8, false, NW, NTT, RTT);                                                \
   } while (0)
-  // Many workgroups (several rounds of them) cover each other's latency, and few wavefronts in each leave the fewest partial
-  // sums to add; few workgroups need their wavefronts to keep the loads in flight.  Weights from HBM, int4 / int8 in us:
-  //   64 groups x 4 rows, K 2048, N 4096 (4096 workgroups of 64 columns): 2 wavefronts x 64 columns 53.7 / 97.7 (5.2 and
-  //     5.6 TB/s), 4 x 64 63.7 / 96.5, 8 x 32 80.3 / 119.7, 4 x 16 90.6 / 128.4
-  //   8 groups x 2 rows, K 2048, N 3072 (384): 4 x 64 8.3, 8 x 32 9.2, 2 x 64 11.6
-  //   8 groups x 2 rows, K 4096, N 1024 (128): 8 x 32 6.6 / 9.9, 4 x 64 10.4 / 15.8, 2 x 64 15.8 / 20.4
-  // Two row tiles pay for themselves where groups of more than 16 rows are common (64 groups of 8 / 12 / 16 / 30 rows on
-  // average, int4: one tile 62.6 / 76.3 / 86.0 / 132.2, two 68.0 / 74.3 / 80.5 / 120.4).
-  //   What counts is the workgroups that have rows: with a few rows over many groups most groups are empty (rows that fall
-  // anywhere: exp(-M / G) of them).  One row tile, 2 x 64 / 4 x 64 / 8 x 32 / 4 x 32 columns: int4 64 groups x 0.4 rows, K 3840, N 1024 (320)
-  // 18.1 / 15.1 / 13.6 / 13.8; 32 x 4.3, K 3968, N 1728 (852) 26.7 / 27.9 / 27.6 / 27.7; int8 32 x 0.3, K 2816, N 1984 (243) 18.3 / 16.3 / 13.3 /
-  // 16.0, two tiles 4 x 64 17.1; 16 x 2.5, K 3072, N 1600 (367) 22.5 / 20.0 / 19.6 / 18.8, 20.7; 8 x 1.9, K 2176, N 7488 (792) 27.3 / 29.2 /
-  // 29.3 / 27.6, 31.0.  Two row tiles, by the tiles there are: 8 x 15.5, K 2432, N 2048 (256) 8 x 32 columns 16.7, 8 x 64 13.0, 4 x 64 14.2.
+  // Launch shape: wavefronts x columns, in tiles of 16 or 32 rows.  The sizes are on the device: rows that fall on the groups at random leave
+  // exp(-M / G) of these empty, and sizes spread like an exponential give 1 / (exp(TR / (M / G)) - 1) tiles of TR rows behind a group's first.
+  // w and w32 are the workgroups of 64 columns that have rows, in tiles of 16 and of 32 rows, two of which have one CU each.  Of them:
+  //   * about one round of the CUs or less is bound by latency: eight wavefronts share K, 32 columns make twice the workgroups (8 groups x 0.25
+  //     rows, K 1920, N 1728: 8 x 32 columns 5.2 us, 4 x 32 5.7, 4 x 64 6.5, 2 x 64 8.8; a long K longer so: 16 x 4, K 4864, N 1088 14.2 / 16.5 /
+  //     16.1 / 22.9), where 32-row tiles fit one round and 16-row tiles do not in those (8 x 17, K 5504, N 960, bytes 8 x 32 24.1, with two row
+  //     tiles 19.2), up to two of them with 64 columns;
+  //   * a few hundred fill the chip sooner with four wavefronts and 32 columns, and leave less to empty workgroups (16 groups x 0.25 rows, K
+  //     1024, N 3712, int4 5.9 us, 8 x 32 7.8, 4 x 64 6.2);
+  //   * more take 64 columns, which read an activation half as often; bytes, which wait for HBM longer, only from 4 rows per group on;
+  //   * thousands over a short K take two wavefronts, which have the fewest partial sums to add (8 x 23, K 1280, N 59328, int4 129 against
+  //     164; 64 x 4, K 2048, N 7168 86 against 95);
+  //   * the second row tile pays for its registers where the second pass over the weights it saves is long and common (64 x 25, K 4736, N
+  //     896, int4 one tile 75, two 64; bytes sooner: 64 x 9, K 6144, N 1664 142 and 131).
+  // 5620 shapes (4 to 128 groups x 0.25 to 64 rows, K 768 to 6144, N 512 to 65536, uneven sizes, weights from HBM): the choice is 2 % (int4) and
+  // 3 % (bytes) behind the best of the eight shapes on average; most of that are sizes that no rule over their sum can know.  Each
+  // threshold may move by a fifth within 0.2 % of that.
   const double per_group = static_cast<double>(M) / static_cast<double>(G), cols = static_cast<double>((N + 63) / 64);
-  const double wgs = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
-  const double tiles = static_cast<double>(G) * std::max(1.0, per_group / 32 + 0.5) * cols;
-  // int4, uneven groups, 4 x 64 / 2 x 64 columns with one row tile, 4 x 64 / 2 x 64 with two: second passes over some groups cost less than an
-  // empty tile in most (64 groups of 12 / 16 rows, K 2048, N 4096 73.0 / 70.2 / 81.0 / 74.8, 85.9 / 81.2 / 85.8 / 78.4; 64, 1024, 2048 21.4 / 20.6 /
-  // 26.3 / 24.9, 25.7 / 24.1 / 28.0 / 26.2; 64, 1920, 1024 20.8 / 23.1 / 23.4 / 23.6, 24.6 / 26.3 / 25.6 / 26.6; 16, 1408, 3072 14.8 / 13.3 / 18.1 /
-  // 15.0, 16.7 / 15.3 / 19.4 / 16.1; 8, 4096, 4096 19.0 / 21.1 / 20.5 / 27.3, 22.0 / 22.0 / 22.1 / 28.1).
-  const bool one = M <= 10 * G || (b_qtype == QWIX_INT4 && tiles >= 320 && per_group <= (wgs >= 3000 ? 14 : 16));
-  if (!one) {
-    if (2 * tiles <= 256) QWIX_GEMVG_LAUNCH(8, 2, 2);
-    else if (tiles <= 256) QWIX_GEMVG_LAUNCH(8, 4, 2);
-    else if (b_qtype == QWIX_INT4 && tiles >= 1024) QWIX_GEMVG_LAUNCH(2, 4, 2);
-    else QWIX_GEMVG_LAUNCH(4, 4, 2);
-  } else {
-    if (b_qtype == QWIX_INT4) {
-      // Two wavefronts or four, one row tile: 64 groups of 1 / 6 rows, K 4096, N 1024 2 x 64 columns 22.6 / 31.7, 4 x 64 20.5 / 32.9; 32, 2048, 2048
-      // 6 / 9.8 rows 15.6 / 19.0, 16.9 / 18.8; 64, 1920, 1024 9.8 rows 22.0, 19.7; 16, 2048, 8192 3 / 8 rows 30.4 / 34.5, 28.2 / 33.4; 8, 2048, 14336
-      // 29.1 / 30.1, 26.4 / 29.3; 64, 2048, 4096 8 rows 58.7, 60.4.
-      const bool two_waves = per_group > 10 ? wgs >= 1500 : wgs >= 3000 || (wgs >= 800 && wgs < 1500 && per_group < 7.5);
-      if (wgs < (K >= 2048 ? 320 : 260)) QWIX_GEMVG_LAUNCH(8, 2, 1);  // (4 x 64 over K 1664, 303: 8.3 against 9.3; over K 1408, 217: 6.4 against 5.7)
-      else if (two_waves) QWIX_GEMVG_LAUNCH(2, 4, 1);
-      else QWIX_GEMVG_LAUNCH(4, 4, 1);
-    } else {
-      // Bytes, four wavefronts, 32 columns / 64 / 64 and two row tiles, uneven groups: 64 columns read an activation half as often, which
-      // counts the more rows there are (16 groups, K 1024, N 8192, 3 / 7 rows 29.0 / 26.7 / 32.2, 33.5 / 30.1 / 35.2; 64, 1920, 1024, 2.5 / 8
-      // rows 25.3 / 26.6 / 28.7, 31.4 / 30.1 / 30.0) and the more rounds of the CUs stream (64, 2048, 4096, 1 row 63.1 / 61.5 / 67.7); 32 fill
-      // a chip that 64 leave idle (32, 3072, 1216, 2.5 / 8 rows 26.9 / 28.7 / 33.6, 30.8 / 31.3 / 33.2).  Second passes over a long K cost more
-      // than the empty tile of most groups once some groups have them (64, 4096, 1024, 8 / 10 rows 58.1 / 57.5 / 56.3, 63.8 / 60.8 / 57.5).
-      if (wgs < 300) QWIX_GEMVG_LAUNCH(8, 2, 1);
-      else if (per_group >= 9.25 && K > 3072) QWIX_GEMVG_LAUNCH(4, 4, 2);
-      else if (wgs >= 1750 || (wgs >= 690 && per_group >= 4.5) || (wgs >= 500 && per_group >= 7.5)) QWIX_GEMVG_LAUNCH(4, 4, 1);
-      else QWIX_GEMVG_LAUNCH(4, 2, 1);
-    }
+  const double live = static_cast<double>(G) * (1.0 - std::exp(-per_group)) * cols;
+  auto later = [&](double tr) { return static_cast<double>(G) / std::expm1(std::min(50.0, tr / per_group)) * cols; };
+  const double w = live + later(16), w32 = live + later(32), launched = w + 0.2 * (static_cast<double>(G) * cols - live);
+  const bool int4 = b_qtype == QWIX_INT4, long_k = K >= 2048;
+  if (w > 154 && w32 <= 143) QWIX_GEMVG_LAUNCH(8, 2, 2);
+  else if (per_group >= 12 && w32 > 143 && w32 <= 256) QWIX_GEMVG_LAUNCH(8, 4, 2);
+  else if (launched < (long_k ? 320 : 256)) QWIX_GEMVG_LAUNCH(8, 2, 1);
+  else if (int4 ? w < (K >= 2560 ? 300 : 384) : w < 384 || (per_group < 4 && w < 1300)) QWIX_GEMVG_LAUNCH(4, 2, 1);
+  else {
+    const bool two = !int4 ? per_group >= 8 && w >= (long_k || per_group >= 12 ? 512 : 2500)
+                           : per_group >= 20 ? K >= 1536 && w >= (long_k ? 1024 : 4500) : per_group >= 9 && long_k && w >= 5500;
+    const double few_from = !int4 ? (K < 1536 ? 3000 : HUGE_VAL) : two ? 4500 : K < 1536 ? 900 : K < 3072 ? 3000 : HUGE_VAL;
+    if (w >= few_from) { if (two) QWIX_GEMVG_LAUNCH(2, 4, 2); else QWIX_GEMVG_LAUNCH(2, 4, 1); }
+    else if (two) QWIX_GEMVG_LAUNCH(4, 4, 2);
+    else QWIX_GEMVG_LAUNCH(4, 4, 1);
   }
 #undef QWIX_GEMVG_LAUNCH
 #undef QWIX_GEMVG_KERNEL

@@ -190,14 +190,16 @@ def test_ragged_dot_weight_only_experts(sizes, wq_type, tiled):
 @pytest.mark.parametrize('G,K,N,M,sizes', [
     (4, 128, 200, 40, (0, 17, 16, 1)),           # few workgroups (8 wavefronts), one K block, rows left over
     (4, 384, 72, 100, (33, 0, 70, 50)),          # two row tiles, an odd number of K blocks, sizes past the last row
-    (8, 256, 2568, 60, (1, 15, 0, 16, 3, 17, 2, 0)),   # 4 wavefronts x 64 columns, a column tile that ends early
-    (64, 256, 1000, 128, tuple(i % 4 for i in range(64))),        # several rounds: 2 wavefronts x 64 columns
-    (64, 384, 1000, 1100, tuple((7 * i) % 35 for i in range(64))),  # the same with two row tiles, several passes
+    (8, 256, 2568, 60, (1, 15, 0, 16, 3, 17, 2, 0)),   # 4 wavefronts x 32 columns, a column tile that ends early
+    (64, 256, 1000, 128, tuple(i % 4 for i in range(64))),        # several rounds: int4 4 wavefronts x 64 columns, bytes x 32
+    (64, 384, 1000, 1100, tuple((7 * i) % 35 for i in range(64))),  # int4: 2 wavefronts x 64 columns; bytes: 4, two row tiles; several passes
+    (4, 256, 1480, 80, (40, 0, 23, 17)),               # two row tiles on eight wavefronts, 32 columns
+    (16, 256, 4400, 740, tuple((37 * i) % 93 for i in range(16))),   # bytes: 2 wavefronts, two row tiles
     (8, 640, 1032, 120, (40, 0, 33, 16, 1, 17, 2, 3)),             # two row tiles, 64 columns on eight wavefronts
     (32, 640, 1032, 12, (3, 0, 1) + (0,) * 20 + (5, 2) + (0,) * 7),   # most groups empty
     (64, 384, 1000, 420, tuple((5 * i) % 18 for i in range(64))),  # bytes: 4 wavefronts x 64 columns, second passes of one row
     (64, 384, 2000, 800, tuple((11 * i) % 26 for i in range(64))),  # int4: 2 wavefronts, one row tile, second passes of up to 9 rows
-    (64, 384, 1000, 770, tuple((11 * i) % 25 for i in range(64))),  # int4: 4 wavefronts
+    (64, 384, 1000, 770, tuple((11 * i) % 25 for i in range(64))),
 ])
 @pytest.mark.parametrize('wq_type,tiled,dtype', [('int4', {1: 128}, O.BF16), ('int8', {1: 128}, O.BF16), ('int8', None, O.F32),
                                                  ('float8_e4m3fn', {1: 128}, O.BF16), ('int4', None, O.F32)])
@@ -233,6 +235,22 @@ def _grouped_reference(x, wq, sizes):
       want[start:stop] = x[start:stop].to(torch.float64) @ w[g]
     start = stop
   return want
+
+
+@pytest.mark.parametrize('G,N,M', [(64, 520, 1400), (16, 4232, 960)])
+def test_ragged_dot_weight_only_second_row_tile_over_a_long_contraction(G, N, M):
+  """int4 weights take two row tiles only where K is long: four wavefronts, and two where there are thousands of workgroups (tolerance:
+  f32 sums of a few thousand products)."""
+  import qwix_amd
+  gen = torch.Generator().manual_seed(G)
+  sizes = torch.bincount(torch.multinomial(torch.rand(G, generator=gen) + 0.2, M, replacement=True, generator=gen), minlength=G).tolist()
+  print('case long contraction', G, N, M, flush=True)
+  _, x = util.make((M, 2048), O.BF16, seed=95)
+  g = torch.Generator(device=util.DEV).manual_seed(N)
+  wq = qwix_amd.quantize(torch.randn(G, 2048, N, generator=g, device=util.DEV).to(torch.bfloat16), 'int4', channelwise_axes=[0, 2], tiled_axes={1: 128})
+  out = qwix_amd.core.ragged_dot._weight_only_groups(x, wq, _sizes(sizes), torch.float32)
+  want = _grouped_reference(x, wq, sizes)
+  assert float((out.to(torch.float64) - want).abs().max()) <= 1e-5 * float(want.abs().max())
 
 
 @pytest.mark.parametrize('G,N,M,sizes', [
