@@ -991,16 +991,18 @@ def _equal_ranges(n: int, k: int, group: int) -> bool:
 
 
 def fused_wq_min_rows(n: int, int4: bool = True, k: int = 0, group: int = 0) -> int:
-  """Rows above which the dequantizing tile GEMM beats the decode kernel (`qwix_hip_gemv_wq`).  The time of one row
-  tile does not depend on the rows (K 4096, up to 128 rows, tiles of 128 x 64: int4 29 / 26 us at N 14336 / 4096, int8
-  29 / 25 us; 129-256 rows, tiles of 256 x 64: 45 us); the decode kernel's grows with them in steps of 16 rows and
-  falls with N (K 4096, int4, 64 / 80 / 96 / 128 rows: N 14336 26 / 35 / 38 / 48 us, N 4096 21 / 23 / 28 / 35 us; int8,
-  32 / 48 / 64 / 80 rows: N 14336 23 / 31 / 35 / 46 us, N 4096 12 / 17 / 21 / 26 us).
-  Where the tile GEMM cuts K into ranges (given `k` and `group`: few tiles, `qwix_hip_gemm_bf16_wq_ws`) it wins earlier.
-  Weights from HBM, decode kernel at 32 / 48 / 64 rows against the tile GEMM's one time up to 128 rows: int4 K 4096,
-  N 4096 12 / 15 / 21 against 15 us; K 8192, N 8192 23 / 29 / 40 against 33; K 14336, N 4096 34 / 45 / 64 against 31;
-  int8 13 / 17 / 21 against 15; 25 / 40 / 48 against 34; 35 / 55 / 67 against 32.  Only where the ranges can be equal: for the
-  others, which end in a shorter range, more rows keep their weights unrounded (`streamed_rows`)."""
+  """Rows above which the dequantizing tile GEMM runs in place of the decode kernel (`qwix_hip_gemv_wq`).  The time of the tile GEMM
+  hardly depends on the rows up to 128, that of the decode kernel grows with them in steps.  us, weights from HBM, groups of 128, the
+  decode kernel at 32 / 48 / 64 / 80 / 96 rows against the tile GEMM at 64: K 4096, N 14336 int4 16.6 / 20.6 / 27.1 / 34.8 / 38.8
+  against 27.9, int8 21.1 / 31.5 / 35.2 / 45.9 / 49.1 against 29.5; K 8192, N 28672 int4 50.6 / 77.0 / 93.7 / 112 / 131 against
+  108, int8 66 / 111 / 124 / 163 / 184 against 106.
+  Where the tile GEMM cuts K into ranges (given `k` and `group`: few tiles, `qwix_hip_gemm_bf16_wq_ws`) it runs earlier: K 8192, N 8192
+  int4 23.9 / 25.5 / 27.1 / 35.2 / 47.4 against 32.9, int8 28.0 / 33.5 / 34.5 / 54.7 / 62.1 against 34.8; K 14336, N 4096 int4 35.0 /
+  35.6 / 36.6 / 40.5 / 41.6 against 29.9, int8 34.3 / 40.4 / 41.2 / 54.4 / 55.3 against 31.6.  Only where the ranges can be equal: for the
+  others, which end in a shorter range, more rows keep their weights unrounded (`streamed_rows`).
+  The lines were drawn for a slower decode kernel and have stayed: for K up to 4096 and few columns today's is ahead beyond them (K 4096, N
+  4096 int4 11.8 / 12.2 / 12.5 / 14.6 / 14.7 against 14.9, at 128 rows 15.0 against 17.0; int8 12.6 / 14.6 / 14.7 / 19.1 / 19.5
+  against 15.5).  Moving them changes which calls round their weights to bf16, to fewer."""
   if k and group and _equal_ranges(n, k, group):
     return 48 if int4 else 32
   if int4:

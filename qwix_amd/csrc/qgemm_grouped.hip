@@ -965,13 +965,13 @@ int launch_grouped_dma(const GroupedArgs& p, hipStream_t st) {
   return check_launch("qgemm_grouped (dma)");
 }
 
-// Decode batches (at most 32 rows) of the sub-channel GEMM with groups of 128 and one scale per token: the NWV
+// Decode batches of the sub-channel GEMM with groups of 128, and more rows where tiles of 128 x 64 are few (takes_decode): the NWV
 // wavefronts of a workgroup share one 32 x 32 output tile and split K by groups (wavefront w takes groups w, w + NWV,
 // ...).  Each wavefront streams its own slabs through a private three-stage ring in LDS (direct-to-LDS loads, its own
 // vmcnt waits, no barrier in the loop), multiplies a group with four MFMAs, folds it into f32 sums with the group's
 // weight scale (parked in LDS at the start), and the partial sums meet in LDS once, at the end.  Against the
-// tile kernels that is two slabs in flight per wavefront and N / 32 workgroups of independent wavefronts where
-// a decode batch left the tile kernel one 16-MFMA chain per slab: the arithmetic per output element is the same
+// tile kernels that is two slabs in flight per wavefront and a workgroup of independent wavefronts per 32 columns (and 32 rows)
+// where a decode batch left the tile kernel one 16-MFMA chain per slab: the arithmetic per output element is the same
 // (exact int32 partial per group, f32 fold, per-token scale and rounding at the end), the groups are added in another
 // order.  SAG: activation scales per row and group as well, parked beside the weights' and multiplied into the partial
 // first, as the tile kernel does.
@@ -1277,8 +1277,9 @@ inline double decode_us(int64_t M, int64_t N, int64_t K, int b_qtype, bool sag) 
 // 17.1, 32.1 -> 29.4, 22.2 -> 20.7, 12.2 -> 10.6); int8 N 18176 over K 8192 (149 MB) 49.3 against 50.5.
 // More rows, where the narrow tiles are few: a workgroup's wavefronts then share K where a tile walks it alone, or in ranges with a second
 // launch.  Weights from HBM, the best of these -> this, us: int4 71 x 2048 over K 3584 16.1 -> 8.2, 71 x 1088 over K 4352 17.6 -> 7.9;
-// int8 84 x 2304 over K 6912 14.3 -> 10.9; scales on both sides, int8 318 x 1280 over K 3328 16.6 -> 15.1, e4m3 178 x 1312 over K 2560
-// 14.1 -> 7.9; int8 238 x 4008 over K 2048 13.7 against 20.2.  f32 weight scales keep the tiles' order of the groups, in which the run that
+// int8 84 x 2304 over K 6912 14.3 -> 10.9; scales on both sides, e4m3 178 x 1312 over K 2560
+// 14.1 -> 7.9; int8 238 x 4008 over K 2048 13.7 against 20.2.  Where the estimates are close the tiles keep the call (scales on both sides, int8
+// 318 x 1280 over K 3328 16.6 against 15.1).  f32 weight scales keep the tiles' order of the groups, in which the run that
 // dumps its partials gives equal bits.
 inline bool rows_share_k(int64_t M, int64_t N, int64_t K, int64_t group, int b_qtype, bool sag, int sb_dtype) {
   if (M <= 32 || sb_dtype != QWIX_BF16 || group != Fast::kBK || K / Fast::kBK < 4 || K > 16384 || (sag && b_qtype == QWIX_INT4) ||

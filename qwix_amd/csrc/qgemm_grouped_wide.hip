@@ -3,9 +3,9 @@
 //
 //   out[m,n] = cast( sum_g (acc_g[m,n] * sa[m,g]) * sb[g,n] ),  acc_g = sum_{k in g} a[m,k] b[n,k]
 //
-// Bound by what goes on beside the MFMAs: a fold of every accumulator per group (one FMA; with OUTER convert and FMA), 160 KB of LDS
-// fragment reads and 64 KB of direct-to-LDS loads per 256 x 256 x 128 slab, all issued by the same eight wavefronts.  Against the 128 x 256
-// tile of qgemm_grouped.hip (wavefronts of 128 x 32):
+// Bound by what goes on beside the MFMAs: a fold of every accumulator per group (one FMA; with OUTER convert and FMA), 192 KB of LDS
+// fragment reads and 64 KB of direct-to-LDS loads per 256 x 256 x 128 slab (int4 weights: 160 and 48 KB), all issued by the same eight
+// wavefronts.  Against the 128 x 256 tile of qgemm_grouped.hip (wavefronts of 128 x 32):
 //   * wavefronts of 32 TM x 64: 1.5 instead of 2.5 KB of fragments per two MFMAs, half the loads per product at TM 4;
 //   * a slab's fragments of a row tile are all in registers; its two column tiles' MFMAs alternate and are folded behind them, so only
 //     two of the tiles' partials exist at a time and 128 sums fit a lane;
@@ -36,8 +36,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ auto buffer_bytes(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
 }
-
-constexpr size_t kLdsMax = 160 * 1024;
 
 __device__ __forceinline__ float load_scale(const void* p, int dtype, int64_t i) {
   return dtype == QWIX_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p)[i]) : reinterpret_cast<const float*>(p)[i];

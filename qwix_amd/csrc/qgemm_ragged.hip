@@ -35,8 +35,9 @@ __global__ void __launch_bounds__(512)
     return;
   }
   const Epilogue e = group_epilogue(ep, rg, g);
-  // The last tile of a group is no higher than its rows need: 64, 128 or 192 rows cost 0.4, 0.6 and 0.8 of 256.  8192 rows in 8 groups, N 14336
-  // over K 4096, int8 507 -> 470 us; 2843 in 32, N 1984 over K 1792 37.6 -> 29.2; 2097 in 8, N 13248 over K 1536 85.7 -> 72.1.
+  // The last tile of a group is no higher than its rows need: 64, 128 or 192 rows cost 0.4, 0.6 and 0.8 of 256.  2843 rows in 32 groups, N 1984
+  // over K 1792, int8 37.6 -> 29.2 us; 2097 in 8, N 13248 over K 1536 85.7 -> 72.1; where groups are many tiles high little is left to gain (8192
+  // in 8, N 14336 over K 4096, four draws of the sizes, int8 484 to 496 -> 471 to 491).
   const uint8_t* bg = B + g * rg.b_group_stride;
   const int rows = m_lim - m0;
   if (rows <= 64) qgemm_pp_tile<QT, OUT, EPI, 1>(A, lda, bg, ldb, m0, n0, m_lim, N, K, e, out, ldo);
