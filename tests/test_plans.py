@@ -169,11 +169,13 @@ def test_recorder_refuses_sums_kept_per_weight(stand_in):
   assert not rec.ok and len(rec.calls) == 1 and recorded[0] is not None
 
 
-@pytest.mark.parametrize('act,weight,both,dtype,split', [
-    ('int8', 'int8', True, torch.bfloat16, True), ('int8', 'int8', True, torch.float32, False), ('int8', 'int4', True, torch.bfloat16, False),
-    ('int8', 'int4', False, torch.float32, True), ('float8_e4m3fn', 'float8_e4m3fn', True, torch.bfloat16, True),
-    ('float8_e4m3fn', 'float8_e4m3fn', True, torch.float32, False)])
-def test_sub_channel_calls_that_are_not_split_get_no_workspace(stand_in, monkeypatch, act, weight, both, dtype, split):
+@pytest.mark.parametrize('M,K,N,act,weight,both,dtype,split', [
+    (318, 3328, 1280, 'int8', 'int8', True, torch.bfloat16, True), (318, 3328, 1280, 'float8_e4m3fn', 'float8_e4m3fn', True, torch.bfloat16, True),
+    (100, 4096, 264, 'int8', 'int8', True, torch.bfloat16, False),  # (few tiles: the wavefronts share K)
+    (100, 4096, 264, 'int8', 'int8', True, torch.float32, False), (100, 4096, 264, 'int8', 'int4', True, torch.bfloat16, False),
+    (100, 4096, 264, 'int8', 'int4', False, torch.float32, True), (100, 4096, 264, 'float8_e4m3fn', 'float8_e4m3fn', True, torch.bfloat16, False),
+    (100, 4096, 264, 'float8_e4m3fn', 'float8_e4m3fn', True, torch.float32, False)])
+def test_sub_channel_calls_that_are_not_split_get_no_workspace(stand_in, monkeypatch, M, K, N, act, weight, both, dtype, split):
   from qwix_amd.core import dot_general as dg
   from qwix_amd.core.qarray import Int4Tensor, QArray
   real = ctypes.CDLL(_lib.LIB_PATH)
@@ -186,7 +188,6 @@ def test_sub_channel_calls_that_are_not_split_get_no_workspace(stand_in, monkeyp
       fn.restype, fn.argtypes = _lib.SIGNATURES[name]
       return fn
   monkeypatch.setattr(_lib, 'load', Sizes)
-  M, K, N = 100, 4096, 264
   values = lambda t, *shape: torch.zeros(*shape, dtype=torch.int8 if t == 'int8' else torch.float8_e4m3fn)
   wv = Int4Tensor(torch.zeros(N, K // 2, dtype=torch.uint8).t(), (K, N), 0) if weight == 'int4' else values(weight, N, K).t()
   x = QArray(values(act, M, K), torch.ones(M, K // 128 if both else 1, dtype=dtype), None, act)
