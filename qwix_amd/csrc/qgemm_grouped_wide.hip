@@ -12,7 +12,7 @@
 //   * one barrier per slab, in the middle: by then every wavefront has read all of the slab's b and the slab before it is done with, so
 //     three stages of a and two of b hold a slab in use, one that has landed and one on its way, and the first fragments of the next
 //     slab are requested under the last row tile of this one.
-// Arithmetic, order and results are those of the 128 x 256 tile, bit for bit.  Measured on one box, that tile -> this one, us:
+// Arithmetic, order and results are those of the 128 x 256 tile, bit for bit.  Measured on one card, that tile -> this one, us:
 // 4096^3, one scale per row, int8 90 -> 74, e4m3 79 -> 65; scales on both sides, int8 105 -> 88, e4m3 94 -> 78; 2048 x 8192 over K
 // 8192, int4 155 -> 134; 450 x 20480 over K 1536, int8 on both sides 43 -> 20 (TM 2); 1823 x 5056 over K 4096, int4 77 -> 50 (TM 3).
 // Of 88 us (int8, both sides) 15 are the loads' and 19 the fold's, found by leaving them out; without both it is the 60 us that the

@@ -34,7 +34,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // Swizzle key of the kernels in this file: 16-byte chunk c of the 128-byte LDS row r sits at chunk position
 // c ^ swz8(r).  Eight consecutive rows then cover all eight chunk positions; over the sixteen rows that the LDS
 // serves per clock for a ds_read_b128 this still leaves two-way bank conflicts, which the sixteen-row key of
-// common.h (swz128) removes.  Measured side by side on one box, the conflict-free key is nevertheless 2-5 %
+// common.h (swz128) removes.  Measured side by side on one card, the conflict-free key is nevertheless 2-5 %
 // SLOWER here (int8 4096^3: 72.1 against 70.3 us; 8192^3: 494 against 485 us; the 8-expert ragged GEMM 578
 // against 551 us; e4m3 and the one-tile-row kernel unchanged): these kernels run at the board's power limit,
 // where faster fragment reads buy nothing and cost clock.  So the eight-row key stays.
